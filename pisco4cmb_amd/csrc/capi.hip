@@ -124,6 +124,7 @@ int pisco::pair_params(int nside_sky, const float *I, const float *Q, const floa
     p.fc = fast_consts(p.hb);
     p.fc64 = fast_consts64(p.hb);
     p.beam = beam8;
+    p.strips = 1;
     p.ra = ra;
     p.dec = dec;
     p.pa = pa;
@@ -140,6 +141,19 @@ int pisco::forward_lanes_auto(const PairParams &p)
     const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
     const double dp = (double)p.hs.npix * s * s;   /* expected pixels per disc */
     return dp < 1000.0 ? 8 : dp < 3000.0 ? 16 : 64;
+}
+
+/* Strips by the beam's size: a strip of a large beam stays in an XCD's 4 MB
+ * L2, and each strip costs a table build per sample.  Forward at sky NSIDE 512,
+ * ms for 1, 2, 3, 4 strips: 2.9 MB 1.12, 0.89, 1.04; 4.2 MB 1.99, 1.18, 1.29;
+ * 5.7 MB 1.60, 1.11, 1.03; 7.5 MB 2.24, 1.64, 1.45, 1.42; 11.7 MB 4.05, 3.03,
+ * 2.69, 2.46, and 6 strips 0.98 of 4.  The sky adjoint pays each strip with a
+ * set of windows; 1, 2, 3 strips: 5.7 MB 1.38, 1.48, 1.65; 11.7 MB 2.81, 2.56,
+ * 2.96 (3.6e5 samples: 20.5, 14.0, 16.1). */
+int pisco::strips_auto(const PairParams &p, bool adjoint)
+{
+    const double mb = 32.0 * p.npix_beam / (1 << 20);
+    return (int)std::min<double>(kMaxStrips, std::ceil(mb / (adjoint ? 8.0 : 2.2)));
 }
 
 struct pisco_ctx {
@@ -191,6 +205,7 @@ struct pisco_ctx {
     DevBuf<unsigned> fxwork;      /* deterministic mode: max row sum, max |g| */
     DevBuf<double> fxscale;       /* deterministic mode: the scale (device) */
     DevBuf<int> support;          /* last non-zero beam row (device) */
+    DevBuf<char> strip;           /* strip_workspace */
     DevBuf<float> sky4;           /* the forward's packed sky: I, Q, U, 0 per pixel */
     DevBuf<float4> recs;          /* beam adjoint: visit records (16 bytes each) */
     DevBuf<long> recidx;          /* beam adjoint: record offsets per sample and band */
@@ -201,7 +216,7 @@ struct pisco_ctx {
     template <typename F> void each_buf(F f)
     {
         f(I); f(Q); f(U); f(V); f(beam); f(ra); f(dec); f(pa); f(tod); f(cot); f(acc); f(fout);
-        f(fxwork); f(fxscale); f(support); f(sky4); f(recs); f(recidx);
+        f(fxwork); f(fxscale); f(support); f(strip); f(sky4); f(recs); f(recidx);
         f(recvmax); f(recpart);
     }
 };
@@ -295,6 +310,23 @@ int adj_lanes(const pisco_ctx *c, const PairParams &p)
     return disc_pixels(p) < 1000.0 ? 8 : 64;
 }
 
+/* Strips for a launch of one wave per sample, whose launches then take at most
+ * kStripLaunch samples.  A frozen context without the workspace takes whole
+ * discs. */
+int use_strips(pisco_ctx *c, PairParams &p, long &chunk, bool adjoint)
+{
+    p.strips = strips_auto(p, adjoint);
+    const size_t bytes = strip_bytes(p.strips);
+    if (p.strips == 1 || (bytes > c->strip.cap && c->strip.frozen)) {
+        p.strips = 1;
+        return PISCO_OK;
+    }
+    CHK(c->strip.ensure(bytes));
+    strip_workspace(p, c->strip.p);
+    chunk = std::min(chunk, kStripLaunch);
+    return PISCO_OK;
+}
+
 /* Launches op over samples p.s_begin .. p.s_end in chunks of ptgPerConv (or
  * one launch). */
 int run_pair(pisco_ctx *c, int op, PairParams p, hipStream_t st, bool sky_packed = false,
@@ -320,6 +352,8 @@ int run_pair(pisco_ctx *c, int op, PairParams p, hipStream_t st, bool sky_packed
     long chunk = (c->cfg.ptgPerConv > 0) ? c->cfg.ptgPerConv : n - s0;
     if (chunk < (1L << 20))
         chunk = std::max<long>(chunk, std::min<long>(n - s0, 1L << 20));
+    if (fwd && !c->beam_interp && lanes == 64)
+        CHK(use_strips(c, p, chunk, false));
     for (long s = s0; s < n; s += chunk) {
         p.s_begin = s;
         p.s_end = std::min(n, s + chunk);
@@ -327,6 +361,8 @@ int run_pair(pisco_ctx *c, int op, PairParams p, hipStream_t st, bool sky_packed
             HIPCHK(launch_pair_interp(op, p, st));
         else if (lanes < 64)
             HIPCHK(launch_fwd_sub(lanes, p, st, op == OP_FWD_V));
+        else if (fwd)
+            HIPCHK(launch_forward(p, st, op == OP_FWD_V));
         else
             HIPCHK(launch_pair(op, p, st));
     }
@@ -348,34 +384,37 @@ int det_scale(pisco_ctx *c, const float *const *beams, const long *npix, int nbe
     return PISCO_OK;
 }
 
-/* Samples per LDS window of a single-pair sky adjoint over discs of radius
- * rho with `lanes` lanes per sample: the tuning value, or (auto) the largest
- * power of two in [16, 512] that keeps a window at about 96,000 expected
- * visits, and at least one sample per lane group of every wave of the block
- * (16 x 64 / lanes).  Each window costs three block-wide passes besides its
- * visits; at 6,000 pixels per disc 16 samples per window measured fastest,
- * at 135 pixels 256 samples took 0.64x the time of 16 (one sample per wave)
- * and, with 8 lanes per sample, 0.97x the time of 128; at 540 pixels with 8
- * lanes, 32 samples took 2.0x the time of 128. */
-int adj_chunk(const pisco_ctx *c, int nside_sky, double rho, int lanes)
+/* Samples per LDS window of a single-pair sky adjoint with `lanes` lanes per
+ * sample: the tuning value, or (auto) the largest power of two in [16, 512]
+ * that keeps a window at about 96,000 expected visits, and at least two
+ * samples per lane group of the block's 8 waves (16 x 64 / lanes).  Each window
+ * costs three block-wide passes besides its visits: 540 pixels per disc, 8
+ * lanes: 32, 64, 128 samples 0.99, 0.65, 0.57 ms.  With strips 8 samples: the
+ * samples in flight are fewer and the strip of the beam that they meet is
+ * smaller (16: 15.9 ms, 8: 14.0 ms at 6,000 pixels per disc). */
+int adj_chunk(const pisco_ctx *c, const PairParams &p, int lanes)
 {
     if (c->adjmap_chunk > 0)
         return c->adjmap_chunk;
-    const double s = pl_sin(0.5 * std::min(rho, kPi));
-    const double disc = 12.0 * nside_sky * nside_sky * s * s;   /* npix (1 - cos rho) / 2 */
+    if (lanes == 64 && strips_auto(p, true) > 1)
+        return kAdjWaves;
     int chunk = 16;
-    while (chunk < 512 && 2.0 * chunk * disc <= 96000.0)
+    while (chunk < 512 && 2.0 * chunk * disc_pixels(p) <= 96000.0)
         chunk *= 2;
-    const int fill = 16 * (64 / std::max(lanes, 1));   /* lane groups of a 16-wave block */
-    return std::max(chunk, std::min(fill, 512));
+    return std::max(chunk, std::min(16 * (64 / std::max(lanes, 1)), 512));
 }
 
 /* The window capacity that fits the LDS next to the per-wave tables. */
-int fit_cap(int cap, int rw, int group, bool det)
+int fit_cap(int cap, int rw, int group, bool det, int lanes)
 {
-    while (cap > 256 && adjmap_lds_bytes(cap, rw, group, det) > 163840)
-        cap -= 256;
-    return cap;
+    auto fit = [&](size_t bytes) {
+        int k = cap;
+        while (k > 256 && adjmap_lds_bytes(k, rw, group, det, lanes) > bytes)
+            k -= 256;
+        return k;
+    };
+    const int two = fit(81920);   /* two blocks per CU */
+    return two >= 1024 || two == cap ? two : fit(163840);
 }
 
 /* The batched launches compute the nearest-pixel convolution only. */
@@ -384,6 +423,29 @@ int no_interp(pisco_ctx *c)
     if (c->beam_interp)
         return fail(PISCO_ERR_INVALID,
                     "beam interpolation is available for single-pair launches only");
+    return PISCO_OK;
+}
+
+/* The LDS-window sky adjoint of one pair over samples p.s_begin .. p.s_end. */
+int run_adjmap(pisco_ctx *c, PairParams p, int chunk, int cap, const double *scale, int lanes,
+               hipStream_t st)
+{
+    const long n = p.s_end;
+    long step = n - p.s_begin;
+    if (lanes == 64)
+        CHK(use_strips(c, p, step, true));
+    for (long s = p.s_begin; s < n; s += step) {
+        p.s_begin = s;
+        p.s_end = std::min(n, s + step);
+        hipError_t e = launch_adjmap_lds(p, chunk, cap, c->adjmap_rw, c->adjmap_blocks, st, nullptr,
+                                         0.0, 1, scale, lanes);
+        if (e != hipSuccess) {
+            char d[256];
+            adjmap_describe(d, sizeof d, cap, c->adjmap_rw);
+            return fail(PISCO_ERR_DEVICE, "sky adjoint launch failed: %s (%s)",
+                        hipGetErrorString(e), d);
+        }
+    }
     return PISCO_OK;
 }
 
@@ -489,7 +551,7 @@ int pisco_set_tuning(pisco_ctx *c, const char *key, long value)
     } else if (k == "adjmap_cap" || k == "adjmap_rw") {
         int cap = k == "adjmap_cap" ? (int)value : c->adjmap_cap;
         int rw = k == "adjmap_rw" ? (int)value : c->adjmap_rw;
-        if (value < 1 || adjmap_lds_bytes(cap, rw, 0, false) > 163840)
+        if (value < 1 || kAdjTableBytes + 276 + 12 * ((size_t)cap + rw) > 163840)
             return fail(PISCO_ERR_INVALID, "LDS window does not fit 160 KiB");
         c->adjmap_cap = cap;
         c->adjmap_rw = rw;
@@ -1110,22 +1172,15 @@ int pisco_dev_adjoint_map(pisco_ctx *c, void *stream, int nside_sky, int nside_b
     }
     if (g_a || g_b) {
         if ((c->adjmap_chunk != 0 || det) && !c->beam_interp) {
-            const int nb = c->adjmap_blocks;   /* 0: one block per window */
-            const int chunk = adj_chunk(c, nside_sky, p.rho_max, adj_lanes(c, p));
-            const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, 0, det);
+            const int lanes = adj_lanes(c, p);
+            const int chunk = adj_chunk(c, p, lanes);
+            const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, 0, det, lanes);
             if (c->adjmap_support) {
                 CHK(c->support.ensure(1));
                 HIPCHK(launch_beam_support(beam8, npix_beam, c->support.p, st));
                 p.beam_last = c->support.p;
             }
-            hipError_t e = launch_adjmap_lds(p, chunk, cap, c->adjmap_rw, nb, st, nullptr, 0.0, 1,
-                                             scale, adj_lanes(c, p));
-            if (e != hipSuccess) {
-                char d[256];
-                adjmap_describe(d, sizeof d, cap, c->adjmap_rw);
-                return fail(PISCO_ERR_DEVICE, "sky adjoint launch failed: %s (%s)",
-                            hipGetErrorString(e), d);
-            }
+            CHK(run_adjmap(c, p, chunk, cap, scale, lanes, st));
         } else {
             CHK(run_pair(c, OP_ADJ_MAP, p, st));
         }
@@ -1319,9 +1374,7 @@ int pisco_batch_create(pisco_ctx *c, int npairs, const pisco_batch_pair *pairs,
         b.beam = q.beam8;
         b.npix = (int)q.npix_beam;
         b.nside = q.nside_beam;
-        FastConsts fc = fast_consts(hpx_make(q.nside_beam));
-        b.nside_f = fc.nside;
-        b.marg_k = fc.marg_k;
+        b.nside_f = (float)q.nside_beam;
         b.rho_max = pisco_beam_rho_max(q.nside_beam, q.npix_beam);
         b.cos_rmax = cos_radius(b.rho_max);
         const double sh = pl_sin(0.5 * b.rho_max);
@@ -1415,7 +1468,6 @@ int setup_batch(pisco_ctx *c, const pisco_batch *b, int nside_sky, const float *
     p.pairs = b->table;
     p.npairs = b->npad;
     p.ngroups = b->npad;
-    p.fc = fast_consts(hpx_make(1));     /* only the rho > 1e-6 band is read */
     p.fc64 = fast_consts64(hpx_make(1)); /* only the crho thresholds are read */
     p.ra = ra;
     p.dec = dec;
@@ -1530,8 +1582,6 @@ int batch_adjoint_pairwise(pisco_ctx *c, hipStream_t st, const pisco_batch *b, i
                            long ptg_stride, const float *g, const double *scale)
 {
     const long npix = 12L * nside_sky * nside_sky;
-    const int nb = c->adjmap_blocks;   /* 0: one block per window */
-    const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, 0, scale != nullptr);
     CHK(c->cot.ensure(std::max<long>(nsamples, 1)));
     CHK(c->support.ensure(1));
     for (const BatchPair &q : b->host) {
@@ -1552,11 +1602,8 @@ int batch_adjoint_pairwise(pisco_ctx *c, hipStream_t st, const pisco_batch *b, i
             p.beam_last = c->support.p;
         }
         const int lanes = adj_lanes(c, p);
-        hipError_t e = launch_adjmap_lds(p, adj_chunk(c, nside_sky, p.rho_max, lanes), cap,
-                                         c->adjmap_rw, nb, st, nullptr, 0.0, 1, scale, lanes);
-        if (e != hipSuccess)
-            return fail(PISCO_ERR_DEVICE, "per-pair sky adjoint launch failed: %s",
-                        hipGetErrorString(e));
+        const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, 0, scale != nullptr, lanes);
+        CHK(run_adjmap(c, p, adj_chunk(c, p, lanes), cap, scale, lanes, st));
     }
     return PISCO_OK;
 }
@@ -1716,7 +1763,7 @@ int pisco_dev_batched_adjoint_map(pisco_ctx *c, void *stream, const pisco_batch 
     const bool det = det_single(c);
     const int grp = c->batch_adj_group;
     /* the window capacity that fits next to the group's per-wave tables */
-    const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, grp, det);
+    const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, grp, det, 64);
     const double *scale = nullptr;
     if (det)
         CHK(batch_det_scale(c, st, b, nsamples, g, &scale));

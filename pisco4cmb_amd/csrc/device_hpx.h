@@ -618,61 +618,234 @@ __host__ __device__ inline int beam_pixel(const Hpx &hb, const Centre &c, double
  *
  * The kernels evaluate the visit geometry in float32 and keep the beam pixel
  * it gives only where no floor of ang2pix can flip; any other visit is
- * re-evaluated by the exact FP64 path (beam_pixel).  Either way the pixel is
- * the one the CPU path computes.
+ * re-evaluated by the FP64 form below (beam_pixel_f64).  Either way the pixel
+ * is the one the CPU path computes.
  *
- * Geometry in haversine form (no cancellation).  With dD = dec_p - dec_c and
- * h2 = 1 - cos(dra) = 2 sin^2(dra/2):
- *   1 - cos rho = (1 - cos dD) + cos dec_c cos dec_p h2,
- *   1 - cos dD  = sin^2 dD / (1 + cos dD),
- *   ya = sin dra cos dec_p,  xa =  sin dD + cos dec_p sin dec_c h2,
- *   yb = sin dra cos dec_c,  xb = -sin dD + cos dec_c sin dec_p h2,
- * alpha = atan2(ya, xa), beta = atan2(yb, xb) (sphtrigo.cpp:41-42).  sin dD
- * and cos dD come from FP64 products of the ring's and the sample's sin/cos
- * dec; everything after that is float.  In the polar branch of ang2pix
- * (cos rho > 2/3) the floors are jp = (int)(tp*tmp), jm = (int)((1-tp)*tmp)
- * and ip = (int)(tt*(jp+jm+1)), with tt = (2 - 2 alpha/pi - 2 psi/pi) mod 4,
- * tp = frac(tt), tmp = nside*sqrt(3 (1 - cos rho)).
+ * What depends only on the ring and the sample is evaluated once per ring, in
+ * FP64, when the walk's run table is built (run_geo), and rounded to float.
+ * With dD = dec_p - dec_c, x = dra/2:
+ *   1 - cos rho = (1 - cos dD) + 2 cos dec_c cos dec_p sin^2 x,
+ *   ya = 2 sin x cos x cos dec_p,  xa = sin dD + 2 cos dec_p sin dec_c sin^2 x,
+ * alpha = atan2(ya, xa) (sphtrigo.cpp:42).  x is linear in the pixel's
+ * position in the ring: x = k b + a0 with k the (integer) distance from the
+ * ring position nearest to the centre's right ascension, so that its relative
+ * error stays at float rounding right up to the centre.
  *
- * Error of the float values against the CPU path's (float32 emulation over
- * 4e6 random visits, discs of 5 degrees, a quarter of them near the poles):
- *   tt   <= 6.0e-7 absolute              bound used: 4e-6
- *   tmp  <= 2.6e-7 relative              bound used: 2e-6
- * plus the CPU path's own rounding of acos(crho) (|crho error| <= 7e-16), which
- * moves its tmp by <= 1.05e-15 nside / sqrt(3 (1 - cos rho)); bound used: 100
- * times that (marg_k).  A floor is kept only if its argument is farther from
- * an integer than these bounds.  rho > 1e-6 (sphtrigo.cpp:40) is decided in
- * float outside 0.5e-6 < rho < 1.5e-6 and by the exact path inside.
+ * In the polar branch of ang2pix (cos rho > 2/3) the floors are jp =
+ * (int)(tp*tmp), jm = (int)((1-tp)*tmp) and ip = (int)(tt*(jp+jm+1)), with
+ * tt = (2/pi) sigma mod 4, tp = frac(tt), tmp = nside*sqrt(3 (1 - cos rho)).
+ * sigma = pi - (alpha + psi): the vector (xa, ya) is turned by psi and its
+ * octant gives tt without a range reduction.
  *
- * chi is needed as float cos(2 chi), sin(2 chi): with chi = beta + alpha + psi
- * - pi (mod 2 pi), e^{2 i chi} = w^2/|w|^2 e^{2 i psi}, w = (xb + i yb)(xa +
- * i ya), evaluated in float (error <= 9.2e-7 measured). */
+ * Errors against FP64, from a float32 emulation over 2e6 visits for each of 21
+ * combinations of sky NSIDE 64-2048, beam NSIDE 512-8192, caps 0.3-34 deg and
+ * centres anywhere, near and at the poles, with the hardware's reciprocal and
+ * square root within 1 ulp:
+ *   tt <= 4.9e-7, tmp <= 4e-7 relative; no floor flipped that lay farther
+ *   than 3.3e-7 tmp from an integer.
+ * Bound used: kFloorMargin tmp + 2e-6 (for the batched kernels, which take
+ * alpha before the turn by psi and reduce tt mod 4, kFloorMarginBatch).  The
+ * CPU path's own rounding of acos(crho) (|crho error| <= 7e-16) moves tmp by
+ * under 1e-7 of that bound for rho > 1e-4; closer visits (and those beyond the
+ * polar branch) take the FP64 form, so the rho > 1e-6 rule of sphtrigo.cpp:40
+ * never meets the float form. */
 struct FastConsts {
-    float omc_lo;   /* 1 - cos(0.5e-6): below, rho <= 1e-6 for sure */
-    float omc_hi;   /* 1 - cos(1.5e-6): above, rho >  1e-6 for sure */
-    float marg_k;   /* 1.2e-13 * nside_beam */
     float nside;    /* nside_beam */
+    float k3;       /* 3 nside_beam^2 */
 };
+
+constexpr float kOmcLo = 5e-9f;           /* 1 - cos(1e-4) */
+constexpr float kOmcHi = 0.33332f;        /* polar branch: cos rho > 2/3 */
+constexpr float kFloorMargin = 2.5e-6f;
+constexpr float kFloorMarginBatch = 4e-6f;
+constexpr int kNeedExact = -2;            /* the floors are not certain */
 
 /* Wave-uniform float constants of one sample. */
 struct SampleF {
-    float cdc, sdc;   /* cos, sin dec of the beam centre */
-    float t0;         /* (pi - psi) * 2/pi mod 4 */
-    float c2p, s2p;   /* cos, sin 2 psi */
+    float cdc, sdc;             /* cos, sin dec of the beam centre */
+    float cps, sps;             /* cos, sin psi */
+    float c2h, c2l, s2h, s2l;   /* cos, sin 2 psi as float pairs */
+    float lim0;                 /* 1/2 - 2e-6, or -1: certify no visit */
 };
 
-__host__ __device__ inline SampleF sample_f32(const Centre &c, double c2psi, double s2psi)
+/* Whether the float form's geometry holds for a beam centre: a declination
+ * within [-pi/2, pi/2] (beyond it query_disc's centre is the reflected point)
+ * and a right ascension small enough that its FP64 reduction is exact to
+ * 1e-11.  Otherwise (NaN included) every visit takes the FP64 form. */
+__host__ __device__ inline bool centre_regular(double ra, double dec)
+{
+    return fabs(ra) < 1e4 && fabs(dec) <= kHalfPi;
+}
+
+__host__ __device__ inline SampleF sample_f32(const Centre &c, double cpsi, double spsi,
+                                              double c2psi, double s2psi)
 {
     SampleF f;
     f.cdc = (float)c.cdc;
     f.sdc = (float)c.sdc;
-    f.t0 = (float)fmodulo((kPi - c.psi) * kInvHalfPi, 4.0);
-    f.c2p = (float)c2psi;
-    f.s2p = (float)s2psi;
+    f.cps = (float)cpsi;
+    f.sps = (float)spsi;
+    f.c2h = (float)c2psi;
+    f.c2l = (float)(c2psi - (double)f.c2h);
+    f.s2h = (float)s2psi;
+    f.s2l = (float)(s2psi - (double)f.s2h);
+    f.lim0 = centre_regular(c.ra, c.dec) ? 0.5f - 2e-6f : -1.0f;
     return f;
 }
 
-constexpr int kNeedExact = -2;   /* beam_pixel_f32: the floors are not certain */
+/* 1/n to ~1e-15 relative: hardware reciprocal estimate + one Newton step
+ * (used only where the value feeds float outputs, never an index). */
+__device__ inline double recip_fast(double n)
+{
+    double r = __builtin_amdgcn_rcp(n);
+    return fma(r, fma(-n, r, 1.0), r);
+}
+
+/* Float geometry of a run of consecutive pixels of one ring, positions j0 ..
+ * j0+len-1, around one sample: x = dra/2 of position j is (j - kc) b + a0. */
+struct RunGeo {
+    float a0, b;
+    int kc;
+    float sD, omD;    /* sin dD, 1 - cos dD */
+    float cdp2;       /* 2 cos dec_p */
+    float kap;        /* sin((dec_p + dec_c)/2) / cos(dD/2) */
+};
+
+__device__ inline RunGeo run_geo(const Hpx &h, const RingRec &rr, int r, const Centre &c, int j0,
+                                 int len)
+{
+    RunGeo g;
+    /* pixel spacing 2 pi / nr and the ring's half-pixel shift */
+    const bool cap = rr.rdiv > 0;
+    const double tpn = cap ? kHalfPi * rr.inv : (kPi * 0.75) * h.fact1;
+    const double nr = cap ? 4.0 * rr.rdiv : 4.0 * h.nside;
+    const double shift = (cap || ((r - h.nside) & 1) == 0) ? 0.5 : 0.0;
+    /* the centre's right ascension on the branch nearest the run's middle */
+    const double mid = ((double)j0 + 0.5 * (double)(len - 1) + shift) * tpn;
+    const double ra = c.ra + kTwoPi * rint((mid - c.ra) * kInvTwoPi);
+    const double kc = rint(ra * (nr * kInvTwoPi) - shift);
+    g.a0 = (float)(0.5 * ((kc + shift) * tpn - ra));
+    g.b = (float)(0.5 * tpn);
+    g.kc = (int)kc;
+    const double sD = fma(rr.sdp, c.cdc, -(rr.cdp * c.sdc));
+    const double rc = recip_fast(1.0 + fma(rr.cdp, c.cdc, rr.sdp * c.sdc));
+    g.sD = (float)sD;
+    g.omD = (float)(sD * sD * rc);
+    g.cdp2 = (float)(2.0 * rr.cdp);
+    g.kap = (float)((c.sdc + rr.sdp) * rc);
+    return g;
+}
+
+/* Position angle free part of a visit. */
+struct VisitGeo {
+    float s2, sc;     /* sin^2 x, sin x cos x */
+    float omc;        /* 1 - cos rho */
+    float xa, ya;
+};
+
+__device__ inline VisitGeo visit_geo(float x, float sD, float omD, float cdp2, float cdc,
+                                     float sdc)
+{
+    VisitGeo v;
+    float sh, ch;
+    plf_sincos(x, &sh, &ch);
+    v.s2 = sh * sh;
+    v.sc = sh * ch;
+    v.omc = fmaf(v.s2, cdp2 * cdc, omD);
+    v.xa = fmaf(v.s2, cdp2 * sdc, sD);
+    v.ya = v.sc * cdp2;
+    return v;
+}
+
+/* e^{2i(alpha + beta)} = (c4, -s4), from Napier's analogy: alpha + beta = pi -
+ * 2 eta (mod 2 pi) with tan eta = kap tan x, so no ill-conditioned direction
+ * at the centre enters.  Error of the result after the turn by 2 psi
+ * (visit_chi): 2.3e-6 |eta| + 6e-8 (float32 emulation). */
+__device__ inline void visit_phase(const VisitGeo &v, float kap, float &c4, float &s4)
+{
+    const float w = (kap * kap) * v.s2, p = 1.0f - v.s2;
+    const float inv = __builtin_amdgcn_rcpf(p + w);
+    const float c = (p - w) * inv, s = (kap * v.sc) * inv;   /* cos 2 eta, sin(2 eta) / 2 */
+    c4 = fmaf(-8.0f * s, s, 1.0f);
+    s4 = 4.0f * (s * c);
+}
+
+/* cos, sin 2 chi, chi = beta + alpha + psi - pi (sphtrigo.cpp:41-53). */
+__device__ inline void visit_chi(const SampleF &f, float c4, float s4, float &c2, float &s2)
+{
+    c2 = fmaf(c4, f.c2h, fmaf(s4, f.s2h, fmaf(c4, f.c2l, s4 * f.s2l)));
+    s2 = fmaf(c4, f.s2h, fmaf(-s4, f.c2h, fmaf(c4, f.s2l, -(s4 * f.c2l))));
+}
+
+/* atan(min(ax, ay) / max(ax, ay)) 2/pi, in [0, 1/2]; fit error 5.6e-8. */
+__device__ inline float quarter_turns(float ax, float ay)
+{
+    const float t = fminf(ax, ay) * __builtin_amdgcn_rcpf(fmaxf(ax, ay));
+    const float z = t * t;
+    float p = -0x1.8ee3fcp-9f;
+    p = fmaf(p, z, 0x1.00234cp-6f);
+    p = fmaf(p, z, -0x1.3869b6p-5f);
+    p = fmaf(p, z, 0x1.03442ep-4f);
+    p = fmaf(p, z, -0x1.6dd48ap-4f);
+    p = fmaf(p, z, 0x1.0462e0p-3f);
+    p = fmaf(p, z, -0x1.b2953cp-3f);
+    p = fmaf(p, z, 0x1.45f304p-1f);
+    return t * p;
+}
+
+/* Beam pixel from tt in [0, 4] and tmp; kNeedExact unless every floor's
+ * argument is farther than 1/2 - lim from an integer. */
+__device__ inline int cap_floors(float tt, float tmp, float omc, float lim)
+{
+    const float tp = __builtin_amdgcn_fractf(tt);
+    const float u1 = tp * tmp, u2 = tmp - u1;
+    const float d1 = __builtin_amdgcn_fractf(u1), d2 = __builtin_amdgcn_fractf(u2);
+    const float irf = ((u1 - d1) + (u2 - d2)) + 1.0f;
+    const float vv = tt * irf;
+    const float dv = __builtin_amdgcn_fractf(vv);
+    const int ir = (int)irf, ip = (int)(vv - dv);
+    const float e = fmaxf(fmaxf(fabsf(d1 - 0.5f), fabsf(d2 - 0.5f)), fabsf(dv - 0.5f));
+    const bool ok = e < lim && omc > kOmcLo && omc < kOmcHi;
+    return ok ? 2 * (int)__umul24((unsigned)ir, (unsigned)(ir - 1)) + ip : kNeedExact;
+}
+
+/* Beam pixel of a visit for the sample's position angle, or kNeedExact. */
+__device__ inline int visit_pixel(const FastConsts &fc, const SampleF &f, const VisitGeo &v)
+{
+    const float xr = fmaf(v.xa, f.cps, -(v.ya * f.sps)), yr = fmaf(v.xa, f.sps, v.ya * f.cps);
+    const float ax = fabsf(xr), ay = fabsf(yr);
+    const float a = quarter_turns(ax, ay);
+    /* sigma's vector is (-xr, yr): tt = 2 - copysign(1 + copysign(m, -xr), yr),
+     * m the quarter turns from the y axis */
+    const float m = ay > ax ? a : 1.0f - a;
+    const float tt = 2.0f - copysignf(1.0f - copysignf(m, xr), yr);
+    const float tmp = __builtin_amdgcn_sqrtf(fc.k3 * v.omc);
+    return cap_floors(tt, tmp, v.omc, fmaf(tmp, -kFloorMargin, f.lim0));
+}
+
+/* |eta| above which cos, sin 2 chi take the FP64 form (visit_chi64): the
+ * forward keeps them within 2.5e-7 of FP64 and the adjoints, whose gradients
+ * are float sums of many visits, within 1e-6. */
+constexpr float kEtaForward = 0.078f;
+constexpr float kEtaAdjoint = 0.38f;
+
+/* cos, sin 2 chi in FP64 (Napier's analogy as visit_phase), rounded to
+ * float. */
+__device__ inline void visit_chi64(const Centre &c, double c2psi, double s2psi, double ra_pix,
+                                   double cdp, double sdp, float &c2, float &s2)
+{
+    double dra = ra_pix - c.ra;
+    dra = fma(-kTwoPi, rint(dra * kInvTwoPi), dra);
+    double sh, ch;
+    pl_sincos(0.5 * dra, &sh, &ch);
+    const double kap = (c.sdc + sdp) * recip_fast(1.0 + fma(cdp, c.cdc, sdp * c.sdc));
+    const double q = kap * sh;
+    const double inv = recip_fast(fma(ch, ch, q * q));
+    const double ce = fma(ch, ch, -(q * q)) * inv, se = 2.0 * (ch * q) * inv;
+    const double c4 = fma(ce, ce, -(se * se)), s4 = 2.0 * (ce * se);
+    c2 = (float)fma(c4, c2psi, s4 * s2psi);
+    s2 = (float)fma(c4, s2psi, -(s4 * c2psi));
+}
 
 struct ExactVisit {
     int bp;
@@ -701,127 +874,11 @@ __device__ __noinline__ ExactVisit beam_visit_exact(int nside_beam, double ra_c,
     return e;
 }
 
-/* The part of a visit's float geometry that reads the sky pixel's ring
- * (FP64 in, float out); the rest (beam_pixel_f32_tail) is float only. */
-struct VisitRing {
-    float xh;         /* dra / 2, dra = ra_pix - ra_centre in [-pi, pi] */
-    float sD, opcD;   /* sin(dec_p - dec_c), 1 + cos(dec_p - dec_c) */
-    float cdp, sdp;   /* cos, sin dec_p */
-};
-
-__device__ inline VisitRing visit_ring_f32(const Centre &c, double ra_pix, double cdp, double sdp)
-{
-    double dra = ra_pix - c.ra;
-    dra = fma(-kTwoPi, rint(dra * kInvTwoPi), dra);
-    VisitRing g;
-    g.xh = (float)(0.5 * dra);
-    g.sD = (float)fma(sdp, c.cdc, -(cdp * c.sdc));
-    g.opcD = 1.0f + (float)fma(cdp, c.cdc, sdp * c.sdc);
-    g.cdp = (float)cdp;
-    g.sdp = (float)sdp;
-    return g;
-}
-
-/* The part of the float mapping that does not depend on the detector's
- * position angle: 1 - cos rho, alpha, and e^{2i(alpha+beta)} (er, ei). */
-struct VisitGeo {
-    float omc;        /* 1 - cos rho */
-    float x3y;        /* sqrt(3 (1 - cos rho)) */
-    float y;          /* 1/sqrt(3 (1 - cos rho)) */
-    float alpha;
-    float er, ei;     /* e^{2i(alpha+beta)} */
-    bool exact;       /* rho within 0.5e-6 of 1e-6, or degenerate: exact path */
-};
-
-__device__ inline VisitGeo visit_geo_f32(const FastConsts &fc, const SampleF &sf,
-                                         const VisitRing &g)
-{
-    VisitGeo v;
-    float sh, ch;
-    plf_sincos(g.xh, &sh, &ch);
-    const float sdra = 2.0f * (sh * ch);
-    const float h2 = 2.0f * (sh * sh);
-    const float omD = (g.sD * g.sD) * __builtin_amdgcn_rcpf(g.opcD);
-    v.omc = fmaf(h2, sf.cdc * g.cdp, omD);
-    const float ya = sdra * g.cdp, xa = fmaf(h2, g.cdp * sf.sdc, g.sD);
-    const float yb = sdra * sf.cdc, xb = fmaf(h2, sf.cdc * g.sdp, -g.sD);
-    const bool big = v.omc > fc.omc_hi;
-    v.exact = !big && !(v.omc < fc.omc_lo);   /* rho within 0.5e-6 of 1e-6 */
-    v.alpha = 0x1.921fb6p+0f;                 /* pi/2 when rho <= 1e-6 */
-    v.er = 1.0f;
-    v.ei = 0.0f;
-    if (big) {
-        v.alpha = plf_atan2_core(ya, xa, __builtin_amdgcn_rcpf(fmaxf(fabsf(xa), fabsf(ya))));
-        const float wr = xb * xa - yb * ya, wi = xb * ya + yb * xa;
-        const float n = wr * wr + wi * wi;
-        if (!(n > 1e-36f))
-            v.exact = true;   /* |w|^2 >= 5e-24 for rho > 1.5e-6 */
-        const float inv = __builtin_amdgcn_rcpf(n);
-        v.er = (wr * wr - wi * wi) * inv;
-        v.ei = 2.0f * (wr * wi) * inv;
-    }
-    const float x3 = 3.0f * v.omc;
-    v.y = __builtin_amdgcn_rsqf(x3);
-    v.x3y = x3 * v.y;
-    return v;
-}
-
-/* The detector's part: its beam pixel (beam map of NSIDE nside with margin
- * factor marg_k) and float cos/sin 2chi, given t0 = (pi - psi) 2/pi mod 4 and
- * cos/sin 2psi of its position angle; kNeedExact where a floor is not
- * certain. */
-__device__ inline int beam_pixel_f32_det(const VisitGeo &v, float t0, float c2p, float s2p,
-                                         float nside, float marg_k, float &c2, float &s2)
-{
-    c2 = v.er * c2p - v.ei * s2p;
-    s2 = v.er * s2p + v.ei * c2p;
-    float tt = fmaf(-v.alpha, 0x1.45f306p-1f /* 2/pi */, t0);
-    tt = (tt < 0.0f) ? tt + 4.0f : tt;
-    tt = (tt >= 4.0f) ? tt - 4.0f : tt;
-    const float tmp = nside * v.x3y;
-    const float tp = tt - (float)(int)tt;
-    const float u1 = tp * tmp, u2 = (1.0f - tp) * tmp;
-    const int jp = (int)u1, jm = (int)u2;
-    const float d1 = u1 - (float)jp, d2 = u2 - (float)jm;
-    const float md = fmaf(tmp, 8e-6f, fmaf(marg_k, v.y, 1e-6f));
-    const int ir = jp + jm + 1;
-    const float vv = tt * (float)ir;
-    const int ip = (int)vv;
-    const float dv = vv - (float)ip;
-    const float mv = fmaf((float)ir, 4.5e-6f, 1e-6f);
-    const bool ok = !v.exact && (v.omc > 0.0f) && (v.omc < 0.33332f) && (d1 > md) &&
-                    (d1 < 1.0f - md) && (d2 > md) && (d2 < 1.0f - md) && (dv > mv) &&
-                    (dv < 1.0f - mv);
-    return ok ? 2 * ir * (ir - 1) + ip : kNeedExact;
-}
-
-/* Beam pixel and float cos/sin 2chi of a visit, or kNeedExact (c2, s2 then
- * unset). */
-__device__ inline int beam_pixel_f32_tail(const FastConsts &fc, const SampleF &sf,
-                                          const VisitRing &g, float &c2, float &s2)
-{
-    const VisitGeo v = visit_geo_f32(fc, sf, g);
-    if (v.exact)
-        return kNeedExact;
-    return beam_pixel_f32_det(v, sf.t0, sf.c2p, sf.s2p, fc.nside, fc.marg_k, c2, s2);
-}
-
-/* Beam pixel and float cos/sin 2chi of the visit of the sky pixel at
- * (ra_pix, cos/sin dec_pix), or kNeedExact (c2, s2 then unset). */
-__device__ inline int beam_pixel_f32(const FastConsts &fc, const Centre &c, const SampleF &sf,
-                                     double ra_pix, double cdp, double sdp, float &c2,
-                                     float &s2)
-{
-    return beam_pixel_f32_tail(fc, sf, visit_ring_f32(c, ra_pix, cdp, sdp), c2, s2);
-}
-
 /* ---- certified double-precision form of the same mapping -----------------
  *
- * A second certified form, used by the forward kernel: on the 5-degree,
- * NSIDE 512 workload the forward measured faster with it than with the
- * single-precision form (its beam gathers saw a 77% instead of 54% L2 hit
- * rate).  Its margins are ~1e-12 relative, so it practically never needs the
- * exact path, and it evaluates that path in place instead of deferring. */
+ * Maps the visits that the single-precision form declines, and the visits of
+ * the banded beam adjoint.  Its margins are ~1e-12 relative, so it practically
+ * never needs the exact path, and it evaluates that path in place. */
 
 /* The CPU path obtains the beam pixel from rho = acos(crho) through
  * z = cos(rho) (and sin(rho) within 0.01 rad of the pole); in the polar branch
@@ -885,28 +942,10 @@ __device__ inline void wave_sincos(double x, double *s, double *c)
     *c = pl_cos_kernel(x, 0.0);
 }
 
-/* 1/n to ~1e-15 relative: hardware reciprocal estimate + one Newton step
- * (used only where the value feeds float outputs, never an index). */
-__device__ inline double recip_fast(double n)
-{
-    double r = __builtin_amdgcn_rcp(n);
-    return fma(r, fma(-n, r, 1.0), r);
-}
-
-/* Bound on |alpha_f - alpha| for alpha_f = plf_atan2_core of the FP64
- * arguments rounded to float (float32 emulation over 4e6 arguments of every
- * direction and magnitude, the reciprocal estimate within +-1 ulp: at most
- * 3.6e-7 rad), with a factor of four of margin. */
-constexpr double kAlphaF32Err = 1.5e-6;
-
-/* sigma -> the polar-branch floors of loc2pix (beam_pixel_f64's tail).
- * et bounds the error of tt = sigma 2/pi (mod 4) coming from an approximate
- * alpha (0 for the exact alpha): every floor that depends on tt must then be
- * farther than its error from an integer.  An uncertain floor gives
- * kNeedExact when DEFER, else the exact path's pixel. */
-template <bool DEFER>
+/* sigma -> the polar-branch floors of loc2pix (beam_pixel_f64's tail); the
+ * exact path's pixel where a floor is uncertain. */
 __device__ inline int beam_floors(const Hpx &hb, double crho, double sigma, double tmp, double y,
-                                  double marg_k, double et)
+                                  double marg_k)
 {
     double tt = fmodulo(sigma * kInvHalfPi, 4.0);
     double tp = tt - (int)tt;
@@ -915,25 +954,15 @@ __device__ inline int beam_floors(const Hpx &hb, double crho, double sigma, doub
     int jp = (int)u1, jm = (int)u2;
     double d1 = u1 - jp, d2 = u2 - jm;
     /* margin: nside * 4.4e-14 / sqrt(omc) + 3e-13 tmp + 1e-10, with
-     * 1/sqrt(omc) = sqrt(3) * y; plus et * tmp for the floors of tp * tmp */
-    double md = fma(marg_k, y, fma(fma(et, 1.0, 3e-13), tmp, 1e-10));
+     * 1/sqrt(omc) = sqrt(3) * y */
+    double md = fma(marg_k, y, fma(3e-13, tmp, 1e-10));
     bool ok = (crho > kTwoThird + 1e-12) && (d1 > md) && (d1 < 1.0 - md) && (d2 > md) &&
               (d2 < 1.0 - md);
     int ir = jp + jm + 1;
-    double vv = tt * ir;
-    int ip = (int)vv;
-    if (et > 0.0) {
-        /* the quadrant (int)tt and ip = (int)(tt ir) */
-        double mv = fma(et, (double)ir, 1e-12);
-        double dv = vv - ip;
-        ok = ok && (tp > et) && (tp < 1.0 - et) && (dv > mv) && (dv < 1.0 - mv);
-    }
+    int ip = (int)(tt * ir);
     if (ok)
         return 2 * ir * (ir - 1) + ip;
-    if constexpr (DEFER)
-        return kNeedExact;
-    else
-        return beam_pixel_exact_rho(hb.nside, crho, sigma);
+    return beam_pixel_exact_rho(hb.nside, crho, sigma);
 }
 
 __device__ inline double sigma_of(double alpha, double psi)
@@ -946,12 +975,6 @@ __device__ inline double sigma_of(double alpha, double psi)
     return sigma;
 }
 
-/* FLOAT_ALPHA: alpha from the float atan2 of the FP64 arguments, its floors
- * certified against kAlphaF32Err, and kNeedExact for a visit whose floors
- * cannot be certified (the caller defers it to this function's exact form);
- * otherwise alpha from the FP64 atan2, the CPU path's own (sphtrigo.cpp:42),
- * and the exact path in place for an uncertain floor. */
-template <bool FLOAT_ALPHA = false>
 __device__ inline int beam_pixel_f64(const Hpx &hb, const FastConsts64 &fc, const Centre &c,
                                       double c2psi, double s2psi, double ra_pix,
                                       double cdp, double sdp, float &c2, float &s2)
@@ -997,19 +1020,9 @@ __device__ inline int beam_pixel_f64(const Hpx &hb, const FastConsts64 &fc, cons
     y = y * fma(-0.5 * x3, y * y, 1.5);
     y = y * fma(-0.5 * x3, y * y, 1.5);
     double tmp = (x3 > 0.0) ? hb.nside * (x3 * y) : 0.0;
-    if constexpr (FLOAT_ALPHA) {
-        double alpha = kHalfPi;
-        if (big) {
-            const float yf = (float)ya, xf = (float)xa;
-            alpha = (double)plf_atan2_core(
-                yf, xf, __builtin_amdgcn_rcpf(fmaxf(fabsf(xf), fabsf(yf))));
-        }
-        return beam_floors<true>(hb, crho, sigma_of(alpha, c.psi), tmp, y, fc.marg_k,
-                                 big ? kAlphaF32Err * kInvHalfPi : 0.0);
-    } else {
-        double alpha = big ? pl_atan2(ya, xa) : kHalfPi;
-        return beam_floors<false>(hb, crho, sigma_of(alpha, c.psi), tmp, y, fc.marg_k, 0.0);
-    }
+    /* alpha from the FP64 atan2, the CPU path's own (sphtrigo.cpp:42) */
+    double alpha = big ? pl_atan2(ya, xa) : kHalfPi;
+    return beam_floors(hb, crho, sigma_of(alpha, c.psi), tmp, y, fc.marg_k);
 }
 
 /* get_interpol (Healpix_Base::get_interpol; the device port in the reference

@@ -79,14 +79,12 @@ __device__ inline long xcd_remap(long b, long nblk)
     return (x < r) ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
 }
 
-/* Run table of one wave for one pass over (up to) 64 rings, and the wave's
- * queue of visits deferred to the exact FP64 mapping (sky pixel, ring). */
+/* Run table of one wave for one pass over (up to) 64 rings (beam
+ * interpolation). */
 struct RunTable {
     int pref[kMaxRuns + 1];  /* visit offset of each run; pref[nrun] = total */
     int pix0[kMaxRuns];
     int ring[kMaxRuns];
-    int qpix[2 * kWaveSize];
-    int qring[2 * kWaveSize];
 };
 
 /* Builds the run table for rings r0 .. r0+63 (clipped to the disc); returns
@@ -122,366 +120,31 @@ __device__ inline int build_runs(const Hpx &hs, const Disc &d, int r0, int lane,
     return total;
 }
 
-/* Beam pixel and float cos/sin(2 chi) of the visit of sky pixel pix (ring r,
- * ring record rr) from the sample with beam-centre constants c, sf; or
- * kNeedExact. */
-__device__ inline int visit_beam(const PairParams &p, const Centre &c, const SampleF &sf,
-                                 const RingRec &rr, int r, int pix, float &c2, float &s2)
-{
-    double ra_pix = ring_phi(p.hs, rr, r, pix);
-    return beam_pixel_f32(p.fc, c, sf, ra_pix, rr.cdp, rr.sdp, c2, s2);
-}
-
-/* Wave-uniform double constants of one sample (double-precision mapping). */
-struct SampleD {
-    double c2psi, s2psi;   /* cos, sin 2 psi */
-};
-
-/* A visit whose beam pixel lies inside the beam, with what `use` needs. */
-struct Pending {
-    int pix, bp, r, sp;
-    float c2, s2;
-    float4 v0;        /* A0 A1 A2 B0 */
-    float2 v1;        /* B1 B2 */
-    float2 v2;        /* A3 B3 (forward with the V term only) */
-    float sI, sQ, sU; /* sky of the visit (forward only) */
-    float sV;         /* sky V of the visit (forward with the V term only) */
-    bool live;
-};
-
-/* The TOD terms of one visit, a and b: the float expression of
- * convolver.cpp:157-164 and, with VT, the V terms the reference's GPU kernel
- * adds (V A3, V B3; cudaConv2.cu:204,214,217-218), appended last. */
-template <bool VT>
-__device__ inline void visit_tod(const Pending &e, float &ta, float &tb)
-{
-    const float A0 = e.v0.x, A1 = e.v0.y, A2 = e.v0.z;
-    const float B0 = e.v0.w, B1 = e.v1.x, B2 = e.v1.y;
-    const float c2 = e.c2, s2 = e.s2;
-    if constexpr (VT) {
-        ta = e.sI * (A0) + e.sQ * (A1 * c2 - A2 * s2) + e.sU * (A2 * c2 + A1 * s2) +
-             e.sV * e.v2.x;
-        tb = e.sI * (B0) + e.sQ * (-B1 * c2 + B2 * s2) + e.sU * (-B2 * c2 - B1 * s2) +
-             e.sV * e.v2.y;
-    } else {
-        ta = e.sI * (A0) + e.sQ * (A1 * c2 - A2 * s2) + e.sU * (A2 * c2 + A1 * s2);
-        tb = e.sI * (B0) + e.sQ * (-B1 * c2 + B2 * s2) + e.sU * (-B2 * c2 - B1 * s2);
-    }
-}
-
-__device__ inline int lanes_below(unsigned long long m)
-{
-    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                          __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-}
-
-/* Maps queue entries base .. base+cnt-1 (cnt <= 64), one per lane, with the
- * certified double-precision form (beam_pixel_f64, whose own fallback is the
- * exact FP64 path; the beam pixel is the exact path's either way) and hands
- * the visits inside the beam to use().  Called with every lane of the wave
- * active.  The double-precision form costs about a quarter of the exact
- * path: draining through it measured 2% faster on the 5-degree, NSIDE 512
- * sky adjoint. */
-template <bool LOAD_SKY, typename Use, bool VT = false>
-__device__ inline void drain_exact(const PairParams &p, RunTable &t, int base, int cnt, int lane,
-                                   const Centre &c, double c2psi, double s2psi, Use &use)
-{
-    wave_sync();
-    if (lane < cnt) {
-        const int pix = t.qpix[base + lane], r = t.qring[base + lane];
-        const RingRec rr = p.rings[r];
-        const double ra_pix = ring_phi(p.hs, rr, r, pix);
-        ExactVisit e;
-        e.bp = beam_pixel_f64(p.hb, p.fc64, c, c2psi, s2psi, ra_pix, rr.cdp, rr.sdp, e.c2, e.s2);
-        if ((unsigned)e.bp < (unsigned)p.npix_beam) {
-            Pending q;
-            q.pix = pix;
-            q.r = r;
-            q.sp = rr.startpix;
-            q.bp = e.bp;
-            q.c2 = e.c2;
-            q.s2 = e.s2;
-            const float *row = p.beam + 8 * (long)e.bp;
-            q.v0 = *(const float4 *)row;
-            q.v1 = *(const float2 *)(row + 4);
-            if constexpr (VT)
-                q.v2 = *(const float2 *)(row + 6);
-            if (LOAD_SKY) {
-                const float4 sv = p.sky4[pix];
-                q.sI = sv.x;
-                q.sQ = sv.y;
-                q.sU = sv.z;
-                q.sV = sv.w;
-            }
-            q.live = true;
-            use(q);
-        }
-    }
-    /* Leave no load of this (rare) path outstanding: otherwise the merge of
-     * the paths at the caller's loop head looks as if those loads might still
-     * be pending, and the compiler would wait for the main path's in-flight
-     * loads there too. */
-    __builtin_amdgcn_s_waitcnt(0);
-    wave_sync();
-}
-
-/* The walk over the visits of one ring pass: lane-strided, with every lane
- * running the same number of iterations (the deferred-visit queue is drained
- * by the whole wave).  Software pipelined by hand: the ring record of the
- * lane's next visit is loaded while the current one is computed, and the
- * beam/sky loads of a visit are issued at the end of its iteration and
- * consumed (by `use`) after the next visit's geometry.  The record is used
- * before the next loads are issued into it, so no register copy of a pending
- * load is needed.  In the forward every global load of the main path is
- * issued unconditionally (lanes without a visit load row 0 / pixel 0 and
- * discard it): a load skipped on some path makes the in-order load counter
- * ambiguous at the loop head, and the compiler then waits for all loads
- * there instead of only for the ring record (the adjoints, with fewer loads
- * per visit, measured faster with conditional loads).  Visits whose floors
- * the fast form cannot certify (the float mapping, or the FP64 form with its
- * float alpha) go to the queue (qn entries, wave-uniform); a full batch of 64
- * is drained at once.  use(q) is called once per visit whose beam pixel lies
- * inside the beam. */
-template <bool LOAD_SKY, bool MAP64, typename Use, bool VT = false, bool LOAD_BEAM = true>
-__device__ inline void walk_visits(const PairParams &p, RunTable &t, int total, int lane,
-                                   const Centre &c, const SampleF &sf, const SampleD &sd,
-                                   int &qn, Use &use)
-{
-    if (total <= 0)
-        return;
-    int s = 0;
-    int v = lane;
-    if (v < total)
-        while (v >= t.pref[s + 1])
-            s++;
-    RingRec rr = p.rings[t.ring[s]];
-    /* complete this first load here: a load still pending on the loop-entry
-     * edge would make the compiler wait for the in-flight beam/sky loads at
-     * every use of the ring record inside the loop */
-    __builtin_amdgcn_s_waitcnt(0);
-    Pending q;
-    q.live = false;
-    for (int v0 = 0; v0 < total; v0 += kWaveSize, v += kWaveSize) {
-        const bool act = v < total;
-        /* a lane past the end repeats the first visit of its run, discarded */
-        const int pix = t.pix0[s] + (act ? v - t.pref[s] : 0);
-        const int r = t.ring[s];
-        float c2, s2;
-        int bp, startpix;
-        if constexpr (MAP64) {
-            const RingRec cur = rr;
-            const int vn = v + kWaveSize;
-            if (vn < total)
-                while (vn >= t.pref[s + 1])
-                    s++;
-            rr = p.rings[t.ring[s]];   /* prefetch of the next visit's record */
-            startpix = cur.startpix;
-            bp = beam_pixel_f64<true>(p.hb, p.fc64, c, sd.c2psi, sd.s2psi,
-                                      ring_phi(p.hs, cur, r, pix), cur.cdp, cur.sdp, c2, s2);
-        } else {
-            /* the part of the geometry that reads the ring record, then the
-             * prefetch of the next visit's record into the same registers */
-            const VisitRing g = visit_ring_f32(c, ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp);
-            startpix = rr.startpix;
-            const int vn = v + kWaveSize;
-            if (vn < total)
-                while (vn >= t.pref[s + 1])
-                    s++;
-            rr = p.rings[t.ring[s]];
-            bp = beam_pixel_f32_tail(p.fc, sf, g, c2, s2);
-        }
-        bp = act ? bp : -1;
-        {   /* visits whose floors the fast form cannot certify: queued */
-            const unsigned long long m = __ballot(bp == kNeedExact);
-            if (m) {
-                if (bp == kNeedExact) {
-                    const int pos = qn + lanes_below(m);
-                    t.qpix[pos] = pix;
-                    t.qring[pos] = r;
-                }
-                qn += __popcll(m);
-            }
-        }
-        if (q.live)
-            use(q);
-        {
-            /* drain here, where the previous visit is consumed and the next
-             * loads are not yet issued: little is live across the exact
-             * path's out-of-line call */
-            if (qn >= kWaveSize) {
-                drain_exact<LOAD_SKY, Use, VT>(p, t, qn - kWaveSize, kWaveSize, lane, c, sd.c2psi,
-                                               sd.s2psi, use);
-                qn -= kWaveSize;
-            }
-        }
-        q.live = (unsigned)bp < (unsigned)p.npix_beam;   /* rejects -1 and kNeedExact */
-        q.pix = pix;
-        q.r = r;
-        q.sp = startpix;
-        q.bp = bp;
-        q.c2 = c2;
-        q.s2 = s2;
-        if constexpr (LOAD_SKY) {
-            /* forward: loads issued unconditionally (row 0 / pixel 0 when
-             * the visit is dead), see above */
-            if constexpr (LOAD_BEAM) {
-                const float *row = p.beam + 8 * (long)(q.live ? bp : 0);
-                q.v0 = *(const float4 *)row;
-                q.v1 = *(const float2 *)(row + 4);
-                if constexpr (VT)
-                    q.v2 = *(const float2 *)(row + 6);
-            }
-            const int sp = q.live ? pix : 0;
-            const float4 sv = p.sky4[sp];
-            q.sI = sv.x;
-            q.sQ = sv.y;
-            q.sU = sv.z;
-            q.sV = sv.w;
-        } else if constexpr (LOAD_BEAM) {
-            if (q.live) {
-                /* adjoints: only live visits load (measured faster there) */
-                const float *row = p.beam + 8 * (long)bp;
-                q.v0 = *(const float4 *)row;
-                q.v1 = *(const float2 *)(row + 4);
-            }
-        }
-    }
-    if (q.live)
-        use(q);
-}
-
-/* Wave-uniform copy of a float (to scalar registers). */
-__device__ inline float unif(float x)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
-}
-
-/* Per-sample setup shared by the visit kernels: beam-centre constants in
- * scalar registers and the sample's disc. */
-__device__ inline void sample_setup(const PairParams &p, long i, float pa_i, Centre &c,
-                                    SampleF &sf, SampleD &sd, Disc &d)
-{
-    c = centre_make(p.ra[i], p.dec[i], pa_i);
-    c.ra = uni(c.ra);
-    c.dec = uni(c.dec);
-    c.psi = uni(c.psi);
-    c.cdc = uni(c.cdc);
-    c.sdc = uni(c.sdc);
-    double s2psi, c2psi;
-    pl_sincos(2.0 * c.psi, &s2psi, &c2psi);
-    sd.c2psi = uni(c2psi);
-    sd.s2psi = uni(s2psi);
-    sf = sample_f32(c, c2psi, s2psi);
-    sf.cdc = unif(sf.cdc);
-    sf.sdc = unif(sf.sdc);
-    sf.t0 = unif(sf.t0);
-    sf.c2p = unif(sf.c2p);
-    sf.s2p = unif(sf.s2p);
-    disc_setup(p.hs, kHalfPi - c.dec, c.ra, p.rho_max, p.cos_rmax, d);
-}
-
-/* One sample of one detector pair (pa of the sample given): forward TOD,
- * or the direct-atomic adjoints. */
-template <int OP>
-__device__ inline void pair_sample(const PairParams &p, long i, float pa_i, RunTable &t,
-                                   int lane)
-{
-    constexpr bool FWD = OP == OP_FWD || OP == OP_FWD_V;
-    Centre c;
-    SampleF sf;
-    SampleD sd;
-    Disc d;
-    sample_setup(p, i, pa_i, c, sf, sd, d);
-    double ga = 0.0, gb = 0.0;
-    if (!FWD) {
-        ga = uni(p.g_a ? (double)p.g_a[i] : 0.0);
-        gb = uni(p.g_b ? (double)p.g_b[i] : 0.0);
-    }
-    double acc_a = 0.0, acc_b = 0.0;
-    auto use = [&](const Pending &q) {
-        const float A0 = q.v0.x, A1 = q.v0.y, A2 = q.v0.z;
-        const float B0 = q.v0.w, B1 = q.v1.x, B2 = q.v1.y;
-        const float c2 = q.c2, s2 = q.s2;
-        const int pix = q.pix, bp = q.bp;
-        if (FWD) {
-            float ta, tb;
-            visit_tod<OP == OP_FWD_V>(q, ta, tb);
-            acc_a += ta;
-            acc_b += tb;
-        } else if (OP == OP_ADJ_MAP) {
-            double cc = c2, ss = s2;
-            double vI = ga * A0 + gb * B0;
-            double vQ = ga * (A1 * cc - A2 * ss) + gb * (-B1 * cc + B2 * ss);
-            double vU = ga * (A2 * cc + A1 * ss) + gb * (-B2 * cc - B1 * ss);
-            unsafeAtomicAdd(&p.gI[pix], vI);
-            unsafeAtomicAdd(&p.gQ[pix], vQ);
-            unsafeAtomicAdd(&p.gU[pix], vU);
-        } else {
-            double cc = c2, ss = s2;
-            double qq = p.Q[pix], u = p.U[pix], sI = p.I[pix];
-            double *g = p.gbeam + 8 * (long)bp;
-            unsafeAtomicAdd(&g[0], ga * sI);
-            unsafeAtomicAdd(&g[1], ga * (qq * cc + u * ss));
-            unsafeAtomicAdd(&g[2], ga * (-qq * ss + u * cc));
-            unsafeAtomicAdd(&g[3], gb * sI);
-            unsafeAtomicAdd(&g[4], gb * (-qq * cc - u * ss));
-            unsafeAtomicAdd(&g[5], gb * (qq * ss - u * cc));
-        }
-    };
-
-    int qn = 0;   /* deferred visits (wave-uniform) */
-    for (int r0 = d.r_first; r0 <= d.r_last; r0 += kWaveSize) {
-        int total = build_runs(p.hs, d, r0, lane, t);
-        walk_visits<FWD, FWD, decltype(use), OP == OP_FWD_V>(p, t, total, lane, c, sf, sd, qn,
-                                                             use);
-        wave_sync();
-    }
-    if (qn > 0)
-        drain_exact<FWD, decltype(use), OP == OP_FWD_V>(p, t, 0, qn, lane, c, sd.c2psi, sd.s2psi,
-                                                       use);
-    if (FWD) {
-        acc_a = wave_sum(acc_a);
-        acc_b = wave_sum(acc_b);
-        if (lane == 0) {
-            if (p.tod_a)
-                p.tod_a[i] = (float)acc_a;
-            if (p.tod_b)
-                p.tod_b[i] = (float)acc_b;
-        }
-    }
-}
-
-/* 4 waves per SIMD (128 VGPRs): with the float alpha and its deferral queue
- * the forward needs about 100 VGPRs; under the 96 of 5 waves per SIMD it
- * spilled and ran 15% slower at the 5-degree, NSIDE 512 headline. */
-template <int OP>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_pair(PairParams p)
-{
-    __shared__ RunTable tables[kWavesPerBlock];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-    const int lane = threadIdx.x % kWaveSize;
-    long lb = xcd_remap(blockIdx.x, gridDim.x);
-    long i = p.s_begin + lb * kWavesPerBlock + wave;
-    if (i >= p.s_end)
-        return;
-    pair_sample<OP>(p, i, p.pa[i], tables[wave], lane);
-}
-
-/* ---- small-disc forward: several samples per wave -------------------------
+/* ---- the walk over a disc's visits ----------------------------------------
  *
- * For discs of a few hundred pixels the per-sample part of k_pair<OP_FWD>
- * (beam-centre constants, disc set-up, the ring step, the final reduction)
- * runs on all 64 lanes for one sample and costs more than the visits.  Here
- * a wave holds G = 64/SUB samples of SUB lanes each: that part runs once for
- * the G samples, each lane group walks its own disc SUB visits at a time, and
- * a SUB-lane reduction gives each sample's TOD.  The mapping (certified FP64
- * form), the per-visit values and the FP64 accumulation are those of
- * k_pair<OP_FWD>. */
-template <int SUB>
-struct SubTable {
-    int pref[2 * SUB + 1];   /* visit offset of each run; pref[nrun] = total */
-    int pix0[2 * SUB];
-    int ring[2 * SUB];
+ * A lane group of SUB lanes (64: the whole wave) walks the visits of its
+ * sample's disc SUB at a time, in passes of at most RPP runs of consecutive
+ * pixels (0 to 2 per ring).  A pass's table holds, per run, the float geometry
+ * of the ring around the sample (run_geo), so that a visit reads two LDS
+ * records and does no FP64.  `bits` marks the visits that start a run: a lane
+ * finds its run by counting the marks below it (its wave's visits are
+ * consecutive), where a search through the run offsets would be a chain of
+ * dependent LDS reads.  The marks cover a segment of VCAP visits from seg0 on:
+ * bit v - 1 - seg0 marks a run that starts at visit v > seg0. */
+template <int SUB_, int RPP_, int VCAP_>
+struct VisitTable {
+    static constexpr int SUB = SUB_, RPP = RPP_, VCAP = VCAP_;
+    float4 rec[RPP][2];      /* a0, b, mid, pixoff (int bits); sD, omD, cdp2, kap */
+    unsigned bits[VCAP / 32];
+    int pref[RPP + 1];       /* visit offset of each run; pref[nrun] = total */
+    int ring[RPP];
+};
+
+/* What a pass covers: its visits and runs, the first ring of the next pass,
+ * and whether some visit's |eta| may exceed the caller's bound. */
+struct Pass {
+    int total, nrun, next;
+    bool wide;
 };
 
 template <int SUB>
@@ -496,6 +159,425 @@ __device__ inline int seg_incl_scan(int x, int sl)
     return x;
 }
 
+/* The runs of ring r, as ring positions: query_disc's ranges, a whole ring
+ * split where dra passes pi (each run then lies on one branch of dra). */
+__device__ inline int disc_runs(const Hpx &h, const Disc &d, const Centre &c, int r, int startpix,
+                                int j0[2], int len[2])
+{
+    int ns = disc_ring(h, d, r, j0, len);
+    j0[0] -= startpix;
+    j0[1] -= startpix;
+    const int nr = 4 * (r < h.nside ? r : (r > 3 * h.nside ? 4 * h.nside - r : h.nside));
+    if (ns == 1 && len[0] == nr) {
+        const bool shifted = r < h.nside || r > 3 * h.nside || ((r - h.nside) & 1) == 0;
+        double t = (c.ra + kPi) * kInvTwoPi;
+        t -= floor(t);
+        int ja = (int)ceil(t * nr - (shifted ? 0.5 : 0.0));
+        ja = ja < 0 ? 0 : ja;
+        if (ja > 0 && ja < nr) {
+            len[0] = ja;
+            j0[1] = ja;
+            len[1] = nr - ja;
+            ns = 2;
+        }
+    }
+    return ns;
+}
+
+/* Builds the table of the pass that starts at ring r0 (up to d.r_last) for
+ * the lane group; every lane of the group returns the same Pass. */
+template <typename T>
+__device__ inline Pass build_pass(const Hpx &hs, const RingRec *rings, const Disc &d,
+                                  const Centre &c, int r0, int r_last, int sl, float eta_max, T &t)
+{
+    constexpr int SUB = T::SUB, RPP = T::RPP;
+    constexpr int kWords = T::VCAP / 32;
+    const int lane = (int)__lane_id();
+    for (int w = sl; w < kWords; w += SUB)
+        t.bits[w] = 0u;
+    wave_sync();
+    int carry = 0;            /* visits << 8 | runs of the rounds before */
+    Pass ps;
+    ps.next = r0;
+    bool wide = false, more = true;
+#pragma unroll 1
+    for (int q = 0; q < (RPP + SUB - 1) / SUB; q++) {
+        const int r = r0 + q * SUB + sl;
+        const bool in = more && r <= r_last;
+        RingRec rr;
+        int j0[2] = {0, 0}, ln[2] = {0, 0};
+        int ns = 0;
+        if (in) {
+            rr = rings[r];
+            ns = disc_runs(hs, d, c, r, rr.startpix, j0, ln);
+        }
+        const int mine = ns + (((ns > 0 ? ln[0] : 0) + (ns > 1 ? ln[1] : 0)) << 8);
+        const int incl = carry + seg_incl_scan<SUB>(mine, sl);
+        /* the rings whose runs still fit the table (a prefix of the lanes) */
+        const bool fit = more && (incl & 255) <= RPP;
+        unsigned long long fm = __ballot(fit);
+        if constexpr (SUB < kWaveSize)
+            fm = (fm >> (lane & ~(SUB - 1))) & ((1ull << SUB) - 1ull);
+        const int nfit = __popcll(fm);
+        int run = (incl & 255) - ns;
+        int off = (incl >> 8) - (mine >> 8);
+#pragma unroll
+        for (int k = 0; k < 2; k++) {   /* constant indices keep j0, ln in registers */
+            if (fit && k < ns) {
+                const RunGeo g = run_geo(hs, rr, r, c, j0[k], ln[k]);
+                const int mid = off - j0[k] + g.kc;
+                t.rec[run][0] = make_float4(g.a0, g.b, (float)mid,
+                                            __int_as_float(rr.startpix + j0[k] - off));
+                t.rec[run][1] = make_float4(g.sD, g.omD, g.cdp2, g.kap);
+                t.pref[run] = off;
+                t.ring[run] = r;
+                const float x0 = fabsf(fmaf((float)(off - mid), g.b, g.a0));
+                const float x1 = fabsf(fmaf((float)(off + ln[k] - mid), g.b, g.a0));
+                const float xm = fmaxf(x0, x1);
+                wide = wide || !(fabsf(g.kap) * xm < eta_max) || xm > 0.7f;
+                if (off > 0 && off <= T::VCAP)   /* the first segment's marks */
+                    atomicOr(&t.bits[(off - 1) >> 5], 1u << ((off - 1) & 31));
+                run++;
+                off += ln[k];
+            }
+        }
+        const int last = __shfl(incl, nfit > 0 ? nfit - 1 : 0, SUB);
+        carry = nfit > 0 ? last : carry;
+        ps.next += nfit;
+        more = more && nfit == SUB;
+    }
+    ps.nrun = carry & 255;
+    ps.total = carry >> 8;
+    unsigned long long wm = __ballot(wide);
+    if constexpr (SUB < kWaveSize)   /* a sample's results do not depend on its neighbours */
+        wm = (wm >> (lane & ~(SUB - 1))) & ((1ull << SUB) - 1ull);
+    ps.wide = wm != 0ull;
+    if (sl == 0)
+        t.pref[ps.nrun] = ps.total;
+    wave_sync();
+    return ps;
+}
+
+/* Marks the runs of the segment that starts at visit seg0 > 0; returns the
+ * number of runs, besides the first, that start at or before seg0. */
+template <typename T>
+__device__ inline int mark_segment(T &t, int nrun, int seg0, int sl)
+{
+    constexpr int SUB = T::SUB;
+    wave_sync();
+    for (int w = sl; w < T::VCAP / 32; w += SUB)
+        t.bits[w] = 0u;
+    wave_sync();
+    int before = -1;
+    for (int i0 = 0; i0 < T::RPP; i0 += SUB) {
+        const bool in = i0 + sl < nrun;
+        const int o = in ? t.pref[i0 + sl] - seg0 : 1;
+        unsigned long long m = __ballot(in && o <= 0);
+        if constexpr (SUB < kWaveSize)
+            m = (m >> ((int)__lane_id() & ~(SUB - 1))) & ((1ull << SUB) - 1ull);
+        before += __popcll(m);
+        if (in && o > 0 && o <= T::VCAP)
+            atomicOr(&t.bits[(o - 1) >> 5], 1u << ((o - 1) & 31));
+    }
+    wave_sync();
+    return before;
+}
+
+/* A visit whose beam pixel lies inside the beam, with what `use` needs. */
+struct Pending {
+    int v, s;         /* visit and run of the pass */
+    int pix, bp;
+    float c2, s2;
+    float4 v0;        /* A0 A1 A2 B0 */
+    float2 v1;        /* B1 B2 */
+    float2 v2;        /* A3 B3 (forward with the V term only) */
+    float sI, sQ, sU; /* sky of the visit (forward only) */
+    float sV;         /* sky V of the visit (forward with the V term only) */
+    bool live;
+};
+
+/* Adds the TOD terms of one visit, a and b (convolver.cpp:157-164; with VT
+ * the V terms the reference's GPU kernel adds, V A3 and V B3,
+ * cudaConv2.cu:204,214,217-218).  With X + iY = (Q + iU) e^{-2i chi} the
+ * polarised part is A1 X + A2 Y for a and its negative with B for b.  The I
+ * (and V) products are formed exactly in FP64: their float rounding would be
+ * the sum's largest error. */
+template <bool VT>
+__device__ inline void visit_tod(const Pending &e, double &acc_a, double &acc_b)
+{
+    const float X = fmaf(e.sQ, e.c2, e.sU * e.s2), Y = fmaf(e.sU, e.c2, -(e.sQ * e.s2));
+    const float pa = fmaf(e.v0.z, Y, e.v0.y * X), pb = fmaf(e.v1.y, Y, e.v1.x * X);
+    const double I = e.sI;
+    acc_a = fma(I, (double)e.v0.x, acc_a) + (double)pa;
+    acc_b = fma(I, (double)e.v0.w, acc_b) - (double)pb;
+    if constexpr (VT) {
+        acc_a = fma((double)e.sV, (double)e.v2.x, acc_a);
+        acc_b = fma((double)e.sV, (double)e.v2.y, acc_b);
+    }
+}
+
+__device__ inline int lanes_below(unsigned long long m)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+/* What a walk loads and computes per visit. */
+enum {
+    WALK_SKY = 1,      /* the sky values */
+    WALK_BEAM = 2,     /* the beam row */
+    WALK_V = 4,        /* the V columns and the sky's V */
+    WALK_CHI = 8,      /* cos, sin 2 chi */
+};
+
+template <int F>
+__device__ inline void load_visit(const PairParams &p, Pending &q, int bp, int pix)
+{
+    if constexpr (F & WALK_BEAM) {
+        const float *row = p.beam + 8 * (long)bp;
+        q.v0 = *(const float4 *)row;
+        q.v1 = *(const float2 *)(row + 4);
+        if constexpr (F & WALK_V)
+            q.v2 = *(const float2 *)(row + 6);
+    }
+    if constexpr (F & WALK_SKY) {
+        const float4 sv = p.sky4[pix];
+        q.sI = sv.x;
+        q.sQ = sv.y;
+        q.sU = sv.z;
+        q.sV = sv.w;
+    }
+}
+
+__device__ inline void rec_make(const PairParams &p, float ra, float dec, float pa, SampleRec &r)
+{
+    const Centre c = centre_make(ra, dec, pa);
+    double s, co;
+    pl_sincos(c.psi, &s, &co);
+    r.c2psi = fma(co, co, -(s * s));
+    r.s2psi = 2.0 * (s * co);
+    r.sf = sample_f32(c, co, s, r.c2psi, r.s2psi);
+    r.ra = c.ra;
+    r.cdc = c.cdc;
+    r.sdc = c.sdc;
+    r.psi = c.psi;
+    Disc d;
+    disc_setup(p.hs, kHalfPi - c.dec, c.ra, p.rho_max, p.cos_rmax, d);
+    r.phi = d.phi;
+    r.z0 = d.z0;
+    r.xa = d.xa;
+    r.irmin = d.irmin;
+    r.irmax = d.irmax;
+    r.r_first = d.r_first;
+    r.r_last = d.r_last;
+}
+
+__device__ inline Centre rec_centre(const SampleRec &r)
+{
+    Centre c;
+    c.ra = r.ra;
+    c.dec = 0.0;   /* not read by the mappings */
+    c.psi = r.psi;
+    c.cdc = r.cdc;
+    c.sdc = r.sdc;
+    return c;
+}
+
+__device__ inline Disc rec_disc(const PairParams &p, const SampleRec &r)
+{
+    Disc d;
+    d.phi = r.phi;
+    d.z0 = r.z0;
+    d.xa = r.xa;
+    d.cosr = p.cos_rmax;
+    d.irmin = r.irmin;
+    d.irmax = r.irmax;
+    d.r_first = r.r_first;
+    d.r_last = r.r_last;
+    return d;
+}
+
+/* Wave-uniform copy of a float (to scalar registers). */
+__device__ inline float unif(float x)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+}
+
+__device__ inline SampleF unif(const SampleF &f)
+{
+    SampleF u;
+    u.cdc = unif(f.cdc);
+    u.sdc = unif(f.sdc);
+    u.cps = unif(f.cps);
+    u.sps = unif(f.sps);
+    u.c2h = unif(f.c2h);
+    u.c2l = unif(f.c2l);
+    u.s2h = unif(f.s2h);
+    u.s2l = unif(f.s2l);
+    u.lim0 = unif(f.lim0);
+    return u;
+}
+
+/* A wave's samples (NS of them) and its queue of visits deferred to the FP64
+ * form (sky pixel, sample); fewer than 64 entries between drains, and one
+ * iteration adds at most 64. */
+template <int NS_>
+struct WaveState {
+    static constexpr int NS = NS_;
+    SampleRec rec[NS];
+    int qpix[2 * kWaveSize];
+    unsigned char qj[2 * kWaveSize];
+};
+
+/* Maps queue entries base .. base+cnt-1 (cnt <= 64), one per lane, with the
+ * certified double-precision form (beam_pixel_f64, whose own fallback is the
+ * exact FP64 path; the beam pixel is the exact path's either way) and hands
+ * the visits inside the beam to use(q, ring, startpix, sample).  Called with
+ * every lane of the wave active. */
+template <int F, typename WS, typename Use>
+__device__ inline void drain_queue(const PairParams &p, const WS &ws, int base, int cnt, int lane,
+                                   Use &use)
+{
+    wave_sync();
+    if (lane < cnt) {
+        const int pix = ws.qpix[base + lane], j = ws.qj[base + lane];
+        const int r = pix2ring(p.hs, pix);
+        const RingRec rr = p.rings[r];
+        const SampleRec &sr = ws.rec[j];
+        Pending q;
+        q.v = q.s = 0;
+        q.pix = pix;
+        q.live = true;
+        q.bp = beam_pixel_f64(p.hb, p.fc64, rec_centre(sr), sr.c2psi, sr.s2psi,
+                              ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, q.c2, q.s2);
+        if ((unsigned)q.bp < (unsigned)p.npix_beam) {
+            load_visit<F>(p, q, q.bp, pix);
+            use(q, r, rr.startpix, j);
+        }
+    }
+    wave_sync();
+}
+
+/* The lanes of m (visits of sample j) join the queue. */
+template <typename WS>
+__device__ inline void enqueue(WS &ws, int &qn, unsigned long long m, int pix, int j)
+{
+    if ((m >> __lane_id()) & 1ull) {
+        const int pos = qn + lanes_below(m);
+        ws.qpix[pos] = pix;
+        ws.qj[pos] = (unsigned char)j;
+    }
+    qn += __popcll(m);
+}
+
+/* Where a walk of a pass is: its next visit, its segment, and the runs besides
+ * the first that start at or before the next visit's block. */
+struct WalkAt {
+    int v0 = 0, seg0 = 0, base = 0;
+};
+
+/* The walk of one segment of a pass, visits at.v0 .. vend - 1.  Software
+ * pipelined by hand: the next visit's records are read from LDS while the
+ * current one is mapped (two sets of registers, the loop unrolled by two), and
+ * the beam and sky loads of a visit are issued at the end of its iteration and
+ * consumed (by `use`) after the next visit's mapping.  Loads two iterations
+ * ahead measured slower: the L1 holds 256 lines and a wave's iteration takes
+ * 72.  Every global load is issued unconditionally (lanes without a visit load
+ * row 0 / pixel 0 and discard them): a load skipped on some path makes the
+ * in-order load counter ambiguous at the loop head.  Visits whose floors the
+ * float form cannot certify join the queue; the walk returns (at.v0 < vend)
+ * when it holds a batch of 64, so that the FP64 drain, which needs many
+ * registers, is outside the loop.  WIDE: cos, sin 2 chi in FP64 for the lane
+ * groups with `wide`. */
+template <int F, bool WIDE, typename T, typename WS, typename Use>
+__device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int total, int vend,
+                                    bool wide, int sl, int j, const SampleF &sf, WalkAt &at,
+                                    int &qn, Use &use)
+{
+    constexpr int SUB = T::SUB;
+    struct Rec {
+        float4 a, b;
+        int run;
+    };
+    int v0 = at.v0, base = at.base, base0 = base;
+    if (v0 >= vend || qn >= kWaveSize)
+        return;
+    auto fetch = [&](Rec &n, int v) {   /* the records of visit v + sl */
+        const int k = v - at.seg0;
+        if constexpr (SUB == kWaveSize) {
+            const unsigned lo = t.bits[k >> 5], hi = t.bits[(k >> 5) + 1];
+            n.run = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, base));
+            base += __popc(lo) + __popc(hi);
+        } else {
+            const unsigned m = t.bits[k >> 5] >> (k & 31);
+            n.run = base + __popc(m & ((1u << sl) - 1u));
+            base += __popc(SUB == 32 ? m : m & ((1u << (SUB & 31)) - 1u));
+        }
+        n.a = t.rec[n.run][0];
+        n.b = t.rec[n.run][1];
+    };
+    Pending q;
+    q.live = false;
+    float vf = (float)(v0 + sl);
+    auto step = [&](const Rec &r, Rec &n) {
+        base0 = base;
+        if (v0 + SUB < vend)
+            fetch(n, v0 + SUB);
+        const int v = v0 + sl;
+        const bool act = v < total;
+        const int pix = v + __float_as_int(r.a.w);
+        const VisitGeo g =
+            visit_geo(fmaf(vf - r.a.z, r.a.y, r.a.x), r.b.x, r.b.y, r.b.z, sf.cdc, sf.sdc);
+        vf += (float)SUB;
+        v0 += SUB;
+        int bp = visit_pixel(p.fc, sf, g);
+        float c2 = 0.f, s2 = 0.f;
+        if constexpr (F & WALK_CHI) {
+            float c4, s4;
+            visit_phase(g, r.b.w, c4, s4);
+            visit_chi(sf, c4, s4, c2, s2);
+            if constexpr (WIDE) {
+                if (wide) {   /* a wide pass has runs */
+                    const int rg = t.ring[r.run];
+                    const RingRec rr = p.rings[rg];
+                    const SampleRec &sr = ws.rec[j];
+                    visit_chi64(rec_centre(sr), sr.c2psi, sr.s2psi, ring_phi(p.hs, rr, rg, pix),
+                                rr.cdp, rr.sdp, c2, s2);
+                }
+            }
+        }
+        bp = act ? bp : -1;
+        const unsigned long long m = __ballot(bp == kNeedExact);
+        if (q.live)
+            use(q);
+        if (m)
+            enqueue(ws, qn, m, pix, j);
+        q.live = (unsigned)bp < (unsigned)p.npix_beam;   /* rejects -1 and kNeedExact */
+        q.v = v;
+        q.s = r.run;
+        q.pix = pix;
+        q.bp = bp;
+        q.c2 = c2;
+        q.s2 = s2;
+        if constexpr ((F & (WALK_SKY | WALK_BEAM)) != 0)
+            load_visit<F>(p, q, q.live ? bp : 0, q.live ? pix : 0);
+    };
+    Rec ra, rb;
+    fetch(ra, v0);
+    for (;;) {
+        step(ra, rb);
+        if (v0 >= vend || qn >= kWaveSize)
+            break;
+        step(rb, ra);
+        if (v0 >= vend || qn >= kWaveSize)
+            break;
+    }
+    if (q.live)
+        use(q);
+    at.v0 = v0;
+    at.base = base0;
+}
+
 __device__ inline int wave_max_uniform(int x)
 {
 #pragma unroll
@@ -504,252 +586,309 @@ __device__ inline int wave_max_uniform(int x)
     return __builtin_amdgcn_readfirstlane(x);
 }
 
-/* Builds the lane group's run table for its rings d.r_first + ps*SUB ..
- * + SUB-1 (clipped to its nrings rings); returns the group's visit count. */
-template <int SUB>
-__device__ inline int build_sub(const Hpx &hs, const Disc &d, int nrings, int ps, int sl,
-                                SubTable<SUB> &t)
+/* Rings r0 .. r_last of the disc of sample j of the lane group's wave state
+ * (none if r_last < r0), in passes; wave-uniform control flow: groups with
+ * fewer rings, visits or segments idle.  after(ps): called once per pass
+ * between its build and its walk; use(q) per visit inside the beam, use_exact
+ * per deferred one (see drain_queue). */
+template <int F, typename T, typename WS, typename After, typename Use, typename UseExact>
+__device__ inline void walk_rings(const PairParams &p, T &t, WS &ws, int j, int r0, int r_last,
+                                  int sl, const SampleF &sf, float eta_max, int &qn, After &after,
+                                  Use &use, UseExact &use_exact)
 {
-    const int r = d.r_first + ps * SUB + sl;
-    int p0[2] = {0, 0}, ln[2] = {0, 0};
-    int ns = 0;
-    if (ps * SUB + sl < nrings)
-        ns = disc_ring(hs, d, r, p0, ln);
-    const int tot = (ns > 0 ? ln[0] : 0) + (ns > 1 ? ln[1] : 0);
-    const int cnt_in = seg_incl_scan<SUB>(ns, sl);
-    const int tot_in = seg_incl_scan<SUB>(tot, sl);
-    const int cbase = cnt_in - ns;
-    int off = tot_in - tot;
-#pragma unroll
-    for (int k = 0; k < 2; k++) {   /* constant indices keep p0, ln in registers */
-        if (k < ns) {
-            t.pix0[cbase + k] = p0[k];
-            t.ring[cbase + k] = r;
-            t.pref[cbase + k] = off;
-            off += ln[k];
+    constexpr int SUB = T::SUB;
+    const int lane = (int)__lane_id();
+    while (SUB == kWaveSize ? r0 <= r_last : (bool)__any(r0 <= r_last)) {
+        const Pass ps = build_pass(p.hs, p.rings, rec_disc(p, ws.rec[j]), rec_centre(ws.rec[j]), r0,
+                                   r_last, sl, eta_max, t);
+        after(ps);
+        int total = ps.total, wtot;
+        if constexpr (SUB == kWaveSize) {
+            total = __builtin_amdgcn_readfirstlane(total);
+            wtot = total;
+        } else {
+            wtot = wave_max_uniform(total);
         }
+        const bool any_wide = __any(ps.wide);
+        WalkAt at;
+        for (;;) {
+            const int vend = min(wtot, at.seg0 + T::VCAP);
+            if (any_wide)
+                walk_segment<F, true>(p, t, ws, total, vend, ps.wide, sl, j, sf, at, qn, use);
+            else
+                walk_segment<F, false>(p, t, ws, total, vend, false, sl, j, sf, at, qn, use);
+            if (qn >= kWaveSize) {
+                drain_queue<F>(p, ws, qn - kWaveSize, kWaveSize, lane, use_exact);
+                qn -= kWaveSize;
+            }
+            if (at.v0 >= vend) {
+                if (vend >= wtot)
+                    break;
+                at.seg0 = vend;
+                at.base = mark_segment(t, ps.nrun, vend, sl);
+            }
+        }
+        wave_sync();
+        r0 = ps.next;
+        if constexpr (SUB == kWaveSize)
+            r0 = __builtin_amdgcn_readfirstlane(r0);
     }
-    const int nrun = __shfl(cnt_in, SUB - 1, SUB);
-    const int total = __shfl(tot_in, SUB - 1, SUB);
-    if (sl == 0)
-        t.pref[nrun] = total;
-    wave_sync();
-    return total;
 }
 
-/* Per-wave state of the forward's deferred visits in the several-samples-
- * per-wave kernels: the queue (sky pixel, ring, lane group) and, per lane
- * group, its sample's beam-centre constants and the FP64 sums of its
- * deferred visits' TOD. */
-template <int SUB>
-struct SubDefer {
-    static constexpr int G = kWaveSize / SUB;
-    int qpix[2 * kWaveSize];
-    int qring[2 * kWaveSize];
-    int qgrp[2 * kWaveSize];
-    double ra[G], psi[G], cdc[G], sdc[G], c2psi[G], s2psi[G];
-    double acc[G][2];
-};
-
-/* Maps the queued visits base .. base+cnt-1 (cnt <= 64, one per lane) with
- * the FP64-alpha form, each with its own lane group's sample, and adds their
- * TOD to that group's sums (whole wave). */
-template <int SUB, bool VT>
-__device__ inline void drain_sub(const PairParams &p, SubDefer<SUB> &q, int base, int cnt, int lane)
+/* The constants of samples i0 .. i0+cnt-1 (cnt <= NS): from p.samples, or
+ * computed, one sample per lane. */
+template <typename WS>
+__device__ inline void wave_samples(const PairParams &p, WS &ws, long i0, int cnt, float pa_off,
+                                    bool offset, int lane)
 {
-    wave_sync();
-    if (lane < cnt) {
-        const int pix = q.qpix[base + lane], r = q.qring[base + lane], g = q.qgrp[base + lane];
-        Centre c;
-        c.ra = q.ra[g];
-        c.psi = q.psi[g];
-        c.cdc = q.cdc[g];
-        c.sdc = q.sdc[g];
-        c.dec = 0.0;   /* not read by the mapping */
-        const RingRec rr = p.rings[r];
-        Pending e;
-        e.bp = beam_pixel_f64(p.hb, p.fc64, c, q.c2psi[g], q.s2psi[g],
-                              ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, e.c2, e.s2);
-        if ((unsigned)e.bp < (unsigned)p.npix_beam) {
-            const float *row = p.beam + 8 * (long)e.bp;
-            e.v0 = *(const float4 *)row;
-            e.v1 = *(const float2 *)(row + 4);
-            if constexpr (VT)
-                e.v2 = *(const float2 *)(row + 6);
-            const float4 sv = p.sky4[pix];
-            e.sI = sv.x;
-            e.sQ = sv.y;
-            e.sU = sv.z;
-            e.sV = sv.w;
-            float ta, tb;
-            visit_tod<VT>(e, ta, tb);
-            atomicAdd(&q.acc[g][0], (double)ta);
-            atomicAdd(&q.acc[g][1], (double)tb);
-        }
+    if (p.samples) {
+        constexpr int W = sizeof(SampleRec) / sizeof(int);
+        const int *src = (const int *)(p.samples + (i0 - p.s_begin));
+        for (int k = lane; k < cnt * W; k += kWaveSize)
+            ((int *)ws.rec)[k] = src[k];
+    } else if (lane < cnt) {
+        const float pa = p.pa[i0 + lane];
+        rec_make(p, p.ra[i0 + lane], p.dec[i0 + lane], offset ? pa + pa_off : pa, ws.rec[lane]);
     }
-    __builtin_amdgcn_s_waitcnt(0);   /* as in drain_exact */
     wave_sync();
 }
 
-/* The walk of one ring pass of a lane group: its `total` visits, SUB at a
- * time, for wtot (the wave's largest total) iterations' worth, with the
- * software pipelining of walk_visits (next ring record prefetched; a visit's
- * loads consumed one iteration later) and the certified FP64 mapping.  In the
- * forward (LOAD_SKY) every load of the loop is issued unconditionally and the
- * mapping takes its alpha from a float atan2; visits whose floors that
- * cannot certify go to the wave's queue (dq, qn) and are drained 64 at a
- * time.  The adjoints load the beam row of live visits only.  A lane without
- * a visit computes the first visit of its run (or, in a group with no visit,
- * pixel 0 of ring 1) and discards it.  use(q) is called once per visit whose
- * beam pixel lies inside the beam and is not deferred. */
-template <int SUB, bool LOAD_SKY, typename Use, bool VT = false>
-__device__ inline void walk_sub(const PairParams &p, const SubTable<SUB> &t, int total,
-                                int wtot, int sl, const Centre &c, double c2psi, double s2psi,
-                                Use &use, SubDefer<SUB> *dq = nullptr, int *qn = nullptr)
+using WaveTable = VisitTable<kWaveSize, kWaveSize, 4096>;
+constexpr int kWaveSamples = 8;   /* samples per wave of the forward, at most */
+
+/* Samples i0 .. i0+cnt-1 (cnt <= kWaveSamples) of one detector pair, one after
+ * the other on the whole wave; their constants are computed together, one per
+ * lane, and their deferred visits share the FP64 drains.  Forward: strip k of
+ * p.strips of each disc; the sum of a strip of a sample does not depend on the
+ * samples it shares the wave with.  Or the direct-atomic adjoints. */
+template <int OP, typename WS>
+__device__ inline void pair_samples(const PairParams &p, long i0, int cnt, int k, float pa_off,
+                                    bool offset, WaveTable &t, WS &ws, double (*dacc)[2], int lane)
 {
-    if (wtot <= 0)
+    constexpr bool FWD = OP == OP_FWD || OP == OP_FWD_V;
+    constexpr int F = WALK_CHI | (FWD || OP == OP_ADJ_MAP ? WALK_BEAM : 0) | (FWD ? WALK_SKY : 0) |
+                      (OP == OP_FWD_V ? WALK_V : 0);
+    wave_samples(p, ws, i0, cnt, pa_off, offset, lane);
+    if (FWD && lane < 2 * cnt)
+        dacc[lane >> 1][lane & 1] = 0.0;   /* sums of deferred visits */
+    wave_sync();
+    double acc_a = 0.0, acc_b = 0.0, ga = 0.0, gb = 0.0;
+    auto use = [&](const Pending &q) {
+        if constexpr (FWD) {
+            visit_tod<OP == OP_FWD_V>(q, acc_a, acc_b);
+        } else if constexpr (OP == OP_ADJ_MAP) {
+            const float A0 = q.v0.x, A1 = q.v0.y, A2 = q.v0.z;
+            const float B0 = q.v0.w, B1 = q.v1.x, B2 = q.v1.y;
+            double cc = q.c2, ss = q.s2;
+            double vI = ga * A0 + gb * B0;
+            double vQ = ga * (A1 * cc - A2 * ss) + gb * (-B1 * cc + B2 * ss);
+            double vU = ga * (A2 * cc + A1 * ss) + gb * (-B2 * cc - B1 * ss);
+            unsafeAtomicAdd(&p.gI[q.pix], vI);
+            unsafeAtomicAdd(&p.gQ[q.pix], vQ);
+            unsafeAtomicAdd(&p.gU[q.pix], vU);
+        } else {
+            double cc = q.c2, ss = q.s2;
+            double qq = p.Q[q.pix], u = p.U[q.pix], sI = p.I[q.pix];
+            double *g = p.gbeam + 8 * (long)q.bp;
+            unsafeAtomicAdd(&g[0], ga * sI);
+            unsafeAtomicAdd(&g[1], ga * (qq * cc + u * ss));
+            unsafeAtomicAdd(&g[2], ga * (-qq * ss + u * cc));
+            unsafeAtomicAdd(&g[3], gb * sI);
+            unsafeAtomicAdd(&g[4], gb * (-qq * cc - u * ss));
+            unsafeAtomicAdd(&g[5], gb * (qq * ss - u * cc));
+        }
+    };
+    auto use_exact = [&](const Pending &q, int, int, int j) {
+        if constexpr (FWD) {
+            double a = 0.0, b = 0.0;
+            visit_tod<OP == OP_FWD_V>(q, a, b);
+            atomicAdd(&dacc[j][0], a);
+            atomicAdd(&dacc[j][1], b);
+        } else {
+            use(q);   /* the adjoints take one sample per wave */
+        }
+    };
+    auto after = [](const Pass &) {};
+    int qn = 0;
+    double sum_a = 0.0, sum_b = 0.0;   /* lane j: the sums of sample j */
+    for (int j = 0; j < cnt; j++) {
+        const SampleF sf = unif(ws.rec[j].sf);
+        int r0 = __builtin_amdgcn_readfirstlane(ws.rec[j].r_first);
+        int r1 = __builtin_amdgcn_readfirstlane(ws.rec[j].r_last);
+        if constexpr (FWD) {
+            const int m = (r1 - r0 + p.strips) / p.strips;   /* rings per strip */
+            r0 += k * m;
+            r1 = min(r1, r0 + m - 1);
+        } else {
+            ga = uni(p.g_a ? (double)p.g_a[i0] : 0.0);   /* one sample */
+            gb = uni(p.g_b ? (double)p.g_b[i0] : 0.0);
+        }
+        walk_rings<F>(p, t, ws, j, r0, r1, lane, sf, FWD ? kEtaForward : kEtaAdjoint, qn, after,
+                      use, use_exact);
+        if constexpr (FWD) {
+            const double a = wave_sum(acc_a), b = wave_sum(acc_b);
+            sum_a = lane == j ? a : sum_a;
+            sum_b = lane == j ? b : sum_b;
+            acc_a = acc_b = 0.0;
+        }
+    }
+    if (qn > 0)
+        drain_queue<F>(p, ws, 0, qn, lane, use_exact);
+    if constexpr (FWD) {
+        if (lane < cnt) {
+            const long i = i0 + lane;
+            sum_a += dacc[lane][0];
+            sum_b += dacc[lane][1];
+            if (p.strips > 1) {
+                const long n = p.s_end - p.s_begin;
+                p.part[(2 * k) * n + i - p.s_begin] = sum_a;
+                p.part[(2 * k + 1) * n + i - p.s_begin] = sum_b;
+            } else {
+                if (p.tod_a)
+                    p.tod_a[i] = (float)sum_a;
+                if (p.tod_b)
+                    p.tod_b[i] = (float)sum_b;
+            }
+        }
+    }
+}
+
+/* The forward: p.group consecutive samples per wave; or, p.strips > 1, a strip
+ * of the disc of one sample, in chunks of kStripChunk samples and within a
+ * chunk by strip.  The beam rows that a strip of the sky meets are about a
+ * strip of the beam, nearly the same one for samples close in the scan, so that
+ * this part stays in the XCD's L2; with whole discs the waves gather from all
+ * of a 12 MB beam.  The samples in flight have to be close: with 2, 4 and 8
+ * samples per wave (1,024 to 4,096 in flight per XCD) the L2 hit rate fell from
+ * 0.93 to 0.83, 0.71 and 0.56; hence one sample per wave, whose constants
+ * k_samples computes. */
+constexpr int kStripChunk = 4096;
+
+template <int OP>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd(PairParams p)
+{
+    __shared__ WaveTable tables[kWavesPerBlock];
+    __shared__ WaveState<kWaveSamples> states[kWavesPerBlock];
+    __shared__ double dacc[kWavesPerBlock][kWaveSamples][2];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int lane = threadIdx.x % kWaveSize;
+    const long lb = xcd_remap(blockIdx.x, gridDim.x);
+    long i0 = p.s_begin + (lb * kWavesPerBlock + wave) * p.group;
+    int k = 0;
+    if (p.strips > 1) {
+        constexpr int MB = kStripChunk / kWavesPerBlock;
+        const long c = lb / (MB * p.strips);
+        const int rem = (int)(lb - c * (MB * p.strips));
+        k = rem / MB;
+        i0 = p.s_begin + c * kStripChunk + (rem - k * MB) * kWavesPerBlock + wave;
+    }
+    if (i0 >= p.s_end)
         return;
-    const bool any = total > 0;
-    int s = 0;
-    int v = sl;
-    if (v < total)
-        while (v >= t.pref[s + 1])
-            s++;
-    RingRec rr = p.rings[any ? t.ring[s] : 1];
-    __builtin_amdgcn_s_waitcnt(0);   /* as in walk_visits */
-    Pending q;
-    q.live = false;
-    for (int v0 = 0; v0 < wtot; v0 += SUB, v += SUB) {
-        const bool act = v < total;
-        const int r = any ? t.ring[s] : 1;
-        const int pix = any ? t.pix0[s] + (act ? v - t.pref[s] : 0) : 0;
-        const RingRec cur = rr;
-        const int vn = v + SUB;
-        if (vn < total)
-            while (vn >= t.pref[s + 1])
-                s++;
-        rr = p.rings[any ? t.ring[s] : 1];
-        float c2, s2;
-        int bp = beam_pixel_f64<LOAD_SKY>(p.hb, p.fc64, c, c2psi, s2psi,
-                                          ring_phi(p.hs, cur, r, pix), cur.cdp, cur.sdp, c2, s2);
-        bp = act ? bp : -1;
-        if constexpr (LOAD_SKY) {   /* float alpha: uncertain floors to the queue */
-            const unsigned long long m = __ballot(bp == kNeedExact);
-            if (m) {
-                if (bp == kNeedExact) {
-                    const int pos = *qn + lanes_below(m);
-                    dq->qpix[pos] = pix;
-                    dq->qring[pos] = r;
-                    dq->qgrp[pos] = (int)(__lane_id() / SUB);
-                }
-                *qn += __popcll(m);
-            }
-        }
-        if (q.live)
-            use(q);
-        if constexpr (LOAD_SKY) {
-            if (*qn >= kWaveSize) {
-                drain_sub<SUB, VT>(p, *dq, *qn - kWaveSize, kWaveSize, (int)__lane_id());
-                *qn -= kWaveSize;
-            }
-        }
-        q.live = (unsigned)bp < (unsigned)p.npix_beam;
-        q.pix = pix;
-        q.r = r;
-        q.sp = cur.startpix;
-        q.bp = bp;
-        q.c2 = c2;
-        q.s2 = s2;
-        if constexpr (LOAD_SKY) {
-            const float *row = p.beam + 8 * (long)(q.live ? bp : 0);
-            q.v0 = *(const float4 *)row;
-            q.v1 = *(const float2 *)(row + 4);
-            if constexpr (VT)
-                q.v2 = *(const float2 *)(row + 6);
-            const float4 sv = p.sky4[q.live ? pix : 0];
-            q.sI = sv.x;
-            q.sQ = sv.y;
-            q.sU = sv.z;
-            q.sV = sv.w;
-        } else if (q.live) {
-            const float *row = p.beam + 8 * (long)bp;
-            q.v0 = *(const float4 *)row;
-            q.v1 = *(const float2 *)(row + 4);
-        }
-    }
-    if (q.live)
-        use(q);
+    pair_samples<OP>(p, i0, (int)min((long)p.group, p.s_end - i0), k, 0.f, false, tables[wave],
+                     states[wave], dacc[wave], lane);
 }
 
-/* Per-lane-group sample set-up of the several-samples-per-wave kernels:
- * beam-centre constants, cos/sin 2 psi, the disc and its ring count (0 for a
- * group without a sample). */
-__device__ inline int sub_setup(const PairParams &p, long i, bool valid, Centre &c,
-                                double &c2psi, double &s2psi, Disc &d)
+/* The samples' constants, one per thread. */
+__global__ void k_samples(PairParams p)
 {
-    c = centre_make(p.ra[i], p.dec[i], p.pa[i]);
-    pl_sincos(2.0 * c.psi, &s2psi, &c2psi);
-    disc_setup(p.hs, kHalfPi - c.dec, c.ra, p.rho_max, p.cos_rmax, d);
-    return valid && d.r_last >= d.r_first ? d.r_last - d.r_first + 1 : 0;
+    const long i = p.s_begin + (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < p.s_end) {
+        SampleRec r;
+        rec_make(p, p.ra[i], p.dec[i], p.pa[i], r);
+        p.samples[i - p.s_begin] = r;
+    }
 }
+
+/* TOD = the sums of the strips, in strip order. */
+__global__ void k_strip_sum(PairParams p)
+{
+    const long n = p.s_end - p.s_begin;
+    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    for (; i < n; i += (long)gridDim.x * blockDim.x) {
+        double a = 0.0, b = 0.0;
+        for (int k = 0; k < p.strips; k++) {
+            a += p.part[(2 * k) * n + i];
+            b += p.part[(2 * k + 1) * n + i];
+        }
+        if (p.tod_a)
+            p.tod_a[p.s_begin + i] = (float)a;
+        if (p.tod_b)
+            p.tod_b[p.s_begin + i] = (float)b;
+    }
+}
+
+/* The direct-atomic adjoints, one sample per wave. */
+template <int OP>
+__global__ __launch_bounds__(kBlock) void k_pair(PairParams p)
+{
+    __shared__ WaveTable tables[kWavesPerBlock];
+    __shared__ WaveState<1> states[kWavesPerBlock];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int lane = threadIdx.x % kWaveSize;
+    const long i = p.s_begin + xcd_remap(blockIdx.x, gridDim.x) * kWavesPerBlock + wave;
+    if (i >= p.s_end)
+        return;
+    pair_samples<OP>(p, i, 1, 0, 0.f, false, tables[wave], states[wave], nullptr, lane);
+}
+
+/* ---- small-disc forward: several samples per wave -------------------------
+ *
+ * For discs of a few hundred pixels the per-sample part of k_fwd (the table
+ * build, the final reduction) runs on all 64 lanes for one sample and costs
+ * more than the visits.  Here a wave holds G = 64/SUB samples of SUB lanes
+ * each: that part runs once for the G samples, each lane group walks its own
+ * disc SUB visits at a time, and a SUB-lane reduction gives each sample's TOD.
+ * The mapping, the per-visit values and the FP64 accumulation are those of
+ * k_fwd. */
+template <int SUB>
+using SubTable = VisitTable<SUB, (SUB < 16 ? 16 : SUB), (SUB < 16 ? 512 : 64 * SUB)>;
 
 template <int SUB, bool VT = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd_sub(PairParams p)
 {
     constexpr int G = kWaveSize / SUB;
     __shared__ SubTable<SUB> tables[kWavesPerBlock * G];
-    __shared__ SubDefer<SUB> defers[kWavesPerBlock];
+    __shared__ WaveState<G> states[kWavesPerBlock];
+    __shared__ double dacc[kWavesPerBlock][G][2];   /* sums of deferred visits */
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int lane = threadIdx.x % kWaveSize;
     const int grp = lane / SUB, sl = lane % SUB;
-    SubTable<SUB> &t = tables[wave * G + grp];
-    SubDefer<SUB> &dq = defers[wave];
     const long lb = xcd_remap(blockIdx.x, gridDim.x);
     const long w0 = p.s_begin + (lb * kWavesPerBlock + wave) * G;   /* the wave's first sample */
     if (w0 >= p.s_end)
         return;   /* wave-uniform */
-    const long i = w0 + grp;
-    const bool valid = i < p.s_end;
-    Centre c;
-    double c2psi, s2psi;
-    Disc d;
-    const int nrings = sub_setup(p, valid ? i : w0, valid, c, c2psi, s2psi, d);
-    const int npass = (wave_max_uniform(nrings) + SUB - 1) / SUB;
-    if (sl == 0) {   /* the group's constants and sums of deferred visits */
-        dq.ra[grp] = c.ra;
-        dq.psi[grp] = c.psi;
-        dq.cdc[grp] = c.cdc;
-        dq.sdc[grp] = c.sdc;
-        dq.c2psi[grp] = c2psi;
-        dq.s2psi[grp] = s2psi;
-        dq.acc[grp][0] = 0.0;
-        dq.acc[grp][1] = 0.0;
-    }
-    wave_sync();
-    int qn = 0;   /* queued visits (wave-uniform) */
+    const int cnt = (int)min((long)G, p.s_end - w0);
+    WaveState<G> &ws = states[wave];
+    if (lane < 2 * G)
+        dacc[wave][lane >> 1][lane & 1] = 0.0;
+    wave_samples(p, ws, w0, cnt, 0.f, false, lane);
+    const int j = grp < cnt ? grp : 0;   /* a group without a sample idles */
+    const SampleF sf = ws.rec[j].sf;
     double acc_a = 0.0, acc_b = 0.0;
-    auto use = [&](const Pending &e) {
-        float ta, tb;
-        visit_tod<VT>(e, ta, tb);
-        acc_a += ta;
-        acc_b += tb;
+    auto use = [&](const Pending &e) { visit_tod<VT>(e, acc_a, acc_b); };
+    auto use_exact = [&](const Pending &e, int, int, int g) {
+        double a = 0.0, b = 0.0;
+        visit_tod<VT>(e, a, b);
+        atomicAdd(&dacc[wave][g][0], a);
+        atomicAdd(&dacc[wave][g][1], b);
     };
-    for (int ps = 0; ps < npass; ps++) {
-        const int total = build_sub<SUB>(p.hs, d, nrings, ps, sl, t);
-        walk_sub<SUB, true, decltype(use), VT>(p, t, total, wave_max_uniform(total), sl, c, c2psi,
-                                               s2psi, use, &dq, &qn);
-        wave_sync();
-    }
+    auto after = [](const Pass &) {};
+    constexpr int F = WALK_SKY | WALK_BEAM | WALK_CHI | (VT ? WALK_V : 0);
+    int qn = 0;
+    walk_rings<F>(p, tables[wave * G + grp], ws, j, ws.rec[j].r_first,
+                  grp < cnt ? ws.rec[j].r_last : ws.rec[j].r_first - 1, sl, sf, kEtaForward, qn,
+                  after, use, use_exact);
     if (qn > 0)
-        drain_sub<SUB, VT>(p, dq, 0, qn, lane);
+        drain_queue<F>(p, ws, 0, qn, lane, use_exact);
 #pragma unroll
     for (int m = SUB / 2; m > 0; m >>= 1) {
         acc_a += __shfl_xor(acc_a, m, SUB);
         acc_b += __shfl_xor(acc_b, m, SUB);
     }
-    if (valid && sl == 0) {
-        acc_a += dq.acc[grp][0];
-        acc_b += dq.acc[grp][1];
+    if (grp < cnt && sl == 0) {
+        const long i = w0 + grp;
+        acc_a += dacc[wave][grp][0];
+        acc_b += dacc[wave][grp][1];
         if (p.tod_a)
             p.tod_a[i] = (float)acc_a;
         if (p.tod_b)
@@ -781,11 +920,13 @@ __global__ __launch_bounds__(kBlock) void k_pair_interp(PairParams p)
     if (i >= p.s_end)
         return;
     RunTable &t = tables[wave];
-    Centre c;
-    SampleF sf;
-    SampleD sd;
+    Centre c = centre_make(p.ra[i], p.dec[i], p.pa[i]);
+    c.ra = uni(c.ra);
+    c.psi = uni(c.psi);
+    c.cdc = uni(c.cdc);
+    c.sdc = uni(c.sdc);
     Disc d;
-    sample_setup(p, i, p.pa[i], c, sf, sd, d);
+    disc_setup(p.hs, kHalfPi - uni(c.dec), c.ra, p.rho_max, p.cos_rmax, d);
     double ga = 0.0, gb = 0.0;
     if (OP != OP_FWD) {
         ga = p.g_a ? (double)p.g_a[i] : 0.0;
@@ -913,15 +1054,16 @@ __device__ inline PairParams batch_pair_params(const BatchParams &b, const Batch
     p.npix_beam = q.npix;
     p.rho_max = q.rho_max;
     p.cos_rmax = q.cos_rmax;
-    p.fc.omc_lo = b.fc.omc_lo;
-    p.fc.omc_hi = b.fc.omc_hi;
-    p.fc.marg_k = q.marg_k;
     p.fc.nside = q.nside_f;
+    p.fc.k3 = 3.0f * q.nside_f * q.nside_f;
     p.fc64.crho_big = b.fc64.crho_big;
     p.fc64.crho_small = b.fc64.crho_small;
     p.fc64.marg_k = 100.0 * 4.4e-16 * q.nside * 1.7320508075688772;
     p.beam = q.beam;
     p.beam_last = nullptr;
+    p.strips = 1;
+    p.samples = nullptr;
+    p.part = nullptr;
     /* a pointing per pair (ptg_stride > 0) is found by the pair's caller index */
     const long po = (long)(q.out < 0 ? 0 : q.out) * b.ptg_stride;
     p.ra = b.ra + po;
@@ -941,27 +1083,32 @@ __device__ inline PairParams batch_pair_params(const BatchParams &b, const Batch
     return p;
 }
 
-/* Batched form of k_pair: one wave per (pair, sample) item in the order of
- * batch_item; each item is exactly the single-pair computation with
+/* Batched form of k_fwd: one wave per (pair, kPairSamples samples) item in the
+ * order of batch_item; each item is exactly the single-pair computation with
  * pa = (float)(pa + pa_offset). */
-template <int OP>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8)))
+constexpr int kPairSamples = 4;
+
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_batch_pair(BatchParams b)
 {
-    __shared__ RunTable tables[kWavesPerBlock];
+    __shared__ WaveTable tables[kWavesPerBlock];
+    __shared__ WaveState<kPairSamples> states[kWavesPerBlock];
+    __shared__ double dacc[kWavesPerBlock][kPairSamples][2];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int lane = threadIdx.x % kWaveSize;
     const long lb = xcd_remap(blockIdx.x, gridDim.x);
     const long w = lb * kWavesPerBlock + wave;
+    const long n = b.s_end - b.s_begin;
     long k, j;
-    if (!batch_item(w, b.s_end - b.s_begin, b.npairs, k, j))
+    if (!batch_item(w, (n + kPairSamples - 1) / kPairSamples, b.npairs, k, j))
         return;
     const BatchPair &q = b.pairs[k];
     if (q.out < 0)
         return;   /* inert padding */
-    const long i = b.s_begin + j;
+    const long i0 = b.s_begin + j * kPairSamples;
     const PairParams p = batch_pair_params(b, q);
-    pair_sample<OP>(p, i, p.pa[i] + q.pa_off, tables[wave], lane);
+    pair_samples<OP_FWD>(p, i0, (int)min((long)kPairSamples, b.s_end - i0), 0, q.pa_off, true,
+                         tables[wave], states[wave], dacc[wave], lane);
 }
 
 /* ---- batched forward: many detector pairs on one pointing ----------------
@@ -981,14 +1128,13 @@ void k_batch_pair(BatchParams b)
  * evaluated exactly, their sums kept in LDS.  The pair table is padded to a
  * multiple of G with inert pairs (npix 0, never members). */
 
-/* Per-wave LDS of a group of G pairs; the queue holds < 64 entries between
- * drains and one visit adds at most G x 64. */
-template <int G>
+/* Per-wave LDS of a group of G pairs.  A queue entry is a sky pixel (below
+ * 2^30) with the pair in the group in its top two bits; the queue holds < 64
+ * entries between drains and one visit adds at most G x 64. */
+template <int G, typename T>
 struct BatchTable {
-    RunTable rt;                       /* run table (its own queue is not used) */
-    int qpix[(G + 1) * kWaveSize];     /* queue: sky pixel, ring, pair in the group */
-    int qring[(G + 1) * kWaveSize];
-    int qpair[(G + 1) * kWaveSize];
+    T vt;
+    unsigned queue[(G + 1) * kWaveSize];
     double acc[G][2];                  /* forward: exact-path sums of each pair */
     double psi[G];                     /* psi of each pair at this sample */
     float ga[G], gb[G];                /* adjoint: cotangents of each pair */
@@ -1028,27 +1174,32 @@ __device__ inline bool batch_exact_visit(const BatchParams &p, const BatchPair &
 /* Wave-uniform constants of the pairs d0 .. d0+G-1 at one sample. */
 template <int G>
 struct BatchConsts {
-    float T0[G], C2P[G], S2P[G];   /* (pi - psi) 2/pi mod 4, cos/sin 2 psi */
+    float T0[G];                   /* (pi - psi) 2/pi mod 4 */
+    float C2H[G], C2L[G], S2H[G], S2L[G];   /* cos, sin 2 psi as float pairs */
     float GA[G], GB[G];            /* adjoint cotangents */
-    float NSF[G], MK[G], CUT_IN[G], CUT_OUT[G];
+    float NSF[G], CUT_IN[G], CUT_OUT[G];
+    float lim0;
     int NPIX[G];
     const float *BEAM[G];
 };
 
-template <int G, bool ADJ>
-__device__ inline void batch_consts(const BatchParams &p, BatchTable<G> &bt, long i, int d0,
-                                    int lane, BatchConsts<G> &K)
+__device__ inline float lane_float(float x, int k)
 {
-    float t0l = 0.f, c2l = 1.f, s2l = 0.f, gal = 0.f, gbl = 0.f;
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), k));
+}
+
+template <int G, bool ADJ, typename BT>
+__device__ inline void batch_consts(const BatchParams &p, BT &bt, long i, int d0, int lane,
+                                    const Centre &c, BatchConsts<G> &K)
+{
+    float t0l = 0.f, gal = 0.f, gbl = 0.f;
+    double s2 = 0.0, c2 = 1.0;
     if (lane < G) {   /* lane k: pair d0 + k */
         const BatchPair &q = p.pairs[d0 + lane];
         const float pa_k = p.pa[i] + q.pa_off;   /* the pair's own pa */
         const double psi = -(double)pa_k;
-        double s2, c2;
         pl_sincos(2.0 * psi, &s2, &c2);
         t0l = (float)fmodulo((kPi - psi) * kInvHalfPi, 4.0);
-        c2l = (float)c2;
-        s2l = (float)s2;
         if (ADJ && q.out >= 0) {
             const long row = 2 * (long)q.out * p.nsamples;
             gal = p.g[row + i];
@@ -1060,55 +1211,64 @@ __device__ inline void batch_consts(const BatchParams &p, BatchTable<G> &bt, lon
         bt.ga[lane] = gal;
         bt.gb[lane] = gbl;
     }
+    const float c2h = (float)c2, s2h = (float)s2;
+    const float c2l = (float)(c2 - (double)c2h), s2l = (float)(s2 - (double)s2h);
+    /* an irregular centre: every visit of every pair to the exact path */
+    const bool reg = centre_regular(c.ra, c.dec);
+    K.lim0 = reg ? 0.5f - 2e-6f : -1.0f;
 #pragma unroll
     for (int k = 0; k < G; k++) {
-        K.T0[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, t0l), k));
-        K.C2P[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c2l), k));
-        K.S2P[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s2l), k));
-        K.GA[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gal), k));
-        K.GB[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gbl), k));
+        K.T0[k] = lane_float(t0l, k);
+        K.C2H[k] = lane_float(c2h, k);
+        K.C2L[k] = lane_float(c2l, k);
+        K.S2H[k] = lane_float(s2h, k);
+        K.S2L[k] = lane_float(s2l, k);
+        K.GA[k] = lane_float(gal, k);
+        K.GB[k] = lane_float(gbl, k);
         const BatchPair &q = p.pairs[d0 + k];
         K.NSF[k] = q.nside_f;
-        K.MK[k] = q.marg_k;
-        K.CUT_IN[k] = q.omc_cut * (1.0f - 4e-6f);
-        K.CUT_OUT[k] = q.omc_cut * (1.0f + 4e-6f);
+        K.CUT_IN[k] = reg ? q.omc_cut * (1.0f - 4e-6f) : -1.0f;
+        K.CUT_OUT[k] = reg ? q.omc_cut * (1.0f + 4e-6f) : INFINITY;
         K.NPIX[k] = q.npix;
         K.BEAM[k] = q.beam;
     }
     wave_sync();
 }
 
-/* A visit of the group waiting for its loads: per pair the beam row and
- * chi, and the visit's sky values / pixel. */
+/* A visit of the group waiting for its loads: per pair the beam row, and the
+ * visit's sky values, phase e^{2i(alpha+beta)} = (c4, -s4) and place. */
 template <int G>
 struct BatchPend {
     float4 q0[G];
     float2 q1[G];
-    float qc[G], qs[G];
+    float c4, s4;
     float sI, sQ, sU;
-    int pix, r, sp;
+    int pix, v, s;
     unsigned live;   /* bit k: pair k has this visit inside its beam */
 };
 
 /* The walk over the visits of the group's union disc (the disc of its first
- * pair), pipelined as walk_visits: per visit the shared float geometry, then
- * each pair's tail (membership, beam pixel, gather); consume(q) receives a
- * visit once its loads are due (after the next visit's geometry).  Queued
- * visits (uncertain membership or beam pixel) are drained 64 at a time by the
- * whole wave; exact(k, pix, r, sp, e, v0, v1) receives those inside pair k's
- * disc and beam. */
-template <int G, bool LOAD_SKY, typename Consume, typename Exact>
-__device__ inline void batch_walk(const BatchParams &p, BatchTable<G> &bt, const Disc &d, int lane,
-                                  const Centre &c, const SampleF &sf, const BatchConsts<G> &K,
-                                  int d0, Consume &consume, Exact &exact)
+ * pair; d clipped by the caller), pipelined as walk_pass: per visit the shared
+ * float geometry, then each pair's tail (membership, beam pixel, gather);
+ * consume(q) receives a visit once its loads are due (after the next visit's
+ * geometry).  Queued visits (uncertain membership or beam pixel) are drained
+ * 64 at a time by the whole wave; exact(k, pix, r, sp, e, v0, v1) receives
+ * those inside pair k's disc and beam. */
+template <int G, bool LOAD_SKY, typename BT, typename After, typename Consume, typename Exact>
+__device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, int lane,
+                                  const Centre &c, const BatchConsts<G> &K, int d0, float eta_max,
+                                  After &after, Consume &consume, Exact &exact)
 {
-    RunTable &t = bt.rt;
+    auto &t = bt.vt;
+    constexpr int VCAP = std::remove_reference<decltype(t)>::type::VCAP;
+    const float cdc = unif((float)c.cdc), sdc = unif((float)c.sdc);
     int qn = 0;
     auto drain = [&](int base, int cnt) {
         wave_sync();
         if (lane < cnt) {
-            const int pix = bt.qpix[base + lane], r = bt.qring[base + lane];
-            const int k = bt.qpair[base + lane];
+            const unsigned e_ = bt.queue[base + lane];
+            const int pix = (int)(e_ & 0x3fffffffu), k = (int)(e_ >> 30);
+            const int r = pix2ring(p.hs, pix);
             ExactVisit e;
             float4 v0;
             float2 v1;
@@ -1119,33 +1279,60 @@ __device__ inline void batch_walk(const BatchParams &p, BatchTable<G> &bt, const
         __builtin_amdgcn_s_waitcnt(0);
         wave_sync();
     };
-    for (int r0 = d.r_first; r0 <= d.r_last; r0 += kWaveSize) {
-        const int total = build_runs(p.hs, d, r0, lane, t);
+    for (int r0 = d.r_first; r0 <= d.r_last;) {
+        const Pass ps = build_pass(p.hs, p.rings, d, c, r0, d.r_last, lane, eta_max, t);
+        after(ps);
+        r0 = __builtin_amdgcn_readfirstlane(ps.next);
+        const int total = __builtin_amdgcn_readfirstlane(ps.total);
         if (total <= 0)
             continue;
-        int s = 0;
-        int v = lane;
-        if (v < total)
-            while (v >= t.pref[s + 1])
-                s++;
-        RingRec rr = p.rings[t.ring[s]];
-        __builtin_amdgcn_s_waitcnt(0);
+        const bool marked = total <= VCAP;
+        int base = 0, s = 0;
+        float4 n0, n1;
+        auto fetch = [&](int v0) {   /* as walk_pass */
+            if (marked) {
+                const unsigned lo = t.bits[v0 >> 5], hi = t.bits[(v0 >> 5) + 1];
+                s = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, base));
+                base += __popc(lo) + __popc(hi);
+            } else {
+                const int v = v0 + lane;
+                if (v < total)
+                    while (v >= t.pref[s + 1])
+                        s++;
+            }
+            n0 = t.rec[s][0];
+            n1 = t.rec[s][1];
+        };
+        fetch(0);
         BatchPend<G> q;
         q.live = 0;
         q.sI = q.sQ = q.sU = 0.f;
-        q.pix = q.r = q.sp = 0;
-        for (int v0 = 0; v0 < total; v0 += kWaveSize, v += kWaveSize) {
+        q.pix = q.v = q.s = 0;
+        float vf = (float)lane;
+        for (int v0 = 0; v0 < total; v0 += kWaveSize, vf += (float)kWaveSize) {
+            const float4 r0_ = n0, r1_ = n1;
+            const int run = s;
+            if (v0 + kWaveSize < total)
+                fetch(v0 + kWaveSize);
+            const int v = v0 + lane;
             const bool act = v < total;
-            const int pix = t.pix0[s] + (act ? v - t.pref[s] : 0);
-            const int r = t.ring[s];
-            const VisitRing g = visit_ring_f32(c, ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp);
-            const int startpix = rr.startpix;
-            const int vn = v + kWaveSize;
-            if (vn < total)
-                while (vn >= t.pref[s + 1])
-                    s++;
-            rr = p.rings[t.ring[s]];
-            const VisitGeo vg = visit_geo_f32(p.fc, sf, g);
+            const int pix = v + __float_as_int(r0_.w);
+            const VisitGeo g =
+                visit_geo(fmaf(vf - r0_.z, r0_.y, r0_.x), r1_.x, r1_.y, r1_.z, cdc, sdc);
+            float c4, s4;
+            visit_phase(g, r1_.w, c4, s4);
+            if (ps.wide) {
+                const int r = t.ring[run];
+                const RingRec rr = p.rings[r];
+                visit_chi64(c, 1.0, 0.0, ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, c4, s4);
+                s4 = -s4;
+            }
+            /* alpha in quarter turns, in [-2, 2] */
+            const float ax = fabsf(g.xa), ay = fabsf(g.ya);
+            const float a = quarter_turns(ax, ay);
+            const float m = ay > ax ? a : 1.0f - a;   /* from the y axis */
+            const float al = copysignf(1.0f - copysignf(m, g.xa), g.ya);
+            const float x3y = __builtin_amdgcn_sqrtf(3.0f * g.omc);
 
             if (q.live)
                 consume(q);
@@ -1160,35 +1347,30 @@ __device__ inline void batch_walk(const BatchParams &p, BatchTable<G> &bt, const
             q.live = 0;
 #pragma unroll
             for (int k = 0; k < G; k++) {
-                const bool in = act && vg.omc < K.CUT_IN[k];
-                const bool edge = act && !in && !(vg.omc > K.CUT_OUT[k]);
-                float c2 = 0.f, s2 = 0.f;
-                int bp = -1;
-                if (in)
-                    bp = beam_pixel_f32_det(vg, K.T0[k], K.C2P[k], K.S2P[k], K.NSF[k], K.MK[k],
-                                            c2, s2);
+                const bool in = act && g.omc < K.CUT_IN[k];
+                const bool edge = act && !in && !(g.omc > K.CUT_OUT[k]);
+                const float tt = 4.0f * __builtin_amdgcn_fractf(0.25f * (K.T0[k] - al));
+                const float tmp = K.NSF[k] * x3y;
+                int bp = cap_floors(tt, tmp, g.omc, fmaf(tmp, -kFloorMarginBatch, K.lim0));
+                bp = in ? bp : -1;
                 const bool defer = edge || bp == kNeedExact;
-                const unsigned long long m = __ballot(defer);
-                if (m) {
-                    if (defer) {
-                        const int pos = qn + lanes_below(m);
-                        bt.qpix[pos] = pix;
-                        bt.qring[pos] = r;
-                        bt.qpair[pos] = k;
-                    }
-                    qn += __popcll(m);
+                const unsigned long long md = __ballot(defer);
+                if (md) {
+                    if (defer)
+                        bt.queue[qn + lanes_below(md)] = (unsigned)pix | ((unsigned)k << 30);
+                    qn += __popcll(md);
                 }
                 const bool live = (unsigned)bp < (unsigned)K.NPIX[k];
                 q.live |= live ? (1u << k) : 0u;
-                q.qc[k] = c2;
-                q.qs[k] = s2;
                 const float *row = K.BEAM[k] + 8 * (long)(live ? bp : 0);
                 q.q0[k] = *(const float4 *)row;
                 q.q1[k] = *(const float2 *)(row + 4);
             }
+            q.c4 = c4;
+            q.s4 = s4;
             q.pix = pix;
-            q.r = r;
-            q.sp = startpix;
+            q.v = v;
+            q.s = run;
             if (LOAD_SKY) {
                 const float4 sv = p.sky4[act ? pix : 0];
                 q.sI = sv.x;
@@ -1211,18 +1393,17 @@ template <int G>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_batch_fwd(BatchParams p)
 {
-    __shared__ BatchTable<G> tabs[kWavesPerBlock];
+    using BT = BatchTable<G, VisitTable<kWaveSize, kWaveSize, 4096>>;
+    __shared__ BT tabs[kWavesPerBlock];
     /* each lane's FP64 TOD sums of the group's pairs in LDS, one slot per
      * lane (the same additions in the same order as in registers).  In
      * registers they spilled, and the spill traffic went through the vector
-     * memory path this gather-bound kernel is limited by: 49.1 -> 40.8 ms at
-     * 32 pairs of FWHM 0.2-1 deg, beam NSIDE 2048, 2.5e5 samples, even with
-     * the LDS now allowing three waves per SIMD instead of four. */
+     * memory path this gather-bound kernel is limited by. */
     __shared__ double accb_s[kWavesPerBlock][G][kWaveSize];
     __shared__ double acca_s[kWavesPerBlock][G][kWaveSize];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int lane = threadIdx.x % kWaveSize;
-    BatchTable<G> &bt = tabs[wave];
+    BT &bt = tabs[wave];
     double (*accb)[kWaveSize] = accb_s[wave];
     double (*acca)[kWaveSize] = acca_s[wave];
 
@@ -1239,11 +1420,8 @@ void k_batch_fwd(BatchParams p)
     c.dec = uni(c.dec);
     c.cdc = uni(c.cdc);
     c.sdc = uni(c.sdc);
-    SampleF sf;
-    sf.cdc = unif((float)c.cdc);
-    sf.sdc = unif((float)c.sdc);
     BatchConsts<G> K;
-    batch_consts<G, false>(p, bt, i, d0, lane, K);
+    batch_consts<G, false>(p, bt, i, d0, lane, c, K);
     Disc d;
     disc_setup(p.hs, kHalfPi - c.dec, c.ra, p.pairs[d0].rho_max, p.pairs[d0].cos_rmax, d);
 
@@ -1252,16 +1430,22 @@ void k_batch_fwd(BatchParams p)
         acca[k][lane] = 0.0;
         accb[k][lane] = 0.0;
     }
+    /* as visit_tod, the sky turned by the visit's phase once for the group
+     * and by each pair's 2 psi */
     auto consume = [&](const BatchPend<G> &q) {
+        const float Qr = fmaf(q.sQ, q.c4, -(q.sU * q.s4)), Ur = fmaf(q.sU, q.c4, q.sQ * q.s4);
+        const double I = q.sI;
 #pragma unroll
         for (int k = 0; k < G; k++) {
             if (q.live & (1u << k)) {
-                const float A0 = q.q0[k].x, A1 = q.q0[k].y, A2 = q.q0[k].z, B0 = q.q0[k].w;
-                const float B1 = q.q1[k].x, B2 = q.q1[k].y, cc = q.qc[k], ss = q.qs[k];
-                const float ta = q.sI * A0 + q.sQ * (A1 * cc - A2 * ss) + q.sU * (A2 * cc + A1 * ss);
-                acca[k][lane] = acca[k][lane] + (double)ta;
-                const float tb = q.sI * B0 + q.sQ * (-B1 * cc + B2 * ss) + q.sU * (-B2 * cc - B1 * ss);
-                accb[k][lane] = accb[k][lane] + (double)tb;
+                const float X = fmaf(Qr, K.C2H[k],
+                                     fmaf(Ur, K.S2H[k], fmaf(Qr, K.C2L[k], Ur * K.S2L[k])));
+                const float Y = fmaf(Ur, K.C2H[k],
+                                     fmaf(-Qr, K.S2H[k], fmaf(Ur, K.C2L[k], -(Qr * K.S2L[k]))));
+                const float ta = fmaf(q.q0[k].z, Y, q.q0[k].y * X);
+                const float tb = fmaf(q.q1[k].y, Y, q.q1[k].x * X);
+                acca[k][lane] = fma(I, (double)q.q0[k].x, acca[k][lane]) + (double)ta;
+                accb[k][lane] = fma(I, (double)q.q0[k].w, accb[k][lane]) - (double)tb;
             }
         }
     };
@@ -1270,15 +1454,21 @@ void k_batch_fwd(BatchParams p)
         (void)r;
         (void)sp;
         const float4 sv = p.sky4[pix];
-        const float sI = sv.x, sQ = sv.y, sU = sv.z;
-        const float ta =
-            sI * v0.x + sQ * (v0.y * e.c2 - v0.z * e.s2) + sU * (v0.z * e.c2 + v0.y * e.s2);
-        const float tb =
-            sI * v0.w + sQ * (-v1.x * e.c2 + v1.y * e.s2) + sU * (-v1.y * e.c2 - v1.x * e.s2);
-        atomicAdd(&bt.acc[k][0], (double)ta);
-        atomicAdd(&bt.acc[k][1], (double)tb);
+        Pending q;
+        q.sI = sv.x;
+        q.sQ = sv.y;
+        q.sU = sv.z;
+        q.c2 = e.c2;
+        q.s2 = e.s2;
+        q.v0 = v0;
+        q.v1 = v1;
+        double ta = 0.0, tb = 0.0;
+        visit_tod<false>(q, ta, tb);
+        atomicAdd(&bt.acc[k][0], ta);
+        atomicAdd(&bt.acc[k][1], tb);
     };
-    batch_walk<G, true>(p, bt, d, lane, c, sf, K, d0, consume, exact);
+    auto after = [](const Pass &) {};
+    batch_walk<G, true>(p, bt, d, lane, c, K, d0, kEtaForward, after, consume, exact);
     wave_sync();
 #pragma unroll
     for (int k = 0; k < G; k++) {
@@ -1308,7 +1498,11 @@ struct AdjLayout {
     int chunk;       /* samples per chunk */
     int cap;         /* LDS pixel capacity of the window */
     int rw;          /* ring capacity of the window tables */
+    int group;       /* samples per wave at a time, one wave per sample (at most kAdjSamples) */
     long nchunks;
+    /* strips of rings that a chunk's discs are cut into (p.strips), taken in
+     * groups of strip_group chunks and within a group by strip */
+    int strips, strip_group;
     /* batch mode (pairs != NULL): every pair of b.pairs adds into the same
      * windows; the windows use radius rho_w (the pairs' union support) */
     const BatchPair *pairs;
@@ -1321,21 +1515,26 @@ struct AdjLayout {
     const double *fx_scale;
 };
 
-#ifndef PISCO_ADJ_WAVES
-#define PISCO_ADJ_WAVES 16
-#endif
-constexpr int kAdjWaves = PISCO_ADJ_WAVES;   /* waves per block of the sky adjoint */
+__host__ __device__ inline long adj_items(const AdjLayout &L)
+{
+    return (L.nchunks + L.strip_group - 1) / L.strip_group * L.strip_group * L.strips;
+}
+
 constexpr int kAdjBlock = kAdjWaves * kWaveSize;
+/* The beam adjoint's band kernels: one block per CU. */
+constexpr int kBandWaves = 16;
+constexpr int kBandBlock = kBandWaves * kWaveSize;
 
 /* rint(v * s) as a two's-complement 64-bit integer, for |v * s| < 2^51 and s
  * a power of two (v * s is then exact): adding 1.5 * 2^52 rounds it to the
  * nearest integer, ties to even as rint does (1.5 * 2^52 is even), and
  * leaves that integer in the low bits of the sum's mantissa, whose exponent
- * is fixed.  Two instructions instead of rint and a 64-bit conversion. */
+ * is fixed (its low word is zero, so the subtraction is one of the high
+ * words).  Two instructions instead of rint and a 64-bit conversion. */
 __device__ inline unsigned long long fix64(float v, double s)
 {
-    const double t = fma((double)v, s, 0x1.8p52);
-    return (unsigned long long)__double_as_longlong(t) - 0x4338000000000000ull;
+    const unsigned long long t = (unsigned long long)__double_as_longlong(fma((double)v, s, 0x1.8p52));
+    return (unsigned long long)((unsigned)(t >> 32) - 0x43380000u) << 32 | (unsigned)t;
 }
 constexpr int kBigI = 0x3fffffff;
 /* A chunk whose window exceeds the LDS capacity is split into at most this
@@ -1343,30 +1542,51 @@ constexpr int kBigI = 0x3fffffff;
 constexpr int kMaxSlabs = 63;
 constexpr int kAdjCtl = 4 + kMaxSlabs + 1;   /* ints of the control block */
 
-/* I,Q,U gradient of one visit, in float: the values are accumulated in float
- * LDS windows, so FP64 products would be rounded away there anyway. */
+/* I,Q,U gradient of one visit, in float: each is rounded to the windows'
+ * resolution (or accumulated in float) anyway.  The polarised part is
+ * (P + iR) e^{2i chi} with P + iR = ga (A1 + iA2) - gb (B1 + iB2). */
 __device__ inline void adj_visit_values(float ga, float gb, float4 v0, float2 v1, float c2,
                                         float s2, float &vI, float &vQ, float &vU)
 {
-    float A0 = v0.x, A1 = v0.y, A2 = v0.z, B0 = v0.w, B1 = v1.x, B2 = v1.y;
-    vI = ga * A0 + gb * B0;
-    vQ = ga * (A1 * c2 - A2 * s2) + gb * (-B1 * c2 + B2 * s2);
-    vU = ga * (A2 * c2 + A1 * s2) + gb * (-B2 * c2 - B1 * s2);
+    vI = fmaf(gb, v0.w, ga * v0.x);
+    const float P = fmaf(-gb, v1.x, ga * v0.y), R = fmaf(-gb, v1.y, ga * v0.z);
+    vQ = fmaf(P, c2, -(R * s2));
+    vU = fmaf(R, c2, P * s2);
 }
 
-/* Per-wave LDS table of the sky adjoint: a run table, or the batch table of
- * a group of BG >= 2 pairs. */
-template <int BG>
-struct AdjWaveTable {
-    using type = BatchTable<BG>;
+/* Where a run's visits lie in the chunk's LDS window: visit v is entry v + x
+ * of the window of its ring, which has (y >> 16) entries and starts at slot
+ * y & 0xffff (the slab's capacity and a ring's pixels are below 2^16). */
+template <typename T>
+struct WindowTable : T {
+    int2 win[T::RPP];
+};
+
+/* Samples that a wave of the sky adjoint takes one after the other. */
+constexpr int kAdjSamples = 2;
+
+/* Per-wave LDS of the sky adjoint. */
+template <int BG, int SUB>
+struct AdjWave {   /* BG >= 2: a group of BG pairs */
+    using VT = WindowTable<VisitTable<kWaveSize, 32, 3072>>;
+    BatchTable<BG, VT> bt;
+};
+template <int SUB>
+struct AdjWave<0, SUB> {   /* several samples per wave */
+    using VT = WindowTable<VisitTable<SUB, SUB, 32 * SUB>>;
+    VT vt[kWaveSize / SUB];
+    WaveState<kWaveSize / SUB> ws;
+    float g[kWaveSize / SUB][2];   /* cotangents */
 };
 template <>
-struct AdjWaveTable<0> {
-    using type = RunTable;
+struct AdjWave<0, kWaveSize> {
+    using VT = WindowTable<VisitTable<kWaveSize, 40, 1536>>;
+    VT vt;
+    WaveState<kAdjSamples> ws;
+    float g[kAdjSamples][2];
 };
 template <>
-struct AdjWaveTable<1> {
-    using type = RunTable;
+struct AdjWave<1, kWaveSize> : AdjWave<0, kWaveSize> {
 };
 
 /* BG: 0 one pair; 1 a batch, one wave per (pair, sample); 2, 4 a batch, one
@@ -1377,13 +1597,11 @@ struct AdjWaveTable<1> {
  * depend on the order of the additions; the result is the same bits for any
  * schedule and launch shape (for a given grouping of the pairs). */
 template <int BG, bool DET = false, int SUB = kWaveSize>
-__global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayout L)
+__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_adjmap_lds(PairParams p, AdjLayout L)
 {
-    static_assert(SUB == kWaveSize || (BG == 0 && sizeof(SubTable<SUB>) * (kWaveSize / SUB) <=
-                                                      sizeof(RunTable)),
-                  "several samples per wave: single pair, tables within the run table");
+    static_assert(SUB == kWaveSize || BG == 0, "several samples per wave: single pair");
     constexpr bool BATCH = BG > 0;
-    using WT = typename AdjWaveTable<BG>::type;
+    using WT = AdjWave<BG, SUB>;
     extern __shared__ __align__(16) unsigned char smem[];
     WT *wtab = (WT *)smem;
     int *win_lo = (int *)(wtab + kAdjWaves);
@@ -1404,7 +1622,6 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayou
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWaveSize);
     const int lane = tid % kWaveSize;
-    RunTable &t = *(RunTable *)&wtab[wave];   /* the first member of either table */
 
     /* Window radius.  A visit adds a non-zero value only if its beam pixel
      * is at or before row `last`, i.e. lies in a beam ring <= R of that row.
@@ -1431,7 +1648,13 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayou
     }
 
     long lb = xcd_remap(blockIdx.x, gridDim.x);
-    for (long ch = lb; ch < L.nchunks; ch += gridDim.x) {
+    const long nitems = adj_items(L);
+    for (long item = lb; item < nitems; item += gridDim.x) {
+        const long per = (long)L.strip_group * L.strips, cg = item / per;
+        const int rem = (int)(item - cg * per), strip = rem / L.strip_group;
+        const long ch = cg * L.strip_group + (rem - strip * L.strip_group);
+        if (ch >= L.nchunks)
+            continue;
         long s0 = p.s_begin + ch * L.chunk;
         long s1 = s0 + L.chunk < p.s_end ? s0 + L.chunk : p.s_end;
         int ns = (int)(s1 - s0);
@@ -1452,8 +1675,29 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayou
             }
         }
         __syncthreads();
-        const int R0 = __builtin_amdgcn_readfirstlane(ctl[0]);
-        const int nring = __builtin_amdgcn_readfirstlane(ctl[1]) - R0 + 1;
+        int R0 = __builtin_amdgcn_readfirstlane(ctl[0]);
+        int nring = __builtin_amdgcn_readfirstlane(ctl[1]) - R0 + 1;
+        /* this strip of the window rings; the first strip also takes the disc
+         * rings before them and the last one those after */
+        const int per_strip = (nring + L.strips - 1) / L.strips;
+        int first = -kBigI, last = kBigI;
+        if (L.strips > 1) {
+            if (nring <= 0) {
+                if (strip > 0)
+                    continue;
+            } else {
+                const int a = R0 + min(strip * per_strip, nring);
+                const int b = R0 + min((strip + 1) * per_strip, nring);   /* one past */
+                if (strip > 0)
+                    first = a;
+                if (strip < L.strips - 1)
+                    last = b - 1;
+                R0 = a;
+                nring = b - a;
+                if (first > last)
+                    continue;
+            }
+        }
         /* no window ring (a disc of radius rho_w can miss every ring centre
          * while the rho_max discs still have visits) or too many: global
          * atomics for this chunk */
@@ -1478,8 +1722,8 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayou
                                        0.f);
                 Disc d;
                 disc_setup(p.hs, kHalfPi - c.dec, c.ra, rho_w, cos_w, d);
-                const int r_end = j < ns ? d.r_last : d.r_first - 1;
-                for (int r = d.r_first + lane % SUB; r <= r_end; r += SUB) {
+                const int r_end = j < ns ? min(d.r_last, R0 + nring - 1) : -1;
+                for (int r = max(d.r_first, R0) + lane % SUB; r <= r_end; r += SUB) {
                     int lo, hi, ipix1, nr;
                     int kind = disc_ring_span(p.hs, d, r, lo, hi, ipix1, nr);
                     if (kind == 0)
@@ -1571,8 +1815,8 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayou
         const int base0 = fallback ? 0 : __builtin_amdgcn_readfirstlane(win_base[k0]);
         const int Ws = fallback ? 0 : __builtin_amdgcn_readfirstlane(win_base[k1]) - base0;
         const bool sfall = fallback || Ws > L.cap;
-        const int rlo = (fallback || si == 0) ? -kBigI : R0 + k0;
-        const int rhi = (fallback || si == nslab - 1) ? kBigI : R0 + k1 - 1;
+        const int rlo = (fallback || si == 0) ? first : R0 + k0;
+        const int rhi = (fallback || si == nslab - 1) ? last : R0 + k1 - 1;
         auto clamp = [&](Disc &d) {
             d.r_first = d.r_first > rlo ? d.r_first : rlo;
             d.r_last = d.r_last < rhi ? d.r_last : rhi;
@@ -1590,20 +1834,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayou
         /* pass 2: visits; adds I,Q,U of one visit to the LDS window (or, when no
          * window holds the pixel, to the global FP64 gradient) */
         const int W = sfall ? 0 : Ws;
-        auto scatter = [&](int pix, int r, int sp, float vI, float vQ, float vU) {
-            if (vI == 0.f && vQ == 0.f && vU == 0.f)
-                return;   /* adds nothing */
-            const int k = r - R0;
-            int slot = -1;
-            if (!sfall && k >= k0 && k < k1) {
-                int nr = 4 * (r < p.hs.nside ? r
-                              : (r > 3 * p.hs.nside ? 4 * p.hs.nside - r : p.hs.nside));
-                int off = pix - sp - win_lo[k];
-                if (off < 0)
-                    off += nr;
-                if (off < win_hi[k])   /* inside the ring's window */
-                    slot = win_base[k] - base0 + off;
-            }
+        auto add = [&](int slot, int pix, float vI, float vQ, float vU) {
             if constexpr (DET) {
                 const unsigned long long fI = fix64(vI, fxs);
                 const unsigned long long fQ = fix64(vQ, fxs);
@@ -1627,9 +1858,56 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayou
                 unsafeAtomicAdd(&p.gU[pix], (double)vU);
             }
         };
+        /* the windows of a pass's runs (`n` lanes of a lane group fill them).
+         * A ring's window may hold a second copy of the run's positions, nr
+         * pixels away; visits there (a run nearly a ring long) take the
+         * global atomics. */
+        auto fill_windows = [&](auto &vt, const Pass &ps, int l, int n) {
+            for (int i = l; i < ps.nrun; i += n) {
+                const int r = vt.ring[i], k = r - R0;
+                int2 w = make_int2(0, 0);
+                if (!sfall && k >= k0 && k < k1) {
+                    int sp, nr;
+                    bool shf;
+                    ring_info(p.hs, r, sp, nr, shf);
+                    const int off = vt.pref[i];
+                    const int j0 = __float_as_int(vt.rec[i][0].w) + off - sp;
+                    const int len = win_hi[k];
+                    int lo = win_lo[k];
+                    const int dm = j0 + (vt.pref[i + 1] - off) / 2 - (lo + len / 2);
+                    lo += dm > nr / 2 ? nr : (dm < -(nr / 2) ? -nr : 0);
+                    w = make_int2(j0 - off - lo, (len << 16) | (win_base[k] - base0));
+                }
+                vt.win[i] = w;
+            }
+            wave_sync();
+        };
+        /* a visit of the walk, through its run's window */
+        auto scatter = [&](const int2 w, int v, int pix, float vI, float vQ, float vU) {
+            const int off = v + w.x;
+            const int slot = (unsigned)off < (unsigned)w.y >> 16 ? (w.y & 0xffff) + off : -1;
+            add(slot, pix, vI, vQ, vU);
+        };
+        /* a deferred visit, by its pixel and ring */
+        auto scatter_pix = [&](int pix, int r, int sp, float vI, float vQ, float vU) {
+            if (vI == 0.f && vQ == 0.f && vU == 0.f)
+                return;   /* adds nothing */
+            const int k = r - R0;
+            int slot = -1;
+            if (!sfall && k >= k0 && k < k1) {
+                int nr = 4 * (r < p.hs.nside ? r
+                              : (r > 3 * p.hs.nside ? 4 * p.hs.nside - r : p.hs.nside));
+                int off = pix - sp - win_lo[k];
+                if (off < 0)
+                    off += nr;
+                if (off < win_hi[k])   /* inside the ring's window */
+                    slot = win_base[k] - base0 + off;
+            }
+            add(slot, pix, vI, vQ, vU);
+        };
         if constexpr (BG >= 2) {
             /* one wave per (group, sample), groups outermost */
-            BatchTable<BG> &bt = wtab[wave];
+            auto &bt = wtab[wave].bt;
             const int ngr = L.npairs / BG;
             for (int j = wave; j < ns * ngr; j += kAdjWaves) {
                 const int jg = j / ns;
@@ -1640,108 +1918,138 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjmap_lds(PairParams p, AdjLayou
                 c.dec = uni(c.dec);
                 c.cdc = uni(c.cdc);
                 c.sdc = uni(c.sdc);
-                SampleF sf;
-                sf.cdc = unif((float)c.cdc);
-                sf.sdc = unif((float)c.sdc);
                 BatchConsts<BG> K;
-                batch_consts<BG, true>(L.b, bt, i, d0, lane, K);
+                batch_consts<BG, true>(L.b, bt, i, d0, lane, c, K);
                 Disc d;
                 disc_setup(p.hs, kHalfPi - c.dec, c.ra, L.pairs[d0].rho_max,
                            L.pairs[d0].cos_rmax, d);
                 clamp(d);
+                /* the pairs' gradients are summed in the frame turned by the
+                 * visit's phase, which is undone once */
                 auto consume = [&](const BatchPend<BG> &q) {
-                    float vI = 0.f, vQ = 0.f, vU = 0.f;
+                    float vI = 0.f, zr = 0.f, zi = 0.f;
 #pragma unroll
                     for (int k = 0; k < BG; k++) {
                         if (q.live & (1u << k)) {
-                            float dI, dQ, dU;
-                            adj_visit_values(K.GA[k], K.GB[k], q.q0[k], q.q1[k], q.qc[k],
-                                             q.qs[k], dI, dQ, dU);
-                            vI += dI;
-                            vQ += dQ;
-                            vU += dU;
+                            const float4 v0 = q.q0[k];
+                            const float2 v1 = q.q1[k];
+                            const float ga = K.GA[k], gb = K.GB[k];
+                            vI = fmaf(gb, v0.w, fmaf(ga, v0.x, vI));
+                            const float P = fmaf(-gb, v1.x, ga * v0.y);
+                            const float R = fmaf(-gb, v1.y, ga * v0.z);
+                            zr = fmaf(P, K.C2H[k], fmaf(-R, K.S2H[k], zr));
+                            zi = fmaf(R, K.C2H[k], fmaf(P, K.S2H[k], zi));
                         }
                     }
-                    scatter(q.pix, q.r, q.sp, vI, vQ, vU);
+                    if (vI != 0.f || zr != 0.f || zi != 0.f)
+                        scatter(bt.vt.win[q.s], q.v, q.pix, vI, fmaf(zr, q.c4, zi * q.s4),
+                                fmaf(zi, q.c4, -(zr * q.s4)));
                 };
                 auto exact = [&](int k, int pix, int r, int sp, const ExactVisit &e,
                                  const float4 &v0, const float2 &v1) {
                     float vI, vQ, vU;
                     adj_visit_values(bt.ga[k], bt.gb[k], v0, v1, e.c2, e.s2, vI, vQ, vU);
-                    scatter(pix, r, sp, vI, vQ, vU);
+                    scatter_pix(pix, r, sp, vI, vQ, vU);
                 };
-                batch_walk<BG, false>(L.b, bt, d, lane, c, sf, K, d0, consume, exact);
+                auto after = [&](const Pass &ps) { fill_windows(bt.vt, ps, lane, kWaveSize); };
+                batch_walk<BG, false>(L.b, bt, d, lane, c, K, d0, kEtaAdjoint, after, consume,
+                                      exact);
             }
         } else if constexpr (SUB < kWaveSize) {
             /* single pair, small discs: 64/SUB samples per wave, SUB lanes
-             * each, with the FP64 mapping (as k_fwd_sub) */
+             * each (as k_fwd_sub) */
             constexpr int G = kWaveSize / SUB;
             const int grp = lane / SUB, sl = lane % SUB;
-            SubTable<SUB> &tg = ((SubTable<SUB> *)&wtab[wave])[grp];
+            auto &tg = wtab[wave].vt[grp];
+            auto &ws = wtab[wave].ws;
             for (int j0 = wave * G; j0 < ns; j0 += kAdjWaves * G) {
-                const int j = j0 + grp;
-                const bool valid = j < ns;
-                const long i = s0 + (valid ? j : j0);
-                Centre c;
-                double c2psi, s2psi;
-                Disc d;
-                int nrings = sub_setup(p, i, valid, c, c2psi, s2psi, d);
-                clamp(d);
-                nrings = nrings > 0 && d.r_last >= d.r_first ? d.r_last - d.r_first + 1 : 0;
-                const float ga = (valid && p.g_a) ? p.g_a[i] : 0.f;
-                const float gb = (valid && p.g_b) ? p.g_b[i] : 0.f;
+                const int cnt = min(G, ns - j0);
+                const long i0 = s0 + j0;
+                wave_samples(p, ws, i0, cnt, 0.f, false, lane);
+                const int j = grp < cnt ? grp : 0;
+                const SampleF sf = ws.rec[j].sf;
+                const float ga = p.g_a ? p.g_a[i0 + j] : 0.f;
+                const float gb = p.g_b ? p.g_b[i0 + j] : 0.f;
+                if (sl == 0) {
+                    wtab[wave].g[grp][0] = ga;
+                    wtab[wave].g[grp][1] = gb;
+                }
                 auto use = [&](const Pending &q) {
                     float vI, vQ, vU;
                     adj_visit_values(ga, gb, q.v0, q.v1, q.c2, q.s2, vI, vQ, vU);
-                    scatter(q.pix, q.r, q.sp, vI, vQ, vU);
+                    if (vI != 0.f || vQ != 0.f || vU != 0.f)
+                        scatter(tg.win[q.s], q.v, q.pix, vI, vQ, vU);
                 };
-                const int npass = (wave_max_uniform(nrings) + SUB - 1) / SUB;
-                for (int ps = 0; ps < npass; ps++) {
-                    const int total = build_sub<SUB>(p.hs, d, nrings, ps, sl, tg);
-                    walk_sub<SUB, false>(p, tg, total, wave_max_uniform(total), sl, c, c2psi,
-                                         s2psi, use);
-                    wave_sync();
-                }
+                auto use_exact = [&](const Pending &q, int r, int sp, int g) {
+                    float vI, vQ, vU;
+                    adj_visit_values(wtab[wave].g[g][0], wtab[wave].g[g][1], q.v0, q.v1, q.c2,
+                                     q.s2, vI, vQ, vU);
+                    scatter_pix(q.pix, r, sp, vI, vQ, vU);
+                };
+                auto after = [&](const Pass &ps) { fill_windows(tg, ps, sl, SUB); };
+                const int r0 = max(ws.rec[j].r_first, rlo);
+                const int r1 = grp < cnt ? min(ws.rec[j].r_last, rhi) : r0 - 1;
+                int qn = 0;
+                constexpr int F = WALK_BEAM | WALK_CHI;
+                walk_rings<F>(p, tg, ws, j, r0, r1, sl, sf, kEtaAdjoint, qn, after, use, use_exact);
+                if (qn > 0)
+                    drain_queue<F>(p, ws, 0, qn, lane, use_exact);
+                wave_sync();   /* the next samples' constants replace these */
             }
         } else {
-        /* one wave per (pair, sample), pairs outermost */
+        /* one wave per (pair, kAdjSamples samples), pairs outermost */
+        auto &t = wtab[wave].vt;
+        auto &ws = wtab[wave].ws;
         const int np = BATCH ? L.npairs : 1;
-        for (int j = wave; j < ns * np; j += kAdjWaves) {
-            const int jp = j / ns;
-            const long i = s0 + (j - jp * ns);
-            float pa_i;
+        const int nq = (ns + L.group - 1) / L.group;
+        for (int jq = wave; jq < nq * np; jq += kAdjWaves) {
+            const int jp = jq / nq;
+            const int j0 = (jq - jp * nq) * L.group, cnt = min(L.group, ns - j0);
+            const long i0 = s0 + j0;
             PairParams pp;
             if constexpr (BATCH) {
                 const BatchPair &q = L.pairs[jp];
                 if (q.out < 0)
                     continue;   /* inert padding (uniform per wave) */
                 pp = batch_pair_params(L.b, q);
-                pa_i = pp.pa[i] + q.pa_off;
+                wave_samples(pp, ws, i0, cnt, q.pa_off, true, lane);
             } else {
                 pp = p;
-                pa_i = p.pa[i];
+                wave_samples(p, ws, i0, cnt, 0.f, false, lane);
             }
-            Centre c;
-            SampleF sf;
-            SampleD sd;
-            Disc d;
-            sample_setup(pp, i, pa_i, c, sf, sd, d);
-            clamp(d);
-            const float ga = unif(pp.g_a ? pp.g_a[i] : 0.f);
-            const float gb = unif(pp.g_b ? pp.g_b[i] : 0.f);
+            if (lane < cnt) {
+                wtab[wave].g[lane][0] = pp.g_a ? pp.g_a[i0 + lane] : 0.f;
+                wtab[wave].g[lane][1] = pp.g_b ? pp.g_b[i0 + lane] : 0.f;
+            }
+            wave_sync();
+            float ga = 0.f, gb = 0.f;
             auto use = [&](const Pending &q) {
                 float vI, vQ, vU;
                 adj_visit_values(ga, gb, q.v0, q.v1, q.c2, q.s2, vI, vQ, vU);
-                scatter(q.pix, q.r, q.sp, vI, vQ, vU);
+                if (vI != 0.f || vQ != 0.f || vU != 0.f)
+                    scatter(t.win[q.s], q.v, q.pix, vI, vQ, vU);
             };
+            auto use_exact = [&](const Pending &q, int r, int sp, int g) {
+                float vI, vQ, vU;
+                adj_visit_values(wtab[wave].g[g][0], wtab[wave].g[g][1], q.v0, q.v1, q.c2, q.s2, vI,
+                                 vQ, vU);
+                scatter_pix(q.pix, r, sp, vI, vQ, vU);
+            };
+            auto after = [&](const Pass &ps) { fill_windows(t, ps, lane, kWaveSize); };
             int qn = 0;
-            for (int r0 = d.r_first; r0 <= d.r_last; r0 += kWaveSize) {
-                int total = build_runs(pp.hs, d, r0, lane, t);
-                walk_visits<false, false>(pp, t, total, lane, c, sf, sd, qn, use);
-                wave_sync();
+            constexpr int F = WALK_BEAM | WALK_CHI;
+            for (int j = 0; j < cnt; j++) {
+                const SampleF sf = unif(ws.rec[j].sf);
+                ga = unif(wtab[wave].g[j][0]);
+                gb = unif(wtab[wave].g[j][1]);
+                const int r0 = max(__builtin_amdgcn_readfirstlane(ws.rec[j].r_first), rlo);
+                const int r1 = min(__builtin_amdgcn_readfirstlane(ws.rec[j].r_last), rhi);
+                walk_rings<F>(pp, t, ws, j, r0, r1, lane, sf, kEtaAdjoint, qn, after, use,
+                              use_exact);
             }
             if (qn > 0)
-                drain_exact<false>(pp, t, 0, qn, lane, c, sd.c2psi, sd.s2psi, use);
+                drain_queue<F>(pp, ws, 0, qn, lane, use_exact);
+            wave_sync();   /* the next samples' constants replace these */
         }
         }
         __syncthreads();
@@ -2006,14 +2314,14 @@ __device__ inline void walk_band_sub(const PairParams &p, const SubBandTable<SUB
 }
 
 template <int SUB>
-__global__ __launch_bounds__(kAdjBlock) void k_adjbeam_band_sub(PairParams p, BeamBands B)
+__global__ __launch_bounds__(kBandBlock) void k_adjbeam_band_sub(PairParams p, BeamBands B)
 {
     constexpr int G = kWaveSize / SUB;
     static_assert(sizeof(SubBandTable<SUB>) * G <= sizeof(BandRunTable),
                   "lane-group tables within the wave's run table");
     extern __shared__ __align__(16) unsigned char smem[];
     BandRunTable *tabs = (BandRunTable *)smem;
-    float *acc = (float *)(tabs + kAdjWaves);
+    float *acc = (float *)(tabs + kBandWaves);
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWaveSize);
     const int lane = tid % kWaveSize;
@@ -2028,12 +2336,12 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjbeam_band_sub(PairParams p, Be
         bool inner;
         double r_in, c_in, r_out, c_out;
         band_annulus_radii(p.hb, p.rho_max, p.cos_rmax, lo, nrow, inner, r_in, c_in, r_out, c_out);
-        for (int i = tid; i < 6 * nrow; i += kAdjBlock)
+        for (int i = tid; i < 6 * nrow; i += kBandBlock)
             acc[i] = 0.f;
         __syncthreads();
         const long s0 = p.s_begin + ch * B.chunk;
         const long s1 = s0 + B.chunk < p.s_end ? s0 + B.chunk : p.s_end;
-        for (long j0 = s0 + (long)wave * G; j0 < s1; j0 += (long)kAdjWaves * G) {
+        for (long j0 = s0 + (long)wave * G; j0 < s1; j0 += (long)kBandWaves * G) {
             const long i = j0 + grp;
             const bool valid = i < s1;
             const long iv = valid ? i : j0;
@@ -2071,7 +2379,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjbeam_band_sub(PairParams p, Be
             }
         }
         __syncthreads();
-        for (int rr = tid; rr < nrow; rr += kAdjBlock) {
+        for (int rr = tid; rr < nrow; rr += kBandBlock) {
             const float *a = acc + 6 * rr;
             double *g = p.gbeam + 8 * (long)(lo + rr);
 #pragma unroll
@@ -2083,11 +2391,11 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjbeam_band_sub(PairParams p, Be
     }
 }
 
-__global__ __launch_bounds__(kAdjBlock) void k_adjbeam_band(PairParams p, BeamBands B)
+__global__ __launch_bounds__(kBandBlock) void k_adjbeam_band(PairParams p, BeamBands B)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     BandRunTable *tabs = (BandRunTable *)smem;
-    float *acc = (float *)(tabs + kAdjWaves);
+    float *acc = (float *)(tabs + kBandWaves);
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWaveSize);
     const int lane = tid % kWaveSize;
@@ -2104,12 +2412,12 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjbeam_band(PairParams p, BeamBa
         double r_in, c_in, r_out, c_out;
         band_annulus_radii(p.hb, p.rho_max, p.cos_rmax, lo, nrow, inner, r_in, c_in, r_out,
                            c_out);
-        for (int i = tid; i < 6 * nrow; i += kAdjBlock)
+        for (int i = tid; i < 6 * nrow; i += kBandBlock)
             acc[i] = 0.f;
         __syncthreads();
         const long s0 = p.s_begin + ch * B.chunk;
         const long s1 = s0 + B.chunk < p.s_end ? s0 + B.chunk : p.s_end;
-        for (long i = s0 + wave; i < s1; i += kAdjWaves) {
+        for (long i = s0 + wave; i < s1; i += kBandWaves) {
             const float ga = unif(p.g_a ? p.g_a[i] : 0.f);
             const float gb = unif(p.g_b ? p.g_b[i] : 0.f);
             if (ga == 0.f && gb == 0.f)
@@ -2149,7 +2457,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjbeam_band(PairParams p, BeamBa
         }
         __syncthreads();
         /* add the band to the FP64 gradient */
-        for (int rr = tid; rr < nrow; rr += kAdjBlock) {
+        for (int rr = tid; rr < nrow; rr += kBandBlock) {
             const float *a = acc + 6 * rr;
             double *g = p.gbeam + 8 * (long)(lo + rr);
 #pragma unroll
@@ -2245,12 +2553,13 @@ __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_beamrec(PairParams p, RecParams R)
 {
     constexpr int NW = WRITE ? kRecWriteWaves : kWavesPerBlock;   /* waves (samples) per block */
-    __shared__ RunTable tables[NW];
+    __shared__ WaveTable tables[NW];
+    __shared__ WaveState<1> states[NW];
     /* counts: one row per wave (sample); write cursors: one row per block */
     __shared__ unsigned curs[WRITE ? 1 : NW][kRecMaxBands];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int lane = threadIdx.x % kWaveSize;
-    RunTable &t = tables[wave];
+    WaveTable &t = tables[wave];
     const long j0 = xcd_remap(blockIdx.x, gridDim.x) * NW;
     const long j = j0 + wave;
     const long i = p.s_begin + j;
@@ -2280,11 +2589,12 @@ void k_beamrec(PairParams p, RecParams R)
     const float ga = unif(p.g_a ? p.g_a[i] : 0.f);
     const float gb = unif(p.g_b ? p.g_b[i] : 0.f);
     if (ga != 0.f || gb != 0.f) {   /* else it adds nothing (wave-uniform) */
-        Centre c;
-        SampleF sf;
-        SampleD sd;
-        Disc d;
-        sample_setup(p, i, p.pa[i], c, sf, sd, d);
+        auto &ws = states[wave];
+        wave_samples(p, ws, i, 1, 0.f, false, lane);
+        const SampleF sf = unif(ws.rec[0].sf);
+        const int r0 = __builtin_amdgcn_readfirstlane(ws.rec[0].r_first);
+        const int r1 = __builtin_amdgcn_readfirstlane(ws.rec[0].r_last);
+        auto after = [](const Pass &) {};
         int qn = 0;
         if constexpr (WRITE) {
             const unsigned smp_key = (unsigned)j << kRecRowBits;
@@ -2296,28 +2606,23 @@ void k_beamrec(PairParams p, RecParams R)
                 BeamRec r;
                 r.key = (unsigned)(q.bp - b * R.rows) | smp_key;
                 r.sI = q.sI;
-                r.X = q.sQ * q.c2 + q.sU * q.s2;
-                r.Y = -q.sQ * q.s2 + q.sU * q.c2;
+                r.X = fmaf(q.sQ, q.c2, q.sU * q.s2);
+                r.Y = fmaf(q.sU, q.c2, -(q.sQ * q.s2));
                 R.brec[slot] = r;
             };
-            for (int r0 = d.r_first; r0 <= d.r_last; r0 += kWaveSize) {
-                const int total = build_runs(p.hs, d, r0, lane, t);
-                walk_visits<true, false, decltype(write), false, false>(p, t, total, lane, c, sf,
-                                                                        sd, qn, write);
-                wave_sync();
-            }
+            auto write_exact = [&](const Pending &q, int, int, int) { write(q); };
+            constexpr int F = WALK_SKY | WALK_CHI;
+            walk_rings<F>(p, t, ws, 0, r0, r1, lane, sf, kEtaAdjoint, qn, after, write,
+                          write_exact);
             if (qn > 0)
-                drain_exact<true>(p, t, 0, qn, lane, c, sd.c2psi, sd.s2psi, write);
+                drain_queue<F>(p, ws, 0, qn, lane, write_exact);
         } else {
             auto count = [&](const Pending &q) { atomicAdd(&cur[rec_band(R, q.bp)], 1u); };
-            for (int r0 = d.r_first; r0 <= d.r_last; r0 += kWaveSize) {
-                const int total = build_runs(p.hs, d, r0, lane, t);
-                walk_visits<false, false, decltype(count), false, false>(p, t, total, lane, c, sf,
-                                                                         sd, qn, count);
-                wave_sync();
-            }
+            auto count_exact = [&](const Pending &q, int, int, int) { count(q); };
+            walk_rings<0>(p, t, ws, 0, r0, r1, lane, sf, kEtaAdjoint, qn, after, count,
+                          count_exact);
             if (qn > 0)
-                drain_exact<false>(p, t, 0, qn, lane, c, sd.c2psi, sd.s2psi, count);
+                drain_queue<0>(p, ws, 0, qn, lane, count_exact);
         }
     }
     if constexpr (!WRITE) {
@@ -2373,7 +2678,7 @@ __global__ __launch_bounds__(kScanBlock) void k_band_scan(RecParams R, long nsam
  * rounded once to a multiple of 2^-k and summed as a 64-bit integer, with k
  * the largest integer such that the block's records, each |v| <= gmax *
  * smax * (1 + 1e-3), cannot sum past 2^62 in magnitude. */
-__global__ __launch_bounds__(kAdjBlock) void k_beamrec_sum(PairParams p, RecParams R)
+__global__ __launch_bounds__(kBandBlock) void k_beamrec_sum(PairParams p, RecParams R)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned long long *acc = (unsigned long long *)smem;
@@ -2400,7 +2705,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_beamrec_sum(PairParams p, RecPara
     /* every sum below 2^62 and (for fix64) every single value below 2^50 */
     const int e = (int)std::ceil(std::log2((double)(j1 - k0) * vmax));
     const double scale = std::ldexp(1.0, std::min(62 - e, 49 - ilogb(vmax)));
-    for (int k = tid; k < 6 * nrow; k += kAdjBlock)
+    for (int k = tid; k < 6 * nrow; k += kBandBlock)
         acc[k] = 0ull;
     __syncthreads();
     /* an absent cotangent reads the other one and adds zeros (with neither
@@ -2413,15 +2718,15 @@ __global__ __launch_bounds__(kAdjBlock) void k_beamrec_sum(PairParams p, RecPara
     BeamRec nx[kRecUnroll];
 #pragma unroll
     for (int u = 0; u < kRecUnroll; u++) {
-        const long k = k0 + u * kAdjBlock + tid;
+        const long k = k0 + u * kBandBlock + tid;
         nx[u] = R.brec[r0 + (k < j1 ? k : k0)];
     }
-    for (long kk = k0; kk < j1; kk += (long)kRecUnroll * kAdjBlock) {
+    for (long kk = k0; kk < j1; kk += (long)kRecUnroll * kBandBlock) {
         BeamRec r[kRecUnroll];
         float ga[kRecUnroll], gb[kRecUnroll];
 #pragma unroll
         for (int u = 0; u < kRecUnroll; u++) {
-            const long k = kk + u * kAdjBlock + tid;
+            const long k = kk + u * kBandBlock + tid;
             r[u] = nx[u];
             if (k >= j1)
                 r[u].sI = r[u].X = r[u].Y = 0.f;   /* adds zeros */
@@ -2437,7 +2742,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_beamrec_sum(PairParams p, RecPara
         }
 #pragma unroll
         for (int u = 0; u < kRecUnroll; u++) {
-            const long kn = kk + u * kAdjBlock + tid + (long)kRecUnroll * kAdjBlock;
+            const long kn = kk + u * kBandBlock + tid + (long)kRecUnroll * kBandBlock;
             nx[u] = R.brec[r0 + (kn < j1 ? kn : k0)];
         }
 #pragma unroll
@@ -2454,7 +2759,7 @@ __global__ __launch_bounds__(kAdjBlock) void k_beamrec_sum(PairParams p, RecPara
     __syncthreads();
     const double inv = 1.0 / scale;
     double *dst = R.part + ((long)part * p.npix_beam + lo) * 6;
-    for (int k = tid; k < 6 * nrow; k += kAdjBlock)
+    for (int k = tid; k < 6 * nrow; k += kBandBlock)
         dst[k] += (double)(long long)acc[k] * inv;
 }
 
@@ -2701,16 +3006,13 @@ __global__ void k_disc(Hpx h, long n, const float *ra, const float *dec, double 
 /* Sky pixel -> (beam pixel, chi) for pixel lists laid out as offsets/pixels
  * (the quantity kernel 1 of the reference computes, cudaConv2.cu:59-128).
  * mode 0: the exact FP64 mapping, chi[k] = chi.
- * mode 1: what the adjoint kernels use: the float form, and the exact
- *         mapping where the float form cannot certify the pixel; chi[k]
- *         receives float cos(2chi), sin(2chi) packed as two floats.
+ * mode 1: what the adjoint kernels use: the float form, and the FP64 form
+ *         where the float form cannot certify the pixel; chi[k] receives
+ *         float cos(2chi), sin(2chi) packed as two floats.
  * mode 2: the float form alone; bpix[k] = kNeedExact (-2) where it declines.
- * mode 3: the certified double-precision form of the small-disc kernels and
- *         of the deferred-visit drain (output as mode 1).
- * mode 4: what the one-wave-per-sample forward uses: the double-precision
- *         form with the float alpha, and mode 3 where it declines.
- * mode 5: the double-precision form with the float alpha alone; bpix[k] =
- *         kNeedExact where it declines. */
+ * mode 3: the FP64 form of the deferred-visit drain (output as mode 1).
+ * modes 4, 5: as 1 and 2 with the forward kernels' bound for cos(2chi),
+ *         sin(2chi) in float. */
 __global__ void k_match(Hpx hs, const RingRec *rings, Hpx hb, FastConsts fc, FastConsts64 fc64,
                         int mode, long n,
                         const float *ra, const float *dec, const float *pa,
@@ -2719,35 +3021,34 @@ __global__ void k_match(Hpx hs, const RingRec *rings, Hpx hb, FastConsts fc, Fas
     long i = (long)blockIdx.x;
     if (i >= n)
         return;
-    Centre c = centre_make(ra[i], dec[i], pa[i]);
-    double s2psi, c2psi;
-    pl_sincos(2.0 * c.psi, &s2psi, &c2psi);
-    const SampleF sf = sample_f32(c, c2psi, s2psi);
+    const Centre c = centre_make(ra[i], dec[i], pa[i]);
+    double spsi, cpsi;
+    pl_sincos(c.psi, &spsi, &cpsi);
+    const double c2psi = fma(cpsi, cpsi, -(spsi * spsi)), s2psi = 2.0 * (spsi * cpsi);
+    const SampleF sf = sample_f32(c, cpsi, spsi, c2psi, s2psi);
     for (long k = offsets[i] + threadIdx.x; k < offsets[i + 1]; k += blockDim.x) {
         int pix = pixels[k];
         int r = pix2ring(hs, pix);
         RingRec rr = rings[r];
         if (mode > 0) {
             float c2 = 0.f, s2 = 0.f;
-            double ra_pix = ring_phi(hs, rr, r, pix);
-            int bp;
-            if (mode >= 4) {
-                bp = beam_pixel_f64<true>(hb, fc64, c, c2psi, s2psi, ra_pix, rr.cdp, rr.sdp, c2,
-                                          s2);
-                if (bp == kNeedExact && mode == 4)
-                    bp = beam_pixel_f64(hb, fc64, c, c2psi, s2psi, ra_pix, rr.cdp, rr.sdp, c2, s2);
-            } else if (mode == 3) {
+            const double ra_pix = ring_phi(hs, rr, r, pix);
+            int bp = kNeedExact;
+            if (mode != 3) {
+                const int j = pix - rr.startpix;
+                const RunGeo g = run_geo(hs, rr, r, c, j, 1);
+                const float x = fmaf((float)(j - g.kc), g.b, g.a0);
+                const VisitGeo v = visit_geo(x, g.sD, g.omD, g.cdp2, sf.cdc, sf.sdc);
+                bp = visit_pixel(fc, sf, v);
+                float c4, s4;
+                visit_phase(v, g.kap, c4, s4);
+                visit_chi(sf, c4, s4, c2, s2);
+                if (!(fabsf(g.kap * x) < (mode >= 4 ? kEtaForward : kEtaAdjoint)) ||
+                    fabsf(x) > 0.7f)
+                    visit_chi64(c, c2psi, s2psi, ra_pix, rr.cdp, rr.sdp, c2, s2);
+            }
+            if (bp == kNeedExact && (mode == 1 || mode == 3 || mode == 4))
                 bp = beam_pixel_f64(hb, fc64, c, c2psi, s2psi, ra_pix, rr.cdp, rr.sdp, c2, s2);
-            } else {
-                bp = beam_pixel_f32(fc, c, sf, ra_pix, rr.cdp, rr.sdp, c2, s2);
-            }
-            if (bp == kNeedExact && mode == 1) {
-                ExactVisit e =
-                    beam_visit_exact(hb.nside, c.ra, c.psi, c.cdc, c.sdc, ra_pix, rr.cdp, rr.sdp);
-                bp = e.bp;
-                c2 = e.c2;
-                s2 = e.s2;
-            }
             bpix[k] = bp;
             float2 *o = (float2 *)&chi[k];
             *o = make_float2(c2, s2);
@@ -2812,12 +3113,39 @@ hipError_t launch_pair(int op, const PairParams &p, hipStream_t st)
         return hipSuccess;
     unsigned g = nblocks(n, kWavesPerBlock);
     switch (op) {
-    case OP_FWD: hipLaunchKernelGGL(k_pair<OP_FWD>, dim3(g), dim3(kBlock), 0, st, p); break;
-    case OP_FWD_V: hipLaunchKernelGGL(k_pair<OP_FWD_V>, dim3(g), dim3(kBlock), 0, st, p); break;
     case OP_ADJ_MAP: hipLaunchKernelGGL(k_pair<OP_ADJ_MAP>, dim3(g), dim3(kBlock), 0, st, p); break;
     case OP_ADJ_BEAM: hipLaunchKernelGGL(k_pair<OP_ADJ_BEAM>, dim3(g), dim3(kBlock), 0, st, p); break;
     default: return hipErrorInvalidValue;
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_forward(const PairParams &p0, hipStream_t st, bool vterm)
+{
+    const long n = p0.s_end - p0.s_begin;
+    if (n <= 0)
+        return hipSuccess;
+    PairParams p = p0;
+    if (!p.samples)
+        p.strips = 1;
+    long nb;
+    if (p.strips > 1) {
+        p.group = 1;
+        nb = (n + kStripChunk - 1) / kStripChunk * (kStripChunk / kWavesPerBlock) * p.strips;
+        hipLaunchKernelGGL(k_samples, dim3(nblocks(n, 64)), dim3(64), 0, st, p);
+    } else {
+        /* samples per wave: as many as leave two rounds of resident waves */
+        p.group = kWaveSamples;
+        while (p.group > 1 && n / p.group < 8192)
+            p.group >>= 1;
+        nb = nblocks(n, kWavesPerBlock * p.group);
+    }
+    if (vterm)
+        hipLaunchKernelGGL(k_fwd<OP_FWD_V>, dim3((unsigned)nb), dim3(kBlock), 0, st, p);
+    else
+        hipLaunchKernelGGL(k_fwd<OP_FWD>, dim3((unsigned)nb), dim3(kBlock), 0, st, p);
+    if (p.strips > 1)
+        hipLaunchKernelGGL(k_strip_sum, dim3(gs_blocks(n)), dim3(256), 0, st, p);
     return hipGetLastError();
 }
 
@@ -2877,8 +3205,9 @@ hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st)
     const unsigned g = nblocks(batch_items(n, p.ngroups), kWavesPerBlock);
     switch (group) {
     case 1:
-        hipLaunchKernelGGL(k_batch_pair<OP_FWD>,
-                           dim3(nblocks(batch_items(n, p.npairs), kWavesPerBlock)),
+        hipLaunchKernelGGL(k_batch_pair,
+                           dim3(nblocks(batch_items((n + kPairSamples - 1) / kPairSamples, p.npairs),
+                                        kWavesPerBlock)),
                            dim3(kBlock), 0, st, p);
         break;
     case 2: hipLaunchKernelGGL(k_batch_fwd<2>, dim3(g), dim3(kBlock), 0, st, p); break;
@@ -2888,11 +3217,15 @@ hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st)
     return hipGetLastError();
 }
 
-size_t adjmap_lds_bytes(int cap, int rw, int group, bool det)
+/* Table bytes that the limits of cap and rw allow for. */
+static_assert(sizeof(AdjWave<0, kWaveSize>) * kAdjWaves <= kAdjTableBytes);
+size_t adjmap_lds_bytes(int cap, int rw, int group, bool det, int lanes)
 {
-    const size_t wt = group == 2 ? sizeof(BatchTable<2>)
-                      : group == 4 ? sizeof(BatchTable<4>)
-                                   : sizeof(RunTable);
+    const size_t wt = group == 2   ? sizeof(AdjWave<2, kWaveSize>)
+                      : group == 4 ? sizeof(AdjWave<4, kWaveSize>)
+                      : lanes == 8 ? sizeof(AdjWave<0, 8>)
+                      : lanes == 16 ? sizeof(AdjWave<0, 16>)
+                                    : sizeof(AdjWave<0, kWaveSize>);
     return wt * kAdjWaves + sizeof(int) * (3 * (size_t)rw + 1 + kAdjCtl) +
            (det ? 8 + 8 * 3 * (size_t)cap : sizeof(float) * 3 * (size_t)cap);
 }
@@ -2946,7 +3279,15 @@ hipError_t launch_adjmap_lds(const PairParams &p, int chunk, int cap, int rw, in
     L.chunk = chunk;
     L.cap = cap;
     L.rw = rw;
+    L.group = std::max(1, std::min(kAdjSamples, chunk / kAdjWaves));
     L.nchunks = (n + chunk - 1) / chunk;
+    L.strips = 1;
+    L.strip_group = 1;
+    if (p.samples) {
+        L.strips = p.strips;
+        L.strip_group = std::max(1, kStripChunk / chunk);
+        hipLaunchKernelGGL(k_samples, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, p);
+    }
     if (batch) {
         L.pairs = batch->pairs;
         L.npairs = batch->npairs;
@@ -2957,12 +3298,12 @@ hipError_t launch_adjmap_lds(const PairParams &p, int chunk, int cap, int rw, in
     const int bg = batch ? group : 0;
     const bool det = fx_scale != nullptr;
     L.fx_scale = fx_scale;
-    const size_t bytes = adjmap_lds_bytes(cap, rw, bg, det);
+    const size_t bytes = adjmap_lds_bytes(cap, rw, bg, det, bg == 0 ? lanes : kWaveSize);
     /* nblocks 0: one block per window.  Blocks start in index order, so the
      * windows in flight on an XCD stay consecutive in the scan; persistent
      * blocks (one per CU) drift apart over the launch, and measured 10%
      * slower on the 5-degree, NSIDE 512 sky adjoint. */
-    const long g = nblocks > 0 ? std::min<long>(L.nchunks, nblocks) : L.nchunks;
+    const long g = nblocks > 0 ? std::min<long>(adj_items(L), nblocks) : adj_items(L);
     if (bg == 0 && lanes != kWaveSize) {   /* several samples per wave */
         switch (lanes) {
         case 8:
@@ -2994,7 +3335,7 @@ hipError_t launch_adjmap_lds(const PairParams &p, int chunk, int cap, int rw, in
 
 int adjbeam_band_rows()
 {
-    return (int)((163840 - sizeof(BandRunTable) * kAdjWaves) / (6 * sizeof(float)));
+    return (int)((163840 - sizeof(BandRunTable) * kBandWaves) / (6 * sizeof(float)));
 }
 
 hipError_t launch_adjbeam_bands(const PairParams &p, int chunk, int rows, int nblocks, int ncu,
@@ -3015,7 +3356,7 @@ hipError_t launch_adjbeam_bands(const PairParams &p, int chunk, int rows, int nb
     const long fill = n * B.nband / (2L * std::max(ncu, 1));
     B.chunk = (int)std::max<long>(std::min<long>(chunk, std::max<long>(fill, 64)), 1);
     B.nchunks = (n + B.chunk - 1) / B.chunk;
-    const size_t bytes = sizeof(BandRunTable) * kAdjWaves + 6 * sizeof(float) * (size_t)B.rows;
+    const size_t bytes = sizeof(BandRunTable) * kBandWaves + 6 * sizeof(float) * (size_t)B.rows;
     if (lanes != 64 && lanes != 8)
         return hipErrorInvalidValue;
     const void *fn = lanes == 8 ? (const void *)k_adjbeam_band_sub<8> : (const void *)k_adjbeam_band;
@@ -3026,10 +3367,10 @@ hipError_t launch_adjbeam_bands(const PairParams &p, int chunk, int rows, int nb
     const long items = B.nchunks * B.nband;
     const long g = nblocks > 0 ? std::min<long>(items, nblocks) : items;   /* 0: one per item */
     if (lanes == 8)
-        hipLaunchKernelGGL(k_adjbeam_band_sub<8>, dim3((unsigned)g), dim3(kAdjBlock), bytes, st, p,
+        hipLaunchKernelGGL(k_adjbeam_band_sub<8>, dim3((unsigned)g), dim3(kBandBlock), bytes, st, p,
                            B);
     else
-        hipLaunchKernelGGL(k_adjbeam_band, dim3((unsigned)g), dim3(kAdjBlock), bytes, st, p, B);
+        hipLaunchKernelGGL(k_adjbeam_band, dim3((unsigned)g), dim3(kBandBlock), bytes, st, p, B);
     return hipGetLastError();
 }
 
@@ -3106,7 +3447,7 @@ hipError_t launch_adjbeam_records(const PairParams &p0, const RecPlan &pl, void 
                            (long)pl.nband);
         const dim3 g3((unsigned)((ns + kRecWriteWaves - 1) / kRecWriteWaves));
         hipLaunchKernelGGL(k_beamrec<true>, g3, dim3(kRecWriteWaves * kWaveSize), 0, st, p, R);
-        hipLaunchKernelGGL(k_beamrec_sum, dim3((unsigned)(pl.nband * pl.nsplit)), dim3(kAdjBlock),
+        hipLaunchKernelGGL(k_beamrec_sum, dim3((unsigned)(pl.nband * pl.nsplit)), dim3(kBandBlock),
                            bytes, st, p, R);
     }
     hipLaunchKernelGGL(k_beamrec_reduce, dim3(gs_blocks(6 * (long)p0.npix_beam)), dim3(256), 0, st,
@@ -3259,15 +3600,11 @@ hipError_t launch_match(const Hpx &hs, const RingRec *rings, const Hpx &hb, int 
     return hipGetLastError();
 }
 
-/* Constants of beam_pixel_f32 for a beam map.  The rho > 1e-6 band edges are
- * 1 - cos(x) = x^2/2 (the x^4/24 term is below float resolution). */
 FastConsts fast_consts(const Hpx &hb)
 {
     FastConsts f;
-    f.omc_lo = (float)(0.5 * 0.5e-6 * 0.5e-6);
-    f.omc_hi = (float)(0.5 * 1.5e-6 * 1.5e-6);
-    f.marg_k = (float)(1.2e-13 * hb.nside);
     f.nside = (float)hb.nside;
+    f.k3 = 3.0f * f.nside * f.nside;
     return f;
 }
 

@@ -14,6 +14,15 @@ namespace pisco {
  * (V A3, V B3, cudaConv2.cu:204,214,217-218); p.sky4 then carries V. */
 enum { OP_FWD = 0, OP_ADJ_MAP = 1, OP_ADJ_BEAM = 2, OP_FWD_V = 3 };
 
+/* A sample's constants, kept in LDS: the walk's loop holds only the floats in
+ * registers, the rest is read by the table builds and the FP64 drains. */
+struct SampleRec {
+    double ra, cdc, sdc, psi, c2psi, s2psi;   /* Centre; cos, sin 2 psi */
+    double phi, z0, xa;                       /* Disc */
+    int irmin, irmax, r_first, r_last;
+    SampleF sf;
+};
+
 /* One launch over samples [s_begin, s_end) of a detector pair a/b that
  * share pointing and beam geometry. */
 struct PairParams {
@@ -28,9 +37,16 @@ struct PairParams {
     Hpx hb;
     int npix_beam;
     double rho_max, cos_rmax;
-    FastConsts fc;            /* single-precision mapping (sky adjoint, beam adjoint) */
-    FastConsts64 fc64;        /* double-precision mapping (forward) */
+    FastConsts fc;            /* single-precision mapping */
+    FastConsts64 fc64;        /* double-precision mapping (visits the float form declines) */
     const float *beam;
+    /* strips of rings that a disc is cut into (1: not cut), with the constants
+     * of the launch's samples and, forward, the strips' sums [strip][a, b]
+     * [sample of the launch]; samples per wave of the forward */
+    int strips;
+    SampleRec *samples;
+    double *part;
+    int group;
     /* device int: index of the last beam row whose A0 A1 A2 B0 B1 B2 are not
      * all zero (-1: none), or NULL.  Only sizes the sky adjoint's LDS
      * windows; every visit of the rho_max disc is still computed. */
@@ -54,7 +70,7 @@ struct BatchPair {
     const float *beam;
     int npix;               /* beam pixels */
     int nside;              /* beam NSIDE */
-    float nside_f, marg_k;  /* FastConsts of this beam NSIDE */
+    float nside_f;          /* (float)nside */
     float omc_cut;          /* 1 - cos(rho_max) */
     float pa_off;           /* pa of the pair = (float)(pa + pa_off) */
     double rho_max, cos_rmax;
@@ -70,7 +86,6 @@ struct BatchParams {
     const float4 *sky4;       /* forward: I, Q, U, 0 per pixel */
     const BatchPair *pairs;   /* device, sorted by rho_max descending */
     int npairs, ngroups;      /* ngroups = ceil(npairs / G) */
-    FastConsts fc;            /* rho > 1e-6 band (omc_lo, omc_hi) */
     FastConsts64 fc64;        /* crho thresholds of the double-precision form */
     const float *ra, *dec, *pa;
     long ptg_stride;          /* 0: shared pointing; else pair `out` at out * ptg_stride */
@@ -136,11 +151,32 @@ hipError_t launch_focal_plane(const FocalPlaneParams &q, hipStream_t st);
 
 hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st);
 
+/* The direct-atomic adjoints. */
 hipError_t launch_pair(int op, const PairParams &p, hipStream_t st);
+/* The forward, one wave per sample and strip.  With p.strips > 1 at most
+ * kStripLaunch samples, p.samples and p.part in a workspace of
+ * strip_bytes(p.strips) bytes (strip_workspace); whole discs if p.samples is
+ * NULL. */
+hipError_t launch_forward(const PairParams &p, hipStream_t st, bool vterm = false);
+constexpr long kStripLaunch = 1L << 17;
+constexpr int kMaxStrips = 8;
+/* Waves per block of the sky adjoint: two blocks per CU, so that one block's
+ * window passes, clears and flushes overlap the other's walk. */
+constexpr int kAdjWaves = 8;
+constexpr size_t kAdjTableBytes = 24640;   /* their tables, one wave per sample, at most */
+constexpr size_t strip_bytes(int strips)
+{
+    return kStripLaunch * (sizeof(SampleRec) + 2 * strips * sizeof(double));
+}
+inline void strip_workspace(PairParams &p, void *ws)
+{
+    p.samples = (SampleRec *)ws;
+    p.part = (double *)((char *)ws + kStripLaunch * sizeof(SampleRec));
+}
 /* The beam-interpolation mode of the same operations (k_pair_interp). */
 hipError_t launch_pair_interp(int op, const PairParams &p, hipStream_t st);
 /* Forward with 64/sub samples per wave, sub = 8, 16 or 32 lanes each (small
- * discs); same results as launch_pair(OP_FWD), or OP_FWD_V with vterm. */
+ * discs); same results as launch_forward. */
 hipError_t launch_fwd_sub(int sub, const PairParams &p, hipStream_t st, bool vterm = false);
 /* Beam adjoint in LDS bands of beam rows (work items: band x chunk of
  * samples); p.gbeam accumulates in FP64, p.sky4 holds the packed sky.  rows:
@@ -192,8 +228,8 @@ hipError_t launch_adjmap_lds(const PairParams &p, int chunk, int cap, int rw, in
                              double rho_w = 0.0, int group = 1,
                              const double *fx_scale = nullptr, int lanes = 64);
 /* group: 0 one pair, 1 per-pair batch items, 2 or 4 pairs per wave; det: the
- * deterministic mode's integer windows */
-size_t adjmap_lds_bytes(int cap, int rw, int group = 0, bool det = false);
+ * deterministic mode's integer windows; lanes per sample (group 0) */
+size_t adjmap_lds_bytes(int cap, int rw, int group = 0, bool det = false, int lanes = 64);
 /* Deterministic sky adjoint: *scale (device) from the beams (beam8 rows)
  * and the cotangents (g_a, g_b of nsamples floats, either may be NULL);
  * count = the most contributions a pixel can receive; work holds 2 unsigned
@@ -247,6 +283,8 @@ int set_error(int code, const char *msg);
 int pair_params(int nside_sky, const float *I, const float *Q, const float *U, int nside_beam,
                 long npix_beam, const float *beam8, long nsamples, const float *ra,
                 const float *dec, const float *pa, PairParams &p);
+/* Strips of the kernels with one wave per sample (PairParams::strips). */
+int strips_auto(const PairParams &p, bool adjoint);
 /* Lanes per sample of the nearest-pixel forward from the expected disc size
  * npix (1 - cos rho_max) / 2: 8 below 1,000 pixels, 16 below 3,000, else 64. */
 int forward_lanes_auto(const PairParams &p);

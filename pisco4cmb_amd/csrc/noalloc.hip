@@ -4,12 +4,12 @@
  * memory the library allocates, for callers that cannot allocate device
  * memory during the call (code under graph capture, serving loops).
  *
- * The forward's workspace is the sky ring table (one RingRec per ring) and
- * the sky packed as one float4 (I, Q, U, 0) per pixel.  Both live in
- * `scratch`, sized for sky NSIDE up to kNoAllocMaxNside: 4 N RingRec records
- * and 12 N^2 float4 pixels, 48.1 MiB at N = 512.  Every call rewrites both
- * parts completely before the forward reads them, so nothing needs clearing;
- * the forward writes each TOD sample once.  Every call on a device shares
+ * The forward's workspace is the sky ring table (one RingRec per ring), the
+ * sky packed as one float4 (I, Q, U, 0) per pixel and the workspace of the
+ * forward's strips.  They live in `scratch`, sized for sky NSIDE
+ * up to kNoAllocMaxNside: 4 N RingRec records and 12 N^2 float4 pixels, 48.1
+ * MiB at N = 512, and 32 MiB for the strips.  Every call rewrites what the forward
+ * reads, so nothing needs clearing; the forward writes each TOD sample once.  Every call on a device shares
  * that device's copy of the array: calls that overlap in time on one device
  * (on different streams, or from different host threads) race.
  */
@@ -31,7 +31,8 @@ constexpr int kNoAllocMaxNside = 512;
 constexpr size_t kRingBytes = sizeof(RingRec) * 4 * (size_t)kNoAllocMaxNside;
 constexpr size_t kSkyOffset = (kRingBytes + 255) / 256 * 256;
 constexpr size_t kSkyBytes = sizeof(float4) * 12 * (size_t)kNoAllocMaxNside * kNoAllocMaxNside;
-constexpr size_t kScratchBytes = kSkyOffset + kSkyBytes;
+constexpr size_t kStripOffset = (kSkyOffset + kSkyBytes + 255) / 256 * 256;
+constexpr size_t kScratchBytes = kStripOffset + strip_bytes(kMaxStrips);
 constexpr long kChunk = 1L << 22;   /* samples per launch, as the torch binding's contexts */
 constexpr int kMaxDevices = 64;
 
@@ -119,10 +120,14 @@ int pisco_dev_forward_noalloc(void *stream, int nside_sky, const float *I, const
     p.tod_a = tod_a;
     p.tod_b = tod_b;
     const int lanes = forward_lanes_auto(p);
-    for (long s = 0; s < nsamples; s += kChunk) {
+    p.strips = lanes < 64 ? 1 : strips_auto(p, false);
+    if (p.strips > 1)
+        strip_workspace(p, base + kStripOffset);
+    const long chunk = p.strips > 1 ? kStripLaunch : kChunk;
+    for (long s = 0; s < nsamples; s += chunk) {
         p.s_begin = s;
-        p.s_end = std::min(nsamples, s + kChunk);
-        e = lanes < 64 ? launch_fwd_sub(lanes, p, st) : launch_pair(OP_FWD, p, st);
+        p.s_end = std::min(nsamples, s + chunk);
+        e = lanes < 64 ? launch_fwd_sub(lanes, p, st) : launch_forward(p, st);
         if (e != hipSuccess)
             return errorf(PISCO_ERR_DEVICE, "forward launch failed: %s", hipGetErrorString(e));
     }
