@@ -141,7 +141,9 @@ struct VisitTable {
 };
 
 /* What a pass covers: its visits and runs, the first ring of the next pass,
- * and whether some visit's |eta| may exceed the caller's bound. */
+ * and whether some run is wide: the |eta| of its visits may exceed the caller's
+ * bound.  Wide runs hold ~ring: which form a visit takes does not depend on the
+ * pass it is in. */
 struct Pass {
     int total, nrun, next;
     bool wide;
@@ -230,11 +232,12 @@ __device__ inline Pass build_pass(const Hpx &hs, const RingRec *rings, const Dis
                                             __int_as_float(rr.startpix + j0[k] - off));
                 t.rec[run][1] = make_float4(g.sD, g.omD, g.cdp2, g.kap);
                 t.pref[run] = off;
-                t.ring[run] = r;
                 const float x0 = fabsf(fmaf((float)(off - mid), g.b, g.a0));
                 const float x1 = fabsf(fmaf((float)(off + ln[k] - mid), g.b, g.a0));
                 const float xm = fmaxf(x0, x1);
-                wide = wide || !(fabsf(g.kap) * xm < eta_max) || xm > 0.7f;
+                const bool w = !(fabsf(g.kap) * xm < eta_max) || xm > 0.7f;
+                t.ring[run] = w ? ~r : r;
+                wide = wide || w;
                 if (off > 0 && off <= T::VCAP)   /* the first segment's marks */
                     atomicOr(&t.bits[(off - 1) >> 5], 1u << ((off - 1) & 31));
                 run++;
@@ -256,6 +259,13 @@ __device__ inline Pass build_pass(const Hpx &hs, const RingRec *rings, const Dis
         t.pref[ps.nrun] = ps.total;
     wave_sync();
     return ps;
+}
+
+template <typename T>
+__device__ inline int run_ring(const T &t, int i)
+{
+    const int r = t.ring[i];
+    return r < 0 ? ~r : r;
 }
 
 /* Marks the runs of the segment that starts at visit seg0 > 0; returns the
@@ -487,8 +497,8 @@ struct WalkAt {
  * in-order load counter ambiguous at the loop head.  Visits whose floors the
  * float form cannot certify join the queue; the walk returns (at.v0 < vend)
  * when it holds a batch of 64, so that the FP64 drain, which needs many
- * registers, is outside the loop.  WIDE: cos, sin 2 chi in FP64 for the lane
- * groups with `wide`. */
+ * registers, is outside the loop.  WIDE: cos, sin 2 chi in FP64 for the wide
+ * runs of the lane groups with `wide`. */
 template <int F, bool WIDE, typename T, typename WS, typename Use>
 __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int total, int vend,
                                     bool wide, int sl, int j, const SampleF &sf, WalkAt &at,
@@ -537,8 +547,8 @@ __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int
             visit_phase(g, r.b.w, c4, s4);
             visit_chi(sf, c4, s4, c2, s2);
             if constexpr (WIDE) {
-                if (wide) {   /* a wide pass has runs */
-                    const int rg = t.ring[r.run];
+                const int rg = wide ? ~t.ring[r.run] : -1;   /* a wide pass has runs */
+                if (rg >= 0) {
                     const RingRec rr = p.rings[rg];
                     const SampleRec &sr = ws.rec[j];
                     visit_chi64(rec_centre(sr), sr.c2psi, sr.s2psi, ring_phi(p.hs, rr, rg, pix),
@@ -1321,8 +1331,8 @@ __device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, i
                 visit_geo(fmaf(vf - r0_.z, r0_.y, r0_.x), r1_.x, r1_.y, r1_.z, cdc, sdc);
             float c4, s4;
             visit_phase(g, r1_.w, c4, s4);
-            if (ps.wide) {
-                const int r = t.ring[run];
+            const int r = ps.wide ? ~t.ring[run] : -1;
+            if (r >= 0) {
                 const RingRec rr = p.rings[r];
                 visit_chi64(c, 1.0, 0.0, ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, c4, s4);
                 s4 = -s4;
@@ -1864,7 +1874,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(4, 4)
          * global atomics. */
         auto fill_windows = [&](auto &vt, const Pass &ps, int l, int n) {
             for (int i = l; i < ps.nrun; i += n) {
-                const int r = vt.ring[i], k = r - R0;
+                const int r = run_ring(vt, i), k = r - R0;
                 int2 w = make_int2(0, 0);
                 if (!sfall && k >= k0 && k < k1) {
                     int sp, nr;
@@ -3134,9 +3144,9 @@ hipError_t launch_forward(const PairParams &p0, hipStream_t st, bool vterm)
         nb = (n + kStripChunk - 1) / kStripChunk * (kStripChunk / kWavesPerBlock) * p.strips;
         hipLaunchKernelGGL(k_samples, dim3(nblocks(n, 64)), dim3(64), 0, st, p);
     } else {
-        /* samples per wave: as many as leave two rounds of resident waves */
+        /* samples per wave: as many as leave 16 rounds of resident waves */
         p.group = kWaveSamples;
-        while (p.group > 1 && n / p.group < 8192)
+        while (p.group > 1 && n / p.group < 65536)
             p.group >>= 1;
         nb = nblocks(n, kWavesPerBlock * p.group);
     }
