@@ -133,16 +133,6 @@ int pisco::pair_params(int nside_sky, const float *I, const float *Q, const floa
     return PISCO_OK;
 }
 
-/* Measured on MI355X over 1e6 CES samples: 8 lanes took 0.59x the time of 64
- * at 135 pixels per disc and 0.88x at 540; 16 lanes 0.98x at 1,500; 64 lanes
- * were fastest at 6,000. */
-int pisco::forward_lanes_auto(const PairParams &p)
-{
-    const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
-    const double dp = (double)p.hs.npix * s * s;   /* expected pixels per disc */
-    return dp < 1000.0 ? 8 : dp < 3000.0 ? 16 : 64;
-}
-
 /* Strips by the beam's size: a strip of a large beam stays in an XCD's 4 MB
  * L2, and each strip costs a table build per sample.  Forward at sky NSIDE 512,
  * ms for 1, 2, 3, 4 strips: 2.9 MB 1.12, 0.89, 1.04; 4.2 MB 1.99, 1.18, 1.29;
@@ -154,6 +144,24 @@ int pisco::strips_auto(const PairParams &p, bool adjoint)
 {
     const double mb = 32.0 * p.npix_beam / (1 << 20);
     return (int)std::min<double>(kMaxStrips, std::ceil(mb / (adjoint ? 8.0 : 2.2)));
+}
+
+/* Lanes per sample of the forward.  Several samples per wave share the table
+ * builds, and neighbouring samples meet the same lines of the sky and the beam.
+ * ms for 8, 16, 32, 64 lanes over 1e5 samples: 240 pixels per disc 0.18, 0.21,
+ * 0.24, 0.24; 960: 0.51, 0.54, 0.57, 0.58; 2,160: 1.04, 1.05, 1.09, 1.23; 16,
+ * 32, 64 lanes at 6,000 pixels over 3.6e5 samples 7.99, 8.44, 9.37, but over
+ * 6e4, fewer waves, 1.79, 1.64, 1.69; at 54,000 over 2e4 7.9, 6.8, 6.1.  The
+ * rule may not look at the number of samples: a sample's sum would depend on
+ * it.  A beam that needs strips takes the one-wave kernel: 2.9 MB, 1,500
+ * pixels 0.93, 0.96, 0.96, 0.86. */
+int pisco::forward_lanes_auto(const PairParams &p)
+{
+    const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
+    const double dp = (double)p.hs.npix * s * s;   /* expected pixels per disc */
+    if (strips_auto(p, false) > 1)
+        return 64;
+    return dp < 1000.0 ? 8 : dp < 3000.0 ? 16 : dp < 30000.0 ? 32 : 64;
 }
 
 struct pisco_ctx {
@@ -300,14 +308,20 @@ int fwd_lanes(const pisco_ctx *c, const PairParams &p)
 }
 
 /* Lanes per sample of the single-pair sky adjoint: the tuning value, or
- * (auto) from the expected disc size.  8 lanes took 0.80x the time of 64 at
- * 135 pixels per disc and 0.95x at 540; at 1,500 pixels 16 lanes equalled
- * 64 and 8 took 1.23x. */
+ * (auto) from the expected disc size and, where 8 lanes would leave waves idle,
+ * the number of samples.  Best ms over 1e5 samples for 8, 16, 64 lanes: 374
+ * pixels per disc 0.46, 0.51, 0.61; 540: 0.64, 0.60, 0.69; 960: 1.01, 1.00,
+ * 1.00; 1,500: 1.31, 1.24, 1.26; 135 pixels, 1e4 samples: 0.113, 0.108, 0.121.
+ * 16 and 64 lanes over 6e4 samples: 6,000 pixels 1.83, 1.95; 8,600: 3.29, 3.30.
+ * Strips are of one-wave samples. */
 int adj_lanes(const pisco_ctx *c, const PairParams &p)
 {
     if (c->adjmap_lanes > 0)
         return c->adjmap_lanes;
-    return disc_pixels(p) < 1000.0 ? 8 : 64;
+    const double dp = disc_pixels(p);
+    if (dp >= 10000.0 || strips_auto(p, true) > 1)
+        return 64;
+    return dp >= 450.0 || p.s_end - p.s_begin < 16384 ? 16 : 8;
 }
 
 /* Strips for a launch of one wave per sample, whose launches then take at most
@@ -385,23 +399,29 @@ int det_scale(pisco_ctx *c, const float *const *beams, const long *npix, int nbe
 }
 
 /* Samples per LDS window of a single-pair sky adjoint with `lanes` lanes per
- * sample: the tuning value, or (auto) the largest power of two in [16, 512]
- * that keeps a window at about 96,000 expected visits, and at least two
- * samples per lane group of the block's 8 waves (16 x 64 / lanes).  Each window
- * costs three block-wide passes besides its visits: 540 pixels per disc, 8
- * lanes: 32, 64, 128 samples 0.99, 0.65, 0.57 ms.  With strips 8 samples: the
- * samples in flight are fewer and the strip of the beam that they meet is
- * smaller (16: 15.9 ms, 8: 14.0 ms at 6,000 pixels per disc). */
+ * sample: the tuning value, or (auto) the largest power of two up to 128 that
+ * keeps a window at 40,000 expected visits, but at least a sample per lane
+ * group of the block's waves; fewer, down to 16, where there would be less than
+ * one window per CU.  Each window costs three block-wide passes besides its
+ * visits, and a larger one more LDS.  ms for 16, 32, 64, 128 samples: 8 lanes,
+ * 374 pixels 1.04, 0.63, 0.46, 0.48; 16 lanes, 960 pixels 1.24, 1.00, 1.03,
+ * 1.12; 64 lanes, 1,500 pixels 1.26, 1.42, 1.45, 1.73; 8 lanes, 94 pixels, 1e4
+ * samples 0.135, 0.098, 0.097, 0.119.  With strips 8 samples: the samples in
+ * flight are fewer and the strip of the beam that they meet is smaller (16:
+ * 15.9 ms, 8: 14.0 ms at 6,000 pixels per disc). */
 int adj_chunk(const pisco_ctx *c, const PairParams &p, int lanes)
 {
     if (c->adjmap_chunk > 0)
         return c->adjmap_chunk;
     if (lanes == 64 && strips_auto(p, true) > 1)
         return kAdjWaves;
-    int chunk = 16;
-    while (chunk < 512 && 2.0 * chunk * disc_pixels(p) <= 96000.0)
+    const double dp = disc_pixels(p);
+    int chunk = std::max(16, kAdjWaves * (64 / lanes));
+    while (chunk < 128 && 2.0 * chunk * dp <= 40000.0)
         chunk *= 2;
-    return std::max(chunk, std::min(16 * (64 / std::max(lanes, 1)), 512));
+    while (chunk > 16 && p.s_end - p.s_begin < 256L * chunk)
+        chunk /= 2;
+    return chunk;
 }
 
 /* The window capacity that fits the LDS next to the per-wave tables. */
