@@ -1864,12 +1864,16 @@ int map_accumulate(pisco_skymap *m, hipStream_t st, long nsamples, const float *
                    const float *pol, const float *data)
 {
     const long total = nsamples * (long)ndet;
-    const long chunk = std::min<long>(m->chunk, total);
-    const long nh = 256L * map_tiles((int)chunk);
+    /* one pointing for all detectors, in one pass: only it is sorted */
+    const bool shared = ptg_stride == 0 && ndet > 1 && nsamples <= m->chunk;
+    const long chunk = shared ? nsamples : std::min<long>(m->chunk, total);
+    const long nh = 256L * map_sort_tiles((int)chunk);
     CHK(m->keys.ensure(3 * chunk));
     CHK(m->vals.ensure(2 * chunk));
-    CHK(m->terms.ensure(2 * chunk));
-    CHK(m->tdata.ensure(chunk));
+    if (!shared) {
+        CHK(m->terms.ensure(2 * chunk));
+        CHK(m->tdata.ensure(chunk));
+    }
     CHK(m->hist.ensure(2 * nh + 1 + map_tiles((int)nh)));
     MapScratch s;
     for (int k = 0; k < 3; k++)
@@ -1892,6 +1896,23 @@ int map_accumulate(pisco_skymap *m, hipStream_t st, long nsamples, const float *
         CHK(m->ppix.ensure(nsamples));
         HIPCHK(launch_map_ptg_pixel(h, ra, dec, nsamples, m->ppix.p, st));
         s.ppix = m->ppix.p;
+    }
+    if (shared) {
+        MapChunk c;
+        c.ra = ra;
+        c.dec = dec;
+        c.pa = pa;
+        c.pol = pol;
+        c.data = data;
+        c.nsamples = nsamples;
+        c.ptg_stride = 0;
+        c.t0 = 0;
+        c.len = (int)nsamples;
+        hipError_t e = launch_map_shared(h, c, ndet, s, m->acc.p, st);
+        if (e != hipSuccess)
+            return fail(PISCO_ERR_DEVICE, "map accumulation launch failed: %s",
+                        hipGetErrorString(e));
+        return PISCO_OK;
     }
     for (long t0 = 0; t0 < total; t0 += chunk) {
         MapChunk c;

@@ -117,17 +117,23 @@ struct MapScratch {
     int *count;               /* [npix] */
     int *off;                 /* [npix + 1] */
     int *tsum;                /* [map_tiles(npix)] */
-    int *hist, *hoff;         /* [256 * map_tiles(chunk)] (+1 for hoff) */
-    int *htsum;               /* [map_tiles(256 * map_tiles(chunk))] */
+    int *hist, *hoff;         /* [256 * map_sort_tiles(chunk)] (+1 for hoff) */
+    int *htsum;               /* [map_tiles(256 * map_sort_tiles(chunk))] */
     const int *ppix;          /* [nsamples] pixels of a shared pointing, or NULL */
     unsigned long long *skipped;
 };
 /* scan tiles of an array of n counts (4096 per tile) */
 int map_tiles(int n);
+/* tiles of the sort of up to n samples, at most */
+int map_sort_tiles(int n);
 /* radix passes of 8 bits that order the pixels of a map of npix pixels */
 int map_sort_passes(int npix);
 hipError_t launch_map_accumulate(const Hpx &h, const MapChunk &c, const MapScratch &s,
                                  double *acc, hipStream_t st);
+/* All samples of a pointing shared by ndet detectors (s.ppix, c.nsamples below
+ * 2^30, the scratch of that many samples; no terms). */
+hipError_t launch_map_shared(const Hpx &h, const MapChunk &c, int ndet, const MapScratch &s,
+                             double *acc, hipStream_t st);
 /* ppix[s] = pixel of pointing s (-1: skipped), for a pointing shared by
  * every detector */
 hipError_t launch_map_ptg_pixel(const Hpx &h, const float *ra, const float *dec, long n,

@@ -18,6 +18,9 @@
  *   5. k_mm_walk     one thread per pixel adds its samples' terms, in that
  *                    order, onto the pixel's sums: nine dependent FP64 adds
  *                    per sample
+ * With a pointing shared by the detectors the sort is of the pointing samples
+ * alone, and steps 4 and 5 are one kernel (k_mm_shared).
+ *
  * Only the 6 distinct entries of the symmetric AtA are kept: the reference's
  * AtA[1] and AtA[3] (and [2]/[6], [5]/[7]) receive the same terms in the
  * same order and are therefore equal.
@@ -224,15 +227,21 @@ __global__ __launch_bounds__(kTileThreads) void k_mm_tile_scan(const int *count,
  * the block's waves), so every pass is stable and the result lists each
  * pixel's samples in increasing sample index. */
 
-/* hist[d * nb + b] = number of items of tile b whose digit is d */
+/* hist[d * nb + b] = number of items of tile b whose digit is d.  PER: items
+ * per thread of a tile, kTilePer or fewer where that many would leave CUs
+ * idle. */
+constexpr int kSmallPer = 4;
+constexpr int kSmallSort = 1 << 20;
+
+template <int PER>
 __global__ __launch_bounds__(kTileThreads) void k_rs_hist(const unsigned *keys, int n, int shift,
                                                           int nb, int *hist)
 {
     __shared__ int h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
-    long base = (long)blockIdx.x * kTile;
-    for (int k = 0; k < kTilePer; k++) {
+    long base = (long)blockIdx.x * (kTileThreads * PER);
+    for (int k = 0; k < PER; k++) {
         long i = base + k * kTileThreads + threadIdx.x;
         if (i < n)
             atomicAdd(&h[(keys[i] >> shift) & 255u], 1);
@@ -243,7 +252,7 @@ __global__ __launch_bounds__(kTileThreads) void k_rs_hist(const unsigned *keys, 
 
 /* Scatter of one pass: hoff = exclusive scan of hist (digit-major).  FIRST:
  * the values are the item indices themselves. */
-template <bool FIRST>
+template <bool FIRST, int PER>
 __global__ __launch_bounds__(kTileThreads) void k_rs_scatter(const unsigned *kin, const int *vin,
                                                              int n, int shift, int nb,
                                                              const int *hoff, unsigned *kout,
@@ -258,8 +267,8 @@ __global__ __launch_bounds__(kTileThreads) void k_rs_scatter(const unsigned *kin
         wcnt[q][tid] = 0;
     __syncthreads();
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const long base = (long)blockIdx.x * kTile;
-    for (int k = 0; k < kTilePer; k++) {
+    const long base = (long)blockIdx.x * (kTileThreads * PER);
+    for (int k = 0; k < PER; k++) {
         long i = base + k * kTileThreads + tid;
         bool valid = i < n;
         unsigned key = valid ? kin[i] : 0u;
@@ -374,6 +383,165 @@ __global__ void k_mm_walk(int npix, const int *off, const double2 *tcs, const fl
     acc[MM_D * np + p] = sd;
     acc[MM_CD * np + p] = scd;
     acc[MM_SD * np + p] = ssd;
+}
+
+/* ---- pointing shared by the detectors ------------------------------------ */
+
+/* Lists the positions of the sorted keys that start a pixel: the pixels with at
+ * least `many` samples at heads[0 ..], the others at heads[n - 1], heads[n - 2],
+ * ... (any order); their numbers in nheads[0], nheads[1].  Counts the skipped
+ * samples of every detector.  One atomic per block and list. */
+constexpr int kHeadThreads = 1024;
+
+__global__ __launch_bounds__(kHeadThreads) void k_mm_heads(const unsigned *keys, int n, int ndet,
+                                                           int many, int *heads, int *nheads,
+                                                           unsigned long long *skipped)
+{
+    __shared__ int num[3], base[2];
+    const int i = blockIdx.x * kHeadThreads + threadIdx.x, lane = threadIdx.x & 63;
+    if (threadIdx.x < 3)
+        num[threadIdx.x] = 0;
+    __syncthreads();
+    const unsigned key = i < n ? keys[i] : 0xffffffffu;
+    const bool head = key != 0xffffffffu && (i == 0 || keys[i - 1] != key);
+    const bool heavy = head && many <= n - i && keys[i + many - 1] == key;
+    const unsigned long long mh = __ballot(heavy), ml = __ballot(head && !heavy);
+    const unsigned long long ms = __ballot(i < n && key == 0xffffffffu);
+    int wh = 0, wl = 0;
+    if (lane == 0) {
+        wh = atomicAdd(&num[0], __popcll(mh));
+        wl = atomicAdd(&num[1], __popcll(ml));
+        atomicAdd(&num[2], __popcll(ms));
+    }
+    wh = __shfl(wh, 0, 64);
+    wl = __shfl(wl, 0, 64);
+    __syncthreads();
+    if (threadIdx.x < 2)
+        base[threadIdx.x] = num[threadIdx.x] ? atomicAdd(&nheads[threadIdx.x], num[threadIdx.x]) : 0;
+    if (threadIdx.x == 2 && num[2])
+        atomicAdd(skipped, (unsigned long long)ndet * num[2]);
+    __syncthreads();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (heavy)
+        heads[base[0] + wh + __popcll(mh & below)] = i;
+    else if (head)
+        heads[n - 1 - (base[1] + wl + __popcll(ml & below))] = i;
+}
+
+/* A pixel's nine sums over ndet detectors by the m pointing samples that hit
+ * it, detector-major as skymap.cpp visits them.  A group of GP lanes per pixel:
+ * each lane forms the terms of one (detector, sample) in LDS, then lane l < 9
+ * adds the group's terms onto sum l in order.  The order allows no other
+ * parallelism within a pixel, so a pixel with many samples takes a whole wave:
+ * the cycles per term are the latency of the loads, the sine and the cosine
+ * over GP, and one add.  Two iterations' loads are in flight: the index of a
+ * sample, and what it points to. */
+template <int GP>
+__device__ inline void shared_pixel(const MapChunk &c, int ndet, const unsigned *keys,
+                                    const int *vals, int n, int b, long npix, double *acc,
+                                    double *e, int l)
+{
+    /* the two factors of this lane's sum: of 1, cos 2psi, sin 2psi, datum */
+    constexpr int kA[9] = {0, 1, 2, 1, 1, 2, 0, 1, 2}, kB[9] = {0, 0, 0, 1, 2, 2, 3, 3, 3};
+    int fa = 0, fb = 0;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        fa = l == k ? kA[k] : fa;
+        fb = l == k ? kB[k] : fb;
+    }
+    const unsigned p = keys[b];
+    int m = 0;   /* samples of the pixel */
+    for (int j = b;; j += GP) {
+        const bool same = j + l < n && keys[j + l] == p;
+        const unsigned long long mask = __ballot(same) >> ((threadIdx.x & 63) - l);
+        const unsigned long long gaps = GP == 64 ? ~mask : ~mask & ((1ull << (GP & 63)) - 1ull);
+        m += gaps ? __ffsll((long long)gaps) - 1 : GP;
+        if (gaps)
+            break;
+    }
+    const int dstep = GP / m, kstep = GP - dstep * m;
+    auto step = [&](int &dt, int &kk) {
+        dt += dstep;
+        kk += kstep;
+        if (kk >= m) {
+            kk -= m;
+            dt++;
+        }
+    };
+    int det = l / m, k = l - det * m, s = 0;   /* the (detector, sample) loaded next */
+    int det0 = 0, k0 = 0;                      /* the group's first one of this iteration */
+    float pol = 0.f, pa = 0.f, d = 0.f;
+    auto load_index = [&]() {
+        if (det < ndet)
+            s = vals[b + k];
+    };
+    auto load = [&]() {
+        if (det < ndet) {
+            pol = c.pol[det];
+            pa = c.pa[s];
+            d = c.data[det * c.nsamples + s];
+        }
+    };
+    double sum = l < 9 ? acc[l * npix + p] : 0.0;
+    load_index();
+    load();
+    bool act = det < ndet;
+    step(det, k);
+    load_index();
+    while (det0 < ndet) {
+        const double psi = -((double)pol + (double)pa), dd = d;
+        const bool now = act;
+        step(det0, k0);
+        load();
+        act = det < ndet;
+        step(det, k);
+        load_index();
+        double s2, c2;
+        pl_sincos(2.0 * psi, &s2, &c2);
+        e[4 * l] = now ? 1.0 : 0.0;   /* zero terms leave a sum as it is */
+        e[4 * l + 1] = now ? c2 : 0.0;
+        e[4 * l + 2] = now ? s2 : 0.0;
+        e[4 * l + 3] = now ? dd : 0.0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (l < 9) {
+#pragma unroll 16
+            for (int i = 0; i < GP; i++)
+                sum += e[4 * i + fa] * e[4 * i + fb];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (l < 9)
+        acc[l * npix + p] = sum;
+}
+
+/* The first kHeavyBlocks blocks take the pixels with many samples, a wave each;
+ * the others those with few, 16 lanes each. */
+constexpr int kHeavyBlocks = 512;
+constexpr int kFewLanes = 16;
+constexpr int kManyTerms = 1024;   /* (detector, sample) pairs of a pixel with many */
+
+__global__ __launch_bounds__(256) void k_mm_shared(MapChunk c, int ndet, const unsigned *keys,
+                                                   const int *vals, int n, const int *heads,
+                                                   const int *nheads, long npix, double *acc)
+{
+    constexpr int GP = kFewLanes, G = 256 / GP;
+    __shared__ double ent[G][4 * GP + 4];   /* groups on different banks */
+    static_assert(sizeof ent >= 4 * 256 * sizeof(double), "also four whole waves");
+    if (blockIdx.x < kHeavyBlocks) {
+        const int w = threadIdx.x / 64;
+        const int nh = nheads[0];
+        for (int h = blockIdx.x * 4 + w; h < nh; h += kHeavyBlocks * 4)
+            shared_pixel<64>(c, ndet, keys, vals, n, heads[h], npix, acc, &ent[0][0] + 256 * w,
+                             threadIdx.x % 64);
+    } else {
+        const int g = threadIdx.x / GP;
+        const int nl = nheads[1], step = (gridDim.x - kHeavyBlocks) * G;
+        for (int h = (blockIdx.x - kHeavyBlocks) * G + g; h < nl; h += step)
+            shared_pixel<GP>(c, ndet, keys, vals, n, heads[n - 1 - h], npix, acc, ent[g],
+                             threadIdx.x % GP);
+    }
 }
 
 namespace {
@@ -536,6 +704,51 @@ int map_sort_passes(int npix)
     return p;
 }
 
+namespace {
+
+/* Sorts keys0[0..n) (values: their indices) by pixel into a buffer pair of s,
+ * whose index is returned. */
+template <int PER>
+int launch_sort_per(const unsigned *keys0, int n, int npix, const MapScratch &s, hipStream_t st)
+{
+    const int nb = grid_for(n, kTileThreads * PER);
+    const int passes = map_sort_passes(npix);
+    const unsigned *kin = keys0;
+    const int *vin = nullptr;
+    int dst = 1;
+    for (int pass = 0; pass < passes; pass++) {
+        dst = (pass & 1) ? 2 : 1;
+        hipLaunchKernelGGL(k_rs_hist<PER>, dim3(nb), dim3(kTileThreads), 0, st, kin, n, 8 * pass,
+                           nb, s.hist);
+        launch_scan(s.hist, 256 * nb, s.htsum, s.hoff, st);
+        if (pass == 0)
+            hipLaunchKernelGGL((k_rs_scatter<true, PER>), dim3(nb), dim3(kTileThreads), 0, st, kin,
+                               vin, n, 8 * pass, nb, (const int *)s.hoff, s.keys[dst],
+                               s.vals[dst]);
+        else
+            hipLaunchKernelGGL((k_rs_scatter<false, PER>), dim3(nb), dim3(kTileThreads), 0, st, kin,
+                               vin, n, 8 * pass, nb, (const int *)s.hoff, s.keys[dst],
+                               s.vals[dst]);
+        kin = s.keys[dst];
+        vin = s.vals[dst];
+    }
+    return dst;
+}
+
+int launch_sort(const unsigned *keys0, int n, int npix, const MapScratch &s, hipStream_t st)
+{
+    return n < kSmallSort ? launch_sort_per<kSmallPer>(keys0, n, npix, s, st)
+                          : launch_sort_per<kTilePer>(keys0, n, npix, s, st);
+}
+
+} // namespace
+
+int map_sort_tiles(int n)
+{
+    const int small = std::min(n, kSmallSort - 1);
+    return std::max(grid_for(small, kTileThreads * kSmallPer), grid_for(n, kTileThreads * kTilePer));
+}
+
 hipError_t launch_map_accumulate(const Hpx &h, const MapChunk &c, const MapScratch &s,
                                  double *acc, hipStream_t st)
 {
@@ -543,34 +756,35 @@ hipError_t launch_map_accumulate(const Hpx &h, const MapChunk &c, const MapScrat
         return hipSuccess;
     const int npix = h.npix;
     const int n = c.len;
-    const int nb = map_tiles(n);
     hipLaunchKernelGGL(k_mm_fill_i32, dim3(std::min(grid_for(npix, 256), 4096)), dim3(256), 0,
                        st, s.count, (long)npix, 0);
     hipLaunchKernelGGL(k_mm_pixel, dim3(grid_for(n, 256)), dim3(256), 0, st, h, c,
                        (const int *)s.ppix, s.keys[0], s.count, s.skipped);
     launch_scan(s.count, npix, s.tsum, s.off, st);
-    /* radix passes: keys[0] (values implicit) -> buffers 1, 2, 1, ... */
-    const int passes = map_sort_passes(npix);
-    int src = 0;
-    for (int pass = 0; pass < passes; pass++) {
-        int dst = (pass & 1) ? 2 : 1;
-        hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(kTileThreads), 0, st,
-                           (const unsigned *)s.keys[src], n, 8 * pass, nb, s.hist);
-        launch_scan(s.hist, 256 * nb, s.htsum, s.hoff, st);
-        if (pass == 0)
-            hipLaunchKernelGGL(k_rs_scatter<true>, dim3(nb), dim3(kTileThreads), 0, st,
-                               (const unsigned *)s.keys[src], (const int *)nullptr, n, 8 * pass,
-                               nb, (const int *)s.hoff, s.keys[dst], s.vals[dst]);
-        else
-            hipLaunchKernelGGL(k_rs_scatter<false>, dim3(nb), dim3(kTileThreads), 0, st,
-                               (const unsigned *)s.keys[src], (const int *)s.vals[src], n,
-                               8 * pass, nb, (const int *)s.hoff, s.keys[dst], s.vals[dst]);
-        src = dst;
-    }
+    const int src = launch_sort(s.keys[0], n, npix, s, st);
     hipLaunchKernelGGL(k_mm_terms, dim3(grid_for(n, 256)), dim3(256), 0, st, c,
                        (const int *)s.vals[src], (const int *)(s.off + npix), s.tcs, s.td);
     hipLaunchKernelGGL(k_mm_walk, dim3(grid_for(npix, 256)), dim3(256), 0, st, npix,
                        (const int *)s.off, (const double2 *)s.tcs, (const float *)s.td, acc);
+    return hipGetLastError();
+}
+
+hipError_t launch_map_shared(const Hpx &h, const MapChunk &c, int ndet, const MapScratch &s,
+                             double *acc, hipStream_t st)
+{
+    const int n = (int)c.nsamples;
+    if (n <= 0 || ndet <= 0)
+        return hipSuccess;
+    const int src = launch_sort((const unsigned *)s.ppix, n, h.npix, s, st);
+    int *heads = (int *)s.keys[0], *nheads = s.count;
+    const int many = std::max(2, (kManyTerms + ndet - 1) / ndet);
+    hipLaunchKernelGGL(k_mm_fill_i32, dim3(1), dim3(64), 0, st, nheads, 2L, 0);
+    hipLaunchKernelGGL(k_mm_heads, dim3(grid_for(n, kHeadThreads)), dim3(kHeadThreads), 0, st,
+                       (const unsigned *)s.keys[src], n, ndet, many, heads, nheads, s.skipped);
+    hipLaunchKernelGGL(k_mm_shared, dim3(kHeavyBlocks + std::min(grid_for(n, 256 / kFewLanes), 4096)),
+                       dim3(256), 0, st, c, ndet, (const unsigned *)s.keys[src],
+                       (const int *)s.vals[src], n, (const int *)heads, (const int *)nheads,
+                       (long)h.npix, acc);
     return hipGetLastError();
 }
 
