@@ -386,14 +386,11 @@ int run_pair(pisco_ctx *c, int op, PairParams p, hipStream_t st, bool sky_packed
 /* Deterministic sky adjoint: the scale (device) for the given beams and
  * cotangents, count = the number of contributions a pixel can receive at
  * most (samples x pairs). */
-int det_scale(pisco_ctx *c, const float *const *beams, const long *npix, int nbeams,
-              const float *g_a, const float *g_b, long ng, long count, hipStream_t st,
-              const double **scale)
+int det_scale(pisco_ctx *c, const FixSource &f, long count, hipStream_t st, const double **scale)
 {
     CHK(c->fxwork.ensure(2));
     CHK(c->fxscale.ensure(1));
-    HIPCHK(launch_fix_scale(beams, npix, nbeams, g_a, g_b, ng, count, c->fxwork.p, c->fxscale.p,
-                            st));
+    HIPCHK(launch_fix_scale(f, count, c->fxwork.p, c->fxscale.p, st));
     *scale = c->fxscale.p;
     return PISCO_OK;
 }
@@ -1186,9 +1183,8 @@ int pisco_dev_adjoint_map(pisco_ctx *c, void *stream, int nside_sky, int nside_b
     const bool det = det_single(c);
     const double *scale = nullptr;
     if (det) {
-        const float *bl[1] = {beam8};
-        const long nl[1] = {npix_beam};
-        CHK(det_scale(c, bl, nl, 1, g_a, g_b, nsamples, nsamples, st, &scale));
+        const FixSource f = {beam8, npix_beam, nullptr, 0, g_a, g_b, nsamples};
+        CHK(det_scale(c, f, nsamples, st, &scale));
     }
     if (g_a || g_b) {
         if ((c->adjmap_chunk != 0 || det) && !c->beam_interp) {
@@ -1206,9 +1202,7 @@ int pisco_dev_adjoint_map(pisco_ctx *c, void *stream, int nside_sky, int nside_b
         }
     }
     if (det) {
-        HIPCHK(launch_fix_to_f32(p.gI, scale, gI, npix, st));
-        HIPCHK(launch_fix_to_f32(p.gQ, scale, gQ, npix, st));
-        HIPCHK(launch_fix_to_f32(p.gU, scale, gU, npix, st));
+        HIPCHK(launch_fix_to_f32(c->acc.p, scale, {{gI, gQ, gU}}, npix, st));
     } else {
         HIPCHK(launch_f64_to_f32(p.gI, gI, npix, st));
         HIPCHK(launch_f64_to_f32(p.gQ, gQ, npix, st));
@@ -1538,14 +1532,8 @@ std::vector<int> batch_ranges(const pisco_ctx *c, const pisco_batch *b)
 int batch_det_scale(pisco_ctx *c, hipStream_t st, const pisco_batch *b, long nsamples,
                     const float *g, const double **scale)
 {
-    std::vector<const float *> bl;
-    std::vector<long> nl;
-    for (int k = 0; k < b->npad; k++) {
-        bl.push_back(b->host[k].beam);
-        nl.push_back(b->host[k].out < 0 ? 0 : b->host[k].npix);
-    }
-    return det_scale(c, bl.data(), nl.data(), (int)bl.size(), g, nullptr,
-                     2L * b->npairs * nsamples, (long)b->npairs * nsamples, st, scale);
+    const FixSource f = {nullptr, 0, b->table, b->npad, g, nullptr, 2L * b->npairs * nsamples};
+    return det_scale(c, f, (long)b->npairs * nsamples, st, scale);
 }
 
 /* Whether a batched launch runs pair by pair (the single-pair kernels, one
@@ -1732,10 +1720,10 @@ int pisco_dev_batched_adjoint_map_pp(pisco_ctx *c, void *stream, const pisco_bat
      * one FP64 gradient */
     CHK(batch_adjoint_pairwise(c, st, b, nside_sky, nsamples, ra, dec, pa, nsamples, g, scale));
     float *out[3] = {gI, gQ, gU};
-    for (int k = 0; k < 3; k++) {
-        if (det)
-            HIPCHK(launch_fix_to_f32(c->acc.p + k * npix, scale, out[k], npix, st));
-        else
+    if (det) {
+        HIPCHK(launch_fix_to_f32(c->acc.p, scale, {{out[0], out[1], out[2]}}, npix, st));
+    } else {
+        for (int k = 0; k < 3; k++)
             HIPCHK(launch_f64_to_f32(c->acc.p + k * npix, out[k], npix, st));
     }
     return PISCO_OK;
@@ -1766,10 +1754,10 @@ int pisco_dev_batched_adjoint_map(pisco_ctx *c, void *stream, const pisco_batch 
         if (det_single(c))
             CHK(batch_det_scale(c, st, b, nsamples, g, &scale));
         CHK(batch_adjoint_pairwise(c, st, b, nside_sky, nsamples, ra, dec, pa, 0, g, scale));
-        for (int k = 0; k < 3; k++) {
-            if (scale)
-                HIPCHK(launch_fix_to_f32(c->acc.p + k * npix, scale, out[k], npix, st));
-            else
+        if (scale) {
+            HIPCHK(launch_fix_to_f32(c->acc.p, scale, {{out[0], out[1], out[2]}}, npix, st));
+        } else {
+            for (int k = 0; k < 3; k++)
                 HIPCHK(launch_f64_to_f32(c->acc.p + k * npix, out[k], npix, st));
         }
         return PISCO_OK;
@@ -1818,10 +1806,10 @@ int pisco_dev_batched_adjoint_map(pisco_ctx *c, void *stream, const pisco_batch 
             return fail(PISCO_ERR_DEVICE, "batched sky adjoint launch failed: %s",
                         hipGetErrorString(e));
     }
-    for (int k = 0; k < 3; k++) {
-        if (det)
-            HIPCHK(launch_fix_to_f32(c->acc.p + k * npix, scale, out[k], npix, st));
-        else
+    if (det) {
+        HIPCHK(launch_fix_to_f32(c->acc.p, scale, {{out[0], out[1], out[2]}}, npix, st));
+    } else {
+        for (int k = 0; k < 3; k++)
             HIPCHK(launch_f64_to_f32(c->acc.p + k * npix, out[k], npix, st));
     }
     return PISCO_OK;

@@ -2787,6 +2787,31 @@ __global__ void k_beamrec_reduce(const double *part, int nsplit, long npix, doub
     }
 }
 
+/* Blocks of the maxima over long arrays: an atomic to one address takes about
+ * 12 ns, so each block makes one per maximum (one per wave of 8,192 blocks took
+ * 0.37 ms over 3.8e6 floats). */
+constexpr int kMaxBlocks = 512;
+
+/* The block's maximum of v >= 0 onto *out, as float bits.  Every thread of a
+ * block of at most 1024 calls it. */
+__device__ inline void block_max(float v, unsigned *out)
+{
+    __shared__ float part[16];
+#pragma unroll
+    for (int m = kWaveSize / 2; m > 0; m >>= 1)
+        v = fmaxf(v, __shfl_xor(v, m, kWaveSize));
+    __syncthreads();   /* part may be in use by a call before */
+    if (threadIdx.x % kWaveSize == 0)
+        part[threadIdx.x / kWaveSize] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < (int)blockDim.x / kWaveSize; w++)
+            v = fmaxf(v, part[w]);
+        if (v > 0.f)
+            atomicMax(out, __float_as_uint(v));
+    }
+}
+
 /* vmax[0] = max |g_a|, |g_b| over the samples; vmax[1] = max over sky
  * pixels of max(|I|, |Q| + |U|) (bounds |I|, |X| and |Y| of every record).
  * vmax must hold zeros on entry; non-negative floats order as their bits. */
@@ -2805,15 +2830,8 @@ __global__ void k_rec_vmax(PairParams p, float *vmax)
         const float4 v = p.sky4[j];
         sk = fmaxf(sk, fmaxf(fabsf(v.x), fabsf(v.y) + fabsf(v.z)));
     }
-#pragma unroll
-    for (int m = kWaveSize / 2; m > 0; m >>= 1) {
-        g = fmaxf(g, __shfl_xor(g, m, kWaveSize));
-        sk = fmaxf(sk, __shfl_xor(sk, m, kWaveSize));
-    }
-    if (threadIdx.x % kWaveSize == 0) {
-        atomicMax((unsigned *)&vmax[0], __float_as_uint(g));
-        atomicMax((unsigned *)&vmax[1], __float_as_uint(sk));
-    }
+    block_max(g, (unsigned *)&vmax[0]);
+    block_max(sk, (unsigned *)&vmax[1]);
 }
 
 __global__ void k_fill_f64_n(double *x, long n)
@@ -2825,10 +2843,11 @@ __global__ void k_fill_f64_n(double *x, long n)
 
 __global__ void k_fill_i32(int *x, int v) { *x = v; }
 
-/* Last row with a non-zero value in columns 0..5 (wave max, one atomic per
- * wave). */
+/* Last row with a non-zero value in columns 0..5 (block max, one atomic
+ * per block). */
 __global__ void k_beam_support(const float4 *beam8, long npix, int *last)
 {
+    __shared__ int part[16];
     int best = -1;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     for (; i < npix; i += (long)gridDim.x * blockDim.x) {
@@ -2840,8 +2859,15 @@ __global__ void k_beam_support(const float4 *beam8, long npix, int *last)
 #pragma unroll
     for (int m = kWaveSize / 2; m > 0; m >>= 1)
         best = max(best, __shfl_xor(best, m, kWaveSize));
-    if (threadIdx.x % kWaveSize == 0 && best >= 0)
-        atomicMax(last, best);
+    if (threadIdx.x % kWaveSize == 0)
+        part[threadIdx.x / kWaveSize] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < (int)blockDim.x / kWaveSize; w++)
+            best = max(best, part[w]);
+        if (best >= 0)
+            atomicMax(last, best);
+    }
 }
 
 /* Ring records of every ring, indexed by ring number 1 .. 4N-1 (entry 0
@@ -2878,33 +2904,33 @@ __global__ void k_pack_sky(const float *I, const float *Q, const float *U, const
 
 /* Deterministic sky adjoint: out[0] = max over beam rows of the sum of |A0
  * A1 A2 B0 B1 B2|, out[1] = max |g| (as float bits; atomicMax on the bits of
- * non-negative floats orders them as the values). */
-__global__ void k_absmax_rows(const float *beam8, long npix, unsigned *out)
+ * non-negative floats orders them as the values).  gridDim.y: the beams. */
+__global__ void k_absmax(FixSource f, unsigned *out)
 {
-    float best = 0.f;
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    for (; i < npix; i += (long)gridDim.x * blockDim.x) {
-        const float *r = beam8 + 8 * i;
-        float v = fabsf(r[0]) + fabsf(r[1]) + fabsf(r[2]) + fabsf(r[3]) + fabsf(r[4]) +
-                  fabsf(r[5]);
-        best = fmaxf(best, v);
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long stride = (long)gridDim.x * blockDim.x;
+    const float *beam8 = f.beam8;
+    long npix = f.npix;
+    if (f.pairs) {
+        const BatchPair &q = f.pairs[blockIdx.y];
+        beam8 = q.beam;
+        npix = q.out < 0 ? 0 : q.npix;   /* inert padding */
     }
-    for (int m = kWaveSize / 2; m > 0; m >>= 1)
-        best = fmaxf(best, __shfl_xor(best, m, kWaveSize));
-    if (threadIdx.x % kWaveSize == 0)
-        atomicMax(out, __float_as_uint(best));
-}
-
-__global__ void k_absmax(const float *x, long n, unsigned *out)
-{
-    float best = 0.f;
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    for (; i < n; i += (long)gridDim.x * blockDim.x)
-        best = fmaxf(best, fabsf(x[i]));
-    for (int m = kWaveSize / 2; m > 0; m >>= 1)
-        best = fmaxf(best, __shfl_xor(best, m, kWaveSize));
-    if (threadIdx.x % kWaveSize == 0)
-        atomicMax(out, __float_as_uint(best));
+    float rows = 0.f, g = 0.f;
+    for (long i = t; i < npix; i += stride) {
+        const float4 r = *(const float4 *)(beam8 + 8 * i);
+        const float2 s = *(const float2 *)(beam8 + 8 * i + 4);
+        rows = fmaxf(rows, fabsf(r.x) + fabsf(r.y) + fabsf(r.z) + fabsf(r.w) + fabsf(s.x) +
+                               fabsf(s.y));
+    }
+    for (long i = blockIdx.y * stride + t; i < f.n; i += gridDim.y * stride) {
+        if (f.g_a)
+            g = fmaxf(g, fabsf(f.g_a[i]));
+        if (f.g_b)
+            g = fmaxf(g, fabsf(f.g_b[i]));
+    }
+    block_max(rows, out);
+    block_max(g, out + 1);
 }
 
 /* scale = 2^k, the largest power of two with count * bound * scale <= 2^62,
@@ -2926,12 +2952,14 @@ __global__ void k_fix_scale(const unsigned *m, long count, double *scale)
     *scale = s;
 }
 
-__global__ void k_fix_to_f32(const unsigned long long *x, const double *scale, float *y, long n)
+__global__ void k_fix_to_f32(const unsigned long long *x, const double *scale, F32Planes y, long n)
 {
     const double inv = 1.0 / *scale;
+    float *out = y.p[blockIdx.y];
+    x += blockIdx.y * n;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     for (; i < n; i += (long)gridDim.x * blockDim.x)
-        y[i] = (float)((double)(long long)x[i] * inv);
+        out[i] = (float)((double)(long long)x[i] * inv);
 }
 
 __global__ void k_fill_u32(unsigned *x, int n, unsigned v)
@@ -3444,7 +3472,7 @@ hipError_t launch_adjbeam_records(const PairParams &p0, const RecPlan &pl, void 
     hipLaunchKernelGGL(k_fill_f64_n, dim3(gs_blocks((long)pl.npart)), dim3(256), 0, st, part,
                        (long)pl.npart);
     hipLaunchKernelGGL(k_fill_f64_n, dim3(1), dim3(64), 0, st, (double *)vmax, 1L);
-    hipLaunchKernelGGL(k_rec_vmax, dim3(1024), dim3(256), 0, st, p0, vmax);
+    hipLaunchKernelGGL(k_rec_vmax, dim3(kMaxBlocks), dim3(256), 0, st, p0, vmax);
     for (long s0 = p0.s_begin; s0 < p0.s_end; s0 += pl.chunk) {
         PairParams p = p0;
         p.s_begin = s0;
@@ -3483,7 +3511,7 @@ hipError_t launch_beam_support(const float *beam8, long npix, int *last, hipStre
 {
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(1), 0, st, last, -1);
     if (npix > 0)
-        hipLaunchKernelGGL(k_beam_support, dim3(gs_blocks(npix)), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_beam_support, dim3(std::min<unsigned>(gs_blocks(npix), kMaxBlocks)), dim3(256), 0, st,
                            (const float4 *)beam8, npix, last);
     return hipGetLastError();
 }
@@ -3521,32 +3549,25 @@ hipError_t launch_pack_sky(const float *I, const float *Q, const float *U, long 
     return hipGetLastError();
 }
 
-hipError_t launch_fix_scale(const float *const *beams, const long *npix, int nbeams,
-                            const float *g_a, const float *g_b, long nsamples, long count,
-                            unsigned *work, double *scale, hipStream_t st)
+hipError_t launch_fix_scale(const FixSource &f, long count, unsigned *work, double *scale,
+                            hipStream_t st)
 {
+    const int ny = f.pairs ? f.npairs : 1;
+    const long most = std::max(f.pairs ? 1L << 20 : f.npix, (f.n + ny - 1) / ny);
+    const unsigned nx = std::min<unsigned>(gs_blocks(most), std::max(1, kMaxBlocks / ny));
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, work, 2, 0u);
-    for (int k = 0; k < nbeams; k++)
-        if (npix[k] > 0)
-            hipLaunchKernelGGL(k_absmax_rows, dim3(gs_blocks(npix[k])), dim3(256), 0, st,
-                               beams[k], npix[k], work);
-    if (g_a && nsamples > 0)
-        hipLaunchKernelGGL(k_absmax, dim3(gs_blocks(nsamples)), dim3(256), 0, st, g_a, nsamples,
-                           work + 1);
-    if (g_b && nsamples > 0)
-        hipLaunchKernelGGL(k_absmax, dim3(gs_blocks(nsamples)), dim3(256), 0, st, g_b, nsamples,
-                           work + 1);
+    hipLaunchKernelGGL(k_absmax, dim3(nx, ny), dim3(256), 0, st, f, work);
     hipLaunchKernelGGL(k_fix_scale, dim3(1), dim3(1), 0, st, (const unsigned *)work, count,
                        scale);
     return hipGetLastError();
 }
 
-hipError_t launch_fix_to_f32(const double *x, const double *scale, float *y, long n,
+hipError_t launch_fix_to_f32(const double *x, const double *scale, const F32Planes &y, long n,
                              hipStream_t st)
 {
     if (n <= 0)
         return hipSuccess;
-    hipLaunchKernelGGL(k_fix_to_f32, dim3(gs_blocks(n)), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_fix_to_f32, dim3(gs_blocks(n), 3), dim3(256), 0, st,
                        (const unsigned long long *)x, scale, y, n);
     return hipGetLastError();
 }

@@ -236,15 +236,25 @@ hipError_t launch_adjmap_lds(const PairParams &p, int chunk, int cap, int rw, in
 /* group: 0 one pair, 1 per-pair batch items, 2 or 4 pairs per wave; det: the
  * deterministic mode's integer windows; lanes per sample (group 0) */
 size_t adjmap_lds_bytes(int cap, int rw, int group = 0, bool det = false, int lanes = 64);
-/* Deterministic sky adjoint: *scale (device) from the beams (beam8 rows)
- * and the cotangents (g_a, g_b of nsamples floats, either may be NULL);
- * count = the most contributions a pixel can receive; work holds 2 unsigned
- * (device). */
-hipError_t launch_fix_scale(const float *const *beams, const long *npix, int nbeams,
-                            const float *g_a, const float *g_b, long nsamples, long count,
-                            unsigned *work, double *scale, hipStream_t st);
-/* y = int64 bits of x / scale */
-hipError_t launch_fix_to_f32(const double *x, const double *scale, float *y, long n,
+/* Deterministic sky adjoint: *scale (device) from the beam rows of one beam or
+ * of the pairs of a batch (device table), and the cotangents g_a and g_b of n
+ * floats (either may be NULL); count = the most contributions a pixel can
+ * receive; work holds 2 unsigned (device). */
+struct FixSource {
+    const float *beam8;
+    long npix;
+    const BatchPair *pairs;   /* or NULL */
+    int npairs;
+    const float *g_a, *g_b;
+    long n;
+};
+hipError_t launch_fix_scale(const FixSource &f, long count, unsigned *work, double *scale,
+                            hipStream_t st);
+/* y.p[k] = int64 bits of plane k of x, divided by *scale; n per plane */
+struct F32Planes {
+    float *p[3];
+};
+hipError_t launch_fix_to_f32(const double *x, const double *scale, const F32Planes &y, long n,
                              hipStream_t st);
 /* Launch resources of the sky-adjoint kernel, for error messages. */
 int adjmap_describe(char *buf, size_t n, int cap, int rw);
