@@ -148,20 +148,20 @@ int pisco::strips_auto(const PairParams &p, bool adjoint)
 
 /* Lanes per sample of the forward.  Several samples per wave share the table
  * builds, and neighbouring samples meet the same lines of the sky and the beam.
- * ms for 8, 16, 32, 64 lanes over 1e5 samples: 240 pixels per disc 0.18, 0.21,
- * 0.24, 0.24; 960: 0.51, 0.54, 0.57, 0.58; 2,160: 1.04, 1.05, 1.09, 1.23; 16,
- * 32, 64 lanes at 6,000 pixels over 3.6e5 samples 7.99, 8.44, 9.37, but over
- * 6e4, fewer waves, 1.79, 1.64, 1.69; at 54,000 over 2e4 7.9, 6.8, 6.1.  The
- * rule may not look at the number of samples: a sample's sum would depend on
- * it.  A beam that needs strips takes the one-wave kernel: 2.9 MB, 1,500
- * pixels 0.93, 0.96, 0.96, 0.86. */
+ * ms for 8, 16, 32, 64 lanes over 1e5 samples: 540 pixels per disc 0.31, 0.33,
+ * 0.39, 0.45; 1,500: 0.76, 0.73, 0.78, 0.78; 2,160: 1.07, 1.01, 1.06, 1.00;
+ * 15,300: 8.17, 6.69, 6.89, 7.56, but over 2e4, fewer waves, 2.98, 2.26, 1.84,
+ * 1.76; 6,000 over 3.6e5 8.12, 7.77, 8.37, 9.08; 54,000 over 2e4 7.9, 6.8, 6.1
+ * for 16, 32, 64.  The rule may not look at the number of samples: a sample's
+ * sum would depend on it.  A beam that needs strips takes the one-wave kernel:
+ * 4.2 MB, 2,160 pixels 1.99 whole, 1.18 in two strips. */
 int pisco::forward_lanes_auto(const PairParams &p)
 {
     const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
     const double dp = (double)p.hs.npix * s * s;   /* expected pixels per disc */
     if (strips_auto(p, false) > 1)
         return 64;
-    return dp < 1000.0 ? 8 : dp < 3000.0 ? 16 : dp < 30000.0 ? 32 : 64;
+    return dp < 1000.0 ? 8 : dp < 10000.0 ? 16 : dp < 30000.0 ? 32 : 64;
 }
 
 struct pisco_ctx {
@@ -373,10 +373,8 @@ int run_pair(pisco_ctx *c, int op, PairParams p, hipStream_t st, bool sky_packed
         p.s_end = std::min(n, s + chunk);
         if (c->beam_interp)
             HIPCHK(launch_pair_interp(op, p, st));
-        else if (lanes < 64)
-            HIPCHK(launch_fwd_sub(lanes, p, st, op == OP_FWD_V));
         else if (fwd)
-            HIPCHK(launch_forward(p, st, op == OP_FWD_V));
+            HIPCHK(launch_forward(lanes, p, st, op == OP_FWD_V));
         else
             HIPCHK(launch_pair(op, p, st));
     }
@@ -1526,6 +1524,19 @@ std::vector<int> batch_ranges(const pisco_ctx *c, const pisco_batch *b)
     return cut;
 }
 
+/* Lanes per sample of the per-pair items: the single-pair rule for the largest
+ * disc.  16 pairs, 540 pixels per disc, 2.5e4 samples: one wave per sample 1.57
+ * ms, 8 lanes 1.38 ms. */
+int pair_lanes(const BatchParams &b, const BatchPair &q)
+{
+    PairParams p;
+    memset(&p, 0, sizeof p);
+    p.hs = b.hs;
+    p.rho_max = q.rho_max;
+    p.npix_beam = q.npix;
+    return forward_lanes_auto(p);
+}
+
 /* The deterministic mode's scale for a batch: every pair's beam, the
  * cotangents of all pairs (2 npairs nsamples values), at most npairs
  * nsamples contributions per pixel. */
@@ -1652,7 +1663,7 @@ int pisco_dev_batched_forward(pisco_ctx *c, void *stream, const pisco_batch *b, 
         for (long s0 = 0; s0 < nsamples; s0 += chunk) {
             p.s_begin = s0;
             p.s_end = std::min(nsamples, s0 + chunk);
-            HIPCHK(launch_batch_forward(G, p, st));
+            HIPCHK(launch_batch_forward(G, p, st, pair_lanes(p, b->host[r0])));
         }
     }
     return PISCO_OK;
@@ -1687,7 +1698,8 @@ int pisco_dev_batched_forward_pp(pisco_ctx *c, void *stream, const pisco_batch *
     for (long s0 = 0; s0 < nsamples; s0 += chunk) {
         p.s_begin = s0;
         p.s_end = std::min(nsamples, s0 + chunk);
-        HIPCHK(launch_batch_forward(1, p, st));   /* per-pair items: no shared geometry */
+        /* per-pair items: no shared geometry */
+        HIPCHK(launch_batch_forward(1, p, st, pair_lanes(p, b->host[0])));
     }
     return PISCO_OK;
 }

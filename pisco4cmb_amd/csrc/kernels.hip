@@ -439,10 +439,29 @@ struct WaveState {
     unsigned char qj[2 * kWaveSize];
 };
 
-/* Maps queue entries base .. base+cnt-1 (cnt <= 64), one per lane, with the
- * certified double-precision form (beam_pixel_f64, whose own fallback is the
- * exact FP64 path; the beam pixel is the exact path's either way) and hands
- * the visits inside the beam to use(q, ring, startpix, sample).  Called with
+/* Maps pixel pix for sample j with the certified double-precision form
+ * (beam_pixel_f64, whose own fallback is the exact FP64 path; the beam pixel is
+ * the exact path's either way) and hands a visit inside the beam to
+ * use(q, ring, startpix, j). */
+template <int F, typename Use>
+__device__ inline void exact_visit(const PairParams &p, const SampleRec &sr, int pix, int j,
+                                   Use &use)
+{
+    const int r = pix2ring(p.hs, pix);
+    const RingRec rr = p.rings[r];
+    Pending q;
+    q.v = q.s = 0;
+    q.pix = pix;
+    q.live = true;
+    q.bp = beam_pixel_f64(p.hb, p.fc64, rec_centre(sr), sr.c2psi, sr.s2psi,
+                          ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, q.c2, q.s2);
+    if ((unsigned)q.bp < (unsigned)p.npix_beam) {
+        load_visit<F>(p, q, q.bp, pix);
+        use(q, r, rr.startpix, j);
+    }
+}
+
+/* Queue entries base .. base+cnt-1 (cnt <= 64), one per lane.  Called with
  * every lane of the wave active. */
 template <int F, typename WS, typename Use>
 __device__ inline void drain_queue(const PairParams &p, const WS &ws, int base, int cnt, int lane,
@@ -450,20 +469,8 @@ __device__ inline void drain_queue(const PairParams &p, const WS &ws, int base, 
 {
     wave_sync();
     if (lane < cnt) {
-        const int pix = ws.qpix[base + lane], j = ws.qj[base + lane];
-        const int r = pix2ring(p.hs, pix);
-        const RingRec rr = p.rings[r];
-        const SampleRec &sr = ws.rec[j];
-        Pending q;
-        q.v = q.s = 0;
-        q.pix = pix;
-        q.live = true;
-        q.bp = beam_pixel_f64(p.hb, p.fc64, rec_centre(sr), sr.c2psi, sr.s2psi,
-                              ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, q.c2, q.s2);
-        if ((unsigned)q.bp < (unsigned)p.npix_beam) {
-            load_visit<F>(p, q, q.bp, pix);
-            use(q, r, rr.startpix, j);
-        }
+        const int j = ws.qj[base + lane];
+        exact_visit<F>(p, ws.rec[j], ws.qpix[base + lane], j, use);
     }
     wave_sync();
 }
@@ -663,139 +670,182 @@ __device__ inline void wave_samples(const PairParams &p, WS &ws, long i0, int cn
     wave_sync();
 }
 
-using WaveTable = VisitTable<kWaveSize, kWaveSize, 4096>;
-constexpr int kWaveSamples = 8;   /* samples per wave of the forward, at most */
+template <int SUB>
+using SubTable = VisitTable<SUB, (SUB < 16 ? 24 : SUB < 64 ? 32 : 64),
+                            (SUB < 16 ? 256 : SUB < 64 ? 1024 : 4096)>;
+using WaveTable = SubTable<kWaveSize>;
 
-/* Samples i0 .. i0+cnt-1 (cnt <= kWaveSamples) of one detector pair, one after
- * the other on the whole wave; their constants are computed together, one per
- * lane, and their deferred visits share the FP64 drains.  Forward: strip k of
- * p.strips of each disc; the sum of a strip of a sample does not depend on the
- * samples it shares the wave with.  Or the direct-atomic adjoints. */
-template <int OP, typename WS>
-__device__ inline void pair_samples(const PairParams &p, long i0, int cnt, int k, float pa_off,
-                                    bool offset, WaveTable &t, WS &ws, double (*dacc)[2], int lane)
+/* ---- forward ---------------------------------------------------------------
+ *
+ * A wave holds G = 64/SUB samples of SUB lanes each, a block kWavesPerBlock
+ * waves.  The deferred visits that do not fill a batch of 64 are mapped once per
+ * block, by the last wave that finishes, so that no wave waits: the FP64 form
+ * costs the same for one lane as for 64 (5-degree discs in 6 strips: 0.10 of the
+ * time).  The first wave computing the constants of the whole block's samples
+ * was no gain: the others wait for it.
+ *
+ * The runs of a table: 24 and 32 for 8 and 16 lanes (16: more passes, each with
+ * a ragged end; 1.29 and 1.15 ms for 1e6 samples of 135 pixels with 16 lanes),
+ * within the 40 KB of LDS that leave four blocks per CU. */
+template <int SUB>
+struct FwdBlock {
+    static constexpr int G = kWaveSize / SUB, NS = kWavesPerBlock * G;
+    SubTable<SUB> tables[NS];
+    SampleRec rec[NS];
+    int qpix[kWavesPerBlock][2 * kWaveSize];
+    unsigned char qj[kWavesPerBlock][2 * kWaveSize];
+    int qn[kWavesPerBlock], done;
+    double sum[NS][2], dsum[NS][2];   /* of the walks, of the deferred visits */
+};
+
+/* A wave's view of its block: the samples of the block, its own queue. */
+struct WaveView {
+    SampleRec *rec;
+    int *qpix;
+    unsigned char *qj;
+};
+
+/* Samples i0 .. i0+ns-1 (ns <= NS), strip k of their discs: their sums to
+ * put(sample, a, b).  Every thread of the block calls it.  A sample's sums do
+ * not depend on the samples it shares the block with. */
+template <int SUB, bool VT, typename Put>
+__device__ inline void forward_block(const PairParams &p, FwdBlock<SUB> &B, long i0, int ns, int k,
+                                     float pa_off, bool offset, Put &put)
 {
-    constexpr bool FWD = OP == OP_FWD || OP == OP_FWD_V;
-    constexpr int F = WALK_CHI | (FWD || OP == OP_ADJ_MAP ? WALK_BEAM : 0) | (FWD ? WALK_SKY : 0) |
-                      (OP == OP_FWD_V ? WALK_V : 0);
-    wave_samples(p, ws, i0, cnt, pa_off, offset, lane);
-    if (FWD && lane < 2 * cnt)
-        dacc[lane >> 1][lane & 1] = 0.0;   /* sums of deferred visits */
-    wave_sync();
-    double acc_a = 0.0, acc_b = 0.0, ga = 0.0, gb = 0.0;
-    auto use = [&](const Pending &q) {
-        if constexpr (FWD) {
-            visit_tod<OP == OP_FWD_V>(q, acc_a, acc_b);
-        } else if constexpr (OP == OP_ADJ_MAP) {
-            const float A0 = q.v0.x, A1 = q.v0.y, A2 = q.v0.z;
-            const float B0 = q.v0.w, B1 = q.v1.x, B2 = q.v1.y;
-            double cc = q.c2, ss = q.s2;
-            double vI = ga * A0 + gb * B0;
-            double vQ = ga * (A1 * cc - A2 * ss) + gb * (-B1 * cc + B2 * ss);
-            double vU = ga * (A2 * cc + A1 * ss) + gb * (-B2 * cc - B1 * ss);
-            unsafeAtomicAdd(&p.gI[q.pix], vI);
-            unsafeAtomicAdd(&p.gQ[q.pix], vQ);
-            unsafeAtomicAdd(&p.gU[q.pix], vU);
-        } else {
-            double cc = q.c2, ss = q.s2;
-            double qq = p.Q[q.pix], u = p.U[q.pix], sI = p.I[q.pix];
-            double *g = p.gbeam + 8 * (long)q.bp;
-            unsafeAtomicAdd(&g[0], ga * sI);
-            unsafeAtomicAdd(&g[1], ga * (qq * cc + u * ss));
-            unsafeAtomicAdd(&g[2], ga * (-qq * ss + u * cc));
-            unsafeAtomicAdd(&g[3], gb * sI);
-            unsafeAtomicAdd(&g[4], gb * (-qq * cc - u * ss));
-            unsafeAtomicAdd(&g[5], gb * (qq * ss - u * cc));
-        }
-    };
-    auto use_exact = [&](const Pending &q, int, int, int j) {
-        if constexpr (FWD) {
-            double a = 0.0, b = 0.0;
-            visit_tod<OP == OP_FWD_V>(q, a, b);
-            atomicAdd(&dacc[j][0], a);
-            atomicAdd(&dacc[j][1], b);
-        } else {
-            use(q);   /* the adjoints take one sample per wave */
-        }
+    constexpr int G = FwdBlock<SUB>::G;
+    constexpr int F = WALK_SKY | WALK_BEAM | WALK_CHI | (VT ? WALK_V : 0);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int lane = threadIdx.x % kWaveSize;
+    const int grp = lane / SUB, sl = lane % SUB;
+    WaveView ws = {B.rec, B.qpix[wave], B.qj[wave]};
+    if (threadIdx.x < 2 * ns)
+        B.dsum[threadIdx.x >> 1][threadIdx.x & 1] = 0.0;
+    if (threadIdx.x == 0)
+        B.done = 0;
+    const int j0 = wave * G;
+    if (j0 < ns) {
+        WaveView own = {B.rec + j0, nullptr, nullptr};
+        wave_samples(p, own, i0 + j0, min(G, ns - j0), pa_off, offset, lane);
+    }
+    __syncthreads();
+    if (j0 >= ns)
+        return;
+    const int j = j0 + grp < ns ? j0 + grp : j0;   /* a group without a sample idles */
+    SampleF sf = B.rec[j].sf;
+    int r0 = B.rec[j].r_first, r1 = B.rec[j].r_last;
+    if constexpr (SUB == kWaveSize) {
+        sf = unif(sf);
+        r0 = __builtin_amdgcn_readfirstlane(r0);
+        r1 = __builtin_amdgcn_readfirstlane(r1);
+        const int m = (r1 - r0 + p.strips) / p.strips;   /* rings per strip */
+        r0 += k * m;
+        r1 = min(r1, r0 + m - 1);
+    } else if (j0 + grp >= ns) {
+        r1 = r0 - 1;
+    }
+    double acc_a = 0.0, acc_b = 0.0;
+    auto use = [&](const Pending &q) { visit_tod<VT>(q, acc_a, acc_b); };
+    auto use_exact = [&](const Pending &q, int, int, int jj) {
+        double a = 0.0, b = 0.0;
+        visit_tod<VT>(q, a, b);
+        atomicAdd(&B.dsum[jj][0], a);
+        atomicAdd(&B.dsum[jj][1], b);
     };
     auto after = [](const Pass &) {};
     int qn = 0;
-    double sum_a = 0.0, sum_b = 0.0;   /* lane j: the sums of sample j */
-    for (int j = 0; j < cnt; j++) {
-        const SampleF sf = unif(ws.rec[j].sf);
-        int r0 = __builtin_amdgcn_readfirstlane(ws.rec[j].r_first);
-        int r1 = __builtin_amdgcn_readfirstlane(ws.rec[j].r_last);
-        if constexpr (FWD) {
-            const int m = (r1 - r0 + p.strips) / p.strips;   /* rings per strip */
-            r0 += k * m;
-            r1 = min(r1, r0 + m - 1);
-        } else {
-            ga = uni(p.g_a ? (double)p.g_a[i0] : 0.0);   /* one sample */
-            gb = uni(p.g_b ? (double)p.g_b[i0] : 0.0);
-        }
-        walk_rings<F>(p, t, ws, j, r0, r1, lane, sf, FWD ? kEtaForward : kEtaAdjoint, qn, after,
-                      use, use_exact);
-        if constexpr (FWD) {
-            const double a = wave_sum(acc_a), b = wave_sum(acc_b);
-            sum_a = lane == j ? a : sum_a;
-            sum_b = lane == j ? b : sum_b;
-            acc_a = acc_b = 0.0;
-        }
+    walk_rings<F>(p, B.tables[j0 + grp], ws, j, r0, r1, sl, sf, kEtaForward, qn, after, use,
+                  use_exact);
+#pragma unroll
+    for (int m = SUB / 2; m > 0; m >>= 1) {
+        acc_a += __shfl_xor(acc_a, m, SUB);
+        acc_b += __shfl_xor(acc_b, m, SUB);
     }
-    if (qn > 0)
-        drain_queue<F>(p, ws, 0, qn, lane, use_exact);
-    if constexpr (FWD) {
-        if (lane < cnt) {
-            const long i = i0 + lane;
-            sum_a += dacc[lane][0];
-            sum_b += dacc[lane][1];
-            if (p.strips > 1) {
-                const long n = p.s_end - p.s_begin;
-                p.part[(2 * k) * n + i - p.s_begin] = sum_a;
-                p.part[(2 * k + 1) * n + i - p.s_begin] = sum_b;
-            } else {
-                if (p.tod_a)
-                    p.tod_a[i] = (float)sum_a;
-                if (p.tod_b)
-                    p.tod_b[i] = (float)sum_b;
+    if (sl == 0 && j0 + grp < ns) {
+        B.sum[j0 + grp][0] = acc_a;
+        B.sum[j0 + grp][1] = acc_b;
+    }
+    if (lane == 0)
+        B.qn[wave] = qn;
+    const int waves = (ns + G - 1) / G;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    int arrived = 0;
+    if (lane == 0)
+        arrived = atomicAdd(&B.done, 1);
+    if (__builtin_amdgcn_readfirstlane(arrived) != waves - 1)
+        return;
+    /* the last wave of the block */
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    int end[kWavesPerBlock], total = 0;
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; w++) {
+        total += w < waves ? __builtin_amdgcn_readfirstlane(B.qn[w]) : 0;
+        end[w] = total;
+    }
+    for (int e0 = 0; e0 < total; e0 += kWaveSize) {
+        const int e = e0 + lane;
+        if (e < total) {
+            int w = 0, first = 0;
+#pragma unroll
+            for (int x = 0; x < kWavesPerBlock - 1; x++) {
+                w = e >= end[x] ? x + 1 : w;
+                first = e >= end[x] ? end[x] : first;
             }
+            const int jj = B.qj[w][e - first];
+            exact_visit<F>(p, B.rec[jj], B.qpix[w][e - first], jj, use_exact);
         }
+        wave_sync();
     }
+    wave_sync();
+    if (lane < ns)
+        put(lane, B.sum[lane][0] + B.dsum[lane][0], B.sum[lane][1] + B.dsum[lane][1]);
 }
 
-/* The forward: p.group consecutive samples per wave; or, p.strips > 1, a strip
- * of the disc of one sample, in chunks of kStripChunk samples and within a
- * chunk by strip.  The beam rows that a strip of the sky meets are about a
- * strip of the beam, nearly the same one for samples close in the scan, so that
- * this part stays in the XCD's L2; with whole discs the waves gather from all
- * of a 12 MB beam.  The samples in flight have to be close: with 2, 4 and 8
- * samples per wave (1,024 to 4,096 in flight per XCD) the L2 hit rate fell from
- * 0.93 to 0.83, 0.71 and 0.56; hence one sample per wave, whose constants
- * k_samples computes. */
+/* The forward of one pair: consecutive samples, whole discs; or (SUB = 64,
+ * p.strips > 1) a strip of each disc, in chunks of kStripChunk samples and
+ * within a chunk by strip.  The beam rows that a strip of the sky meets are
+ * about a strip of the beam, nearly the same one for samples close in the scan,
+ * so that this part stays in the XCD's L2; with whole discs the waves gather
+ * from all of a 12 MB beam.  The samples in flight have to be close: with 2, 4
+ * and 8 samples per wave (1,024 to 4,096 in flight per XCD) the L2 hit rate fell
+ * from 0.93 to 0.83, 0.71 and 0.56; hence one sample per wave, whose constants
+ * k_samples computes once for all strips.
+ *
+ * Bound: a visit gathers a 128-byte line of the beam, 2.15 cycles each per CU
+ * (140 cycles per 64 visits), and takes about 130 vector instructions per 64;
+ * both units are 0.84 to 0.96 busy at 5 degrees. */
 constexpr int kStripChunk = 4096;
 
-template <int OP>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd(PairParams p)
+template <int SUB, bool VT = false>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd_sub(PairParams p)
 {
-    __shared__ WaveTable tables[kWavesPerBlock];
-    __shared__ WaveState<kWaveSamples> states[kWavesPerBlock];
-    __shared__ double dacc[kWavesPerBlock][kWaveSamples][2];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-    const int lane = threadIdx.x % kWaveSize;
+    __shared__ FwdBlock<SUB> B;
+    constexpr int NS = FwdBlock<SUB>::NS;
     const long lb = xcd_remap(blockIdx.x, gridDim.x);
-    long i0 = p.s_begin + (lb * kWavesPerBlock + wave) * p.group;
+    long i0 = p.s_begin + lb * NS;
     int k = 0;
-    if (p.strips > 1) {
-        constexpr int MB = kStripChunk / kWavesPerBlock;
+    if (SUB == kWaveSize && p.strips > 1) {
+        constexpr int MB = kStripChunk / NS;
         const long c = lb / (MB * p.strips);
         const int rem = (int)(lb - c * (MB * p.strips));
         k = rem / MB;
-        i0 = p.s_begin + c * kStripChunk + (rem - k * MB) * kWavesPerBlock + wave;
+        i0 = p.s_begin + c * kStripChunk + (rem - k * MB) * NS;
     }
     if (i0 >= p.s_end)
         return;
-    pair_samples<OP>(p, i0, (int)min((long)p.group, p.s_end - i0), k, 0.f, false, tables[wave],
-                     states[wave], dacc[wave], lane);
+    auto put = [&](int j, double a, double b) {
+        const long i = i0 + j;
+        if (SUB == kWaveSize && p.strips > 1) {
+            const long n = p.s_end - p.s_begin;
+            p.part[(2 * k) * n + i - p.s_begin] = a;
+            p.part[(2 * k + 1) * n + i - p.s_begin] = b;
+        } else {
+            if (p.tod_a)
+                p.tod_a[i] = (float)a;
+            if (p.tod_b)
+                p.tod_b[i] = (float)b;
+        }
+    };
+    forward_block<SUB, VT>(p, B, i0, (int)min((long)NS, p.s_end - i0), k, 0.f, false, put);
 }
 
 /* The samples' constants, one per thread. */
@@ -831,6 +881,7 @@ __global__ void k_strip_sum(PairParams p)
 template <int OP>
 __global__ __launch_bounds__(kBlock) void k_pair(PairParams p)
 {
+    constexpr int F = WALK_CHI | (OP == OP_ADJ_MAP ? WALK_BEAM : 0);
     __shared__ WaveTable tables[kWavesPerBlock];
     __shared__ WaveState<1> states[kWavesPerBlock];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
@@ -838,72 +889,41 @@ __global__ __launch_bounds__(kBlock) void k_pair(PairParams p)
     const long i = p.s_begin + xcd_remap(blockIdx.x, gridDim.x) * kWavesPerBlock + wave;
     if (i >= p.s_end)
         return;
-    pair_samples<OP>(p, i, 1, 0, 0.f, false, tables[wave], states[wave], nullptr, lane);
-}
-
-/* ---- small-disc forward: several samples per wave -------------------------
- *
- * For discs of a few hundred pixels the per-sample part of k_fwd (the table
- * build, the final reduction) runs on all 64 lanes for one sample and costs
- * more than the visits.  Here a wave holds G = 64/SUB samples of SUB lanes
- * each: that part runs once for the G samples, each lane group walks its own
- * disc SUB visits at a time, and a SUB-lane reduction gives each sample's TOD.
- * The mapping, the per-visit values and the FP64 accumulation are those of
- * k_fwd. */
-template <int SUB>
-using SubTable = VisitTable<SUB, (SUB < 16 ? 16 : SUB), (SUB < 16 ? 512 : 64 * SUB)>;
-
-template <int SUB, bool VT = false>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd_sub(PairParams p)
-{
-    constexpr int G = kWaveSize / SUB;
-    __shared__ SubTable<SUB> tables[kWavesPerBlock * G];
-    __shared__ WaveState<G> states[kWavesPerBlock];
-    __shared__ double dacc[kWavesPerBlock][G][2];   /* sums of deferred visits */
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-    const int lane = threadIdx.x % kWaveSize;
-    const int grp = lane / SUB, sl = lane % SUB;
-    const long lb = xcd_remap(blockIdx.x, gridDim.x);
-    const long w0 = p.s_begin + (lb * kWavesPerBlock + wave) * G;   /* the wave's first sample */
-    if (w0 >= p.s_end)
-        return;   /* wave-uniform */
-    const int cnt = (int)min((long)G, p.s_end - w0);
-    WaveState<G> &ws = states[wave];
-    if (lane < 2 * G)
-        dacc[wave][lane >> 1][lane & 1] = 0.0;
-    wave_samples(p, ws, w0, cnt, 0.f, false, lane);
-    const int j = grp < cnt ? grp : 0;   /* a group without a sample idles */
-    const SampleF sf = ws.rec[j].sf;
-    double acc_a = 0.0, acc_b = 0.0;
-    auto use = [&](const Pending &e) { visit_tod<VT>(e, acc_a, acc_b); };
-    auto use_exact = [&](const Pending &e, int, int, int g) {
-        double a = 0.0, b = 0.0;
-        visit_tod<VT>(e, a, b);
-        atomicAdd(&dacc[wave][g][0], a);
-        atomicAdd(&dacc[wave][g][1], b);
+    auto &ws = states[wave];
+    wave_samples(p, ws, i, 1, 0.f, false, lane);
+    const double ga = uni(p.g_a ? (double)p.g_a[i] : 0.0);
+    const double gb = uni(p.g_b ? (double)p.g_b[i] : 0.0);
+    auto use = [&](const Pending &q) {
+        if constexpr (OP == OP_ADJ_MAP) {
+            const float A0 = q.v0.x, A1 = q.v0.y, A2 = q.v0.z;
+            const float B0 = q.v0.w, B1 = q.v1.x, B2 = q.v1.y;
+            double cc = q.c2, ss = q.s2;
+            double vI = ga * A0 + gb * B0;
+            double vQ = ga * (A1 * cc - A2 * ss) + gb * (-B1 * cc + B2 * ss);
+            double vU = ga * (A2 * cc + A1 * ss) + gb * (-B2 * cc - B1 * ss);
+            unsafeAtomicAdd(&p.gI[q.pix], vI);
+            unsafeAtomicAdd(&p.gQ[q.pix], vQ);
+            unsafeAtomicAdd(&p.gU[q.pix], vU);
+        } else {
+            double cc = q.c2, ss = q.s2;
+            double qq = p.Q[q.pix], u = p.U[q.pix], sI = p.I[q.pix];
+            double *g = p.gbeam + 8 * (long)q.bp;
+            unsafeAtomicAdd(&g[0], ga * sI);
+            unsafeAtomicAdd(&g[1], ga * (qq * cc + u * ss));
+            unsafeAtomicAdd(&g[2], ga * (-qq * ss + u * cc));
+            unsafeAtomicAdd(&g[3], gb * sI);
+            unsafeAtomicAdd(&g[4], gb * (-qq * cc - u * ss));
+            unsafeAtomicAdd(&g[5], gb * (qq * ss - u * cc));
+        }
     };
+    auto use_exact = [&](const Pending &q, int, int, int) { use(q); };
     auto after = [](const Pass &) {};
-    constexpr int F = WALK_SKY | WALK_BEAM | WALK_CHI | (VT ? WALK_V : 0);
     int qn = 0;
-    walk_rings<F>(p, tables[wave * G + grp], ws, j, ws.rec[j].r_first,
-                  grp < cnt ? ws.rec[j].r_last : ws.rec[j].r_first - 1, sl, sf, kEtaForward, qn,
-                  after, use, use_exact);
+    walk_rings<F>(p, tables[wave], ws, 0, __builtin_amdgcn_readfirstlane(ws.rec[0].r_first),
+                  __builtin_amdgcn_readfirstlane(ws.rec[0].r_last), lane, unif(ws.rec[0].sf),
+                  kEtaAdjoint, qn, after, use, use_exact);
     if (qn > 0)
         drain_queue<F>(p, ws, 0, qn, lane, use_exact);
-#pragma unroll
-    for (int m = SUB / 2; m > 0; m >>= 1) {
-        acc_a += __shfl_xor(acc_a, m, SUB);
-        acc_b += __shfl_xor(acc_b, m, SUB);
-    }
-    if (grp < cnt && sl == 0) {
-        const long i = w0 + grp;
-        acc_a += dacc[wave][grp][0];
-        acc_b += dacc[wave][grp][1];
-        if (p.tod_a)
-            p.tod_a[i] = (float)acc_a;
-        if (p.tod_b)
-            p.tod_b[i] = (float)acc_b;
-    }
 }
 
 /* ---- beam interpolation mode ----------------------------------------------
@@ -1093,32 +1113,30 @@ __device__ inline PairParams batch_pair_params(const BatchParams &b, const Batch
     return p;
 }
 
-/* Batched form of k_fwd: one wave per (pair, kPairSamples samples) item in the
- * order of batch_item; each item is exactly the single-pair computation with
+/* Batched form of k_fwd_sub: a block per (pair, NS samples) item in the order
+ * of batch_item; each sample is the single-pair computation with
  * pa = (float)(pa + pa_offset). */
-constexpr int kPairSamples = 4;
-
+template <int SUB>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_batch_pair(BatchParams b)
 {
-    __shared__ WaveTable tables[kWavesPerBlock];
-    __shared__ WaveState<kPairSamples> states[kWavesPerBlock];
-    __shared__ double dacc[kWavesPerBlock][kPairSamples][2];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-    const int lane = threadIdx.x % kWaveSize;
+    __shared__ FwdBlock<SUB> B;
+    constexpr int NS = FwdBlock<SUB>::NS;
     const long lb = xcd_remap(blockIdx.x, gridDim.x);
-    const long w = lb * kWavesPerBlock + wave;
     const long n = b.s_end - b.s_begin;
     long k, j;
-    if (!batch_item(w, (n + kPairSamples - 1) / kPairSamples, b.npairs, k, j))
+    if (!batch_item(lb, (n + NS - 1) / NS, b.npairs, k, j))
         return;
     const BatchPair &q = b.pairs[k];
     if (q.out < 0)
         return;   /* inert padding */
-    const long i0 = b.s_begin + j * kPairSamples;
+    const long i0 = b.s_begin + j * NS;
     const PairParams p = batch_pair_params(b, q);
-    pair_samples<OP_FWD>(p, i0, (int)min((long)kPairSamples, b.s_end - i0), 0, q.pa_off, true,
-                         tables[wave], states[wave], dacc[wave], lane);
+    auto put = [&](int l, double x, double y) {
+        p.tod_a[i0 + l] = (float)x;
+        p.tod_b[i0 + l] = (float)y;
+    };
+    forward_block<SUB, false>(p, B, i0, (int)min((long)NS, b.s_end - i0), 0, q.pa_off, true, put);
 }
 
 /* ---- batched forward: many detector pairs on one pointing ----------------
@@ -3158,62 +3176,40 @@ hipError_t launch_pair(int op, const PairParams &p, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_forward(const PairParams &p0, hipStream_t st, bool vterm)
+template <int SUB>
+static void launch_fwd_lanes(const PairParams &p, hipStream_t st, bool vterm)
+{
+    constexpr int NS = FwdBlock<SUB>::NS;
+    const long n = p.s_end - p.s_begin;
+    const unsigned nb = p.strips > 1
+                            ? (unsigned)((n + kStripChunk - 1) / kStripChunk * (kStripChunk / NS) * p.strips)
+                            : nblocks(n, NS);
+    if (vterm)
+        hipLaunchKernelGGL((k_fwd_sub<SUB, true>), dim3(nb), dim3(kBlock), 0, st, p);
+    else
+        hipLaunchKernelGGL((k_fwd_sub<SUB, false>), dim3(nb), dim3(kBlock), 0, st, p);
+}
+
+hipError_t launch_forward(int lanes, const PairParams &p0, hipStream_t st, bool vterm)
 {
     const long n = p0.s_end - p0.s_begin;
     if (n <= 0)
         return hipSuccess;
     PairParams p = p0;
-    if (!p.samples)
+    if (!p.samples || lanes != kWaveSize)
         p.strips = 1;
-    long nb;
-    if (p.strips > 1) {
-        p.group = 1;
-        nb = (n + kStripChunk - 1) / kStripChunk * (kStripChunk / kWavesPerBlock) * p.strips;
+    if (p.strips > 1)
         hipLaunchKernelGGL(k_samples, dim3(nblocks(n, 64)), dim3(64), 0, st, p);
-    } else {
-        /* samples per wave: as many as leave 16 rounds of resident waves */
-        p.group = kWaveSamples;
-        while (p.group > 1 && n / p.group < 65536)
-            p.group >>= 1;
-        nb = nblocks(n, kWavesPerBlock * p.group);
+    switch (lanes) {
+    case 8: launch_fwd_lanes<8>(p, st, vterm); break;
+    case 16: launch_fwd_lanes<16>(p, st, vterm); break;
+    case 32: launch_fwd_lanes<32>(p, st, vterm); break;
+    case 64: launch_fwd_lanes<64>(p, st, vterm); break;
+    default: return hipErrorInvalidValue;
     }
-    if (vterm)
-        hipLaunchKernelGGL(k_fwd<OP_FWD_V>, dim3((unsigned)nb), dim3(kBlock), 0, st, p);
-    else
-        hipLaunchKernelGGL(k_fwd<OP_FWD>, dim3((unsigned)nb), dim3(kBlock), 0, st, p);
     if (p.strips > 1)
         hipLaunchKernelGGL(k_strip_sum, dim3(gs_blocks(n)), dim3(256), 0, st, p);
     return hipGetLastError();
-}
-
-template <bool VT>
-static hipError_t launch_fwd_sub_vt(int sub, const PairParams &p, long n, hipStream_t st)
-{
-    switch (sub) {
-    case 8:
-        hipLaunchKernelGGL((k_fwd_sub<8, VT>), dim3(nblocks(n, kWavesPerBlock * 8)), dim3(kBlock),
-                           0, st, p);
-        break;
-    case 16:
-        hipLaunchKernelGGL((k_fwd_sub<16, VT>), dim3(nblocks(n, kWavesPerBlock * 4)),
-                           dim3(kBlock), 0, st, p);
-        break;
-    case 32:
-        hipLaunchKernelGGL((k_fwd_sub<32, VT>), dim3(nblocks(n, kWavesPerBlock * 2)),
-                           dim3(kBlock), 0, st, p);
-        break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_fwd_sub(int sub, const PairParams &p, hipStream_t st, bool vterm)
-{
-    long n = p.s_end - p.s_begin;
-    if (n <= 0)
-        return hipSuccess;
-    return vterm ? launch_fwd_sub_vt<true>(sub, p, n, st) : launch_fwd_sub_vt<false>(sub, p, n, st);
 }
 
 hipError_t launch_pair_interp(int op, const PairParams &p, hipStream_t st)
@@ -3235,7 +3231,15 @@ hipError_t launch_pair_interp(int op, const PairParams &p, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st)
+template <int SUB>
+static void launch_batch_pairs(const BatchParams &p, long n, hipStream_t st)
+{
+    constexpr int NS = FwdBlock<SUB>::NS;
+    hipLaunchKernelGGL(k_batch_pair<SUB>, dim3((unsigned)batch_items((n + NS - 1) / NS, p.npairs)),
+                       dim3(kBlock), 0, st, p);
+}
+
+hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st, int lanes)
 {
     const long n = p.s_end - p.s_begin;
     if (n <= 0)
@@ -3243,10 +3247,13 @@ hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st)
     const unsigned g = nblocks(batch_items(n, p.ngroups), kWavesPerBlock);
     switch (group) {
     case 1:
-        hipLaunchKernelGGL(k_batch_pair,
-                           dim3(nblocks(batch_items((n + kPairSamples - 1) / kPairSamples, p.npairs),
-                                        kWavesPerBlock)),
-                           dim3(kBlock), 0, st, p);
+        switch (lanes) {
+        case 8: launch_batch_pairs<8>(p, n, st); break;
+        case 16: launch_batch_pairs<16>(p, n, st); break;
+        case 32: launch_batch_pairs<32>(p, n, st); break;
+        case 64: launch_batch_pairs<64>(p, n, st); break;
+        default: return hipErrorInvalidValue;
+        }
         break;
     case 2: hipLaunchKernelGGL(k_batch_fwd<2>, dim3(g), dim3(kBlock), 0, st, p); break;
     case 4: hipLaunchKernelGGL(k_batch_fwd<4>, dim3(g), dim3(kBlock), 0, st, p); break;

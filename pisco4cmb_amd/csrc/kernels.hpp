@@ -42,11 +42,10 @@ struct PairParams {
     const float *beam;
     /* strips of rings that a disc is cut into (1: not cut), with the constants
      * of the launch's samples and, forward, the strips' sums [strip][a, b]
-     * [sample of the launch]; samples per wave of the forward */
+     * [sample of the launch] */
     int strips;
     SampleRec *samples;
     double *part;
-    int group;
     /* device int: index of the last beam row whose A0 A1 A2 B0 B1 B2 are not
      * all zero (-1: none), or NULL.  Only sizes the sky adjoint's LDS
      * windows; every visit of the rho_max disc is still computed. */
@@ -155,15 +154,15 @@ struct FocalPlaneParams {
 };
 hipError_t launch_focal_plane(const FocalPlaneParams &q, hipStream_t st);
 
-hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st);
+hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st, int lanes = 64);
 
 /* The direct-atomic adjoints. */
 hipError_t launch_pair(int op, const PairParams &p, hipStream_t st);
-/* The forward, one wave per sample and strip.  With p.strips > 1 at most
- * kStripLaunch samples, p.samples and p.part in a workspace of
- * strip_bytes(p.strips) bytes (strip_workspace); whole discs if p.samples is
+/* The forward of one pair with 8, 16, 32 or 64 lanes per sample.  With 64 and
+ * p.strips > 1 at most kStripLaunch samples, p.samples and p.part in a workspace
+ * of strip_bytes(p.strips) bytes (strip_workspace); whole discs if p.samples is
  * NULL. */
-hipError_t launch_forward(const PairParams &p, hipStream_t st, bool vterm = false);
+hipError_t launch_forward(int lanes, const PairParams &p, hipStream_t st, bool vterm = false);
 constexpr long kStripLaunch = 1L << 17;
 constexpr int kMaxStrips = 8;
 /* Waves per block of the sky adjoint: two blocks per CU, so that one block's
@@ -181,9 +180,6 @@ inline void strip_workspace(PairParams &p, void *ws)
 }
 /* The beam-interpolation mode of the same operations (k_pair_interp). */
 hipError_t launch_pair_interp(int op, const PairParams &p, hipStream_t st);
-/* Forward with 64/sub samples per wave, sub = 8, 16 or 32 lanes each (small
- * discs); same results as launch_forward. */
-hipError_t launch_fwd_sub(int sub, const PairParams &p, hipStream_t st, bool vterm = false);
 /* Beam adjoint in LDS bands of beam rows (work items: band x chunk of
  * samples); p.gbeam accumulates in FP64, p.sky4 holds the packed sky.  rows:
  * rows per band (0 or more than fits: as many as fit the LDS). */

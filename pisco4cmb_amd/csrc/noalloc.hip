@@ -127,7 +127,7 @@ int pisco_dev_forward_noalloc(void *stream, int nside_sky, const float *I, const
     for (long s = 0; s < nsamples; s += chunk) {
         p.s_begin = s;
         p.s_end = std::min(nsamples, s + chunk);
-        e = lanes < 64 ? launch_fwd_sub(lanes, p, st) : launch_forward(p, st);
+        e = launch_forward(lanes, p, st);
         if (e != hipSuccess)
             return errorf(PISCO_ERR_DEVICE, "forward launch failed: %s", hipGetErrorString(e));
     }

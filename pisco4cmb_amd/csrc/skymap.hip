@@ -397,7 +397,8 @@ __global__ __launch_bounds__(kHeadThreads) void k_mm_heads(const unsigned *keys,
                                                            int many, int *heads, int *nheads,
                                                            unsigned long long *skipped)
 {
-    __shared__ int num[3], base[2];
+    __shared__ int num[3];
+    __shared__ int base[2];
     const int i = blockIdx.x * kHeadThreads + threadIdx.x, lane = threadIdx.x & 63;
     if (threadIdx.x < 3)
         num[threadIdx.x] = 0;
