@@ -2560,14 +2560,55 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_excl(long *x, long n)
         x[n] = part[t];
 }
 
-__device__ inline int rec_band(const RecParams &R, int bp)
+/* Band and row of a beam pixel.  tile == 0: consecutive rows.  Otherwise a band
+ * is a patch of the polar cap: `tile` rings by `tile` pixels of a quadrant (ring
+ * i has i pixels per quadrant), block t of rings and column c <= t, numbered
+ * 2 t (t + 1) + quadrant (t + 1) + c.  A sky pixel is several beam pixels, so
+ * along a sky ring each visit is in another block of consecutive rows (1.5 outer
+ * rings hold 3,400 pixels) and the 64 records of a wave went to 64 lines; of a
+ * patch it crosses about seven visits at a time. */
+__device__ inline int rec_band(const RecParams &R, int bp, int &row)
 {
-    int b = (int)((float)bp * R.inv_rows);
-    if (b * R.rows > bp)
-        b--;
-    else if ((b + 1) * R.rows <= bp)
-        b++;
-    return b;
+    if (R.tile == 0) {
+        int b = (int)((float)bp * R.inv_rows);
+        if (b * R.rows > bp)
+            b--;
+        else if ((b + 1) * R.rows <= bp)
+            b++;
+        row = bp - b * R.rows;
+        return b;
+    }
+    /* ring i = 1, 2, ... starts at 2 i (i - 1); the estimate is off by at most 1 */
+    int i = (int)(0.5f * (1.0f + __builtin_amdgcn_sqrtf(fmaf(2.0f, (float)bp, 1.0f))));
+    int j = bp - 2 * i * (i - 1);
+    if (j < 0) {
+        i--;
+        j += 4 * i;
+    } else if (j >= 4 * i) {
+        j -= 4 * i;
+        i++;
+    }
+    const int q = (j >= i) + (j >= 2 * i) + (j >= 3 * i);
+    j -= q * i;
+    const int t = (int)(((float)i - 0.5f) * R.inv_tile);   /* (i - 1) / tile */
+    const int c = (int)(((float)j + 0.5f) * R.inv_tile);
+    row = (i - 1 - t * R.tile) * R.tile + (j - c * R.tile);
+    return (2 * t + q) * (t + 1) + c;
+}
+
+/* The beam pixel of a row of band b, or -1 if it has none. */
+__device__ inline int rec_pixel(const RecParams &R, int b, int row, int npix)
+{
+    int bp = b * R.rows + row;
+    if (R.tile) {
+        int t = (int)(0.5f * (__builtin_amdgcn_sqrtf(fmaf(2.0f, (float)b, 1.0f)) - 1.0f));
+        t += 2 * (t + 1) * (t + 2) <= b;
+        t -= 2 * t * (t + 1) > b;
+        const int rem = b - 2 * t * (t + 1), q = rem / (t + 1), c = rem - q * (t + 1);
+        const int u = row / R.tile, i = t * R.tile + u + 1, j = c * R.tile + (row - u * R.tile);
+        bp = j < i ? 2 * i * (i - 1) + q * i + j : npix;
+    }
+    return bp < npix ? bp : -1;
 }
 
 /* Steps 1 and 3: one wave per sample of the chunk [p.s_begin, p.s_end),
@@ -2627,12 +2668,13 @@ void k_beamrec(PairParams p, RecParams R)
         if constexpr (WRITE) {
             const unsigned smp_key = (unsigned)j << kRecRowBits;
             auto write = [&](const Pending &q) {
-                const int b = rec_band(R, q.bp);
+                int row;
+                const int b = rec_band(R, q.bp, row);
                 const unsigned slot = atomicAdd(&cur[b], 1u);
                 if (slot >= (unsigned)R.nrec_cap)
                     return;   /* never: both passes count the same visits */
                 BeamRec r;
-                r.key = (unsigned)(q.bp - b * R.rows) | smp_key;
+                r.key = (unsigned)row | smp_key;
                 r.sI = q.sI;
                 r.X = fmaf(q.sQ, q.c2, q.sU * q.s2);
                 r.Y = fmaf(q.sU, q.c2, -(q.sQ * q.s2));
@@ -2645,7 +2687,10 @@ void k_beamrec(PairParams p, RecParams R)
             if (qn > 0)
                 drain_queue<F>(p, ws, 0, qn, lane, write_exact);
         } else {
-            auto count = [&](const Pending &q) { atomicAdd(&cur[rec_band(R, q.bp)], 1u); };
+            auto count = [&](const Pending &q) {
+                int row;
+                atomicAdd(&cur[rec_band(R, q.bp, row)], 1u);
+            };
             auto count_exact = [&](const Pending &q, int, int, int) { count(q); };
             walk_rings<0>(p, t, ws, 0, r0, r1, lane, sf, kEtaAdjoint, qn, after, count,
                           count_exact);
@@ -2712,8 +2757,7 @@ __global__ __launch_bounds__(kBandBlock) void k_beamrec_sum(PairParams p, RecPar
     unsigned long long *acc = (unsigned long long *)smem;
     const int tid = threadIdx.x;
     const int b = blockIdx.x / R.nsplit, part = blockIdx.x % R.nsplit;
-    const int lo = b * R.rows;
-    const int nrow = min(p.npix_beam - lo, R.rows);
+    const int nrow = R.tile ? R.rows : min(p.npix_beam - b * R.rows, R.rows);
     const long r0 = R.bbase[b], cnt = R.bbase[b + 1] - r0;
     /* the part's samples: a share of the chunk's, cut at multiples of the
      * write pass's samples per block, so that the records of a part are the
@@ -2786,9 +2830,18 @@ __global__ __launch_bounds__(kBandBlock) void k_beamrec_sum(PairParams p, RecPar
     }
     __syncthreads();
     const double inv = 1.0 / scale;
-    double *dst = R.part + ((long)part * p.npix_beam + lo) * 6;
-    for (int k = tid; k < 6 * nrow; k += kBandBlock)
-        dst[k] += (double)(long long)acc[k] * inv;
+    double *dst = R.part + (long)part * p.npix_beam * 6;
+    if (R.tile == 0) {
+        dst += (long)b * R.rows * 6;
+        for (int k = tid; k < 6 * nrow; k += kBandBlock)
+            dst[k] += (double)(long long)acc[k] * inv;
+        return;
+    }
+    for (int k = tid; k < 6 * nrow; k += kBandBlock) {
+        const int row = k / 6, bp = rec_pixel(R, b, row, p.npix_beam);
+        if (bp >= 0)
+            dst[6 * (long)bp + (k - 6 * row)] += (double)(long long)acc[k] * inv;
+    }
 }
 
 /* The parts' sums into the FP64 gradient (rows of eight, columns 0..5), in
@@ -3429,6 +3482,21 @@ bool adjbeam_rec_plan(const PairParams &p, int rows, size_t pool_bytes, int ncu,
     pl.nband = (int)((p.npix_beam + pl.rows - 1) / pl.rows);
     if (pl.nband > kRecMaxBands || n <= 0)
         return false;
+    /* patches, where the beam lies in the polar cap and has several */
+    pl.tile = 0;
+    const long nb = p.hb.nside;
+    if (pl.nband > 8 && p.npix_beam <= 2 * nb * (nb + 1)) {
+        const int tile = (int)std::sqrt((double)pl.rows);
+        long rings = 1;
+        while (2 * rings * (rings + 1) < p.npix_beam)
+            rings++;
+        const long blocks = (rings + tile - 1) / tile;
+        if (tile >= 8 && 2 * blocks * (blocks + 1) <= kRecMaxBands) {
+            pl.tile = tile;
+            pl.rows = tile * tile;
+            pl.nband = (int)(2 * blocks * (blocks + 1));
+        }
+    }
     /* Visits per sample, at most: the sky pixels whose centres lie within
      * rho_max are disjoint, each of area 4 pi / npix, and lie inside the cap
      * of radius rho_max + 2 s, s = sqrt(4 pi / npix) (more than any HEALPix
@@ -3463,6 +3531,8 @@ hipError_t launch_adjbeam_records(const PairParams &p0, const RecPlan &pl, void 
     R.rows = pl.rows;
     R.nband = pl.nband;
     R.inv_rows = 1.0f / (float)pl.rows;
+    R.tile = pl.tile;
+    R.inv_tile = pl.tile ? 1.0f / (float)pl.tile : 0.f;
     R.brec = (BeamRec *)recs;
     R.nrec_cap = (long)pl.nrec;
     R.bcnt = idx;

@@ -195,6 +195,8 @@ struct BeamRec;
 struct RecParams {
     int rows, nband;
     float inv_rows;
+    int tile;             /* RecPlan::tile */
+    float inv_tile;
     BeamRec *brec;        /* records in band order, at most chunk x bound */
     long nrec_cap;        /* records brec holds (below 2^31) */
     long *bcnt;           /* [nband][chunk] records per (band, sample), then their offsets */
@@ -206,6 +208,7 @@ struct RecParams {
 };
 struct RecPlan {
     int rows, nband, nsplit;
+    int tile;             /* rings and columns of a band's patch, or 0: consecutive rows */
     long chunk;           /* samples per chunk */
     long bound;           /* visits per sample, at most */
     size_t nrec;          /* records (16 bytes) */
