@@ -795,7 +795,13 @@ __device__ inline float quarter_turns(float ax, float ay)
 
 /* Beam pixel from tt in [0, 4] and tmp; kNeedExact unless every floor's
  * argument is farther than 1/2 - lim from an integer. */
-__device__ inline int cap_floors(float tt, float tmp, float omc, float lim)
+/* A certified pixel of the polar cap: its ring, quadrant, and place in the
+ * quadrant (whole numbers). */
+struct CapPlace {
+    float ring, quad, pos;
+};
+
+__device__ inline int cap_floors(float tt, float tmp, float omc, float lim, CapPlace &place)
 {
     const float tp = __builtin_amdgcn_fractf(tt);
     const float u1 = tp * tmp, u2 = tmp - u1;
@@ -803,6 +809,9 @@ __device__ inline int cap_floors(float tt, float tmp, float omc, float lim)
     const float irf = ((u1 - d1) + (u2 - d2)) + 1.0f;
     const float vv = tt * irf;
     const float dv = __builtin_amdgcn_fractf(vv);
+    place.ring = irf;
+    place.quad = tt - tp;
+    place.pos = fmaf(-place.quad, irf, vv - dv);
     const int ir = (int)irf, ip = (int)(vv - dv);
     const float e = fmaxf(fmaxf(fabsf(d1 - 0.5f), fabsf(d2 - 0.5f)), fabsf(dv - 0.5f));
     const bool ok = e < lim && omc > kOmcLo && omc < kOmcHi;
@@ -810,7 +819,8 @@ __device__ inline int cap_floors(float tt, float tmp, float omc, float lim)
 }
 
 /* Beam pixel of a visit for the sample's position angle, or kNeedExact. */
-__device__ inline int visit_pixel(const FastConsts &fc, const SampleF &f, const VisitGeo &v)
+__device__ inline int visit_pixel(const FastConsts &fc, const SampleF &f, const VisitGeo &v,
+                                  CapPlace &place)
 {
     const float xr = fmaf(v.xa, f.cps, -(v.ya * f.sps)), yr = fmaf(v.xa, f.sps, v.ya * f.cps);
     const float ax = fabsf(xr), ay = fabsf(yr);
@@ -820,7 +830,7 @@ __device__ inline int visit_pixel(const FastConsts &fc, const SampleF &f, const 
     const float m = ay > ax ? a : 1.0f - a;
     const float tt = 2.0f - copysignf(1.0f - copysignf(m, xr), yr);
     const float tmp = __builtin_amdgcn_sqrtf(fc.k3 * v.omc);
-    return cap_floors(tt, tmp, v.omc, fmaf(tmp, -kFloorMargin, f.lim0));
+    return cap_floors(tt, tmp, v.omc, fmaf(tmp, -kFloorMargin, f.lim0), place);
 }
 
 /* |eta| above which cos, sin 2 chi take the FP64 form (visit_chi64): the

@@ -304,6 +304,7 @@ struct Pending {
     float sI, sQ, sU; /* sky of the visit (forward only) */
     float sV;         /* sky V of the visit (forward with the V term only) */
     bool live;
+    CapPlace place;   /* WALK_PLACE only */
 };
 
 /* Adds the TOD terms of one visit, a and b (convolver.cpp:157-164; with VT
@@ -338,6 +339,7 @@ enum {
     WALK_BEAM = 2,     /* the beam row */
     WALK_V = 4,        /* the V columns and the sky's V */
     WALK_CHI = 8,      /* cos, sin 2 chi */
+    WALK_PLACE = 16,   /* the beam pixel's ring, quadrant and position */
 };
 
 template <int F>
@@ -547,7 +549,8 @@ __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int
             visit_geo(fmaf(vf - r.a.z, r.a.y, r.a.x), r.b.x, r.b.y, r.b.z, sf.cdc, sf.sdc);
         vf += (float)SUB;
         v0 += SUB;
-        int bp = visit_pixel(p.fc, sf, g);
+        CapPlace place;
+        int bp = visit_pixel(p.fc, sf, g, place);
         float c2 = 0.f, s2 = 0.f;
         if constexpr (F & WALK_CHI) {
             float c4, s4;
@@ -576,6 +579,8 @@ __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int
         q.bp = bp;
         q.c2 = c2;
         q.s2 = s2;
+        if constexpr (F & WALK_PLACE)
+            q.place = place;
         if constexpr ((F & (WALK_SKY | WALK_BEAM)) != 0)
             load_visit<F>(p, q, q.live ? bp : 0, q.live ? pix : 0);
     };
@@ -1379,7 +1384,8 @@ __device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, i
                 const bool edge = act && !in && !(g.omc > K.CUT_OUT[k]);
                 const float tt = 4.0f * __builtin_amdgcn_fractf(0.25f * (K.T0[k] - al));
                 const float tmp = K.NSF[k] * x3y;
-                int bp = cap_floors(tt, tmp, g.omc, fmaf(tmp, -kFloorMarginBatch, K.lim0));
+                CapPlace place;
+                int bp = cap_floors(tt, tmp, g.omc, fmaf(tmp, -kFloorMarginBatch, K.lim0), place);
                 bp = in ? bp : -1;
                 const bool defer = edge || bp == kNeedExact;
                 const unsigned long long md = __ballot(defer);
@@ -2596,6 +2602,17 @@ __device__ inline int rec_band(const RecParams &R, int bp, int &row)
     return (2 * t + q) * (t + 1) + c;
 }
 
+/* The same from a visit's certified place: whole numbers in float. */
+__device__ inline int rec_band(const RecParams &R, int bp, const CapPlace &e, int &row)
+{
+    if (R.tile == 0)
+        return rec_band(R, bp, row);
+    const float w = (float)R.tile;
+    const float t = floorf((e.ring - 0.5f) * R.inv_tile), c = floorf((e.pos + 0.5f) * R.inv_tile);
+    row = (int)fmaf(fmaf(-t, w, e.ring - 1.0f), w, fmaf(-c, w, e.pos));
+    return (int)fmaf(fmaf(2.0f, t, e.quad), t + 1.0f, c);
+}
+
 /* The beam pixel of a row of band b, or -1 if it has none. */
 __device__ inline int rec_pixel(const RecParams &R, int b, int row, int npix)
 {
@@ -2667,9 +2684,7 @@ void k_beamrec(PairParams p, RecParams R)
         int qn = 0;
         if constexpr (WRITE) {
             const unsigned smp_key = (unsigned)j << kRecRowBits;
-            auto write = [&](const Pending &q) {
-                int row;
-                const int b = rec_band(R, q.bp, row);
+            auto put = [&](const Pending &q, int b, int row) {
                 const unsigned slot = atomicAdd(&cur[b], 1u);
                 if (slot >= (unsigned)R.nrec_cap)
                     return;   /* never: both passes count the same visits */
@@ -2680,8 +2695,17 @@ void k_beamrec(PairParams p, RecParams R)
                 r.Y = fmaf(q.sU, q.c2, -(q.sQ * q.s2));
                 R.brec[slot] = r;
             };
-            auto write_exact = [&](const Pending &q, int, int, int) { write(q); };
-            constexpr int F = WALK_SKY | WALK_CHI;
+            auto write = [&](const Pending &q) {
+                int row;
+                const int b = rec_band(R, q.bp, q.place, row);
+                put(q, b, row);
+            };
+            auto write_exact = [&](const Pending &q, int, int, int) {
+                int row;
+                const int b = rec_band(R, q.bp, row);
+                put(q, b, row);
+            };
+            constexpr int F = WALK_SKY | WALK_CHI | WALK_PLACE;
             walk_rings<F>(p, t, ws, 0, r0, r1, lane, sf, kEtaAdjoint, qn, after, write,
                           write_exact);
             if (qn > 0)
@@ -2689,10 +2713,13 @@ void k_beamrec(PairParams p, RecParams R)
         } else {
             auto count = [&](const Pending &q) {
                 int row;
+                atomicAdd(&cur[rec_band(R, q.bp, q.place, row)], 1u);
+            };
+            auto count_exact = [&](const Pending &q, int, int, int) {
+                int row;
                 atomicAdd(&cur[rec_band(R, q.bp, row)], 1u);
             };
-            auto count_exact = [&](const Pending &q, int, int, int) { count(q); };
-            walk_rings<0>(p, t, ws, 0, r0, r1, lane, sf, kEtaAdjoint, qn, after, count,
+            walk_rings<WALK_PLACE>(p, t, ws, 0, r0, r1, lane, sf, kEtaAdjoint, qn, after, count,
                           count_exact);
             if (qn > 0)
                 drain_queue<0>(p, ws, 0, qn, lane, count_exact);
@@ -3148,7 +3175,8 @@ __global__ void k_match(Hpx hs, const RingRec *rings, Hpx hb, FastConsts fc, Fas
                 const RunGeo g = run_geo(hs, rr, r, c, j, 1);
                 const float x = fmaf((float)(j - g.kc), g.b, g.a0);
                 const VisitGeo v = visit_geo(x, g.sD, g.omD, g.cdp2, sf.cdc, sf.sdc);
-                bp = visit_pixel(fc, sf, v);
+                CapPlace place;
+                bp = visit_pixel(fc, sf, v, place);
                 float c4, s4;
                 visit_phase(v, g.kap, c4, s4);
                 visit_chi(sf, c4, s4, c2, s2);
