@@ -1570,6 +1570,14 @@ __device__ inline unsigned long long fix64(float v, double s)
     const unsigned long long t = (unsigned long long)__double_as_longlong(fma((double)v, s, 0x1.8p52));
     return (unsigned long long)((unsigned)(t >> 32) - 0x43380000u) << 32 | (unsigned)t;
 }
+/* An add to LDS.  The scope differs from that of the global atomics beside it:
+ * with the same one the compiler merged the last add of both branches into one
+ * flat atomic, which waits for all memory. */
+template <typename V>
+__device__ inline void lds_add(V *x, V v)
+{
+    __hip_atomic_fetch_add(x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 constexpr int kBigI = 0x3fffffff;
 /* A chunk whose window exceeds the LDS capacity is split into at most this
  * many slabs of consecutive window rings (see k_adjmap_lds). */
@@ -1874,18 +1882,18 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(4, 4)
                 const unsigned long long fQ = fix64(vQ, fxs);
                 const unsigned long long fU = fix64(vU, fxs);
                 if (slot >= 0) {
-                    atomicAdd(&acc64[slot], fI);
-                    atomicAdd(&acc64[W + slot], fQ);
-                    atomicAdd(&acc64[2 * W + slot], fU);
+                    lds_add(&acc64[slot], fI);
+                    lds_add(&acc64[W + slot], fQ);
+                    lds_add(&acc64[2 * W + slot], fU);
                 } else {   /* no window holds the pixel: global int64 atomics */
                     atomicAdd((unsigned long long *)&p.gI[pix], fI);
                     atomicAdd((unsigned long long *)&p.gQ[pix], fQ);
                     atomicAdd((unsigned long long *)&p.gU[pix], fU);
                 }
             } else if (slot >= 0) {
-                atomicAdd(&acc[slot], vI);
-                atomicAdd(&acc[W + slot], vQ);
-                atomicAdd(&acc[2 * W + slot], vU);
+                lds_add(&acc[slot], vI);
+                lds_add(&acc[W + slot], vQ);
+                lds_add(&acc[2 * W + slot], vU);
             } else {   /* no window holds the pixel: global FP64 atomics */
                 unsafeAtomicAdd(&p.gI[pix], (double)vI);
                 unsafeAtomicAdd(&p.gQ[pix], (double)vQ);
