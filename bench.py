@@ -282,7 +282,7 @@ def main():
 
     dominant = "adjoint_map" if t_adj >= t_fwd else "forward"
     b_dom, t_dom = (b_adj, t_adj) if dominant == "adjoint_map" else (b_fwd, t_fwd)
-    k_dom = "k_adjmap_lds" if dominant == "adjoint_map" else "k_pair<0>"
+    k_dom = "k_adjmap_lds" if dominant == "adjoint_map" else "k_fwd_sub<64, false>"
     # the timed sky adjoint is the integer-sum (deterministic) form
     k_traffic = "k_adjmap_lds_deterministic" if k_dom == "k_adjmap_lds" else k_dom
     achieved = b_dom / t_dom
@@ -318,7 +318,7 @@ def main():
                     "adjoint_float_sums_s": t_adj_float,
                     "frac_hbm_fwd_plus_adj": (b_fwd + b_adj) / (t_fwd + t_adj) / HBM_PEAK,
                     "forward_tod_samples_per_s": k * n / t_fwd,
-                    "forward_measured_limiter": measured_limiter("k_pair<0>"),
+                    "forward_measured_limiter": measured_limiter("k_fwd_sub<64, false>"),
                     "wall_s_timed": wall, "setup_s": setup_s},
     }
     if beam_adj:

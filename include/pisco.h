@@ -126,8 +126,9 @@ int pisco_exec_adjoint_beam(pisco_ctx *ctx, const float *g_a, const float *g_b,
 /* Launch-shape tuning of a context (defaults are the measured best on the
  * NSIDE 512, 5-degree workload; except for beam_interpolation, results do
  * not depend on them).  Keys: "adjmap_chunk" (samples per LDS window of the sky adjoint;
- * 0 selects direct global atomics; -1, the default, picks 16 to 128 from the
- * disc size for single-pair adjoints and 16 for batched ones), "adjmap_cap" (window pixels),
+ * 0 selects direct global atomics; -1, the default, picks 8 to 128 from the
+ * disc, the beam and the number of samples for single-pair adjoints and 16 for
+ * batched ones), "adjmap_cap" (window pixels),
  * "adjmap_rw" (window rings), "adjmap_blocks" (blocks of the adjoint launches,
  * each looping over windows; 0, the default, one block per window), "adjmap_support" (1: windows cover only the discs of the beam's
  * non-zero rows, 0: the full rho_max discs; results are the same either way),
@@ -136,9 +137,11 @@ int pisco_exec_adjoint_beam(pisco_ctx *ctx, const float *g_a, const float *g_b,
  * geometry), "batch_adj_group" (batched sky adjoint: 1, 2 or 4 pairs per
  * wave, as batch_group), "forward_lanes" (single-pair forward: 64 = one
  * sample per wave; 32, 16 or 8 lanes per sample with 64/lanes samples per
- * wave; 0, the default, picks 8 below 1,000 expected pixels per disc, 16
- * below 3,000, else 64), "adjmap_lanes" (single-pair sky adjoint: 64, 16 or
- * 8; 0, the default, picks 8 below 1,000 pixels per disc, else 64),
+ * wave; 0, the default, picks 64 for beams above 2.2 MB, else 8 below 1,000
+ * expected pixels per disc, 16 below 10,000, 32 below 30,000, else 64),
+ * "adjmap_lanes" (single-pair sky adjoint: 64, 16 or 8; 0, the default, picks
+ * 64 for beams above 8 MB or from 10,000 pixels per disc, 16 from 450 pixels or
+ * below 16,384 samples, else 8),
  * "batch_pair_major" (batched launches: 1 runs the pairs one after another
  * with the single-pair kernels, 0 all pairs per chunk of samples; -1, the
  * default, picks 1 when a pair's packed beam exceeds 4 MiB),
@@ -195,7 +198,7 @@ int pisco_dev_forward(pisco_ctx *ctx, void *stream, int nside_sky,
  * cannot allocate device memory during the call (code under graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  It takes no
  * context and allocates nothing: its workspace (the sky's ring table and
- * packed pixels) is a fixed device array of 48.1 MiB that each device the
+ * packed pixels, strips) is a fixed device array of 80.1 MiB that each device the
  * library runs on holds for the life of the process, so the sky NSIDE is at
  * most 512 (a larger one is refused with PISCO_ERR_INVALID; pisco_dev_forward
  * takes any).  Runs on the current device and the given stream with the

@@ -2,15 +2,16 @@
  * kernels.hip -- gfx950 kernels of the pixel-space beam convolution.
  *
  * Work mapping (CDNA4: 64-lane wavefronts, 4 waves per 256-thread block):
- *   one wavefront per pointing sample.  The wave first runs the ring part of
- *   query_disc with one ring per lane (64 rings per pass), turns the 0-2 pixel
- *   runs of each ring into a compact run table in LDS with a wave prefix sum,
- *   and then walks the flattened visit list lane-strided, so that consecutive
- *   lanes read consecutive sky pixels of a ring (coalesced) while the beam
- *   reads are gathers.  Each visit recomputes the FP64 beam-frame mapping
- *   (rho, sigma, chi -> beam pixel) exactly as the CPU path does; sums are
- *   reduced across the wave with shuffles and written by a single lane, so
- *   the forward is deterministic and needs no atomics.
+ *   a lane group (8, 16, 32 or 64 lanes) per pointing sample.  It first runs the
+ *   ring part of query_disc with one ring per lane, turns the 0-2 pixel runs of
+ *   each ring into a table in LDS with a prefix sum over its lanes, and then
+ *   walks the flattened visit list lane-strided, so that consecutive lanes read
+ *   consecutive sky pixels of a ring (coalesced) while the beam reads are
+ *   gathers.  Each visit maps its pixel into the beam frame in certified single
+ *   precision; a visit whose beam pixel that cannot certify is mapped in double
+ *   precision or exactly as the CPU path does.  Sums are reduced across the
+ *   lanes with shuffles, so the forward is deterministic and needs no global
+ *   atomics.
  *
  * Blocks are remapped so that each of the 8 XCDs (each with its own L2) works
  * on one contiguous stretch of the scan: consecutive samples share most of
@@ -129,7 +130,11 @@ __device__ inline int build_runs(const Hpx &hs, const Disc &d, int r0, int lane,
  * records and does no FP64.  `bits` marks the visits that start a run: a lane
  * finds its run by counting the marks below it (its wave's visits are
  * consecutive), where a search through the run offsets would be a chain of
- * dependent LDS reads.  The marks cover a segment of VCAP visits from seg0 on:
+ * dependent LDS reads.  Per 64 visits the forward issues about 130 vector
+ * instructions, where recomputing the ring's geometry per visit in mixed
+ * precision took 279: 1e6 samples of 135 pixels 1.28 and 0.80 ms.  Bound by
+ * vector issue and by the gather's lines, 2.15 cycles each per CU.  The marks
+ * cover a segment of VCAP visits from seg0 on:
  * bit v - 1 - seg0 marks a run that starts at visit v > seg0. */
 template <int SUB_, int RPP_, int VCAP_>
 struct VisitTable {
@@ -940,7 +945,7 @@ __global__ __launch_bounds__(kBlock) void k_pair(PairParams p)
  * double products, divided by the double weight sum), with the values
  * starting from zero at every visit.  A visit with no neighbour in the beam
  * contributes nothing.  The mapping is the exact FP64 rho_sigma_chi of the
- * sky pixel; one wave per sample walks the disc as k_pair does, without the
+ * sky pixel; one wave per sample walks the disc as k_fwd_sub does, without the
  * pipelining of the nearest-pixel kernels.  Sky adjoint and beam adjoint use
  * FP64 atomics; the beam adjoint spreads each visit over the neighbours used
  * with weights w / sum(w). */
@@ -1151,7 +1156,7 @@ void k_batch_pair(BatchParams b)
  * takes one (sample, group of G pairs), in the item order of batch_item; the
  * pairs are sorted by disc radius,
  * so the group's union disc is the disc of its first pair.  Lanes walk the
- * visits of that disc as in k_pair; per visit the parts that do not depend on
+ * visits of that disc as in k_fwd_sub; per visit the parts that do not depend on
  * the pair (sky values, the float geometry: 1 - cos rho, alpha, the chi
  * phase) are computed once and each pair runs only its tail: disc membership
  * (its own rho_max), beam pixel for its position angle, beam gather, sum.
@@ -1518,7 +1523,7 @@ void k_batch_fwd(BatchParams p)
 
 /* ---- adjoint with respect to the sky, LDS-privatised ---------------------
  *
- * A block (16 waves) owns a chunk of K consecutive samples.  Their discs
+ * A block (8 waves) owns a chunk of K consecutive samples.  Their discs
  * overlap almost entirely, so the block first computes, per ring, the pixel
  * window that covers every disc of the chunk (pass 1: ring spans unwrapped
  * around the chunk's first centre, atomic min/max in LDS), lays the windows
@@ -2214,7 +2219,7 @@ __device__ inline int build_band_runs(const Hpx &hs, const Disc &dout, const Dis
 }
 
 /* The walk of one annulus pass: FP64 certified mapping, software pipelined
- * as walk_visits; every load of the loop issued unconditionally.  use(q) is
+ * as walk_segment; every load of the loop issued unconditionally.  use(q) is
  * called for each visit whose beam pixel lies in rows [lo, lo + nrow). */
 template <typename Use>
 __device__ inline void walk_band(const PairParams &p, const BandRunTable &t, int total, int lane,
@@ -2229,7 +2234,7 @@ __device__ inline void walk_band(const PairParams &p, const BandRunTable &t, int
         while (v >= t.pref[s + 1])
             s++;
     RingRec rr = p.rings[t.ring[s]];
-    __builtin_amdgcn_s_waitcnt(0);   /* as in walk_visits */
+    __builtin_amdgcn_s_waitcnt(0);   /* the counter is 0 at the loop head */
     Pending q;
     q.live = false;
     for (int v0 = 0; v0 < total; v0 += kWaveSize, v += kWaveSize) {
@@ -2323,7 +2328,7 @@ __device__ inline void walk_band_sub(const PairParams &p, const SubBandTable<SUB
         while (v >= t.pref[s + 1])
             s++;
     RingRec rr = p.rings[any ? t.ring[s] : 1];
-    __builtin_amdgcn_s_waitcnt(0);   /* as in walk_visits */
+    __builtin_amdgcn_s_waitcnt(0);   /* the counter is 0 at the loop head */
     Pending q;
     q.live = false;
     for (int v0 = 0; v0 < wtot; v0 += SUB, v += SUB) {
