@@ -1076,7 +1076,7 @@ __device__ inline bool batch_item(long w, long nsamp, int nunits, long &unit, lo
 
 __host__ inline long batch_items(long nsamp, int nunits)
 {
-    return (nsamp + kBatchChunk - 1) / kBatchChunk * kBatchChunk * nunits;
+    return nsamp * nunits;   /* the last chunk is short: no idle tail for one XCD */
 }
 
 /* PairParams of one pair of a batch: its beam, beam-map geometry, disc and
