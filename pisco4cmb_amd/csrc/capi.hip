@@ -137,12 +137,16 @@ int pisco::pair_params(int nside_sky, const float *I, const float *Q, const floa
  * L2, and each strip costs a table build per sample.  Forward at sky NSIDE 512,
  * ms for 1, 2, 3, 4 strips: 2.9 MB 1.12, 0.89, 1.04; 4.2 MB 1.99, 1.18, 1.29;
  * 5.7 MB 1.60, 1.11, 1.03; 7.5 MB 2.24, 1.64, 1.45, 1.42; 11.7 MB 4.05, 3.03,
- * 2.69, 2.46, and 6 strips 0.98 of 4.  The sky adjoint pays each strip with a
+ * 2.69, 2.46, and 6 strips 0.98 of 4.  Below 3.2 MB the lane groups do as well
+ * (2.9 MB, 16 lanes 0.87), and strips cost small calls two launches: 2,000
+ * samples of 2.8 MB 0.18 and 0.19.  The sky adjoint pays each strip with a
  * set of windows; 1, 2, 3 strips: 5.7 MB 1.38, 1.48, 1.65; 11.7 MB 2.81, 2.56,
  * 2.96 (3.6e5 samples: 20.5, 14.0, 16.1). */
 int pisco::strips_auto(const PairParams &p, bool adjoint)
 {
     const double mb = 32.0 * p.npix_beam / (1 << 20);
+    if (!adjoint && mb < 3.2)
+        return 1;
     return (int)std::min<double>(kMaxStrips, std::ceil(mb / (adjoint ? 8.0 : 2.2)));
 }
 
@@ -151,17 +155,17 @@ int pisco::strips_auto(const PairParams &p, bool adjoint)
  * ms for 8, 16, 32, 64 lanes over 1e5 samples: 540 pixels per disc 0.31, 0.33,
  * 0.39, 0.45; 1,500: 0.76, 0.73, 0.78, 0.78; 2,160: 1.07, 1.01, 1.06, 1.00;
  * 15,300: 8.17, 6.69, 6.89, 7.56, but over 2e4, fewer waves, 2.98, 2.26, 1.84,
- * 1.76; 6,000 over 3.6e5 8.12, 7.77, 8.37, 9.08; 54,000 over 2e4 7.9, 6.8, 6.1
- * for 16, 32, 64.  The rule may not look at the number of samples: a sample's
- * sum would depend on it.  A beam that needs strips takes the one-wave kernel:
- * 4.2 MB, 2,160 pixels 1.99 whole, 1.18 in two strips. */
+ * 1.76; 6,000 over 3.6e5 8.12, 7.77, 8.37, 9.08.  The rule may not look at the
+ * number of samples (a sample's sum would depend on it), so large discs take a
+ * wave each: few samples would otherwise leave most waves idle.  Strips are of
+ * one-wave samples. */
 int pisco::forward_lanes_auto(const PairParams &p)
 {
     const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
     const double dp = (double)p.hs.npix * s * s;   /* expected pixels per disc */
     if (strips_auto(p, false) > 1)
         return 64;
-    return dp < 1000.0 ? 8 : dp < 10000.0 ? 16 : dp < 30000.0 ? 32 : 64;
+    return dp < 1000.0 ? 8 : dp < 3000.0 ? 16 : 64;
 }
 
 struct pisco_ctx {
@@ -313,15 +317,17 @@ int fwd_lanes(const pisco_ctx *c, const PairParams &p)
  * pixels per disc 0.46, 0.51, 0.61; 540: 0.64, 0.60, 0.69; 960: 1.01, 1.00,
  * 1.00; 1,500: 1.31, 1.24, 1.26; 135 pixels, 1e4 samples: 0.113, 0.108, 0.121.
  * 16 and 64 lanes over 6e4 samples: 6,000 pixels 1.83, 1.95; 8,600: 3.29, 3.30.
+ * 5,700 pixels, 2,000 samples: 16 lanes 0.43 ms, which leave waves idle again.
  * Strips are of one-wave samples. */
 int adj_lanes(const pisco_ctx *c, const PairParams &p)
 {
     if (c->adjmap_lanes > 0)
         return c->adjmap_lanes;
     const double dp = disc_pixels(p);
-    if (dp >= 10000.0 || strips_auto(p, true) > 1)
+    const long n = p.s_end - p.s_begin;
+    if (dp >= 10000.0 || strips_auto(p, true) > 1 || (dp >= 2000.0 && n < 4096))
         return 64;
-    return dp >= 450.0 || p.s_end - p.s_begin < 16384 ? 16 : 8;
+    return dp >= 450.0 || n < 16384 ? 16 : 8;
 }
 
 /* Strips for a launch of one wave per sample, whose launches then take at most
@@ -396,8 +402,8 @@ int det_scale(pisco_ctx *c, const FixSource &f, long count, hipStream_t st, cons
 /* Samples per LDS window of a single-pair sky adjoint with `lanes` lanes per
  * sample: the tuning value, or (auto) the largest power of two up to 128 that
  * keeps a window at 40,000 expected visits, but at least a sample per lane
- * group of the block's waves; fewer, down to 16, where there would be less than
- * one window per CU.  Each window costs three block-wide passes besides its
+ * group of the block's waves; fewer, down to 16 (64 lanes: 8), where there would
+ * be less than one window per CU.  Each window costs three block-wide passes besides its
  * visits, and a larger one more LDS.  ms for 16, 32, 64, 128 samples: 8 lanes,
  * 374 pixels 1.04, 0.63, 0.46, 0.48; 16 lanes, 960 pixels 1.24, 1.00, 1.03,
  * 1.12; 64 lanes, 1,500 pixels 1.26, 1.42, 1.45, 1.73; 8 lanes, 94 pixels, 1e4
@@ -414,7 +420,7 @@ int adj_chunk(const pisco_ctx *c, const PairParams &p, int lanes)
     int chunk = std::max(16, kAdjWaves * (64 / lanes));
     while (chunk < 128 && 2.0 * chunk * dp <= 40000.0)
         chunk *= 2;
-    while (chunk > 16 && p.s_end - p.s_begin < 256L * chunk)
+    while (chunk > (lanes == 64 ? kAdjWaves : 16) && p.s_end - p.s_begin < 256L * chunk)
         chunk /= 2;
     return chunk;
 }
