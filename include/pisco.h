@@ -137,10 +137,11 @@ int pisco_exec_adjoint_beam(pisco_ctx *ctx, const float *g_a, const float *g_b,
  * geometry), "batch_adj_group" (batched sky adjoint: 1, 2 or 4 pairs per
  * wave, as batch_group), "forward_lanes" (single-pair forward: 64 = one
  * sample per wave; 32, 16 or 8 lanes per sample with 64/lanes samples per
- * wave; 0, the default, picks 64 for beams above 2.2 MB, else 8 below 1,000
- * expected pixels per disc, 16 below 10,000, 32 below 30,000, else 64),
+ * wave; 0, the default, picks 64 for beams above 3.2 MB, else 8 below 1,000
+ * expected pixels per disc, 16 below 3,000, else 64),
  * "adjmap_lanes" (single-pair sky adjoint: 64, 16 or 8; 0, the default, picks
- * 64 for beams above 8 MB or from 10,000 pixels per disc, 16 from 450 pixels or
+ * 64 for beams above 8 MB, from 10,000 pixels per disc or from 2,000 with less
+ * than 4,096 samples, 16 from 450 pixels or
  * below 16,384 samples, else 8),
  * "batch_pair_major" (batched launches: 1 runs the pairs one after another
  * with the single-pair kernels, 0 all pairs per chunk of samples; -1, the
