@@ -211,6 +211,8 @@ __device__ inline Pass build_pass(const Hpx &hs, const RingRec *rings, const Dis
     for (int q = 0; q < (RPP + SUB - 1) / SUB; q++) {
         const int r = r0 + q * SUB + sl;
         const bool in = more && r <= r_last;
+        if (q > 0 && !__any(in))
+            break;   /* no lane group has more rings */
         RingRec rr;
         int j0[2] = {0, 0}, ln[2] = {0, 0};
         int ns = 0;
