@@ -1731,6 +1731,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(4, 4)
         const int per_strip = (nring + L.strips - 1) / L.strips;
         int first = -kBigI, last = kBigI;
         if (L.strips > 1) {
+            __syncthreads();   /* every wave has read ctl before the next item sets it */
             if (nring <= 0) {
                 if (strip > 0)
                     continue;
