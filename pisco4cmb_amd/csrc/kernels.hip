@@ -26,6 +26,7 @@
 
 #include "device_hpx.h"
 #include "kernels.hpp"
+#include "visit_marks.h"
 
 namespace pisco {
 
@@ -246,7 +247,7 @@ __device__ inline Pass build_pass(const Hpx &hs, const RingRec *rings, const Dis
                 t.ring[run] = w ? ~r : r;
                 wide = wide || w;
                 if (off > 0 && off <= T::VCAP)   /* the first segment's marks */
-                    atomicOr(&t.bits[(off - 1) >> 5], 1u << ((off - 1) & 31));
+                    atomicOr(&t.bits[mark_word(off)], mark_bit(off));
                 run++;
                 off += ln[k];
             }
@@ -275,8 +276,8 @@ __device__ inline int run_ring(const T &t, int i)
     return r < 0 ? ~r : r;
 }
 
-/* Marks the runs of the segment that starts at visit seg0 > 0; returns the
- * number of runs, besides the first, that start at or before seg0. */
+/* Marks the runs of the segment that starts at visit seg0 > 0; returns the run
+ * of its first visit. */
 template <typename T>
 __device__ inline int mark_segment(T &t, int nrun, int seg0, int sl)
 {
@@ -285,19 +286,19 @@ __device__ inline int mark_segment(T &t, int nrun, int seg0, int sl)
     for (int w = sl; w < T::VCAP / 32; w += SUB)
         t.bits[w] = 0u;
     wave_sync();
-    int before = -1;
+    int started = 0;
     for (int i0 = 0; i0 < T::RPP; i0 += SUB) {
         const bool in = i0 + sl < nrun;
         const int o = in ? t.pref[i0 + sl] - seg0 : 1;
         unsigned long long m = __ballot(in && o <= 0);
         if constexpr (SUB < kWaveSize)
             m = (m >> ((int)__lane_id() & ~(SUB - 1))) & ((1ull << SUB) - 1ull);
-        before += __popcll(m);
+        started += __popcll(m);
         if (in && o > 0 && o <= T::VCAP)
-            atomicOr(&t.bits[(o - 1) >> 5], 1u << ((o - 1) & 31));
+            atomicOr(&t.bits[mark_word(o)], mark_bit(o));
     }
     wave_sync();
-    return before;
+    return segment_base(started);
 }
 
 /* A visit whose beam pixel lies inside the beam, with what `use` needs. */
@@ -536,8 +537,8 @@ __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int
             base += __popc(lo) + __popc(hi);
         } else {
             const unsigned m = t.bits[k >> 5] >> (k & 31);
-            n.run = base + __popc(m & ((1u << sl) - 1u));
-            base += __popc(SUB == 32 ? m : m & ((1u << (SUB & 31)) - 1u));
+            n.run = base + marks_below(m, sl);
+            base += SUB == 32 ? __popc(m) : marks_below(m, SUB);
         }
         n.a = t.rec[n.run][0];
         n.b = t.rec[n.run][1];
