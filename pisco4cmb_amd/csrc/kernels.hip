@@ -27,6 +27,7 @@
 #include "device_hpx.h"
 #include "kernels.hpp"
 #include "visit_marks.h"
+#include "work_items.h"
 
 namespace pisco {
 
@@ -837,11 +838,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     long i0 = p.s_begin + lb * NS;
     int k = 0;
     if (SUB == kWaveSize && p.strips > 1) {
-        constexpr int MB = kStripChunk / NS;
-        const long c = lb / (MB * p.strips);
-        const int rem = (int)(lb - c * (MB * p.strips));
-        k = rem / MB;
-        i0 = p.s_begin + c * kStripChunk + (rem - k * MB) * NS;
+        long strip, blk;
+        if (!work_item(lb, (p.s_end - p.s_begin + NS - 1) / NS, p.strips, kStripChunk / NS, strip,
+                       blk))
+            return;
+        k = (int)strip;
+        i0 = p.s_begin + blk * NS;
     }
     if (i0 >= p.s_end)
         return;
@@ -1055,32 +1057,9 @@ __global__ __launch_bounds__(kBlock) void k_pair_interp(PairParams p)
     }
 }
 
-/* Item order of the batched launches: samples in chunks of kBatchChunk, and
- * within a chunk all items of one pair (or pair group) before the next.  The
- * XCD-aware block order hands each XCD whole chunks, so every XCD sees every
- * pair (the pairs' discs differ widely in size) while consecutive waves
- * share one beam.  Returns false for the padding items of a partial last
- * chunk. */
+/* Samples per chunk of the batched launches (work_item): every XCD sees every
+ * pair, whose discs differ widely in size. */
 constexpr long kBatchChunk = 1024;
-
-__device__ inline bool batch_item(long w, long nsamp, int nunits, long &unit, long &sample)
-{
-    const long per = kBatchChunk * nunits;
-    const long c = w / per;
-    const long rem = w - c * per;
-    const long cs = c * kBatchChunk;
-    const long len = (nsamp - cs) < kBatchChunk ? (nsamp - cs) : kBatchChunk;
-    if (len <= 0 || rem >= len * nunits)
-        return false;
-    unit = rem / len;
-    sample = cs + (rem - unit * len);
-    return true;
-}
-
-__host__ inline long batch_items(long nsamp, int nunits)
-{
-    return nsamp * nunits;   /* the last chunk is short: no idle tail for one XCD */
-}
 
 /* PairParams of one pair of a batch: its beam, beam-map geometry, disc and
  * outputs (TOD rows 2 out, 2 out + 1 of [pairs][2][nsamples]). */
@@ -1127,7 +1106,7 @@ __device__ inline PairParams batch_pair_params(const BatchParams &b, const Batch
 }
 
 /* Batched form of k_fwd_sub: a block per (pair, NS samples) item in the order
- * of batch_item; each sample is the single-pair computation with
+ * of work_item; each sample is the single-pair computation with
  * pa = (float)(pa + pa_offset). */
 template <int SUB>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
@@ -1138,7 +1117,7 @@ void k_batch_pair(BatchParams b)
     const long lb = xcd_remap(blockIdx.x, gridDim.x);
     const long n = b.s_end - b.s_begin;
     long k, j;
-    if (!batch_item(lb, (n + NS - 1) / NS, b.npairs, k, j))
+    if (!work_item(lb, (n + NS - 1) / NS, b.npairs, kBatchChunk, k, j))
         return;
     const BatchPair &q = b.pairs[k];
     if (q.out < 0)
@@ -1156,7 +1135,7 @@ void k_batch_pair(BatchParams b)
  *
  * Detector pairs that share the boresight pointing (each with its own beam,
  * disc radius and position-angle offset) are convolved in one launch.  A wave
- * takes one (sample, group of G pairs), in the item order of batch_item; the
+ * takes one (sample, group of G pairs), in the item order of work_item; the
  * pairs are sorted by disc radius,
  * so the group's union disc is the disc of its first pair.  Lanes walk the
  * visits of that disc as in k_fwd_sub; per visit the parts that do not depend on
@@ -1452,7 +1431,7 @@ void k_batch_fwd(BatchParams p)
     const long lb = xcd_remap(blockIdx.x, gridDim.x);
     const long w = lb * kWavesPerBlock + wave;
     long grp, j;
-    if (!batch_item(w, p.s_end - p.s_begin, p.ngroups, grp, j))
+    if (!work_item(w, p.s_end - p.s_begin, p.ngroups, kBatchChunk, grp, j))
         return;
     const long i = p.s_begin + j;
     const int d0 = (int)grp * G;
@@ -1559,7 +1538,7 @@ struct AdjLayout {
 
 __host__ __device__ inline long adj_items(const AdjLayout &L)
 {
-    return (L.nchunks + L.strip_group - 1) / L.strip_group * L.strip_group * L.strips;
+    return work_items(L.nchunks, L.strips);
 }
 
 constexpr int kAdjBlock = kAdjWaves * kWaveSize;
@@ -1700,11 +1679,10 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(4, 4)
     long lb = xcd_remap(blockIdx.x, gridDim.x);
     const long nitems = adj_items(L);
     for (long item = lb; item < nitems; item += gridDim.x) {
-        const long per = (long)L.strip_group * L.strips, cg = item / per;
-        const int rem = (int)(item - cg * per), strip = rem / L.strip_group;
-        const long ch = cg * L.strip_group + (rem - strip * L.strip_group);
-        if (ch >= L.nchunks)
+        long unit, ch;
+        if (!work_item(item, L.nchunks, L.strips, L.strip_group, unit, ch))
             continue;
+        const int strip = (int)unit;
         long s0 = p.s_begin + ch * L.chunk;
         long s1 = s0 + L.chunk < p.s_end ? s0 + L.chunk : p.s_end;
         int ns = (int)(s1 - s0);
@@ -3279,9 +3257,7 @@ static void launch_fwd_lanes(const PairParams &p, hipStream_t st, bool vterm)
 {
     constexpr int NS = FwdBlock<SUB>::NS;
     const long n = p.s_end - p.s_begin;
-    const unsigned nb = p.strips > 1
-                            ? (unsigned)((n + kStripChunk - 1) / kStripChunk * (kStripChunk / NS) * p.strips)
-                            : nblocks(n, NS);
+    const unsigned nb = (unsigned)work_items(nblocks(n, NS), p.strips);
     if (vterm)
         hipLaunchKernelGGL((k_fwd_sub<SUB, true>), dim3(nb), dim3(kBlock), 0, st, p);
     else
@@ -3333,7 +3309,7 @@ template <int SUB>
 static void launch_batch_pairs(const BatchParams &p, long n, hipStream_t st)
 {
     constexpr int NS = FwdBlock<SUB>::NS;
-    hipLaunchKernelGGL(k_batch_pair<SUB>, dim3((unsigned)batch_items((n + NS - 1) / NS, p.npairs)),
+    hipLaunchKernelGGL(k_batch_pair<SUB>, dim3((unsigned)work_items((n + NS - 1) / NS, p.npairs)),
                        dim3(kBlock), 0, st, p);
 }
 
@@ -3342,7 +3318,7 @@ hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st,
     const long n = p.s_end - p.s_begin;
     if (n <= 0)
         return hipSuccess;
-    const unsigned g = nblocks(batch_items(n, p.ngroups), kWavesPerBlock);
+    const unsigned g = nblocks(work_items(n, p.ngroups), kWavesPerBlock);
     switch (group) {
     case 1:
         switch (lanes) {
