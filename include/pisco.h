@@ -137,11 +137,11 @@ int pisco_exec_adjoint_beam(pisco_ctx *ctx, const float *g_a, const float *g_b,
  * geometry), "batch_adj_group" (batched sky adjoint: 1, 2 or 4 pairs per
  * wave, as batch_group), "forward_lanes" (single-pair forward: 64 = one
  * sample per wave; 32, 16 or 8 lanes per sample with 64/lanes samples per
- * wave; 0, the default, picks 64 for beams above 3.2 MB, else 8 below 1,000
- * expected pixels per disc, 16 below 3,000, else 64),
+ * wave; 0, the default, picks 64 for beams above 3.2 MB with at least 1,200
+ * expected pixels per disc, else 8 below 1,000 pixels, 16 below 3,000, else 64),
  * "adjmap_lanes" (single-pair sky adjoint: 64, 16 or 8; 0, the default, picks
- * 64 for beams above 8 MB, from 10,000 pixels per disc or from 2,000 with less
- * than 4,096 samples, 16 from 450 pixels or
+ * 64 for beams above 8 MB with at least 4,000 pixels per disc, from 10,000
+ * pixels or from 2,000 with less than 4,096 samples, 16 from 450 pixels or
  * below 16,384 samples, else 8),
  * "batch_pair_major" (batched launches: 1 runs the pairs one after another
  * with the single-pair kernels, 0 all pairs per chunk of samples; -1, the
@@ -464,6 +464,13 @@ int pisco_pix2ang(int nside, long pix, double *theta, double *phi);
  * the decomposition so that its coverage can be checked. */
 long pisco_band_annulus(int nside_sky, int nside_beam, long npix_beam, int rows, int band,
                         float ra, float dec, int cover, long cap, int *pix);
+
+/* The automatic launch shape of a single-pair call (tuning keys at their
+ * defaults): lanes per sample and strips per disc of the forward, then of the
+ * sky adjoint over nsamples samples.  Host only; it exposes the rules so that
+ * they can be checked. */
+int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamples,
+                       int shape[4]);
 
 /* E-field magnitude and phase of a perfectly co-polarised elliptical
  * Gaussian beam on the first npix pixels of a beam map

@@ -114,6 +114,7 @@ SIGNATURES = {
     "pisco_pix2ang": (c_int, [c_int, c_long, P, P]),
     "pisco_band_annulus": (c_long, [c_int, c_int, c_long, c_int, c_int, c_float, c_float, c_int,
                                     c_long, P]),
+    "pisco_launch_shape": (c_int, [c_int, c_int, c_long, c_long, P]),
     "pisco_beam_gaussian_fields": (c_int, [c_int, c_long, c_double, c_double, c_double, P,
                                            P, P, P]),
     "pisco_beam_from_fields": (c_int, [c_long, P, P, P, P, P, P, P, P]),

@@ -133,21 +133,35 @@ int pisco::pair_params(int nside_sky, const float *I, const float *Q, const floa
     return PISCO_OK;
 }
 
-/* Strips by the beam's size: a strip of a large beam stays in an XCD's 4 MB
- * L2, and each strip costs a table build per sample.  Forward at sky NSIDE 512,
- * ms for 1, 2, 3, 4 strips: 2.9 MB 1.12, 0.89, 1.04; 4.2 MB 1.99, 1.18, 1.29;
- * 5.7 MB 1.60, 1.11, 1.03; 7.5 MB 2.24, 1.64, 1.45, 1.42; 11.7 MB 4.05, 3.03,
- * 2.69, 2.46, and 6 strips 0.98 of 4.  Below 3.2 MB the lane groups do as well
- * (2.9 MB, 16 lanes 0.87), and strips cost small calls two launches: 2,000
- * samples of 2.8 MB 0.18 and 0.19.  The sky adjoint pays each strip with a
- * set of windows; 1, 2, 3 strips: 5.7 MB 1.38, 1.48, 1.65; 11.7 MB 2.81, 2.56,
- * 2.96 (3.6e5 samples: 20.5, 14.0, 16.1). */
+/* Expected sky pixels per disc, npix (1 - cos rho_max) / 2. */
+static double disc_pixels(const PairParams &p)
+{
+    const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
+    return (double)p.hs.npix * s * s;
+}
+
+/* Strips by the sizes of the beam and the disc: a strip of a large beam stays in
+ * an XCD's 4 MB L2, and each strip costs a table build per sample.  Forward at
+ * sky NSIDE 512, ms for 1, 2, 3, 4 strips: 2.9 MB 1.12, 0.89, 1.04; 4.2 MB 1.99,
+ * 1.18, 1.29; 5.7 MB 1.60, 1.11, 1.03; 7.5 MB 2.24, 1.64, 1.45, 1.42; 11.7 MB
+ * 4.05, 3.03, 2.69, 2.46, and 6 strips 0.98 of 4.  Below 3.2 MB the lane groups do
+ * as well (2.9 MB, 16 lanes 0.87), and strips cost small calls two launches: 2,000
+ * samples of 2.8 MB 0.18 and 0.19.  On a coarse sky the builds outweigh the few
+ * visits of a strip: 11.7 MB over 6e4 samples, ms for whole discs (best lanes), 2,
+ * 3, 4, 6 strips: 94 pixels 0.10, 0.24, 0.33, 0.43, 0.60; 374 pixels 0.26, 0.34,
+ * 0.44, 0.53, 0.74; 1,496 pixels 0.85, 0.75, 0.73, 0.82, 1.05; 3,367 pixels 1.85,
+ * 1.69, 1.43, 1.35, 1.46; hence 600 pixels to a strip.
+ * The sky adjoint pays each strip with a set of windows; 1, 2, 3 strips: 5.7 MB
+ * 1.38, 1.48, 1.65; 11.7 MB 2.81, 2.56, 2.96 (3.6e5 samples: 20.5, 14.0, 16.1).
+ * 11.7 MB over 2.5e5 samples, 16 lanes and 2 strips: 1,496 pixels 3.6, 5.2; 3,367
+ * pixels 7.3, 8.1; hence 2,000 pixels to a strip. */
 int pisco::strips_auto(const PairParams &p, bool adjoint)
 {
     const double mb = 32.0 * p.npix_beam / (1 << 20);
     if (!adjoint && mb < 3.2)
         return 1;
-    return (int)std::min<double>(kMaxStrips, std::ceil(mb / (adjoint ? 8.0 : 2.2)));
+    const double most = std::min<double>(kMaxStrips, disc_pixels(p) / (adjoint ? 2000.0 : 600.0));
+    return std::max(1, (int)std::min(most, std::ceil(mb / (adjoint ? 8.0 : 2.2))));
 }
 
 /* Lanes per sample of the forward.  Several samples per wave share the table
@@ -161,8 +175,7 @@ int pisco::strips_auto(const PairParams &p, bool adjoint)
  * one-wave samples. */
 int pisco::forward_lanes_auto(const PairParams &p)
 {
-    const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
-    const double dp = (double)p.hs.npix * s * s;   /* expected pixels per disc */
+    const double dp = disc_pixels(p);
     if (strips_auto(p, false) > 1)
         return 64;
     return dp < 1000.0 ? 8 : dp < 3000.0 ? 16 : 64;
@@ -295,13 +308,6 @@ int setup_pair(pisco_ctx *c, int nside_sky, const float *I, const float *Q,
     return PISCO_OK;
 }
 
-/* Expected sky pixels in a disc of radius rho_max: npix (1 - cos rho) / 2. */
-double disc_pixels(const PairParams &p)
-{
-    const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
-    return (double)p.hs.npix * s * s;
-}
-
 /* Lanes per sample of the nearest-pixel forward: the tuning value, or
  * (auto) forward_lanes_auto. */
 int fwd_lanes(const pisco_ctx *c, const PairParams &p)
@@ -311,23 +317,27 @@ int fwd_lanes(const pisco_ctx *c, const PairParams &p)
     return forward_lanes_auto(p);
 }
 
-/* Lanes per sample of the single-pair sky adjoint: the tuning value, or
- * (auto) from the expected disc size and, where 8 lanes would leave waves idle,
+/* Lanes per sample of the single-pair sky adjoint
+ * from the expected disc size and, where 8 lanes would leave waves idle,
  * the number of samples.  Best ms over 1e5 samples for 8, 16, 64 lanes: 374
  * pixels per disc 0.46, 0.51, 0.61; 540: 0.64, 0.60, 0.69; 960: 1.01, 1.00,
  * 1.00; 1,500: 1.31, 1.24, 1.26; 135 pixels, 1e4 samples: 0.113, 0.108, 0.121.
  * 16 and 64 lanes over 6e4 samples: 6,000 pixels 1.83, 1.95; 8,600: 3.29, 3.30.
  * 5,700 pixels, 2,000 samples: 16 lanes 0.43 ms, which leave waves idle again.
  * Strips are of one-wave samples. */
-int adj_lanes(const pisco_ctx *c, const PairParams &p)
+int adj_lanes_auto(const PairParams &p)
 {
-    if (c->adjmap_lanes > 0)
-        return c->adjmap_lanes;
     const double dp = disc_pixels(p);
     const long n = p.s_end - p.s_begin;
     if (dp >= 10000.0 || strips_auto(p, true) > 1 || (dp >= 2000.0 && n < 4096))
         return 64;
     return dp >= 450.0 || n < 16384 ? 16 : 8;
+}
+
+/* The tuning value, or adj_lanes_auto. */
+int adj_lanes(const pisco_ctx *c, const PairParams &p)
+{
+    return c->adjmap_lanes > 0 ? c->adjmap_lanes : adj_lanes_auto(p);
 }
 
 /* Strips for a launch of one wave per sample, whose launches then take at most
@@ -557,6 +567,24 @@ int pisco_pix2ang(int nside, long pix, double *theta, double *phi)
     if (!valid_nside(nside) || pix < 0 || pix >= 12L * nside * nside || !theta || !phi)
         return fail(PISCO_ERR_INVALID, "bad argument");
     pix2ang(hpx_make(nside), (int)pix, *theta, *phi);
+    return PISCO_OK;
+}
+
+int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamples, int shape[4])
+{
+    if (!valid_nside(nside_sky) || !valid_nside(nside_beam) || npix_beam < 1 ||
+        npix_beam >= 12L * nside_beam * nside_beam || nsamples < 0 || !shape)
+        return fail(PISCO_ERR_INVALID, "bad argument");
+    PairParams p;
+    memset(&p, 0, sizeof p);
+    p.hs = hpx_make(nside_sky);
+    p.npix_beam = (int)npix_beam;
+    p.rho_max = pisco_beam_rho_max(nside_beam, npix_beam);
+    p.s_end = nsamples;
+    shape[0] = forward_lanes_auto(p);
+    shape[1] = shape[0] == 64 ? strips_auto(p, false) : 1;
+    shape[2] = adj_lanes_auto(p);
+    shape[3] = shape[2] == 64 ? strips_auto(p, true) : 1;
     return PISCO_OK;
 }
 

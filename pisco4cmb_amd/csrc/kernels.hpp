@@ -298,10 +298,12 @@ int set_error(int code, const char *msg);
 int pair_params(int nside_sky, const float *I, const float *Q, const float *U, int nside_beam,
                 long npix_beam, const float *beam8, long nsamples, const float *ra,
                 const float *dec, const float *pa, PairParams &p);
-/* Strips of the kernels with one wave per sample (PairParams::strips). */
+/* Strips of the kernels with one wave per sample (PairParams::strips), from the
+ * beam's bytes and the expected pixels per disc. */
 int strips_auto(const PairParams &p, bool adjoint);
-/* Lanes per sample of the nearest-pixel forward from the expected disc size
- * npix (1 - cos rho_max) / 2: 8 below 1,000 pixels, 16 below 3,000, else 64. */
+/* Lanes per sample of the nearest-pixel forward: 64 with strips, else from the
+ * expected disc size npix (1 - cos rho_max) / 2: 8 below 1,000 pixels, 16 below
+ * 3,000, else 64. */
 int forward_lanes_auto(const PairParams &p);
 
 } /* namespace pisco */

@@ -1,0 +1,33 @@
+"""Strips at the disc sizes that take them by the automatic rule: sky NSIDE 128,
+beam NSIDE 1024, cap 20 deg (11.6 MB, 5,900 pixels per disc; six strips forward,
+two in the adjoint), 4,101 samples (a strip chunk and a partial block), some of
+whose discs hold a pole.  A sample's TOD has the same bits in any launch.
+Tolerance: relative RMS 1e-6 of the oracle, the bound of the other single-pair
+tests."""
+import numpy as np
+import pytest
+
+from test_gpu_strips import Calls, make, rel_rms
+from test_launch_shape import shape
+
+pytestmark = pytest.mark.gpu
+
+
+def test_automatic_strips(oracle):
+    ns, nb, cap, n = 128, 1024, 20.0, 4101
+    assert shape(ns, nb, cap, n) == [64, 6, 64, 2]
+    sky, beam, ra, dec, pa, g = make(ns, nb, cap, n, 11)
+    c = Calls(ns, nb, beam, sky)
+    beams = list(beam.aBeams) + list(beam.bBeams)
+    a, b = c.forward(ra, dec, pa)
+    m = 300   # the oracle's share of the samples: both ends
+    sel = np.r_[0:m, n - m:n]
+    oa, ob = oracle.convolve(ns, *sky[:3], nb, beams, ra[sel], dec[sel], pa[sel])
+    assert rel_rms(a[sel], oa) < 1e-6 and rel_rms(b[sel], ob) < 1e-6
+    for lo, hi in ((0, 1), (5, 1030), (n - 3, n)):
+        x, y = c.forward(ra[lo:hi], dec[lo:hi], pa[lo:hi])
+        assert np.array_equal(x, a[lo:hi]) and np.array_equal(y, b[lo:hi])
+    args = [v[sel] for v in (ra, dec, pa, *g)]
+    ref = oracle.adjoint_map(ns, nb, beams, *args)
+    for x, r in zip(c.adjoint(*args), ref):
+        assert rel_rms(x, r) < 1e-6

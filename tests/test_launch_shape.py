@@ -1,0 +1,46 @@
+"""The automatic launch shapes of single-pair calls (pisco_launch_shape), on the
+CPU: strips only where a strip keeps enough visits to pay for its table build.
+Before they looked at the disc, 94-pixel discs of a 12 MB beam were cut into six
+strips of 15 visits and took eight times as long."""
+import ctypes
+import math
+
+import pytest
+
+from pisco4cmb_amd import pypisco
+from pisco4cmb_amd._lib import check, lib
+
+
+def shape(ns, nb, cap_deg, n=100000):
+    s = (ctypes.c_int * 4)()
+    npix = pypisco.beam_npix_for_radius(nb, math.radians(cap_deg))
+    check(lib.pisco_launch_shape(ns, nb, npix, n, s))
+    return list(s)
+
+
+@pytest.mark.parametrize("ns,nb,cap,fwd,adj", [
+    (64, 4096, 5.0, [8, 1], [8, 1]),        # 94 pixels, 11.7 MB
+    (128, 4096, 5.0, [8, 1], [8, 1]),       # 374
+    (200, 2400, 5.0, [8, 1], [16, 1]),      # 913, 4.0 MB
+    (256, 4096, 5.0, [64, 2], [16, 1]),     # 1,496
+    (384, 4096, 5.0, [64, 5], [16, 1]),     # 3,367
+    (512, 4096, 5.0, [64, 6], [64, 2]),     # 5,985: the headline shape
+    (512, 4096, 2.5, [16, 1], [16, 1]),     # 1,497, 2.9 MB
+    (256, 2048, 1.5, [8, 1], [8, 1]),       # 135
+])
+def test_strips_keep_their_visits(ns, nb, cap, fwd, adj):
+    s = shape(ns, nb, cap)
+    assert s[:2] == fwd and s[2:] == adj
+
+
+def test_forward_shape_is_the_same_for_any_number_of_samples():
+    for ns, nb, cap in ((64, 512, 3.0), (512, 4096, 5.0), (256, 4096, 4.0)):
+        assert len({tuple(shape(ns, nb, cap, n)[:2]) for n in (0, 1, 500, 5000, 10**6)}) == 1
+
+
+def test_bad_arguments():
+    s = (ctypes.c_int * 4)()
+    assert lib.pisco_launch_shape(0, 512, 100, 1, s) != 0
+    assert lib.pisco_launch_shape(64, 512, 0, 1, s) != 0
+    assert lib.pisco_launch_shape(64, 512, 100, -1, s) != 0
+    assert lib.pisco_launch_shape(64, 512, 100, 1, None) != 0
