@@ -173,12 +173,15 @@ int pisco::strips_auto(const PairParams &p, bool adjoint)
  * number of samples (a sample's sum would depend on it), so large discs take a
  * wave each: few samples would otherwise leave most waves idle.  Strips are of
  * one-wave samples. */
-int pisco::forward_lanes_auto(const PairParams &p)
+static int disc_lanes(const PairParams &p)
 {
     const double dp = disc_pixels(p);
-    if (strips_auto(p, false) > 1)
-        return 64;
     return dp < 1000.0 ? 8 : dp < 3000.0 ? 16 : 64;
+}
+
+int pisco::forward_lanes_auto(const PairParams &p)
+{
+    return strips_auto(p, false) > 1 ? 64 : disc_lanes(p);
 }
 
 struct pisco_ctx {
@@ -1558,17 +1561,41 @@ std::vector<int> batch_ranges(const pisco_ctx *c, const pisco_batch *b)
     return cut;
 }
 
-/* Lanes per sample of the per-pair items: the single-pair rule for the largest
- * disc.  16 pairs, 540 pixels per disc, 2.5e4 samples: one wave per sample 1.57
- * ms, 8 lanes 1.38 ms. */
+/* Lanes per sample of a pair's items: the single-pair rule of its own disc (these
+ * items take no strips), and 16 instead of 8 in a short call, whose blocks of 32
+ * samples leave CUs idle.  540 pixels per disc, us for 8, 16, 64 lanes: 4 pairs,
+ * 1,000 samples 66, 49, 37; 3,000 samples 80, 62, 69; 16 pairs, 1,000 samples 80,
+ * 80, 88; 3,000 samples 162, 177, 214; 1e4 samples 411, 458, 620.  A pair's TOD
+ * depends on the other pairs of the batch in nothing, and on the length of the
+ * call in the order of its FP64 sums. */
 int pair_lanes(const BatchParams &b, const BatchPair &q)
 {
     PairParams p;
     memset(&p, 0, sizeof p);
     p.hs = b.hs;
     p.rho_max = q.rho_max;
-    p.npix_beam = q.npix;
-    return forward_lanes_auto(p);
+    const int lanes = disc_lanes(p);
+    return lanes == 8 && b.nsamples < 2048 ? 16 : lanes;
+}
+
+/* Per-pair items of the pairs [r0, r1) of the table, consecutive pairs of the
+ * same lanes per launch. */
+int forward_pairs(BatchParams p, const pisco_batch *b, int r0, int r1, hipStream_t st)
+{
+    for (int k = r0, e; k < r1; k = e) {
+        if (b->host[k].out < 0) {   /* inert padding */
+            e = k + 1;
+            continue;
+        }
+        const int lanes = pair_lanes(p, b->host[k]);
+        for (e = k + 1; e < r1 && b->host[e].out >= 0; e++)
+            if (pair_lanes(p, b->host[e]) != lanes)
+                break;
+        p.pairs = b->table + k;
+        p.npairs = e - k;
+        HIPCHK(launch_batch_forward(1, p, st, lanes));
+    }
+    return PISCO_OK;
 }
 
 /* The deterministic mode's scale for a batch: every pair's beam, the
@@ -1697,7 +1724,10 @@ int pisco_dev_batched_forward(pisco_ctx *c, void *stream, const pisco_batch *b, 
         for (long s0 = 0; s0 < nsamples; s0 += chunk) {
             p.s_begin = s0;
             p.s_end = std::min(nsamples, s0 + chunk);
-            HIPCHK(launch_batch_forward(G, p, st, pair_lanes(p, b->host[r0])));
+            if (G == 1)
+                CHK(forward_pairs(p, b, r0, r1, st));
+            else
+                HIPCHK(launch_batch_forward(G, p, st));
         }
     }
     return PISCO_OK;
@@ -1733,7 +1763,7 @@ int pisco_dev_batched_forward_pp(pisco_ctx *c, void *stream, const pisco_batch *
         p.s_begin = s0;
         p.s_end = std::min(nsamples, s0 + chunk);
         /* per-pair items: no shared geometry */
-        HIPCHK(launch_batch_forward(1, p, st, pair_lanes(p, b->host[0])));
+        CHK(forward_pairs(p, b, 0, b->npad, st));
     }
     return PISCO_OK;
 }
