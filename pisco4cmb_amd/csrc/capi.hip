@@ -213,7 +213,8 @@ struct pisco_ctx {
     int adjmap_rw = 1024;         /* LDS window rings */
     int adjmap_blocks = 0;        /* persistent blocks; 0 = one block per window (work item) */
     int adjmap_support = 1;       /* size LDS windows by the beam's non-zero rows */
-    int batch_group = 4;          /* pairs per wave in batched forwards (1: per-pair items) */
+    int batch_group = 0;          /* pairs per wave in batched forwards (1: per-pair items;
+                                   * 0: by the pairs' discs and beams, group_auto) */
     int batch_adj_group = 4;      /* pairs per wave in batched sky adjoints */
     int beam_interp = 0;          /* 1: beam interpolated from get_interpol neighbours */
     int adjmap_det = -1;          /* sky adjoint sums: 1 integer (deterministic), 0 float,
@@ -719,7 +720,7 @@ int pisco_get_tuning(pisco_ctx *c, const char *key, long *value)
     else if (k == "adjmap_support")
         *value = c->adjmap_support;
     else if (k == "batch_group")
-        *value = c->batch_group;
+        *value = c->batch_group > 0 ? c->batch_group : 4;
     else if (k == "beam_interpolation")
         *value = c->beam_interp;
     else if (k == "adjmap_deterministic")
@@ -1578,21 +1579,61 @@ int pair_lanes(const BatchParams &b, const BatchPair &q)
     return lanes == 8 && b.nsamples < 2048 ? 16 : lanes;
 }
 
-/* Per-pair items of the pairs [r0, r1) of the table, consecutive pairs of the
- * same lanes per launch. */
-int forward_pairs(BatchParams p, const pisco_batch *b, int r0, int r1, hipStream_t st)
+/* Pairs per wave of the four pairs k .. k+3 of a batched forward, 1 with `lanes`
+ * per sample (0: pair_lanes).  A group shares each visit's geometry but gathers
+ * from all its beams, which have to stay in an XCD's 4 MB L2 beside the sky; per-pair
+ * items gather from one.  ms for groups of 4, 2, and items of 16, 64 lanes, 1e5
+ * samples; sky NSIDE 512, 8 and 16 pairs: 960 pixels of 0.47 MB 6.7, 7.3, 6.8, 8.1,
+ * of 1.9 MB 9.2, 8.4, 7.9, 8.1; 2,160 pixels of 1.05 MB 15.7, 14.8, 14.2, 15.3;
+ * 1,750 pixels of 3.4 MB 12.2, 8.2, 8.4, 7.1; 3,830 pixels of 1.9 MB 19.2, 13.9,
+ * 12.9, 14.5.  Sky NSIDE 2048, 4 pairs: 5,500 pixels of 2.7 MB 19.4, 13.0, 13.0,
+ * 11.9; 8,600 pixels of 1.05 MB 15.3, 14.0, 13.7, 14.9; 34,500 pixels of 1.05 MB
+ * 56.2, 49.5, 45.5, 47.8, and of 300 samples 1.33, 0.92, 1.35, 0.60; 3,100 pixels of
+ * 1.5 MB 7.6, 6.0, 6.2, 6.1; sky NSIDE 128, 303 pixels of 2.4 MB, 8 pairs 2.5, 2.4,
+ * 1.6, 2.7.  Groups of 4 stay where items leave the XCDs with unequal discs: 4
+ * pairs of 540 to 960 pixels, up to 1.9 MB, 6,000 samples 0.135, items 0.158. */
+int group_auto(const BatchParams &b, const pisco_batch *bt, int k, int &lanes)
+{
+    PairParams p;
+    memset(&p, 0, sizeof p);
+    p.hs = b.hs;
+    p.rho_max = bt->host[k].rho_max;   /* the largest disc */
+    double mb = 0.0;                   /* the largest beam */
+    for (int j = k; j < k + 4; j++)
+        if (bt->host[j].out >= 0)
+            mb = std::max(mb, 32.0 * bt->host[j].npix / (1 << 20));
+    lanes = 0;
+    const bool few = disc_pixels(p) < 1000.0;
+    if (mb <= (few ? 2.0 : 1.0))
+        return 4;
+    if (!few && mb <= 1.7)
+        return 2;
+    lanes = few ? 16 : 64;
+    return 1;
+}
+
+/* Per-pair items of the pairs [r0, r1) of the table with lanes_all lanes per
+ * sample, or (0) their own, consecutive pairs of the same lanes per launch. */
+int forward_pairs(BatchParams p, const pisco_batch *b, int r0, int r1, int lanes_all,
+                  hipStream_t st)
 {
     for (int k = r0, e; k < r1; k = e) {
         if (b->host[k].out < 0) {   /* inert padding */
             e = k + 1;
             continue;
         }
-        const int lanes = pair_lanes(p, b->host[k]);
+        const int lanes = lanes_all ? lanes_all : pair_lanes(p, b->host[k]);
         for (e = k + 1; e < r1 && b->host[e].out >= 0; e++)
-            if (pair_lanes(p, b->host[e]) != lanes)
+            if (!lanes_all && pair_lanes(p, b->host[e]) != lanes)
                 break;
         p.pairs = b->table + k;
         p.npairs = e - k;
+        /* unequal discs in short turns, so that every XCD sees all of them: 4 pairs
+         * of 2,450 to 4,900 pixels, 6,000 samples 1.22 -> 1.08 ms; equal ones in
+         * long turns, a beam at a time in an XCD's L2: 1,750 pixels of 3.4 MB, 8
+         * pairs, 1e5 samples 7.2 ms, short turns 9.2 */
+        if (lanes_all == 64 && b->host[e - 1].rho_max < 0.84 * b->host[k].rho_max)
+            p.turn = 256;
         HIPCHK(launch_batch_forward(1, p, st, lanes));
     }
     return PISCO_OK;
@@ -1707,7 +1748,6 @@ int pisco_dev_batched_forward(pisco_ctx *c, void *stream, const pisco_batch *b, 
                                       dec, pa, 0, tod);
     BatchParams p;
     CHK(setup_batch(c, b, nside_sky, I, Q, U, nsamples, ra, dec, pa, p));
-    const int G = c->batch_group;
     p.tod = tod;
     hipStream_t st = pick(c, stream);
     CHK(c->sky4.ensure(4 * (size_t)p.hs.npix));
@@ -1717,17 +1757,24 @@ int pisco_dev_batched_forward(pisco_ctx *c, void *stream, const pisco_batch *b, 
     chunk = std::max<long>(chunk, std::min<long>(nsamples, 1L << 20));
     const std::vector<int> cut = batch_ranges(c, b);
     for (size_t r = 0; r + 1 < cut.size(); r++) {   /* ranges of the sorted pair table */
-        const int r0 = cut[r], r1 = cut[r + 1];
-        p.pairs = b->table + r0;
-        p.npairs = r1 - r0;
-        p.ngroups = (r1 - r0) / G;
-        for (long s0 = 0; s0 < nsamples; s0 += chunk) {
-            p.s_begin = s0;
-            p.s_end = std::min(nsamples, s0 + chunk);
-            if (G == 1)
-                CHK(forward_pairs(p, b, r0, r1, st));
-            else
-                HIPCHK(launch_batch_forward(G, p, st));
+        for (int k = cut[r], e; k < cut[r + 1]; k = e) {
+            int lanes = 0, other = 0;
+            const int G = c->batch_group > 0 ? c->batch_group : group_auto(p, b, k, lanes);
+            for (e = k + 4; e < cut[r + 1]; e += 4)
+                if (c->batch_group == 0 &&
+                    (group_auto(p, b, e, other) != G || other != lanes))
+                    break;
+            p.pairs = b->table + k;
+            p.npairs = e - k;
+            p.ngroups = p.npairs / G;
+            for (long s0 = 0; s0 < nsamples; s0 += chunk) {
+                p.s_begin = s0;
+                p.s_end = std::min(nsamples, s0 + chunk);
+                if (G == 1)
+                    CHK(forward_pairs(p, b, k, e, lanes, st));
+                else
+                    HIPCHK(launch_batch_forward(G, p, st));
+            }
         }
     }
     return PISCO_OK;
@@ -1763,7 +1810,7 @@ int pisco_dev_batched_forward_pp(pisco_ctx *c, void *stream, const pisco_batch *
         p.s_begin = s0;
         p.s_end = std::min(nsamples, s0 + chunk);
         /* per-pair items: no shared geometry */
-        CHK(forward_pairs(p, b, 0, b->npad, st));
+        CHK(forward_pairs(p, b, 0, b->npad, 0, st));
     }
     return PISCO_OK;
 }

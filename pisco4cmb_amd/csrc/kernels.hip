@@ -1117,7 +1117,7 @@ void k_batch_pair(BatchParams b)
     const long lb = xcd_remap(blockIdx.x, gridDim.x);
     const long n = b.s_end - b.s_begin;
     long k, j;
-    if (!work_item(lb, (n + NS - 1) / NS, b.npairs, kBatchChunk, k, j))
+    if (!work_item(lb, (n + NS - 1) / NS, b.npairs, b.turn > 0 ? b.turn : kBatchChunk, k, j))
         return;
     const BatchPair &q = b.pairs[k];
     if (q.out < 0)

@@ -85,6 +85,8 @@ struct BatchParams {
     const float4 *sky4;       /* forward: I, Q, U, 0 per pixel */
     const BatchPair *pairs;   /* device, sorted by rho_max descending */
     int npairs, ngroups;      /* ngroups = ceil(npairs / G) */
+    int turn;                 /* per-pair items: blocks of a pair before the next pair's (0:
+                               * kBatchChunk) */
     FastConsts64 fc64;        /* crho thresholds of the double-precision form */
     const float *ra, *dec, *pa;
     long ptg_stride;          /* 0: shared pointing; else pair `out` at out * ptg_stride */
