@@ -465,12 +465,13 @@ int pisco_pix2ang(int nside, long pix, double *theta, double *phi);
 long pisco_band_annulus(int nside_sky, int nside_beam, long npix_beam, int rows, int band,
                         float ra, float dec, int cover, long cap, int *pix);
 
-/* The automatic launch shape of a single-pair call (tuning keys at their
- * defaults): lanes per sample and strips per disc of the forward, then of the
- * sky adjoint over nsamples samples.  Host only; it exposes the rules so that
- * they can be checked. */
+/* The automatic launch shape of a call (tuning keys at their defaults, 256
+ * CUs): lanes per sample and strips per disc of a pair's forward, then of its
+ * sky adjoint over nsamples samples; pixels of an LDS window of that adjoint,
+ * and of a batched one of four such pairs, with integer sums.  Host only; it
+ * exposes the rules so that they can be checked. */
 int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamples,
-                       int shape[4]);
+                       int shape[6]);
 
 /* E-field magnitude and phase of a perfectly co-polarised elliptical
  * Gaussian beam on the first npix pixels of a beam map

@@ -133,12 +133,14 @@ int pisco::pair_params(int nside_sky, const float *I, const float *Q, const floa
     return PISCO_OK;
 }
 
-/* Expected sky pixels per disc, npix (1 - cos rho_max) / 2. */
-static double disc_pixels(const PairParams &p)
+/* Expected sky pixels in a disc of radius rho, npix (1 - cos rho) / 2. */
+static double disc_pixels(const Hpx &hs, double rho)
 {
-    const double s = pl_sin(0.5 * std::min(p.rho_max, kPi));
-    return (double)p.hs.npix * s * s;
+    const double s = pl_sin(0.5 * std::min(rho, kPi));
+    return (double)hs.npix * s * s;
 }
+
+static double disc_pixels(const PairParams &p) { return disc_pixels(p.hs, p.rho_max); }
 
 /* Strips by the sizes of the beam and the disc: a strip of a large beam stays in
  * an XCD's 4 MB L2, and each strip costs a table build per sample.  Forward at
@@ -173,16 +175,19 @@ int pisco::strips_auto(const PairParams &p, bool adjoint)
  * number of samples (a sample's sum would depend on it), so large discs take a
  * wave each: few samples would otherwise leave most waves idle.  Strips are of
  * one-wave samples. */
-static int disc_lanes(const PairParams &p)
+static int disc_lanes(double dp)
 {
-    const double dp = disc_pixels(p);
     return dp < 1000.0 ? 8 : dp < 3000.0 ? 16 : 64;
 }
 
 int pisco::forward_lanes_auto(const PairParams &p)
 {
-    return strips_auto(p, false) > 1 ? 64 : disc_lanes(p);
+    return strips_auto(p, false) > 1 ? 64 : disc_lanes(disc_pixels(p));
 }
+
+/* Defaults of the sky adjoint's windows: pixels and rings of one, samples of a
+ * batched one. */
+constexpr int kAdjCap = 6144, kAdjRings = 1024, kBatchWindow = 16;
 
 struct pisco_ctx {
     pisco_run_config cfg{};
@@ -209,8 +214,8 @@ struct pisco_ctx {
     int ncu = 256;                /* compute units of the device */
     /* tuning (pisco_set_tuning) */
     int adjmap_chunk = -1;        /* samples per LDS window; 0 = direct atomics, -1 = auto */
-    int adjmap_cap = 6144;        /* LDS window pixels */
-    int adjmap_rw = 1024;         /* LDS window rings */
+    int adjmap_cap = kAdjCap;     /* LDS window pixels, at most */
+    int adjmap_rw = kAdjRings;    /* LDS window rings */
     int adjmap_blocks = 0;        /* persistent blocks; 0 = one block per window (work item) */
     int adjmap_support = 1;       /* size LDS windows by the beam's non-zero rows */
     int batch_group = 0;          /* pairs per wave in batched forwards (1: per-pair items;
@@ -414,7 +419,7 @@ int det_scale(pisco_ctx *c, const FixSource &f, long count, hipStream_t st, cons
 }
 
 /* Samples per LDS window of a single-pair sky adjoint with `lanes` lanes per
- * sample: the tuning value, or (auto) the largest power of two up to 128 that
+ * sample: the largest power of two up to 128 that
  * keeps a window at 40,000 expected visits, but at least a sample per lane
  * group of the block's waves; fewer, down to 16 (64 lanes: 8), where there would
  * be less than one window per CU.  Each window costs three block-wide passes besides its
@@ -424,10 +429,8 @@ int det_scale(pisco_ctx *c, const FixSource &f, long count, hipStream_t st, cons
  * samples 0.135, 0.098, 0.097, 0.119.  With strips 8 samples: the samples in
  * flight are fewer and the strip of the beam that they meet is smaller (16:
  * 15.9 ms, 8: 14.0 ms at 6,000 pixels per disc). */
-int adj_chunk(const pisco_ctx *c, const PairParams &p, int lanes)
+int adj_chunk_auto(const PairParams &p, int lanes)
 {
-    if (c->adjmap_chunk > 0)
-        return c->adjmap_chunk;
     if (lanes == 64 && strips_auto(p, true) > 1)
         return kAdjWaves;
     const double dp = disc_pixels(p);
@@ -439,17 +442,48 @@ int adj_chunk(const pisco_ctx *c, const PairParams &p, int lanes)
     return chunk;
 }
 
-/* The window capacity that fits the LDS next to the per-wave tables. */
-int fit_cap(int cap, int rw, int group, bool det, int lanes)
+/* The tuning value, or adj_chunk_auto. */
+int adj_chunk(const pisco_ctx *c, const PairParams &p, int lanes)
+{
+    return c->adjmap_chunk > 0 ? c->adjmap_chunk : adj_chunk_auto(p, lanes);
+}
+
+/* What the sky adjoint's windows are sized by. */
+struct AdjTuning {
+    int cap, rw, ncu;
+};
+AdjTuning adj_tuning(const pisco_ctx *c) { return {c->adjmap_cap, c->adjmap_rw, c->ncu}; }
+
+/* The window capacity that fits the LDS next to the per-wave tables, for a launch
+ * of `blocks` windows of about `pixels` pixels each: with two blocks per CU, whose
+ * passes overlap; with one block, a third of the slabs, where there is at most a
+ * window per CU, or where the smaller windows would come near the 63 slabs that a
+ * window can be cut into (its remaining rings then take global atomics).  Integer
+ * sums, ms for two blocks and one: single pair, 8,600 pixels, 1,000 samples 0.36,
+ * 0.33, 4,000 samples 0.45, 0.53; 138,000 pixels, 4,000 samples 6.0, 5.0; 77,600
+ * pixels 2.7, 3.1; groups of four, 2,160 pixels, 3,500 samples 0.29, 0.26, 2e4 samples
+ * 1.06, 1.09; 77,600 pixels, 12,000 samples 18.6, 15.9. */
+int fit_cap(const AdjTuning &t, int group, bool det, int lanes, long blocks, double pixels)
 {
     auto fit = [&](size_t bytes) {
-        int k = cap;
-        while (k > 256 && adjmap_lds_bytes(k, rw, group, det, lanes) > bytes)
+        int k = t.cap;
+        while (k > 256 && adjmap_lds_bytes(k, t.rw, group, det, lanes) > bytes)
             k -= 256;
         return k;
     };
-    const int two = fit(81920);   /* two blocks per CU */
-    return two >= 1024 || two == cap ? two : fit(163840);
+    const int two = fit(81920);
+    if (two == t.cap)
+        return two;
+    const bool one = two < 1024 || blocks <= t.ncu || pixels > (group ? 36.0 : 56.0) * two;
+    return one ? fit(163840) : two;
+}
+
+/* The same for the sky adjoint of one pair in windows of `chunk` samples. */
+int pair_cap(const AdjTuning &t, const PairParams &p, bool det, int lanes, int chunk)
+{
+    const int strips = lanes == 64 ? strips_auto(p, true) : 1;
+    const long windows = (p.s_end - p.s_begin + chunk - 1) / chunk;
+    return fit_cap(t, 0, det, lanes, windows * strips, disc_pixels(p) / strips);
 }
 
 /* The batched launches compute the nearest-pixel convolution only. */
@@ -574,7 +608,7 @@ int pisco_pix2ang(int nside, long pix, double *theta, double *phi)
     return PISCO_OK;
 }
 
-int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamples, int shape[4])
+int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamples, int shape[6])
 {
     if (!valid_nside(nside_sky) || !valid_nside(nside_beam) || npix_beam < 1 ||
         npix_beam >= 12L * nside_beam * nside_beam || nsamples < 0 || !shape)
@@ -589,6 +623,10 @@ int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamp
     shape[1] = shape[0] == 64 ? strips_auto(p, false) : 1;
     shape[2] = adj_lanes_auto(p);
     shape[3] = shape[2] == 64 ? strips_auto(p, true) : 1;
+    const AdjTuning t = {kAdjCap, kAdjRings, 256};
+    shape[4] = pair_cap(t, p, true, shape[2], adj_chunk_auto(p, shape[2]));
+    shape[5] = fit_cap(t, 4, true, 64, (nsamples + kBatchWindow - 1) / kBatchWindow,
+                       disc_pixels(p));
     return PISCO_OK;
 }
 
@@ -1226,7 +1264,7 @@ int pisco_dev_adjoint_map(pisco_ctx *c, void *stream, int nside_sky, int nside_b
         if ((c->adjmap_chunk != 0 || det) && !c->beam_interp) {
             const int lanes = adj_lanes(c, p);
             const int chunk = adj_chunk(c, p, lanes);
-            const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, 0, det, lanes);
+            const int cap = pair_cap(adj_tuning(c), p, det, lanes, chunk);
             if (c->adjmap_support) {
                 CHK(c->support.ensure(1));
                 HIPCHK(launch_beam_support(beam8, npix_beam, c->support.p, st));
@@ -1571,11 +1609,7 @@ std::vector<int> batch_ranges(const pisco_ctx *c, const pisco_batch *b)
  * call in the order of its FP64 sums. */
 int pair_lanes(const BatchParams &b, const BatchPair &q)
 {
-    PairParams p;
-    memset(&p, 0, sizeof p);
-    p.hs = b.hs;
-    p.rho_max = q.rho_max;
-    const int lanes = disc_lanes(p);
+    const int lanes = disc_lanes(disc_pixels(b.hs, q.rho_max));
     return lanes == 8 && b.nsamples < 2048 ? 16 : lanes;
 }
 
@@ -1594,16 +1628,12 @@ int pair_lanes(const BatchParams &b, const BatchPair &q)
  * pairs of 540 to 960 pixels, up to 1.9 MB, 6,000 samples 0.135, items 0.158. */
 int group_auto(const BatchParams &b, const pisco_batch *bt, int k, int &lanes)
 {
-    PairParams p;
-    memset(&p, 0, sizeof p);
-    p.hs = b.hs;
-    p.rho_max = bt->host[k].rho_max;   /* the largest disc */
-    double mb = 0.0;                   /* the largest beam */
+    const bool few = disc_pixels(b.hs, bt->host[k].rho_max) < 1000.0;   /* the largest disc */
+    double mb = 0.0;                                                    /* the largest beam */
     for (int j = k; j < k + 4; j++)
         if (bt->host[j].out >= 0)
             mb = std::max(mb, 32.0 * bt->host[j].npix / (1 << 20));
     lanes = 0;
-    const bool few = disc_pixels(p) < 1000.0;
     if (mb <= (few ? 2.0 : 1.0))
         return 4;
     if (!few && mb <= 1.7)
@@ -1723,8 +1753,9 @@ int batch_adjoint_pairwise(pisco_ctx *c, hipStream_t st, const pisco_batch *b, i
             p.beam_last = c->support.p;
         }
         const int lanes = adj_lanes(c, p);
-        const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, 0, scale != nullptr, lanes);
-        CHK(run_adjmap(c, p, adj_chunk(c, p, lanes), cap, scale, lanes, st));
+        const int chunk = adj_chunk(c, p, lanes);
+        CHK(run_adjmap(c, p, chunk, pair_cap(adj_tuning(c), p, scale != nullptr, lanes, chunk), scale, lanes,
+                       st));
     }
     return PISCO_OK;
 }
@@ -1890,11 +1921,9 @@ int pisco_dev_batched_adjoint_map(pisco_ctx *c, void *stream, const pisco_batch 
     bp.gQ = c->acc.p + npix;
     bp.gU = c->acc.p + 2 * npix;
     const int nb = c->adjmap_blocks;   /* 0: one block per window */
-    const int chunk = c->adjmap_chunk > 0 ? c->adjmap_chunk : 16;
+    const int chunk = c->adjmap_chunk > 0 ? c->adjmap_chunk : kBatchWindow;
     const bool det = det_single(c);
     const int grp = c->batch_adj_group;
-    /* the window capacity that fits next to the group's per-wave tables */
-    const int cap = fit_cap(c->adjmap_cap, c->adjmap_rw, grp, det, 64);
     const double *scale = nullptr;
     if (det)
         CHK(batch_det_scale(c, st, b, nsamples, g, &scale));
@@ -1923,8 +1952,11 @@ int pisco_dev_batched_adjoint_map(pisco_ctx *c, void *stream, const pisco_batch 
         p.gU = bp.gU;
         p.s_begin = 0;
         p.s_end = nsamples;
-        hipError_t e = launch_adjmap_lds(p, chunk, cap, c->adjmap_rw, nb, st, &bp,
-                                         std::min(b->rho_support, q0.rho_max), grp, scale);
+        const double rho_w = std::min(b->rho_support, q0.rho_max);
+        const int cap = fit_cap(adj_tuning(c), grp, det, 64, (nsamples + chunk - 1) / chunk,
+                                disc_pixels(p.hs, rho_w));
+        hipError_t e = launch_adjmap_lds(p, chunk, cap, c->adjmap_rw, nb, st, &bp, rho_w, grp,
+                                         scale);
         if (e != hipSuccess)
             return fail(PISCO_ERR_DEVICE, "batched sky adjoint launch failed: %s",
                         hipGetErrorString(e));

@@ -12,7 +12,7 @@ from pisco4cmb_amd._lib import check, lib
 
 
 def shape(ns, nb, cap_deg, n=100000):
-    s = (ctypes.c_int * 4)()
+    s = (ctypes.c_int * 6)()
     npix = pypisco.beam_npix_for_radius(nb, math.radians(cap_deg))
     check(lib.pisco_launch_shape(ns, nb, npix, n, s))
     return list(s)
@@ -30,7 +30,7 @@ def shape(ns, nb, cap_deg, n=100000):
 ])
 def test_strips_keep_their_visits(ns, nb, cap, fwd, adj):
     s = shape(ns, nb, cap)
-    assert s[:2] == fwd and s[2:] == adj
+    assert s[:2] == fwd and s[2:4] == adj
 
 
 def test_forward_shape_is_the_same_for_any_number_of_samples():
@@ -38,8 +38,26 @@ def test_forward_shape_is_the_same_for_any_number_of_samples():
         assert len({tuple(shape(ns, nb, cap, n)[:2]) for n in (0, 1, 500, 5000, 10**6)}) == 1
 
 
+@pytest.mark.parametrize("cap", [1.5, 3.0, 4.5, 6.0, 9.0])
+def test_windows_reach_large_discs(cap):
+    """A window that is cut into more slabs of rings than the adjoint has (63)
+    leaves the rest to global atomics; a slab is at least 5/6 full of these
+    discs' rings (at most 1,250 pixels of 7,168)."""
+    ns, nb = 2048, 2048
+    disc = 12.0 * ns * ns * math.sin(math.radians(cap) / 2) ** 2
+    for n in (100, 4000, 100000):
+        for window in shape(ns, nb, cap, n)[4:]:
+            assert 63 * window * 5 / 6 > min(disc, 200000.0)
+
+
+@pytest.mark.parametrize("ns,nb,cap", [(512, 2048, 3.0), (2048, 2048, 3.0)])
+def test_one_window_per_cu_takes_its_whole_lds(ns, nb, cap):
+    for k in (4, 5):
+        assert shape(ns, nb, cap, 1000)[k] > 2 * shape(ns, nb, cap, 100000)[k]
+
+
 def test_bad_arguments():
-    s = (ctypes.c_int * 4)()
+    s = (ctypes.c_int * 6)()
     assert lib.pisco_launch_shape(0, 512, 100, 1, s) != 0
     assert lib.pisco_launch_shape(64, 512, 0, 1, s) != 0
     assert lib.pisco_launch_shape(64, 512, 100, -1, s) != 0
