@@ -127,8 +127,8 @@ int pisco_exec_adjoint_beam(pisco_ctx *ctx, const float *g_a, const float *g_b,
  * NSIDE 512, 5-degree workload; except for beam_interpolation, results do
  * not depend on them).  Keys: "adjmap_chunk" (samples per LDS window of the sky adjoint;
  * 0 selects direct global atomics; -1, the default, picks 8 to 128 from the
- * disc, the beam and the number of samples for single-pair adjoints and 16 for
- * batched ones), "adjmap_cap" (window pixels),
+ * disc, the beam and the number of samples for single-pair adjoints, and for
+ * batched ones 8 below 4,096 samples, else 16), "adjmap_cap" (window pixels),
  * "adjmap_rw" (window rings), "adjmap_blocks" (blocks of the adjoint launches,
  * each looping over windows; 0, the default, one block per window), "adjmap_support" (1: windows cover only the discs of the beam's
  * non-zero rows, 0: the full rho_max discs; results are the same either way),
@@ -467,11 +467,11 @@ long pisco_band_annulus(int nside_sky, int nside_beam, long npix_beam, int rows,
 
 /* The automatic launch shape of a call (tuning keys at their defaults, 256
  * CUs): lanes per sample and strips per disc of a pair's forward, then of its
- * sky adjoint over nsamples samples; pixels of an LDS window of that adjoint,
- * and of a batched one of four such pairs, with integer sums.  Host only; it
+ * sky adjoint over nsamples samples; samples and pixels of an LDS window of that
+ * adjoint, then of a batched one of four such pairs, with integer sums.  Host only; it
  * exposes the rules so that they can be checked. */
 int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamples,
-                       int shape[6]);
+                       int shape[8]);
 
 /* E-field magnitude and phase of a perfectly co-polarised elliptical
  * Gaussian beam on the first npix pixels of a beam map

@@ -185,9 +185,8 @@ int pisco::forward_lanes_auto(const PairParams &p)
     return strips_auto(p, false) > 1 ? 64 : disc_lanes(disc_pixels(p));
 }
 
-/* Defaults of the sky adjoint's windows: pixels and rings of one, samples of a
- * batched one. */
-constexpr int kAdjCap = 6144, kAdjRings = 1024, kBatchWindow = 16;
+/* Defaults of the sky adjoint's windows: pixels and rings. */
+constexpr int kAdjCap = 6144, kAdjRings = 1024;
 
 struct pisco_ctx {
     pisco_run_config cfg{};
@@ -448,6 +447,13 @@ int adj_chunk(const pisco_ctx *c, const PairParams &p, int lanes)
     return c->adjmap_chunk > 0 ? c->adjmap_chunk : adj_chunk_auto(p, lanes);
 }
 
+/* Samples per LDS window of a batched sky adjoint: 16, or a sample per wave where
+ * 16 would leave less than one window per CU.  Groups of four, ms for 8 and 16: 540
+ * pixels, 2,000 samples 0.096, 0.134; 345 pixels of a sky of NSIDE 2048 0.667, 0.702;
+ * 34,500 pixels 1.94, 2.86; 3,500 samples (and the smaller windows then) 0.117, 0.136;
+ * 0.683, 0.700; 2.91, 2.93. */
+int batch_chunk_auto(long nsamples) { return nsamples < 256L * 16 ? kAdjWaves : 16; }
+
 /* What the sky adjoint's windows are sized by. */
 struct AdjTuning {
     int cap, rw, ncu;
@@ -608,7 +614,7 @@ int pisco_pix2ang(int nside, long pix, double *theta, double *phi)
     return PISCO_OK;
 }
 
-int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamples, int shape[6])
+int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamples, int shape[8])
 {
     if (!valid_nside(nside_sky) || !valid_nside(nside_beam) || npix_beam < 1 ||
         npix_beam >= 12L * nside_beam * nside_beam || nsamples < 0 || !shape)
@@ -624,9 +630,10 @@ int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamp
     shape[2] = adj_lanes_auto(p);
     shape[3] = shape[2] == 64 ? strips_auto(p, true) : 1;
     const AdjTuning t = {kAdjCap, kAdjRings, 256};
-    shape[4] = pair_cap(t, p, true, shape[2], adj_chunk_auto(p, shape[2]));
-    shape[5] = fit_cap(t, 4, true, 64, (nsamples + kBatchWindow - 1) / kBatchWindow,
-                       disc_pixels(p));
+    shape[4] = adj_chunk_auto(p, shape[2]);
+    shape[5] = pair_cap(t, p, true, shape[2], shape[4]);
+    shape[6] = batch_chunk_auto(nsamples);
+    shape[7] = fit_cap(t, 4, true, 64, (nsamples + shape[6] - 1) / shape[6], disc_pixels(p));
     return PISCO_OK;
 }
 
@@ -1921,7 +1928,7 @@ int pisco_dev_batched_adjoint_map(pisco_ctx *c, void *stream, const pisco_batch 
     bp.gQ = c->acc.p + npix;
     bp.gU = c->acc.p + 2 * npix;
     const int nb = c->adjmap_blocks;   /* 0: one block per window */
-    const int chunk = c->adjmap_chunk > 0 ? c->adjmap_chunk : kBatchWindow;
+    const int chunk = c->adjmap_chunk > 0 ? c->adjmap_chunk : batch_chunk_auto(nsamples);
     const bool det = det_single(c);
     const int grp = c->batch_adj_group;
     const double *scale = nullptr;

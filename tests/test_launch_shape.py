@@ -12,7 +12,7 @@ from pisco4cmb_amd._lib import check, lib
 
 
 def shape(ns, nb, cap_deg, n=100000):
-    s = (ctypes.c_int * 6)()
+    s = (ctypes.c_int * 8)()
     npix = pypisco.beam_npix_for_radius(nb, math.radians(cap_deg))
     check(lib.pisco_launch_shape(ns, nb, npix, n, s))
     return list(s)
@@ -46,18 +46,26 @@ def test_windows_reach_large_discs(cap):
     ns, nb = 2048, 2048
     disc = 12.0 * ns * ns * math.sin(math.radians(cap) / 2) ** 2
     for n in (100, 4000, 100000):
-        for window in shape(ns, nb, cap, n)[4:]:
+        for window in shape(ns, nb, cap, n)[5::2]:
             assert 63 * window * 5 / 6 > min(disc, 200000.0)
 
 
 @pytest.mark.parametrize("ns,nb,cap", [(512, 2048, 3.0), (2048, 2048, 3.0)])
 def test_one_window_per_cu_takes_its_whole_lds(ns, nb, cap):
-    for k in (4, 5):
+    for k in (5, 7):
         assert shape(ns, nb, cap, 1000)[k] > 2 * shape(ns, nb, cap, 100000)[k]
 
 
+def test_short_calls_fill_the_cus():
+    """At least 256 windows, or windows of a sample per wave."""
+    for n in (1, 300, 4095, 4096, 10**5):
+        for k in (4, 6):
+            s = shape(512, 2048, 3.0, n)
+            assert s[k] == 8 or n >= 256 * s[k] or s[2] < 64 and s[k] == 16
+
+
 def test_bad_arguments():
-    s = (ctypes.c_int * 6)()
+    s = (ctypes.c_int * 8)()
     assert lib.pisco_launch_shape(0, 512, 100, 1, s) != 0
     assert lib.pisco_launch_shape(64, 512, 0, 1, s) != 0
     assert lib.pisco_launch_shape(64, 512, 100, -1, s) != 0
