@@ -128,7 +128,10 @@ int pisco_exec_adjoint_beam(pisco_ctx *ctx, const float *g_a, const float *g_b,
  * not depend on them).  Keys: "adjmap_chunk" (samples per LDS window of the sky adjoint;
  * 0 selects direct global atomics; -1, the default, picks 8 to 128 from the
  * disc, the beam and the number of samples for single-pair adjoints, and for
- * batched ones 8 below 4,096 samples, else 16), "adjmap_cap" (window pixels),
+ * batched ones 8 below 4,096 samples, else 16), "adjmap_cap" (window pixels,
+ * as many of them as fit the LDS; until it is set, the capacity leaves room for
+ * two blocks per CU where that is faster; "adjmap_window", read only, is the
+ * capacity of the last call),
  * "adjmap_rw" (window rings), "adjmap_blocks" (blocks of the adjoint launches,
  * each looping over windows; 0, the default, one block per window), "adjmap_support" (1: windows cover only the discs of the beam's
  * non-zero rows, 0: the full rho_max discs; results are the same either way),

@@ -214,6 +214,8 @@ struct pisco_ctx {
     /* tuning (pisco_set_tuning) */
     int adjmap_chunk = -1;        /* samples per LDS window; 0 = direct atomics, -1 = auto */
     int adjmap_cap = kAdjCap;     /* LDS window pixels, at most */
+    bool adjmap_cap_set = false;  /* the caller's value: as many of them as fit */
+    int adjmap_window = 0;        /* of the last LDS-window sky adjoint */
     int adjmap_rw = kAdjRings;    /* LDS window rings */
     int adjmap_blocks = 0;        /* persistent blocks; 0 = one block per window (work item) */
     int adjmap_support = 1;       /* size LDS windows by the beam's non-zero rows */
@@ -457,8 +459,12 @@ int batch_chunk_auto(long nsamples) { return nsamples < 256L * 16 ? kAdjWaves : 
 /* What the sky adjoint's windows are sized by. */
 struct AdjTuning {
     int cap, rw, ncu;
+    bool cap_set;   /* the caller chose cap */
 };
-AdjTuning adj_tuning(const pisco_ctx *c) { return {c->adjmap_cap, c->adjmap_rw, c->ncu}; }
+AdjTuning adj_tuning(const pisco_ctx *c)
+{
+    return {c->adjmap_cap, c->adjmap_rw, c->ncu, c->adjmap_cap_set};
+}
 
 /* The window capacity that fits the LDS next to the per-wave tables, for a launch
  * of `blocks` windows of about `pixels` pixels each: with two blocks per CU, whose
@@ -477,6 +483,8 @@ int fit_cap(const AdjTuning &t, int group, bool det, int lanes, long blocks, dou
             k -= 256;
         return k;
     };
+    if (t.cap_set)
+        return fit(163840);
     const int two = fit(81920);
     if (two == t.cap)
         return two;
@@ -507,6 +515,7 @@ int run_adjmap(pisco_ctx *c, PairParams p, int chunk, int cap, const double *sca
 {
     const long n = p.s_end;
     long step = n - p.s_begin;
+    c->adjmap_window = cap;
     if (lanes == 64)
         CHK(use_strips(c, p, step, true));
     for (long s = p.s_begin; s < n; s += step) {
@@ -629,7 +638,7 @@ int pisco_launch_shape(int nside_sky, int nside_beam, long npix_beam, long nsamp
     shape[1] = shape[0] == 64 ? strips_auto(p, false) : 1;
     shape[2] = adj_lanes_auto(p);
     shape[3] = shape[2] == 64 ? strips_auto(p, true) : 1;
-    const AdjTuning t = {kAdjCap, kAdjRings, 256};
+    const AdjTuning t = {kAdjCap, kAdjRings, 256, false};
     shape[4] = adj_chunk_auto(p, shape[2]);
     shape[5] = pair_cap(t, p, true, shape[2], shape[4]);
     shape[6] = batch_chunk_auto(nsamples);
@@ -653,6 +662,7 @@ int pisco_set_tuning(pisco_ctx *c, const char *key, long value)
             return fail(PISCO_ERR_INVALID, "LDS window does not fit 160 KiB");
         c->adjmap_cap = cap;
         c->adjmap_rw = rw;
+        c->adjmap_cap_set = c->adjmap_cap_set || k == "adjmap_cap";
     } else if (k == "adjmap_support") {
         if (value != 0 && value != 1)
             return fail(PISCO_ERR_INVALID, "adjmap_support must be 0 or 1");
@@ -758,6 +768,8 @@ int pisco_get_tuning(pisco_ctx *c, const char *key, long *value)
 
     else if (k == "adjmap_cap")
         *value = c->adjmap_cap;
+    else if (k == "adjmap_window")
+        *value = c->adjmap_window;
     else if (k == "adjmap_rw")
         *value = c->adjmap_rw;
     else if (k == "adjmap_blocks")
@@ -1962,6 +1974,7 @@ int pisco_dev_batched_adjoint_map(pisco_ctx *c, void *stream, const pisco_batch 
         const double rho_w = std::min(b->rho_support, q0.rho_max);
         const int cap = fit_cap(adj_tuning(c), grp, det, 64, (nsamples + chunk - 1) / chunk,
                                 disc_pixels(p.hs, rho_w));
+        c->adjmap_window = cap;
         hipError_t e = launch_adjmap_lds(p, chunk, cap, c->adjmap_rw, nb, st, &bp, rho_w, grp,
                                          scale);
         if (e != hipSuccess)

@@ -7,6 +7,7 @@ tests."""
 import numpy as np
 import pytest
 
+from pisco4cmb_amd import pypisco
 from test_gpu_strips import Calls, make, rel_rms
 from test_launch_shape import shape
 
@@ -31,3 +32,23 @@ def test_automatic_strips(oracle):
     ref = oracle.adjoint_map(ns, nb, beams, *args)
     for x, r in zip(c.adjoint(*args), ref):
         assert rel_rms(x, r) < 1e-6
+
+
+def test_window_capacity_is_the_callers():
+    """adjmap_cap gives the launches that it names, as many of its pixels as fit the
+    LDS beside the tables: the capacities of the slab tests are three different ones
+    with integer sums as well."""
+    ns, nb, n = 64, 256, 20
+    sky, beam, ra, dec, pa, g = make(ns, nb, 6.0, n, 12)
+    conv = pypisco.GPUConvolver(pypisco.default_run_config())
+    conv.configure_execution()
+    c = Calls(ns, nb, beam, sky)
+    c.ctx = conv.ctx
+    for det in (0, 1):
+        c.tune(adjmap_deterministic=det, adjmap_lanes=64)
+        used = []
+        for cap in (6144, 2048, 512):
+            c.tune(adjmap_cap=cap)
+            c.adjoint(ra, dec, pa, *g)
+            used.append(conv.get_tuning("adjmap_window"))
+        assert used[1:] == [2048, 512] and 4500 < used[0] <= 6144
