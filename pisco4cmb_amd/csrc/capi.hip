@@ -479,8 +479,8 @@ int fit_cap(const AdjTuning &t, int group, bool det, int lanes, long blocks, dou
 {
     auto fit = [&](size_t bytes) {
         int k = t.cap;
-        while (k > 256 && adjmap_lds_bytes(k, t.rw, group, det, lanes) > bytes)
-            k -= 256;
+        while (k > 16 && adjmap_lds_bytes(k, t.rw, group, det, lanes) > bytes)
+            k -= k > 256 ? 256 : 16;   /* few pixels beside very many rings */
         return k;
     };
     if (t.cap_set)

@@ -52,3 +52,22 @@ def test_window_capacity_is_the_callers():
             c.adjoint(ra, dec, pa, *g)
             used.append(conv.get_tuning("adjmap_window"))
         assert used[1:] == [2048, 512] and 4500 < used[0] <= 6144
+
+
+@pytest.mark.parametrize("lanes", [8, 16, 64])
+def test_window_beside_very_many_rings(oracle, lanes):
+    """cap + rw at the limit that set_tuning accepts (the tables of one wave per
+    sample; those of lane groups are larger): the window shrinks to what is left."""
+    ns, nb, n = 64, 256, 20
+    sky, beam, ra, dec, pa, g = make(ns, nb, 6.0, n, 13)
+    conv = pypisco.GPUConvolver(pypisco.default_run_config())
+    conv.configure_execution()
+    c = Calls(ns, nb, beam, sky)
+    c.ctx = conv.ctx
+    c.tune(adjmap_lanes=lanes, adjmap_cap=256)
+    c.tune(adjmap_rw=9950)
+    ref = oracle.adjoint_map(ns, nb, list(beam.aBeams) + list(beam.bBeams), ra, dec, pa, *g)
+    for det in (0, 1):
+        c.tune(adjmap_deterministic=det)
+        for x, r in zip(c.adjoint(ra, dec, pa, *g), ref):
+            assert rel_rms(x, r) < 1e-6
