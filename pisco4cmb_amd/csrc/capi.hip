@@ -658,7 +658,7 @@ int pisco_set_tuning(pisco_ctx *c, const char *key, long value)
     } else if (k == "adjmap_cap" || k == "adjmap_rw") {
         int cap = k == "adjmap_cap" ? (int)value : c->adjmap_cap;
         int rw = k == "adjmap_rw" ? (int)value : c->adjmap_rw;
-        if (value < 1 || kAdjTableBytes + 276 + 12 * ((size_t)cap + rw) > 163840)
+        if (value < 1 || kAdjTableBytes + 12 * ((size_t)cap + rw) > 163840)
             return fail(PISCO_ERR_INVALID, "LDS window does not fit 160 KiB");
         c->adjmap_cap = cap;
         c->adjmap_rw = rw;

@@ -3336,7 +3336,7 @@ hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st,
     return hipGetLastError();
 }
 
-/* Table bytes that the limits of cap and rw allow for. */
+/* The limits of cap and rw allow for the tables. */
 static_assert(sizeof(AdjWave<0, kWaveSize>) * kAdjWaves <= kAdjTableBytes);
 size_t adjmap_lds_bytes(int cap, int rw, int group, bool det, int lanes)
 {

@@ -170,7 +170,9 @@ constexpr int kMaxStrips = 8;
 /* Waves per block of the sky adjoint: two blocks per CU, so that one block's
  * window passes, clears and flushes overlap the other's walk. */
 constexpr int kAdjWaves = 8;
-constexpr size_t kAdjTableBytes = 24640;   /* their tables, one wave per sample, at most */
+/* What the limits of the window's pixels and rings leave for the tables (the
+ * tables of one wave per sample take less, those of 8 lanes 448 bytes more). */
+constexpr size_t kAdjTableBytes = 41300;
 constexpr size_t strip_bytes(int strips)
 {
     return kStripLaunch * (sizeof(SampleRec) + 2 * strips * sizeof(double));

@@ -71,3 +71,19 @@ def test_window_beside_very_many_rings(oracle, lanes):
         c.tune(adjmap_deterministic=det)
         for x, r in zip(c.adjoint(ra, dec, pa, *g), ref):
             assert rel_rms(x, r) < 1e-6
+
+
+def test_window_limits():
+    """Pixels and rings together up to 10,211; more was refused before the tables
+    became smaller, and is."""
+    conv = pypisco.GPUConvolver(pypisco.default_run_config())
+    conv.configure_execution()
+    for cap, rw, ok in ((6144, 4067, True), (6144, 4068, False), (9187, 1024, True),
+                        (9188, 1024, False), (256, 9955, True), (256, 9956, False)):
+        conv.set_tuning("adjmap_cap", 1)
+        conv.set_tuning("adjmap_rw", rw)
+        if ok:
+            conv.set_tuning("adjmap_cap", cap)
+        else:
+            with pytest.raises(ValueError):
+                conv.set_tuning("adjmap_cap", cap)
