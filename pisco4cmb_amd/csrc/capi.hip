@@ -350,15 +350,28 @@ int adj_lanes(const pisco_ctx *c, const PairParams &p)
     return c->adjmap_lanes > 0 ? c->adjmap_lanes : adj_lanes_auto(p);
 }
 
+/* Whether a buffer may not grow now: the context's buffers are frozen, or the
+ * stream is being captured. */
+bool pinned(const pisco_ctx *c, hipStream_t st)
+{
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return c->frozen || hipStreamIsCapturing(st, &s) != hipSuccess ||
+           s != hipStreamCaptureStatusNone;
+}
+
 /* Strips for a launch of one wave per sample, whose launches then take at most
- * kStripLaunch samples.  A frozen context without the workspace takes whole
- * discs. */
-int use_strips(pisco_ctx *c, PairParams &p, long &chunk, bool adjoint)
+ * kStripLaunch samples.  Where the workspace may not grow, the forward takes a
+ * disc's strips one after the other (the same sums; p.samples stays NULL) and the
+ * adjoint whole discs. */
+int use_strips(pisco_ctx *c, PairParams &p, long &chunk, bool adjoint, hipStream_t st)
 {
     p.strips = strips_auto(p, adjoint);
     const size_t bytes = strip_bytes(p.strips);
-    if (p.strips == 1 || (bytes > c->strip.cap && c->strip.frozen)) {
-        p.strips = 1;
+    if (p.strips == 1)
+        return PISCO_OK;
+    if (bytes > c->strip.cap && pinned(c, st)) {
+        if (adjoint)
+            p.strips = 1;
         return PISCO_OK;
     }
     CHK(c->strip.ensure(bytes));
@@ -393,7 +406,7 @@ int run_pair(pisco_ctx *c, int op, PairParams p, hipStream_t st, bool sky_packed
     if (chunk < (1L << 20))
         chunk = std::max<long>(chunk, std::min<long>(n - s0, 1L << 20));
     if (fwd && !c->beam_interp && lanes == 64)
-        CHK(use_strips(c, p, chunk, false));
+        CHK(use_strips(c, p, chunk, false, st));
     for (long s = s0; s < n; s += chunk) {
         p.s_begin = s;
         p.s_end = std::min(n, s + chunk);
@@ -517,7 +530,7 @@ int run_adjmap(pisco_ctx *c, PairParams p, int chunk, int cap, const double *sca
     long step = n - p.s_begin;
     c->adjmap_window = cap;
     if (lanes == 64)
-        CHK(use_strips(c, p, step, true));
+        CHK(use_strips(c, p, step, true, st));
     for (long s = p.s_begin; s < n; s += step) {
         p.s_begin = s;
         p.s_end = std::min(n, s + step);

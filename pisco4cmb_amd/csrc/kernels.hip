@@ -863,6 +863,37 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     forward_block<SUB, VT>(p, B, i0, (int)min((long)NS, p.s_end - i0), k, 0.f, false, put);
 }
 
+/* The strips of a disc one after the other, where there is no workspace for their
+ * sums (a captured graph holds the context's buffers): the same sums in the same
+ * order as k_fwd_sub and k_strip_sum.  The waves drift apart over the beam. */
+template <bool VT>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd_strips(PairParams p)
+{
+    __shared__ FwdBlock<kWaveSize> B;
+    constexpr int NS = FwdBlock<kWaveSize>::NS;
+    __shared__ double total[NS][2];
+    const long i0 = p.s_begin + xcd_remap(blockIdx.x, gridDim.x) * NS;
+    const int ns = (int)min((long)NS, p.s_end - i0);
+    if (threadIdx.x < 2 * NS)
+        total[threadIdx.x >> 1][threadIdx.x & 1] = 0.0;
+    auto put = [&](int j, double a, double b) {
+        total[j][0] += a;
+        total[j][1] += b;
+    };
+    for (int k = 0; k < p.strips; k++) {
+        __syncthreads();
+        forward_block<kWaveSize, VT>(p, B, i0, ns, k, 0.f, false, put);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < ns) {
+        const long i = i0 + threadIdx.x;
+        if (p.tod_a)
+            p.tod_a[i] = (float)total[threadIdx.x][0];
+        if (p.tod_b)
+            p.tod_b[i] = (float)total[threadIdx.x][1];
+    }
+}
+
 /* The samples' constants, one per thread. */
 __global__ void k_samples(PairParams p)
 {
@@ -3270,8 +3301,16 @@ hipError_t launch_forward(int lanes, const PairParams &p0, hipStream_t st, bool 
     if (n <= 0)
         return hipSuccess;
     PairParams p = p0;
-    if (!p.samples || lanes != kWaveSize)
+    if (lanes != kWaveSize)
         p.strips = 1;
+    if (p.strips > 1 && !p.samples) {
+        const dim3 g(nblocks(n, FwdBlock<kWaveSize>::NS));
+        if (vterm)
+            hipLaunchKernelGGL(k_fwd_strips<true>, g, dim3(kBlock), 0, st, p);
+        else
+            hipLaunchKernelGGL(k_fwd_strips<false>, g, dim3(kBlock), 0, st, p);
+        return hipGetLastError();
+    }
     if (p.strips > 1)
         hipLaunchKernelGGL(k_samples, dim3(nblocks(n, 64)), dim3(64), 0, st, p);
     switch (lanes) {

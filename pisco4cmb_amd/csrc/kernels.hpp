@@ -162,8 +162,8 @@ hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st,
 hipError_t launch_pair(int op, const PairParams &p, hipStream_t st);
 /* The forward of one pair with 8, 16, 32 or 64 lanes per sample.  With 64 and
  * p.strips > 1 at most kStripLaunch samples, p.samples and p.part in a workspace
- * of strip_bytes(p.strips) bytes (strip_workspace); whole discs if p.samples is
- * NULL. */
+ * of strip_bytes(p.strips) bytes (strip_workspace); without one (p.samples NULL)
+ * a disc's strips one after the other, slower and with the same sums. */
 hipError_t launch_forward(int lanes, const PairParams &p, hipStream_t st, bool vterm = false);
 constexpr long kStripLaunch = 1L << 17;
 constexpr int kMaxStrips = 8;
