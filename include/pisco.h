@@ -202,7 +202,7 @@ int pisco_dev_forward(pisco_ctx *ctx, void *stream, int nside_sky,
  * cannot allocate device memory during the call (code under graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  It takes no
  * context and allocates nothing: its workspace (the sky's ring table and
- * packed pixels, strips) is a fixed device array of 80.1 MiB that each device the
+ * packed pixels, strips) is a fixed device array of 56.1 MiB that each device the
  * library runs on holds for the life of the process, so the sky NSIDE is at
  * most 512 (a larger one is refused with PISCO_ERR_INVALID; pisco_dev_forward
  * takes any).  Runs on the current device and the given stream with the

@@ -360,23 +360,26 @@ bool pinned(const pisco_ctx *c, hipStream_t st)
 }
 
 /* Strips for a launch of one wave per sample, whose launches then take at most
- * kStripLaunch samples.  Where the workspace may not grow, the forward takes a
+ * kStripLaunch samples; the workspace is sized for the call, in powers of two.  Where the workspace may not grow, the forward takes a
  * disc's strips one after the other (the same sums; p.samples stays NULL) and the
  * adjoint whole discs. */
 int use_strips(pisco_ctx *c, PairParams &p, long &chunk, bool adjoint, hipStream_t st)
 {
     p.strips = strips_auto(p, adjoint);
-    const size_t bytes = strip_bytes(p.strips);
     if (p.strips == 1)
         return PISCO_OK;
+    long samples = 256;
+    while (samples < std::min(p.s_end - p.s_begin, kStripLaunch))
+        samples *= 2;
+    const size_t bytes = strip_bytes(adjoint ? 0 : p.strips, samples);
     if (bytes > c->strip.cap && pinned(c, st)) {
         if (adjoint)
             p.strips = 1;
         return PISCO_OK;
     }
     CHK(c->strip.ensure(bytes));
-    strip_workspace(p, c->strip.p);
-    chunk = std::min(chunk, kStripLaunch);
+    strip_workspace(p, c->strip.p, samples);
+    chunk = std::min(chunk, samples);
     return PISCO_OK;
 }
 

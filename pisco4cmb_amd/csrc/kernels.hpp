@@ -161,11 +161,11 @@ hipError_t launch_batch_forward(int group, const BatchParams &p, hipStream_t st,
 /* The direct-atomic adjoints. */
 hipError_t launch_pair(int op, const PairParams &p, hipStream_t st);
 /* The forward of one pair with 8, 16, 32 or 64 lanes per sample.  With 64 and
- * p.strips > 1 at most kStripLaunch samples, p.samples and p.part in a workspace
- * of strip_bytes(p.strips) bytes (strip_workspace); without one (p.samples NULL)
+ * p.strips > 1 p.samples and p.part in a workspace of strip_bytes(p.strips, n)
+ * bytes for n samples (strip_workspace); without one (p.samples NULL)
  * a disc's strips one after the other, slower and with the same sums. */
 hipError_t launch_forward(int lanes, const PairParams &p, hipStream_t st, bool vterm = false);
-constexpr long kStripLaunch = 1L << 17;
+constexpr long kStripLaunch = 1L << 17;   /* samples of a launch, at most: 32 MiB */
 constexpr int kMaxStrips = 8;
 /* Waves per block of the sky adjoint: two blocks per CU, so that one block's
  * window passes, clears and flushes overlap the other's walk. */
@@ -173,14 +173,15 @@ constexpr int kAdjWaves = 8;
 /* What the limits of the window's pixels and rings leave for the tables (the
  * tables of one wave per sample take less, those of 8 lanes 448 bytes more). */
 constexpr size_t kAdjTableBytes = 41300;
-constexpr size_t strip_bytes(int strips)
+/* strips 0: the sky adjoint, which keeps the samples' constants only */
+constexpr size_t strip_bytes(int strips, long samples)
 {
-    return kStripLaunch * (sizeof(SampleRec) + 2 * strips * sizeof(double));
+    return samples * (sizeof(SampleRec) + 2 * strips * sizeof(double));
 }
-inline void strip_workspace(PairParams &p, void *ws)
+inline void strip_workspace(PairParams &p, void *ws, long samples)
 {
     p.samples = (SampleRec *)ws;
-    p.part = (double *)((char *)ws + kStripLaunch * sizeof(SampleRec));
+    p.part = (double *)((char *)ws + samples * sizeof(SampleRec));
 }
 /* The beam-interpolation mode of the same operations (k_pair_interp). */
 hipError_t launch_pair_interp(int op, const PairParams &p, hipStream_t st);

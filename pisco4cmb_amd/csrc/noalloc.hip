@@ -8,7 +8,7 @@
  * sky packed as one float4 (I, Q, U, 0) per pixel and the workspace of the
  * forward's strips.  They live in `scratch`, sized for sky NSIDE
  * up to kNoAllocMaxNside: 4 N RingRec records and 12 N^2 float4 pixels, 48.1
- * MiB at N = 512, and 32 MiB for the strips.  Every call rewrites what the forward
+ * MiB at N = 512, and 8 MiB for the strips.  Every call rewrites what the forward
  * reads, so nothing needs clearing; the forward writes each TOD sample once.  Every call on a device shares
  * that device's copy of the array: calls that overlap in time on one device
  * (on different streams, or from different host threads) race.
@@ -31,8 +31,11 @@ constexpr int kNoAllocMaxNside = 512;
 constexpr size_t kRingBytes = sizeof(RingRec) * 4 * (size_t)kNoAllocMaxNside;
 constexpr size_t kSkyOffset = (kRingBytes + 255) / 256 * 256;
 constexpr size_t kSkyBytes = sizeof(float4) * 12 * (size_t)kNoAllocMaxNside * kNoAllocMaxNside;
-constexpr size_t kStripOffset = (kSkyOffset + kSkyBytes + 255) / 256 * 256;
-constexpr size_t kScratchBytes = kStripOffset + strip_bytes(kMaxStrips);
+/* The strips' workspace starts behind the call's sky.  Behind one of NSIDE 512 it
+ * holds 37,000 samples of 6 strips per launch: 2e5 samples of 5 degrees 7.2 ms, with
+ * 4 MiB 7.4, with 32 MiB 7.0 (whole discs 9.3). */
+constexpr size_t kStripBytes = (size_t)8 << 20;
+constexpr size_t kScratchBytes = (kSkyOffset + kSkyBytes + 255) / 256 * 256 + kStripBytes;
 constexpr long kChunk = 1L << 22;   /* samples per launch, as the torch binding's contexts */
 constexpr int kMaxDevices = 64;
 
@@ -121,9 +124,12 @@ int pisco_dev_forward_noalloc(void *stream, int nside_sky, const float *I, const
     p.tod_b = tod_b;
     const int lanes = forward_lanes_auto(p);
     p.strips = lanes < 64 ? 1 : strips_auto(p, false);
-    if (p.strips > 1)
-        strip_workspace(p, base + kStripOffset);
-    const long chunk = p.strips > 1 ? kStripLaunch : kChunk;
+    long chunk = kChunk;
+    if (p.strips > 1) {
+        const size_t off = (kSkyOffset + sizeof(float4) * (size_t)p.hs.npix + 255) / 256 * 256;
+        chunk = std::min(kStripLaunch, (long)((kScratchBytes - off) / strip_bytes(p.strips, 1)));
+        strip_workspace(p, base + off, chunk);
+    }
     for (long s = 0; s < nsamples; s += chunk) {
         p.s_begin = s;
         p.s_end = std::min(nsamples, s + chunk);

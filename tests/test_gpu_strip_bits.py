@@ -107,3 +107,47 @@ def test_captured_after_a_call_without_strips(ctx):
             assert same(ref.bits(), want)
     torch.cuda.synchronize()
     lib.pisco_destroy(other)
+
+
+def test_workspace_is_the_size_of_the_call():
+    """500 samples of five strips need 112 kB; a context held 27 MB for them, and the
+    fixed array of the forward without allocations 32 MiB beside its sky."""
+    import re
+    f = Forward(500)
+    ctx = torch_ops.new_ctx(torch.device("cuda:0"))
+    check(lib.pisco_set_tuning(ctx, b"forward_lanes", 8))
+    f(ctx)                                                  # everything but the strips
+    check(lib.pisco_set_tuning(ctx, b"forward_lanes", 0))
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    f(ctx)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 4 << 20
+    lib.pisco_destroy(ctx)
+    rc = lib.pisco_dev_forward_noalloc(None, 1024, *[s.data_ptr() for s in f.sky[:3]], NB,
+                                       f.beam8.shape[0], f.beam8.data_ptr(), 0, None, None, None,
+                                       None, None)
+    assert rc != 0
+    size = int(re.search(r"(\d+)-byte", lib.pisco_last_error().decode()).group(1))
+    assert size <= 48.2 * 2 ** 20 + (8 << 20)
+
+
+@pytest.mark.parametrize("ns", [64, 512])
+def test_noalloc_launches_of_what_its_workspace_holds(ns):
+    """More samples than one launch's (sky NSIDE 512: 37,000 of six strips): the bits
+    of the forward with allocations."""
+    nb, cap, n = (512, 36.0, 3000) if ns == 64 else (4096, 5.0, 40001)
+    f = Forward(n)
+    if ns == 512:
+        f.sky = [t(x) for x in inputs.iid_sky(ns, seed=4)]
+        npix = pypisco.beam_npix_for_radius(nb, math.radians(cap))
+        f.beam8 = torch.rand((npix, 8), device="cuda")
+    args = (ns, *[s.data_ptr() for s in f.sky[:3]], nb, f.beam8.shape[0], f.beam8.data_ptr(), n,
+            *[x.data_ptr() for x in f.ptg], *[o.data_ptr() for o in f.out])
+    dev = torch.device("cuda:0")
+    check(lib.pisco_dev_forward(torch_ops._ctx(dev), torch_ops._stream(dev), *args))
+    want = f.bits()
+    for o in f.out:
+        o.fill_(float("nan"))
+    check(lib.pisco_dev_forward_noalloc(torch_ops._stream(dev), *args))
+    assert same(f.bits(), want)
