@@ -423,11 +423,10 @@ int pisco_dev_match(pisco_ctx *ctx, void *stream, int nside_sky,
  * construction) -- and writes float cos(2chi), sin(2chi) packed into each
  * 8-byte chi element instead of chi.  Mode 2 is the single-precision form
  * alone: bpix = -2 where it defers to the exact mapping.  Mode 3 is the
- * certified double-precision form of the small-disc kernels (same output
- * layout as mode 1).  Mode 4 is what the one-wave-per-sample forward uses:
- * the double-precision form with a float atan2 for the position angle,
- * and mode 3 where that cannot certify a pixel; mode 5 is that form alone
- * (bpix = -2 where it declines). */
+ * certified double-precision form that maps the deferred visits (same output
+ * layout as mode 1).  Modes 4 and 5 are modes 1 and 2 with the bound for cos,
+ * sin(2chi) in single precision (2.5e-7) of the forward and of the sky adjoint
+ * with several samples per wave. */
 int pisco_dev_match_mode(pisco_ctx *ctx, void *stream, int mode, int nside_sky,
                          int nside_beam, long n, const float *ra,
                          const float *dec, const float *pa, const long *offsets,

@@ -532,6 +532,7 @@ int run_adjmap(pisco_ctx *c, PairParams p, int chunk, int cap, const double *sca
     const long n = p.s_end;
     long step = n - p.s_begin;
     c->adjmap_window = cap;
+    p.eta = c->adjmap_lanes > 0 || disc_pixels(p) < 1000.0 ? kEtaForward : kEtaAdjoint;
     if (lanes == 64)
         CHK(use_strips(c, p, step, true, st));
     for (long s = p.s_begin; s < n; s += step) {

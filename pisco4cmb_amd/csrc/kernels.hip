@@ -562,9 +562,9 @@ __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int
         int bp = visit_pixel(p.fc, sf, g, place);
         float c2 = 0.f, s2 = 0.f;
         if constexpr (F & WALK_CHI) {
-            float c4, s4;
-            visit_phase(g, r.b.w, c4, s4);
-            visit_chi(sf, c4, s4, c2, s2);
+            float d4, s4;
+            visit_phase(g, r.b.w, d4, s4);
+            visit_chi(sf, d4, s4, c2, s2);
             if constexpr (WIDE) {
                 const int rg = wide ? ~t.ring[r.run] : -1;   /* a wide pass has runs */
                 if (rg >= 0) {
@@ -1370,8 +1370,9 @@ __device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, i
             const int pix = v + __float_as_int(r0_.w);
             const VisitGeo g =
                 visit_geo(fmaf(vf - r0_.z, r0_.y, r0_.x), r1_.x, r1_.y, r1_.z, cdc, sdc);
-            float c4, s4;
-            visit_phase(g, r1_.w, c4, s4);
+            float d4, s4;
+            visit_phase(g, r1_.w, d4, s4);
+            float c4 = 1.0f - d4;
             const int r = ps.wide ? ~t.ring[run] : -1;
             if (r >= 0) {
                 const RingRec rr = p.rings[r];
@@ -2051,7 +2052,8 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(4, 4)
                 const int r1 = grp < cnt ? min(ws.rec[j].r_last, rhi) : r0 - 1;
                 int qn = 0;
                 constexpr int F = WALK_BEAM | WALK_CHI;
-                walk_rings<F>(p, tg, ws, j, r0, r1, sl, sf, kEtaAdjoint, qn, after, use, use_exact);
+                walk_rings<F>(p, tg, ws, j, r0, r1, sl, sf, p.eta, qn, after, use,
+                              use_exact);
                 if (qn > 0)
                     drain_queue<F>(p, ws, 0, qn, lane, use_exact);
                 wave_sync();   /* the next samples' constants replace these */
@@ -3173,8 +3175,8 @@ __global__ void k_disc(Hpx h, long n, const float *ra, const float *dec, double 
  *         float cos(2chi), sin(2chi) packed as two floats.
  * mode 2: the float form alone; bpix[k] = kNeedExact (-2) where it declines.
  * mode 3: the FP64 form of the deferred-visit drain (output as mode 1).
- * modes 4, 5: as 1 and 2 with the forward kernels' bound for cos(2chi),
- *         sin(2chi) in float. */
+ * modes 4, 5: as 1 and 2 with the bound of the forward and of the sky adjoint
+ *         with lane groups for cos(2chi), sin(2chi) in float. */
 __global__ void k_match(Hpx hs, const RingRec *rings, Hpx hb, FastConsts fc, FastConsts64 fc64,
                         int mode, long n,
                         const float *ra, const float *dec, const float *pa,
@@ -3203,9 +3205,9 @@ __global__ void k_match(Hpx hs, const RingRec *rings, Hpx hb, FastConsts fc, Fas
                 const VisitGeo v = visit_geo(x, g.sD, g.omD, g.cdp2, sf.cdc, sf.sdc);
                 CapPlace place;
                 bp = visit_pixel(fc, sf, v, place);
-                float c4, s4;
-                visit_phase(v, g.kap, c4, s4);
-                visit_chi(sf, c4, s4, c2, s2);
+                float d4, s4;
+                visit_phase(v, g.kap, d4, s4);
+                visit_chi(sf, d4, s4, c2, s2);
                 if (!(fabsf(g.kap * x) < (mode >= 4 ? kEtaForward : kEtaAdjoint)) ||
                     fabsf(x) > 0.7f)
                     visit_chi64(c, c2psi, s2psi, ra_pix, rr.cdp, rr.sdp, c2, s2);
