@@ -426,7 +426,8 @@ int pisco_dev_match(pisco_ctx *ctx, void *stream, int nside_sky,
  * certified double-precision form that maps the deferred visits (same output
  * layout as mode 1).  Modes 4 and 5 are modes 1 and 2 with the bound for cos,
  * sin(2chi) in single precision (2.5e-7) of the forward and of the sky adjoint
- * with several samples per wave. */
+ * with several samples per wave.  Mode 6 is the batched kernels' single-precision
+ * form alone. */
 int pisco_dev_match_mode(pisco_ctx *ctx, void *stream, int mode, int nside_sky,
                          int nside_beam, long n, const float *ra,
                          const float *dec, const float *pa, const long *offsets,

@@ -836,6 +836,29 @@ __device__ inline int visit_pixel(const FastConsts &fc, const SampleF &f, const 
     return cap_floors(tt, tmp, v.omc, fmaf(tmp, -kFloorMargin, f.lim0), place);
 }
 
+/* The same for the batched kernels, whose pairs share a visit's alpha, in quarter
+ * turns in [-2, 2], and turn it by their own psi: t0 = (pi - psi) 2/pi mod 4. */
+__device__ inline float visit_alpha(const VisitGeo &v)
+{
+    const float ax = fabsf(v.xa), ay = fabsf(v.ya);
+    const float a = quarter_turns(ax, ay);
+    const float m = ay > ax ? a : 1.0f - a;   /* from the y axis */
+    return copysignf(1.0f - copysignf(m, v.xa), v.ya);
+}
+
+__device__ inline float pair_t0(double psi)
+{
+    return (float)fmodulo((kPi - psi) * kInvHalfPi, 4.0);
+}
+
+__device__ inline int pair_pixel(float alpha, float x3y, float omc, float t0, float nside,
+                                 float lim0, CapPlace &place)
+{
+    const float tt = 4.0f * __builtin_amdgcn_fractf(0.25f * (t0 - alpha));
+    const float tmp = nside * x3y;
+    return cap_floors(tt, tmp, omc, fmaf(tmp, -kFloorMarginBatch, lim0), place);
+}
+
 /* |eta| above which cos, sin 2 chi take the FP64 form (visit_chi64): the
  * forward and the sky adjoint with lane groups of discs below 1,000 pixels keep
  * them within 2.2e-7 of FP64, and the other adjoints, whose gradients are float

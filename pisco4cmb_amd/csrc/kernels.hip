@@ -1250,7 +1250,7 @@ __device__ inline void batch_consts(const BatchParams &p, BT &bt, long i, int d0
         const float pa_k = p.pa[i] + q.pa_off;   /* the pair's own pa */
         const double psi = -(double)pa_k;
         pl_sincos(2.0 * psi, &s2, &c2);
-        t0l = (float)fmodulo((kPi - psi) * kInvHalfPi, 4.0);
+        t0l = pair_t0(psi);
         if (ADJ && q.out >= 0) {
             const long row = 2 * (long)q.out * p.nsamples;
             gal = p.g[row + i];
@@ -1379,11 +1379,7 @@ __device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, i
                 visit_chi64(c, 1.0, 0.0, ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, c4, s4);
                 s4 = -s4;
             }
-            /* alpha in quarter turns, in [-2, 2] */
-            const float ax = fabsf(g.xa), ay = fabsf(g.ya);
-            const float a = quarter_turns(ax, ay);
-            const float m = ay > ax ? a : 1.0f - a;   /* from the y axis */
-            const float al = copysignf(1.0f - copysignf(m, g.xa), g.ya);
+            const float al = visit_alpha(g);
             const float x3y = __builtin_amdgcn_sqrtf(3.0f * g.omc);
 
             if (q.live)
@@ -1401,10 +1397,8 @@ __device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, i
             for (int k = 0; k < G; k++) {
                 const bool in = act && g.omc < K.CUT_IN[k];
                 const bool edge = act && !in && !(g.omc > K.CUT_OUT[k]);
-                const float tt = 4.0f * __builtin_amdgcn_fractf(0.25f * (K.T0[k] - al));
-                const float tmp = K.NSF[k] * x3y;
                 CapPlace place;
-                int bp = cap_floors(tt, tmp, g.omc, fmaf(tmp, -kFloorMarginBatch, K.lim0), place);
+                int bp = pair_pixel(al, x3y, g.omc, K.T0[k], K.NSF[k], K.lim0, place);
                 bp = in ? bp : -1;
                 const bool defer = edge || bp == kNeedExact;
                 const unsigned long long md = __ballot(defer);
@@ -3176,7 +3170,8 @@ __global__ void k_disc(Hpx h, long n, const float *ra, const float *dec, double 
  * mode 2: the float form alone; bpix[k] = kNeedExact (-2) where it declines.
  * mode 3: the FP64 form of the deferred-visit drain (output as mode 1).
  * modes 4, 5: as 1 and 2 with the bound of the forward and of the sky adjoint
- *         with lane groups for cos(2chi), sin(2chi) in float. */
+ *         with lane groups for cos(2chi), sin(2chi) in float.
+ * mode 6: the batched kernels' float form alone (as mode 2; chi as mode 5). */
 __global__ void k_match(Hpx hs, const RingRec *rings, Hpx hb, FastConsts fc, FastConsts64 fc64,
                         int mode, long n,
                         const float *ra, const float *dec, const float *pa,
@@ -3204,7 +3199,9 @@ __global__ void k_match(Hpx hs, const RingRec *rings, Hpx hb, FastConsts fc, Fas
                 const float x = fmaf((float)(j - g.kc), g.b, g.a0);
                 const VisitGeo v = visit_geo(x, g.sD, g.omD, g.cdp2, sf.cdc, sf.sdc);
                 CapPlace place;
-                bp = visit_pixel(fc, sf, v, place);
+                bp = mode == 6 ? pair_pixel(visit_alpha(v), __builtin_amdgcn_sqrtf(3.0f * v.omc),
+                                            v.omc, pair_t0(c.psi), (float)hb.nside, sf.lim0, place)
+                               : visit_pixel(fc, sf, v, place);
                 float d4, s4;
                 visit_phase(v, g.kap, d4, s4);
                 visit_chi(sf, d4, s4, c2, s2);

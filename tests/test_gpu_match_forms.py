@@ -58,3 +58,34 @@ def test_gradient_of_small_discs(oracle, lanes, dec):
     err = np.mean(err, axis=0)
     print("I, Q, U", err)
     assert err.max() <= 6.5e-8
+
+
+@pytest.mark.parametrize("ns,nb,cap,n", [(512, 2048, 3.0, 500), (512, 4096, 5.0, 200),
+                                         (2048, 8192, 1.0, 150), (64, 512, 10.0, 500),
+                                         (64, 64, 35.0, 60), (256, 8192, 2.0, 300)])
+@pytest.mark.parametrize("polar", [False, True])
+def test_batched_form(gpu, oracle, ns, nb, cap, n, polar):
+    """The batched kernels' single-precision form: every pixel that it certifies is
+    the oracle's.  It declines where a floor's argument lies within 4e-6 tmp + 2e-6
+    of an integer, tmp <= sqrt(3 (1 - cos cap)) nside, three floors with two sides
+    each, the arguments of ip larger by up to 4: at most 6 x 1.7 times that, and
+    what the pole of the beam and the end of its polar cap add."""
+    rng = np.random.default_rng(ns + nb)
+    if polar:
+        ra, dec, pa = pointings(n, ns, np.array([1.2, -1.3, 1.45, -1.5, 1.55, -1.56, 1.5707]))
+    else:
+        ra, dec, pa = pointings(n, ns, math.pi / 2 - np.arccos(rng.uniform(-1, 1, n)))
+    off, pix = oracle.query_disc_many(ns, ra, dec, math.radians(cap))
+    want, chi = oracle.match(ns, nb, ra, dec, pa, off, pix)
+    bp, c2, s2 = gpu.match_fast(ns, nb, ra, dec, pa, off, pix, mode=6)
+    sure = bp != -2
+    assert np.array_equal(bp[sure], want[sure])
+    assert np.abs(c2 - np.cos(2 * chi))[sure].max() <= 2.5e-7
+    assert np.abs(s2 - np.sin(2 * chi))[sure].max() <= 2.5e-7
+    tmp = math.sqrt(3 * (1 - math.cos(math.radians(cap)))) * nb
+    # a declination beyond the pole has the exact form for every visit
+    regular = np.repeat(np.abs(dec.astype(np.float64)) <= math.pi / 2, np.diff(off))
+    assert not sure[~regular].any()
+    declined = 1 - sure[regular].mean()
+    print("declined %.2e, bound %.2e" % (declined, 10.2 * (4e-6 * tmp + 2e-6)))
+    assert declined <= 10.2 * (4e-6 * tmp + 2e-6) + 2e-3
