@@ -704,6 +704,7 @@ __device__ inline double recip_fast(double n)
 /* Float geometry of a run of consecutive pixels of one ring, positions j0 ..
  * j0+len-1, around one sample: x = dra/2 of position j is (j - kc) b + a0. */
 struct RunGeo {
+    double a0d, bd, kapd;   /* a0, b, kap before the rounding to float */
     float a0, b;
     int kc;
     float sD, omD;    /* sin dD, 1 - cos dD */
@@ -724,15 +725,18 @@ __device__ inline RunGeo run_geo(const Hpx &h, const RingRec &rr, int r, const C
     const double mid = ((double)j0 + 0.5 * (double)(len - 1) + shift) * tpn;
     const double ra = c.ra + kTwoPi * rint((mid - c.ra) * kInvTwoPi);
     const double kc = rint(ra * (nr * kInvTwoPi) - shift);
-    g.a0 = (float)(0.5 * ((kc + shift) * tpn - ra));
-    g.b = (float)(0.5 * tpn);
+    g.a0d = 0.5 * ((kc + shift) * tpn - ra);
+    g.bd = 0.5 * tpn;
+    g.a0 = (float)g.a0d;
+    g.b = (float)g.bd;
     g.kc = (int)kc;
     const double sD = fma(rr.sdp, c.cdc, -(rr.cdp * c.sdc));
     const double rc = recip_fast(1.0 + fma(rr.cdp, c.cdc, rr.sdp * c.sdc));
     g.sD = (float)sD;
     g.omD = (float)(sD * sD * rc);
     g.cdp2 = (float)(2.0 * rr.cdp);
-    g.kap = (float)((c.sdc + rr.sdp) * rc);
+    g.kapd = (c.sdc + rr.sdp) * rc;
+    g.kap = (float)g.kapd;
     return g;
 }
 
@@ -859,7 +863,7 @@ __device__ inline int pair_pixel(float alpha, float x3y, float omc, float t0, fl
     return cap_floors(tt, tmp, omc, fmaf(tmp, -kFloorMarginBatch, lim0), place);
 }
 
-/* |eta| above which cos, sin 2 chi take the FP64 form (visit_chi64): the
+/* |eta| above which cos, sin 2 chi take the FP64 form (visit_phase64): the
  * forward and the sky adjoint with lane groups of discs below 1,000 pixels keep
  * them within 2.2e-7 of FP64, and the other adjoints, whose gradients are float
  * sums of many visits, within 1e-6.  Sky gradient over small discs, relative RMS of Q and U
@@ -870,22 +874,36 @@ __device__ inline int pair_pixel(float alpha, float x3y, float omc, float t0, fl
 constexpr float kEtaForward = 0.078f;
 constexpr float kEtaAdjoint = 0.38f;
 
-/* cos, sin 2 chi in FP64 (Napier's analogy as visit_phase), rounded to
- * float. */
-__device__ inline void visit_chi64(const Centre &c, double c2psi, double s2psi, double ra_pix,
-                                   double cdp, double sdp, float &c2, float &s2)
+/* visit_phase in FP64, rounded to float at the end (with visit_chi: within 1.2e-7),
+ * from h = dra/4 and k2 = 2 kap of the visit: with t = tan h, tan eta = k2 t /
+ * (1 - t^2).  t by a polynomial in h^2 up to h = pi/4 (Chebyshev interpolation,
+ * relative error 1.2e-9). */
+__device__ inline void visit_phase64(double h, double k2, float &d4, float &s4)
+{
+    const double z = h * h;
+    double p = 0x1.21afd124822a5p-8;
+    p = fma(p, z, -0x1.6e08157222680p-17);
+    p = fma(p, z, 0x1.6612cdee32a5fp-7);
+    p = fma(p, z, 0x1.5bfd2464feb1cp-6);
+    p = fma(p, z, 0x1.baf2170033bf3p-5);
+    p = fma(p, z, 0x1.110cd8e996eb4p-3);
+    p = fma(p, z, 0x1.5555655f8048ap-2);
+    p = fma(p, z, 0x1.fffffff6139bfp-1);
+    const double t = h * p, num = k2 * t, den = fma(-t, t, 1.0);
+    const double q = num * num, r = recip_fast(fma(den, den, q));
+    const double ce = fma(den, den, -q) * r, se = 2.0 * (den * num) * r;
+    d4 = (float)(2.0 * (se * se));
+    s4 = (float)(2.0 * (ce * se));
+}
+
+/* The same from the visit's ring. */
+__device__ inline void visit_phase64(const Centre &c, double ra_pix, double cdp, double sdp,
+                                     float &d4, float &s4)
 {
     double dra = ra_pix - c.ra;
     dra = fma(-kTwoPi, rint(dra * kInvTwoPi), dra);
-    double sh, ch;
-    pl_sincos(0.5 * dra, &sh, &ch);
     const double kap = (c.sdc + sdp) * recip_fast(1.0 + fma(cdp, c.cdc, sdp * c.sdc));
-    const double q = kap * sh;
-    const double inv = recip_fast(fma(ch, ch, q * q));
-    const double ce = fma(ch, ch, -(q * q)) * inv, se = 2.0 * (ch * q) * inv;
-    const double c4 = fma(ce, ce, -(se * se)), s4 = 2.0 * (ce * se);
-    c2 = (float)fma(c4, c2psi, s4 * s2psi);
-    s2 = (float)fma(c4, s2psi, -(s4 * c2psi));
+    visit_phase64(0.25 * dra, 2.0 * kap, d4, s4);
 }
 
 struct ExactVisit {

@@ -138,9 +138,27 @@ __device__ inline int build_runs(const Hpx &hs, const Disc &d, int r0, int lane,
  * vector issue and by the gather's lines, 2.15 cycles each per CU.  The marks
  * cover a segment of VCAP visits from seg0 on:
  * bit v - 1 - seg0 marks a run that starts at visit v > seg0. */
-template <int SUB_, int RPP_, int VCAP_>
-struct VisitTable {
+/* A wide run's constants for visit_phase64 (h of position j is (j - kc) b + a0).
+ * With them a wide visit takes about 25 FP64 instructions more than another; from the
+ * ring's record, with a sine and a cosine of full precision, it took a hundred and a
+ * load from memory in the loop.  2e4 samples of 5 degrees at declination 69 degrees
+ * 1.22 -> 0.82 ms (no wide runs 0.71; an FP64 geometry throughout 0.94).  The tables
+ * of 8 lanes and of the sky adjoint have no room for them beside what they hold. */
+struct WideRec {
+    double a0, b, k2;
+};
+template <int N>
+struct WideRecs {   /* of the wide runs, where the LDS has room for them */
+    WideRec wide[N];
+};
+template <>
+struct WideRecs<0> {
+};
+
+template <int SUB_, int RPP_, int VCAP_, bool WIDE_ = false>
+struct VisitTable : WideRecs<WIDE_ ? RPP_ : 0> {
     static constexpr int SUB = SUB_, RPP = RPP_, VCAP = VCAP_;
+    static constexpr bool WIDE = WIDE_;
     float4 rec[RPP][2];      /* a0, b, mid, pixoff (int bits); sD, omD, cdp2, kap */
     unsigned bits[VCAP / 32];
     int pref[RPP + 1];       /* visit offset of each run; pref[nrun] = total */
@@ -246,6 +264,10 @@ __device__ inline Pass build_pass(const Hpx &hs, const RingRec *rings, const Dis
                 const float xm = fmaxf(x0, x1);
                 const bool w = !(fabsf(g.kap) * xm < eta_max) || xm > 0.7f;
                 t.ring[run] = w ? ~r : r;
+                if constexpr (T::WIDE) {
+                    if (w)
+                        t.wide[run] = {0.5 * g.a0d, 0.5 * g.bd, 2.0 * g.kapd};
+                }
                 wide = wide || w;
                 if (off > 0 && off <= T::VCAP)   /* the first segment's marks */
                     atomicOr(&t.bits[mark_word(off)], mark_bit(off));
@@ -554,8 +576,9 @@ __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int
         const int v = v0 + sl;
         const bool act = v < total;
         const int pix = v + __float_as_int(r.a.w);
+        const float at_run = vf - r.a.z;   /* ring positions from the run's kc */
         const VisitGeo g =
-            visit_geo(fmaf(vf - r.a.z, r.a.y, r.a.x), r.b.x, r.b.y, r.b.z, sf.cdc, sf.sdc);
+            visit_geo(fmaf(at_run, r.a.y, r.a.x), r.b.x, r.b.y, r.b.z, sf.cdc, sf.sdc);
         vf += (float)SUB;
         v0 += SUB;
         CapPlace place;
@@ -564,16 +587,20 @@ __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int
         if constexpr (F & WALK_CHI) {
             float d4, s4;
             visit_phase(g, r.b.w, d4, s4);
-            visit_chi(sf, d4, s4, c2, s2);
             if constexpr (WIDE) {
                 const int rg = wide ? ~t.ring[r.run] : -1;   /* a wide pass has runs */
                 if (rg >= 0) {
-                    const RingRec rr = p.rings[rg];
-                    const SampleRec &sr = ws.rec[j];
-                    visit_chi64(rec_centre(sr), sr.c2psi, sr.s2psi, ring_phi(p.hs, rr, rg, pix),
-                                rr.cdp, rr.sdp, c2, s2);
+                    if constexpr (T::WIDE) {
+                        const WideRec &wr = t.wide[r.run];
+                        visit_phase64(fma((double)at_run, wr.b, wr.a0), wr.k2, d4, s4);
+                    } else {
+                        const RingRec rr = p.rings[rg];
+                        visit_phase64(rec_centre(ws.rec[j]), ring_phi(p.hs, rr, rg, pix), rr.cdp,
+                                      rr.sdp, d4, s4);
+                    }
                 }
             }
+            visit_chi(sf, d4, s4, c2, s2);
         }
         bp = act ? bp : -1;
         const unsigned long long m = __ballot(bp == kNeedExact);
@@ -686,7 +713,7 @@ __device__ inline void wave_samples(const PairParams &p, WS &ws, long i0, int cn
 
 template <int SUB>
 using SubTable = VisitTable<SUB, (SUB < 16 ? 24 : SUB < 64 ? 32 : 64),
-                            (SUB < 16 ? 256 : SUB < 64 ? 1024 : 4096)>;
+                            (SUB < 16 ? 256 : SUB < 64 ? 1024 : 4096), (SUB >= 16)>;
 using WaveTable = SubTable<kWaveSize>;
 
 /* ---- forward ---------------------------------------------------------------
@@ -1311,7 +1338,8 @@ __device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, i
                                   After &after, Consume &consume, Exact &exact)
 {
     auto &t = bt.vt;
-    constexpr int VCAP = std::remove_reference<decltype(t)>::type::VCAP;
+    using T = typename std::remove_reference<decltype(t)>::type;
+    constexpr int VCAP = T::VCAP;
     const float cdc = unif((float)c.cdc), sdc = unif((float)c.sdc);
     int qn = 0;
     auto drain = [&](int base, int cnt) {
@@ -1368,17 +1396,22 @@ __device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, i
             const int v = v0 + lane;
             const bool act = v < total;
             const int pix = v + __float_as_int(r0_.w);
+            const float at_run = vf - r0_.z;
             const VisitGeo g =
-                visit_geo(fmaf(vf - r0_.z, r0_.y, r0_.x), r1_.x, r1_.y, r1_.z, cdc, sdc);
+                visit_geo(fmaf(at_run, r0_.y, r0_.x), r1_.x, r1_.y, r1_.z, cdc, sdc);
             float d4, s4;
             visit_phase(g, r1_.w, d4, s4);
-            float c4 = 1.0f - d4;
             const int r = ps.wide ? ~t.ring[run] : -1;
             if (r >= 0) {
-                const RingRec rr = p.rings[r];
-                visit_chi64(c, 1.0, 0.0, ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, c4, s4);
-                s4 = -s4;
+                if constexpr (T::WIDE) {
+                    const WideRec &wr = t.wide[run];
+                    visit_phase64(fma((double)at_run, wr.b, wr.a0), wr.k2, d4, s4);
+                } else {
+                    const RingRec rr = p.rings[r];
+                    visit_phase64(c, ring_phi(p.hs, rr, r, pix), rr.cdp, rr.sdp, d4, s4);
+                }
             }
+            const float c4 = 1.0f - d4;
             const float al = visit_alpha(g);
             const float x3y = __builtin_amdgcn_sqrtf(3.0f * g.omc);
 
@@ -1440,7 +1473,7 @@ template <int G>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_batch_fwd(BatchParams p)
 {
-    using BT = BatchTable<G, VisitTable<kWaveSize, kWaveSize, 4096>>;
+    using BT = BatchTable<G, VisitTable<kWaveSize, kWaveSize, 4096, true>>;
     __shared__ BT tabs[kWavesPerBlock];
     /* each lane's FP64 TOD sums of the group's pairs in LDS, one slot per
      * lane (the same additions in the same order as in registers).  In
@@ -3204,10 +3237,10 @@ __global__ void k_match(Hpx hs, const RingRec *rings, Hpx hb, FastConsts fc, Fas
                                : visit_pixel(fc, sf, v, place);
                 float d4, s4;
                 visit_phase(v, g.kap, d4, s4);
-                visit_chi(sf, d4, s4, c2, s2);
                 if (!(fabsf(g.kap * x) < (mode >= 4 ? kEtaForward : kEtaAdjoint)) ||
                     fabsf(x) > 0.7f)
-                    visit_chi64(c, c2psi, s2psi, ra_pix, rr.cdp, rr.sdp, c2, s2);
+                    visit_phase64(c, ra_pix, rr.cdp, rr.sdp, d4, s4);
+                visit_chi(sf, d4, s4, c2, s2);
             }
             if (bp == kNeedExact && (mode == 1 || mode == 3 || mode == 4))
                 bp = beam_pixel_f64(hb, fc64, c, c2psi, s2psi, ra_pix, rr.cdp, rr.sdp, c2, s2);

@@ -39,7 +39,7 @@ struct PairParams {
     double rho_max, cos_rmax;
     FastConsts fc;            /* single-precision mapping */
     FastConsts64 fc64;        /* double-precision mapping (visits the float form declines) */
-    float eta;                /* sky adjoint with lane groups: bound of visit_chi64 */
+    float eta;                /* sky adjoint with lane groups: bound of visit_phase64 */
     const float *beam;
     /* strips of rings that a disc is cut into (1: not cut), with the constants
      * of the launch's samples and, forward, the strips' sums [strip][a, b]
