@@ -144,8 +144,8 @@ int pisco_exec_adjoint_beam(pisco_ctx *ctx, const float *g_a, const float *g_b,
  * expected pixels per disc, else 8 below 1,000 pixels, 16 below 3,000, else 64),
  * "adjmap_lanes" (single-pair sky adjoint: 64, 16 or 8; 0, the default, picks
  * 64 for beams above 8 MB with at least 4,000 pixels per disc, from 10,000
- * pixels or from 2,000 with less than 4,096 samples, 16 from 450 pixels or
- * below 16,384 samples, else 8),
+ * pixels or below 4,096 samples, 16 from 450 pixels or below 16,384 samples,
+ * else 8),
  * "batch_pair_major" (batched launches: 1 runs the pairs one after another
  * with the single-pair kernels, 0 all pairs per chunk of samples; -1, the
  * default, picks 1 when a pair's packed beam exceeds 4 MiB),

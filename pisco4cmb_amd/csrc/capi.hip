@@ -333,13 +333,15 @@ int fwd_lanes(const pisco_ctx *c, const PairParams &p)
  * pixels per disc 0.46, 0.51, 0.61; 540: 0.64, 0.60, 0.69; 960: 1.01, 1.00,
  * 1.00; 1,500: 1.31, 1.24, 1.26; 135 pixels, 1e4 samples: 0.113, 0.108, 0.121.
  * 16 and 64 lanes over 6e4 samples: 6,000 pixels 1.83, 1.95; 8,600: 3.29, 3.30.
- * 5,700 pixels, 2,000 samples: 16 lanes 0.43 ms, which leave waves idle again.
+ * Below 4,096 samples a wave each, or waves are left idle again: 1,000 samples of
+ * 94 pixels, us for 8, 16, 64 lanes 66, 59, 50; of 540 pixels 130, 97, 70; of 1,620
+ * pixels 280, 189, 101.
  * Strips are of one-wave samples. */
 int adj_lanes_auto(const PairParams &p)
 {
     const double dp = disc_pixels(p);
     const long n = p.s_end - p.s_begin;
-    if (dp >= 10000.0 || strips_auto(p, true) > 1 || (dp >= 2000.0 && n < 4096))
+    if (dp >= 10000.0 || strips_auto(p, true) > 1 || n < 4096)
         return 64;
     return dp >= 450.0 || n < 16384 ? 16 : 8;
 }

@@ -64,6 +64,12 @@ def test_short_calls_fill_the_cus():
             assert s[k] == 8 or n >= 256 * s[k] or s[2] < 64 and s[k] == 16
 
 
+@pytest.mark.parametrize("ns,nb,cap", [(64, 512, 3.0), (256, 2048, 1.5), (512, 4096, 2.5), (512, 4096, 5.0)])
+def test_short_adjoints_take_a_wave_per_sample(ns, nb, cap):
+    for n in (1, 300, 3000, 4095):
+        assert shape(ns, nb, cap, n)[2] == 64
+
+
 def test_bad_arguments():
     s = (ctypes.c_int * 8)()
     assert lib.pisco_launch_shape(0, 512, 100, 1, s) != 0
