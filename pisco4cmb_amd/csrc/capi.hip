@@ -1663,7 +1663,10 @@ int pair_lanes(const BatchParams &b, const BatchPair &q)
  * 56.2, 49.5, 45.5, 47.8, and of 300 samples 1.33, 0.92, 1.35, 0.60; 3,100 pixels of
  * 1.5 MB 7.6, 6.0, 6.2, 6.1; sky NSIDE 128, 303 pixels of 2.4 MB, 8 pairs 2.5, 2.4,
  * 1.6, 2.7.  Groups of 4 stay where items leave the XCDs with unequal discs: 4
- * pairs of 540 to 960 pixels, up to 1.9 MB, 6,000 samples 0.135, items 0.158. */
+ * pairs of 540 to 960 pixels, up to 1.9 MB, 6,000 samples 0.135, items 0.158; and in
+ * calls that fill the CUs' waves once or twice, whose end groups of two stretch: 6
+ * pairs, 34,500 pixels of 1.05 MB, ms for 4, 2: 1,500 samples 2.32, 2.08; 2,100 3.03,
+ * 3.35; 3,000 3.08, 3.67; 5,000 5.13, 5.32; 7,000 6.30, 6.36. */
 int group_auto(const BatchParams &b, const pisco_batch *bt, int k, int &lanes)
 {
     const bool few = disc_pixels(b.hs, bt->host[k].rho_max) < 1000.0;   /* the largest disc */
@@ -1672,7 +1675,7 @@ int group_auto(const BatchParams &b, const pisco_batch *bt, int k, int &lanes)
         if (bt->host[j].out >= 0)
             mb = std::max(mb, 32.0 * bt->host[j].npix / (1 << 20));
     lanes = 0;
-    if (mb <= (few ? 2.0 : 1.0))
+    if (mb <= (few ? 2.0 : 1.0) || (mb <= 1.7 && b.nsamples >= 2048 && b.nsamples < 6144))
         return 4;
     if (!few && mb <= 1.7)
         return 2;

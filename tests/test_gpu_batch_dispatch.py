@@ -1,7 +1,7 @@
 """The batched forward's automatic choice of pairs per wave: pairs whose packed
 beams are large leave the groups of four, whose gathers from four beams then miss
 the L2.  Shapes (sky NSIDE, beam NSIDE, cap; beam, disc): 64, 256, 30 deg (1.6 MiB,
-3,300 pixels: groups of two), 64, 256, 36 deg (2.3 MiB, 4,700: a pair's items), 48,
+3,300 pixels: groups of two, and of four from 2,048 to 6,143 samples), 64, 256, 36 deg (2.3 MiB, 4,700: a pair's items), 48,
 512, 18 deg (2.4 MiB, 680: a pair's items) and 64, 256, 12 deg (0.3 MiB, 540: four).
 
 The choice shows in the order of the FP64 sums: with flat beams and a sky that
@@ -30,10 +30,11 @@ def rel_rms(a, b):
     return float(np.sqrt(np.mean((a - b) ** 2)) / max(np.sqrt(np.mean(b ** 2)), 1e-300))
 
 
-@pytest.mark.parametrize("ns,nb,cap,group", [(64, 256, 30.0, 2), (64, 256, 36.0, 1),
-                                             (48, 512, 18.0, 1), (64, 256, 12.0, 4)])
-def test_default_group(ns, nb, cap, group):
-    n = 300
+@pytest.mark.parametrize("ns,nb,cap,group,n",
+                         [(64, 256, 30.0, 2, 300), (64, 256, 30.0, 2, 2047), (64, 256, 30.0, 4, 2048),
+                          (64, 256, 30.0, 4, 6143), (64, 256, 30.0, 2, 6144), (64, 256, 36.0, 1, 300),
+                          (64, 256, 36.0, 1, 3000), (48, 512, 18.0, 1, 300), (64, 256, 12.0, 4, 300)])
+def test_default_group(ns, nb, cap, group, n):
     sky = [x.copy() for x in inputs.iid_sky(ns, seed=3)[:3]]
     sky[0][::64] = 2.0 ** 60
     sky[0][1::64] = -(2.0 ** 60)
