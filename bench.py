@@ -297,7 +297,8 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32 data/products, f64 index path + accumulation",
+        "dtype": "f32 data; pixel indices in f32 where certified against f64, else f64; "
+                 "I products and accumulation f64",
         "data": "synthetic (seeded power-law sky, Gaussian beams, CES scan)",
         "config": {"workload": "fwd+adjoint-map, sky NSIDE 512, pair, FWHM 0.33 deg, cap "
                                "5 deg, beam NSIDE 4096, %d samples whole-sky CES" % n,

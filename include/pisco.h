@@ -133,12 +133,13 @@ int pisco_exec_adjoint_beam(pisco_ctx *ctx, const float *g_a, const float *g_b,
  * two blocks per CU where that is faster; "adjmap_window", read only, is the
  * capacity of the last call),
  * "adjmap_rw" (window rings), "adjmap_blocks" (blocks of the adjoint launches,
- * each looping over windows; 0, the default, one block per window), "adjmap_support" (1: windows cover only the discs of the beam's
- * non-zero rows, 0: the full rho_max discs; results are the same either way),
+ * each looping over windows; 0, the default, one block per window),
+ * "adjmap_support" (1: windows cover only the discs of the beam's non-zero rows, 0: the full rho_max discs; results are the same either way),
  * "batch_group" (batched forward: 1 = items of one pair, the single-pair
  * computation; 2 or 4 = pairs per wave sharing each visit's geometry; until it is
- * set, 4, and 2 or 1 for pairs whose packed beams exceed 1 MiB), "batch_adj_group" (batched sky adjoint: 1, 2 or 4 pairs per
- * wave, as batch_group), "forward_lanes" (single-pair forward: 64 = one
+ * set, 4, and for pairs whose packed beams exceed 1 MiB 1, 2 or 4 by the beams, the
+ * discs and the number of samples), "batch_adj_group" (batched sky adjoint: 1, 2 or
+ * 4 pairs per wave, as batch_group), "forward_lanes" (single-pair forward: 64 = one
  * sample per wave; 32, 16 or 8 lanes per sample with 64/lanes samples per
  * wave; 0, the default, picks 64 for beams above 3.2 MB with at least 1,200
  * expected pixels per disc, else 8 below 1,000 pixels, 16 below 3,000, else 64),

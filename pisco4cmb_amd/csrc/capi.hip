@@ -362,9 +362,9 @@ bool pinned(const pisco_ctx *c, hipStream_t st)
 }
 
 /* Strips for a launch of one wave per sample, whose launches then take at most
- * kStripLaunch samples; the workspace is sized for the call, in powers of two.  Where the workspace may not grow, the forward takes a
- * disc's strips one after the other (the same sums; p.samples stays NULL) and the
- * adjoint whole discs. */
+ * kStripLaunch samples; the workspace is sized for the call, in powers of
+ * two.  Where it may not grow, the forward takes a disc's strips one after the other
+ * (the same sums; p.samples stays NULL) and the adjoint whole discs. */
 int use_strips(pisco_ctx *c, PairParams &p, long &chunk, bool adjoint, hipStream_t st)
 {
     p.strips = strips_auto(p, adjoint);
@@ -1795,8 +1795,9 @@ int batch_adjoint_pairwise(pisco_ctx *c, hipStream_t st, const pisco_batch *b, i
         }
         const int lanes = adj_lanes(c, p);
         const int chunk = adj_chunk(c, p, lanes);
-        CHK(run_adjmap(c, p, chunk, pair_cap(adj_tuning(c), p, scale != nullptr, lanes, chunk), scale, lanes,
-                       st));
+        CHK(run_adjmap(c, p, chunk,
+                       pair_cap(adj_tuning(c), p, scale != nullptr, lanes, chunk), scale,
+                       lanes, st));
     }
     return PISCO_OK;
 }

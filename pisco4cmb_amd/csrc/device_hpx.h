@@ -650,7 +650,6 @@ __host__ __device__ inline int beam_pixel(const Hpx &hb, const Centre &c, double
  * polar branch) take the FP64 form, so the rho > 1e-6 rule of sphtrigo.cpp:40
  * never meets the float form. */
 struct FastConsts {
-    float nside;    /* nside_beam */
     float k3;       /* 3 nside_beam^2 */
 };
 
@@ -800,14 +799,14 @@ __device__ inline float quarter_turns(float ax, float ay)
     return t * p;
 }
 
-/* Beam pixel from tt in [0, 4] and tmp; kNeedExact unless every floor's
- * argument is farther than 1/2 - lim from an integer. */
 /* A certified pixel of the polar cap: its ring, quadrant, and place in the
  * quadrant (whole numbers). */
 struct CapPlace {
     float ring, quad, pos;
 };
 
+/* Beam pixel from tt in [0, 4] and tmp; kNeedExact unless every floor's
+ * argument is farther than 1/2 - lim from an integer. */
 __device__ inline int cap_floors(float tt, float tmp, float omc, float lim, CapPlace &place)
 {
     const float tp = __builtin_amdgcn_fractf(tt);

@@ -283,7 +283,7 @@ __device__ inline Pass build_pass(const Hpx &hs, const RingRec *rings, const Dis
     ps.nrun = carry & 255;
     ps.total = carry >> 8;
     unsigned long long wm = __ballot(wide);
-    if constexpr (SUB < kWaveSize)   /* a sample's results do not depend on its neighbours */
+    if constexpr (SUB < kWaveSize)   /* the group's own runs decide its form */
         wm = (wm >> (lane & ~(SUB - 1))) & ((1ull << SUB) - 1ull);
     ps.wide = wm != 0ull;
     if (sl == 0)
@@ -747,8 +747,10 @@ struct WaveView {
 };
 
 /* Samples i0 .. i0+ns-1 (ns <= NS), strip k of their discs: their sums to
- * put(sample, a, b).  Every thread of the block calls it.  A sample's sums do
- * not depend on the samples it shares the block with. */
+ * put(sample, a, b).  Every thread of the block calls it.  With one wave
+ * per sample a sample's sums do not depend on the samples it shares the block
+ * with.  Lane groups share a wave's queue of deferred visits, so there the order
+ * in which those few are added in FP64 does. */
 template <int SUB, bool VT, typename Put>
 __device__ inline void forward_block(const PairParams &p, FwdBlock<SUB> &B, long i0, int ns, int k,
                                      float pa_off, bool offset, Put &put)
@@ -1134,7 +1136,6 @@ __device__ inline PairParams batch_pair_params(const BatchParams &b, const Batch
     p.npix_beam = q.npix;
     p.rho_max = q.rho_max;
     p.cos_rmax = q.cos_rmax;
-    p.fc.nside = q.nside_f;
     p.fc.k3 = 3.0f * q.nside_f * q.nside_f;
     p.fc64.crho_big = b.fc64.crho_big;
     p.fc64.crho_small = b.fc64.crho_small;
@@ -1326,7 +1327,7 @@ struct BatchPend {
 };
 
 /* The walk over the visits of the group's union disc (the disc of its first
- * pair; d clipped by the caller), pipelined as walk_pass: per visit the shared
+ * pair; d clipped by the caller), pipelined as walk_segment: per visit the shared
  * float geometry, then each pair's tail (membership, beam pixel, gather);
  * consume(q) receives a visit once its loads are due (after the next visit's
  * geometry).  Queued visits (uncertain membership or beam pixel) are drained
@@ -1368,7 +1369,7 @@ __device__ inline void batch_walk(const BatchParams &p, BT &bt, const Disc &d, i
         const bool marked = total <= VCAP;
         int base = 0, s = 0;
         float4 n0, n1;
-        auto fetch = [&](int v0) {   /* as walk_pass */
+        auto fetch = [&](int v0) {   /* as walk_segment */
             if (marked) {
                 const unsigned lo = t.bits[v0 >> 5], hi = t.bits[(v0 >> 5) + 1];
                 s = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, base));
@@ -1569,10 +1570,12 @@ void k_batch_fwd(BatchParams p)
  * window that covers every disc of the chunk (pass 1: ring spans unwrapped
  * around the chunk's first centre, atomic min/max in LDS), lays the windows
  * out contiguously in LDS (prefix sum), accumulates every visit's I,Q,U
- * gradient into LDS with ds_add_f32 (pass 2: wave per sample, as the
- * forward), and finally adds the non-zero window entries to the FP64 global
- * gradient (one global atomic per pixel and chunk instead of one per visit).
- * A chunk whose windows do not fit falls back to direct global atomics. */
+ * gradient into LDS (pass 2: a wave or a lane group per sample, as the forward;
+ * ds_add_f32, or ds_add_u64 of 64-bit integers in the deterministic mode), and
+ * finally adds the non-zero window entries to the global gradient (one global
+ * atomic per pixel and chunk instead of one per visit).  Windows larger than the
+ * LDS are taken in slabs of whole rings, one walk each; a chunk with too many
+ * rings, or whose samples lie far apart, adds to the global gradient directly. */
 
 struct AdjLayout {
     int chunk;       /* samples per chunk */
@@ -2698,7 +2701,7 @@ __device__ inline int rec_pixel(const RecParams &R, int b, int row, int npix)
 
 /* Steps 1 and 3: one wave per sample of the chunk [p.s_begin, p.s_end),
  * the sky adjoint's walk and certified single-precision mapping (every
- * visit's beam pixel is the exact one; cos/sin 2chi within 9.2e-7), with the
+ * visit's beam pixel is the exact one; cos/sin 2chi within 1e-6), with the
  * deferred visits mapped by the FP64-alpha form.  The count pass loads no
  * beam rows; the write pass loads each visit's sky values, pipelined. */
 template <bool WRITE>
@@ -3823,8 +3826,7 @@ hipError_t launch_match(const Hpx &hs, const RingRec *rings, const Hpx &hb, int 
 FastConsts fast_consts(const Hpx &hb)
 {
     FastConsts f;
-    f.nside = (float)hb.nside;
-    f.k3 = 3.0f * f.nside * f.nside;
+    f.k3 = 3.0f * (float)hb.nside * (float)hb.nside;
     return f;
 }
 
