@@ -636,12 +636,19 @@ __device__ inline void walk_segment(const PairParams &p, const T &t, WS &ws, int
     at.base = base0;
 }
 
-__device__ inline int wave_max_uniform(int x)
+/* The largest x over the wave's lane groups, each of which holds one value.  By
+ * lane reads: the lane addresses of shuffles, formed before the walk, were spilled,
+ * and each of their six steps waited for scratch memory (forward, 2e4 samples of 5
+ * pixels 17.0 and 15.6 us, 2e5 of 136 pixels 179 and 171; sky adjoint, 2e5 of 34
+ * pixels 261 and 242). */
+template <int SUB>
+__device__ inline int group_max_uniform(int x)
 {
+    int m = __builtin_amdgcn_readlane(x, 0);
 #pragma unroll
-    for (int m = kWaveSize / 2; m > 0; m >>= 1)
-        x = max(x, __shfl_xor(x, m, kWaveSize));
-    return __builtin_amdgcn_readfirstlane(x);
+    for (int g = SUB; g < kWaveSize; g += SUB)
+        m = max(m, __builtin_amdgcn_readlane(x, g));
+    return m;
 }
 
 /* Rings r0 .. r_last of the disc of sample j of the lane group's wave state
@@ -665,7 +672,7 @@ __device__ inline void walk_rings(const PairParams &p, T &t, WS &ws, int j, int 
             total = __builtin_amdgcn_readfirstlane(total);
             wtot = total;
         } else {
-            wtot = wave_max_uniform(total);
+            wtot = group_max_uniform<SUB>(total);
         }
         const bool any_wide = __any(ps.wide);
         WalkAt at;
@@ -2475,10 +2482,10 @@ __global__ __launch_bounds__(kBandBlock) void k_adjbeam_band_sub(PairParams p, B
                 atomicAdd(&a[4], -(gb * X));
                 atomicAdd(&a[5], -(gb * Y));
             };
-            const int npass = (wave_max_uniform(nrings) + SUB - 1) / SUB;
+            const int npass = (group_max_uniform<SUB>(nrings) + SUB - 1) / SUB;
             for (int ps = 0; ps < npass; ps++) {
                 const int total = build_band_sub<SUB>(p.hs, dout, din, inner, nrings, ps, sl, t);
-                walk_band_sub<SUB>(p, t, total, wave_max_uniform(total), sl, c, c2psi, s2psi, lo,
+                walk_band_sub<SUB>(p, t, total, group_max_uniform<SUB>(total), sl, c, c2psi, s2psi, lo,
                                    nrow, use);
                 wave_sync();
             }
